@@ -1198,38 +1198,6 @@ __global__ void neighbours_one_kernel(nlh_celllist_dev<TI> c, int64_t i, int64_t
     *count = n;
 }
 
-// neighbours of a range of atoms: one thread per atom, a counting pass and
-// a filling pass at host-scanned offsets, both through the device-side
-// header's traversal (the reference's order, R and S bit for bit)
-template <typename TI>
-__global__ __launch_bounds__(256) void neighbours_count_kernel(nlh_celllist_dev<TI> c, int64_t i_first, int64_t n,
-                                                               int64_t *__restrict__ count)
-{
-    const int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= n) return;
-    int64_t k = 0;
-    nlh_for_each_neighbour(c, i_first + a, [&](TI, const double *, const TI *) { ++k; });
-    count[a] = k;
-}
-
-template <typename TI>
-__global__ __launch_bounds__(256) void neighbours_fill_kernel(nlh_celllist_dev<TI> c, int64_t i_first, int64_t n,
-                                                              const int64_t *__restrict__ off, TI *__restrict__ j,
-                                                              double *__restrict__ R, TI *__restrict__ S)
-{
-    const int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= n) return;
-    int64_t q = off[a];
-    nlh_for_each_neighbour(c, i_first + a, [&](TI jj, const double *RR, const TI *SS) {
-        j[q] = jj;
-        for (int k = 0; k < 3; ++k) {
-            R[3 * q + k] = RR[k];
-            S[3 * q + k] = SS[k];
-        }
-        ++q;
-    });
-}
-
 namespace {
 
 // Cell-list view of system `sys` of the last build (positions, perm and
@@ -1248,30 +1216,46 @@ nlh_celllist_view system_view(const nlh_handle *h, int32_t sys)
     return v;
 }
 
-template <typename TI>
-void neighbours_range_launch(nlh_handle *h, int32_t sys, int64_t i_first, int64_t n)
+// Count, offsets and neighbours of a range of atoms, with one wait.  The
+// neighbours are written in the same go when the outputs of an earlier query
+// hold them all; otherwise the outputs grow and the last pass runs (again).
+void neighbours_range(nlh_handle *h, int32_t sys, int64_t i_first, int64_t n)
 {
-    const auto c = nlh_make_celllist_dev<TI>(system_view(h, sys), h->geoms[sys]);
-    const unsigned blocks = (unsigned)((n + 255) / 256);
-    h->nr_count.ensure(h->stream, (size_t)n * 8);
-    hipLaunchKernelGGL(neighbours_count_kernel<TI>, dim3(blocks), dim3(256), 0, h->stream, c, i_first, n,
-                       h->nr_count.as<int64_t>());
-    HIPC(hipGetLastError());
-    // exclusive scan of the counts on the host (one pass over n values)
-    h->nr_off_host.assign((size_t)n + 1, 0);
-    HIPC(hipMemcpyAsync(h->nr_off_host.data() + 1, h->nr_count.p, (size_t)n * 8, hipMemcpyDeviceToHost, h->stream));
-    HIPC(hipStreamSynchronize(h->stream));
-    for (int64_t a = 0; a < n; ++a) h->nr_off_host[a + 1] += h->nr_off_host[a];
-    const int64_t total = h->nr_off_host[n];
-    const size_t t1 = (size_t)std::max<int64_t>(total, 1), ti = sizeof(TI);
+    const size_t ti = (size_t)h->ti_bytes;
+    h->nr_count.ensure(h->stream, (size_t)n * 4);
     h->nr_off.ensure(h->stream, ((size_t)n + 1) * 8);
-    h->nr_j.ensure(h->stream, t1 * ti);
-    h->nr_R.ensure(h->stream, t1 * 24);
-    h->nr_S.ensure(h->stream, t1 * 3 * ti);
-    HIPC(hipMemcpyAsync(h->nr_off.p, h->nr_off_host.data(), ((size_t)n + 1) * 8, hipMemcpyHostToDevice, h->stream));
-    if (total > 0)
-        hipLaunchKernelGGL(neighbours_fill_kernel<TI>, dim3(blocks), dim3(256), 0, h->stream, c, i_first, n,
-                           h->nr_off.as<int64_t>(), h->nr_j.as<TI>(), h->nr_R.as<double>(), h->nr_S.as<TI>());
+    nlh::LazyRange q{};
+    q.sys = h->sys_d + sys;
+    q.isys = sys;
+    q.i_first = i_first - 1;
+    q.n = n;
+    q.X = h->X_dev;
+    q.rec = h->rec.as<nlh::Rec>();
+    q.wbig = h->wbig.as<int32_t>();
+    q.cell_offsets = h->cell_offsets.p;
+    q.count = h->nr_count.as<int32_t>();
+    q.off = h->nr_off.as<int64_t>();
+    const auto outputs = [&] {
+        q.j = h->nr_j.p;
+        q.R = h->nr_R.as<double>();
+        q.S = h->nr_S.p;
+        q.cap = (int64_t)std::min({h->nr_j.cap / ti, h->nr_R.cap / 24, h->nr_S.cap / (3 * ti)});
+    };
+    outputs();
+    nlh::launch_lazy_range(q, h->ti_bytes, false, h->stream);
+    nlh::launch_range_scan(q, h->stream);
+    if (q.cap > 0) nlh::launch_lazy_range(q, h->ti_bytes, true, h->stream);
+    HIPC(hipGetLastError());
+    h->nr_off_host.resize((size_t)n + 1);
+    HIPC(hipMemcpyAsync(h->nr_off_host.data(), h->nr_off.p, ((size_t)n + 1) * 8, hipMemcpyDeviceToHost, h->stream));
+    HIPC(hipStreamSynchronize(h->stream));
+    const int64_t total = h->nr_off_host[n];
+    if (total <= q.cap) return;
+    h->nr_j.ensure(h->stream, (size_t)total * ti);
+    h->nr_R.ensure(h->stream, (size_t)total * 24);
+    h->nr_S.ensure(h->stream, (size_t)total * 3 * ti);
+    outputs();
+    nlh::launch_lazy_range(q, h->ti_bytes, true, h->stream);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(h->stream));
 }
@@ -1880,8 +1864,7 @@ int nlh_neighbours_range(nlh_handle *h, int32_t sys, int64_t i_first, int64_t n,
         if (!cached) {
             h->nr_valid = false;
             if (n > 0) {
-                if (h->ti_bytes == 8) neighbours_range_launch<int64_t>(h, sys, i_first, n);
-                else neighbours_range_launch<int32_t>(h, sys, i_first, n);
+                neighbours_range(h, sys, i_first, n);
             } else {
                 h->nr_off_host.assign(1, 0);
             }

@@ -359,6 +359,34 @@ __global__ __launch_bounds__(kScanThreads) void scan_pairs_kernel(
     }
 }
 
+// Offsets of a lazy query: exclusive scan of n counts by one block, 8 per
+// thread and turn (a query is a few thousand atoms, and its offsets go to
+// the host next: a scan over several blocks would save nothing).
+__global__ __launch_bounds__(1024) void range_scan_kernel(const int32_t *__restrict__ count, int64_t n,
+                                                          int64_t *__restrict__ off)
+{
+    int64_t carry = 0;
+    for (int64_t base = 0; base < n; base += 1024 * kScanItems) {
+        const int64_t b = base + (int64_t)threadIdx.x * kScanItems;
+        int32_t v[kScanItems];
+        int64_t s = 0;
+#pragma unroll
+        for (int q = 0; q < kScanItems; ++q) {
+            v[q] = b + q < n ? count[b + q] : 0;
+            s += v[q];
+        }
+        int64_t tot;
+        int64_t run = carry + block_excl_scan_n<1024>(s, tot);
+#pragma unroll
+        for (int q = 0; q < kScanItems; ++q) {
+            if (b + q < n) off[b + q] = run;
+            run += v[q];
+        }
+        carry += tot;
+    }
+    if (threadIdx.x == 0) off[n] = carry;
+}
+
 // Per-system `first` arrays for a batch (local, 1-based) and the per-system
 // pair bases.  System s owns entries [atom_base[s] + s, atom_base[s+1] + s] of
 // the concatenated first arrays: thread g writes the entry of atom g (its
@@ -873,6 +901,11 @@ void launch_scan_pairs(const PipelineBufs &b, hipStream_t st)
                                            dim3(blocks_for(std::max<int64_t>(n, (int64_t)b.nsys + 1), 256)),
                                            dim3(256), 0, st, b.pair_off, n, b.sys_atom_base, b.atom_sys, b.nsys,
                                            b.first_out, b.sys_pair_base));
+}
+
+void launch_range_scan(const LazyRange &q, hipStream_t st)
+{
+    hipLaunchKernelGGL(range_scan_kernel, dim3(1), dim3(1024), 0, st, q.count, q.n, q.off);
 }
 
 void launch_sorted_positions(const PipelineBufs &b, double *Xs, hipStream_t st)

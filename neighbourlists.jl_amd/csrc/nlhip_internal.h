@@ -294,6 +294,28 @@ void launch_scan_pairs(const PipelineBufs &b, hipStream_t st);
 bool launch_fill(const PipelineBufs &b, bool want_R, bool wide, hipStream_t st);
 void launch_sorted_positions(const PipelineBufs &b, double *Xs, hipStream_t st);
 
+// A lazy query: the neighbours of atoms i_first .. i_first + n - 1 (0-based)
+// of system isys of the last build.
+struct LazyRange {
+    const SysDev *sys;          // the system
+    int32_t isys;
+    int64_t i_first, n;
+    const double *X;            // positions of the whole build
+    const Rec *rec;
+    const int32_t *wbig;
+    const void *cell_offsets;   // of the whole build, TI, 1-based per system
+    int32_t *count;             // n
+    int64_t *off;               // n + 1: first neighbour of each atom, then the total
+    int64_t cap;                // entries the outputs hold
+    void *j;
+    double *R;
+    void *S;
+};
+// One pass over the range: counts, or (fill) the neighbours at off.
+void launch_lazy_range(const LazyRange &q, int ti_bytes, bool fill, hipStream_t st);
+// off = exclusive scan of count, then the total.
+void launch_range_scan(const LazyRange &q, hipStream_t st);
+
 // Fused build of small systems (b.nunits > 0): the cell list of every
 // system, its pair counts and its slot rows, by one workgroup per work item
 // (a unit of consecutive systems or one part of one); launched by

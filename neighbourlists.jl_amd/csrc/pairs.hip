@@ -176,18 +176,16 @@ struct HomeCell {
     const SysDev *sd;
 };
 
-__device__ __forceinline__ void home_cell(const PairsArgs &A, const SysDev &sd, int cell, HomeCell &H)
+// The grid around the cell at 1-based coordinates (ci0, ci1, ci2).
+__device__ __forceinline__ void home_grid(const SysDev &sd, int ci0, int ci1, int ci2, HomeCell &H)
 {
-    H.hs = A.cell_start[cell];
-    H.he = A.cell_start[cell + 1];
     H.sd = &sd;
     H.n0 = sd.n[0]; H.n1 = sd.n[1]; H.n2 = sd.n[2];
     H.cbase = sd.cell_base;
     H.abase = sd.atom_base;
-    const int lc = cell - H.cbase;
-    H.ci0 = lc % H.n0 + 1;
-    H.ci1 = (lc / H.n0) % H.n1 + 1;
-    H.ci2 = lc / (H.n0 * H.n1) + 1;
+    H.ci0 = ci0;
+    H.ci1 = ci1;
+    H.ci2 = ci2;
     H.nx0 = sd.nxyz[0]; H.nx1 = sd.nxyz[1]; H.nx2 = sd.nxyz[2];
     H.sx = 2 * H.nx0 + 1;
     H.sy = 2 * H.nx1 + 1;
@@ -195,11 +193,21 @@ __device__ __forceinline__ void home_cell(const PairsArgs &A, const SysDev &sd, 
     H.p0 = sd.pbc & 1; H.p1 = (sd.pbc >> 1) & 1; H.p2 = (sd.pbc >> 2) & 1;
 }
 
+__device__ __forceinline__ void home_cell(const PairsArgs &A, const SysDev &sd, int cell, HomeCell &H)
+{
+    H.hs = A.cell_start[cell];
+    H.he = A.cell_start[cell + 1];
+    const int lc = cell - sd.cell_base;
+    home_grid(sd, lc % sd.n[0] + 1, (lc / sd.n[0]) % sd.n[1] + 1, lc / (sd.n[0] * sd.n[1]) + 1, H);
+}
+
 // Neighbour cells sb .. sb+63 of the home cell, one per lane, in the
-// reference order.  Returns the number of candidate atoms in the batch
+// reference order.  cell_atoms(c, start, count) gives the sorted atoms of
+// the system's cell c.  Returns the number of candidate atoms in the batch
 // (wave-uniform); per lane: exclusive prefix, first sorted index, shift.
-__device__ __forceinline__ int segment_batch(const PairsArgs &A, const HomeCell &H, int sb, int &excl, int &start_g,
-                                             uint32_t &shp)
+template <typename F>
+__device__ __forceinline__ int segment_batch(const HomeCell &H, int sb, int &excl, int &start_g, uint32_t &shp,
+                                             F &&cell_atoms)
 {
     const int g = sb + lane_id();
     int cnt_g = 0;
@@ -219,9 +227,7 @@ __device__ __forceinline__ int segment_batch(const PairsArgs &A, const HomeCell 
             wrap_and_shift(a0, H.n0, H.p0, c0, s0);
             wrap_and_shift(a1, H.n1, H.p1, c1, s1);
             wrap_and_shift(a2, H.n2, H.p2, c2, s2);
-            const int gc = H.cbase + (c0 - 1) + (c1 - 1) * H.n0 + (c2 - 1) * H.n0 * H.n1;
-            start_g = A.cell_start[gc];
-            cnt_g = A.cell_start[gc + 1] - start_g;
+            cell_atoms((c0 - 1) + (c1 - 1) * H.n0 + (c2 - 1) * H.n0 * H.n1, start_g, cnt_g);
             shp = pack_wind(s0, s1, s2);
         }
     }
@@ -288,7 +294,10 @@ __device__ __forceinline__ void count_cell(const PairsArgs &A, const SysDev &sd,
         for (int sb = 0; sb < H.nseg; sb += kWave) {
             int excl, start_g;
             uint32_t shp;
-            const int total = segment_batch(A, H, sb, excl, start_g, shp);
+            const int total = segment_batch(H, sb, excl, start_g, shp, [&](int c, int &st, int &n) {
+                st = A.cell_start[H.cbase + c];
+                n = A.cell_start[H.cbase + c + 1] - st;
+            });
             for (int k0 = 0; k0 < total; k0 += kChunksPerPass * kWave) {
                 const int nch = sgpr(min(kChunksPerPass, (total - k0 + kWave - 1) / kWave));
                 Cand c[kChunksPerPass];
@@ -341,6 +350,91 @@ __device__ __forceinline__ void count_cell(const PairsArgs &A, const SysDev &sd,
             }
         }
         if (lane < nh) pair_count[H.abase + hj_lane] = cnt_lane | kRow8Bit;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// lazy queries: the neighbours of a range of atoms
+// ---------------------------------------------------------------------------
+
+// for_each_neighbour (cell_list.jl:779-801) of atoms i_first .. i_first + n - 1
+// of one system, one wave per atom: its neighbour cells one per lane, their
+// atoms flattened in the reference order, 64 candidates tested at a time, so
+// a hit's place is the hits before it.  Without FILL the neighbours are
+// counted, with it they are written from off[a] on (nothing when the total
+// off[n] exceeds cap: the host grows the outputs and runs it again).
+//
+// Latency-bound: a query of a few thousand atoms is one wave per SIMD.  With
+// one thread per atom walking the cells through perm and the positions the
+// two passes over 4,096 atoms of a 50,000-atom cube took 248 us each; a
+// wave per atom reading the sorted records takes 9 and 10 us.
+template <typename TI, bool FILL>
+__global__ __launch_bounds__(kPairsBlock) void lazy_range_kernel(LazyRange Q)
+{
+    const int64_t a = (int64_t)blockIdx.x * kWavesPerPairsBlock + sgpr((int)(threadIdx.x / kWave));
+    if (a >= Q.n) return;   // wave-uniform
+    int64_t run = 0;
+    if (FILL) {
+        if (Q.off[Q.n] > Q.cap) return;
+        run = Q.off[a];
+    }
+    const SysDev &sd = *Q.sys;
+    const int64_t il = Q.i_first + a;   // 0-based, local to the system
+    const double *xi = Q.X + 3 * (sd.atom_base + il);
+    const double hx = xi[0], hy = xi[1], hz = xi[2];
+    int32_t ci[3], wi[3];
+    cell_and_winding(sd, hx, hy, hz, ci, wi);
+    HomeCell H;
+    home_grid(sd, ci[0], ci[1], ci[2], H);
+    const TI *co = static_cast<const TI *>(Q.cell_offsets) + (int64_t)sd.cell_base + Q.isys;
+    const PairsArgs A{Q.sys, nullptr, 1, sd.M, sd.nat, nullptr, Q.rec, Q.wbig};
+    const int lane = lane_id();
+    const double rc2 = sd.rc2;
+    for (int sb = 0; sb < H.nseg; sb += kWave) {
+        int excl, start_g;
+        uint32_t shp;
+        const int total = segment_batch(H, sb, excl, start_g, shp, [&](int c, int &st, int &n) {
+            const int64_t s0 = (int64_t)co[c];
+            st = (int)(sd.atom_base + s0 - 1);
+            n = (int)((int64_t)co[c + 1] - s0);
+        });
+        for (int k0 = 0; k0 < total; k0 += kWave) {
+            const Cand c = load_candidate(A, k0 + lane, total, excl, start_g, shp);
+            const int32_t Sx = c.tx + wi[0], Sy = c.ty + wi[1], Sz = c.tz + wi[2];
+            double cx, cy, cz;
+            cell_shift(sd.C, Sx, Sy, Sz, cx, cy, cz);
+            const double Rx = (c.x - hx) + cx, Ry = (c.y - hy) + cy, Rz = (c.z - hz) + cz;
+            const double r2 = (Rx * Rx + Ry * Ry) + Rz * Rz;
+            const bool hit = c.valid & (r2 < rc2) & !(c.zero_shift & (c.j == (int32_t)il));
+            const uint64_t m = __ballot(hit);
+            if (FILL && hit) {
+                const int64_t q = run + mbcnt64(m);
+                static_cast<TI *>(Q.j)[q] = (TI)(c.j + 1);
+                double *R = Q.R + 3 * q;
+                R[0] = Rx;
+                R[1] = Ry;
+                R[2] = Rz;
+                TI *S = static_cast<TI *>(Q.S) + 3 * q;
+                S[0] = (TI)Sx;
+                S[1] = (TI)Sy;
+                S[2] = (TI)Sz;
+            }
+            run += __popcll(m);
+        }
+    }
+    if (!FILL && lane == 0) Q.count[a] = (int32_t)run;
+}
+
+void launch_lazy_range(const LazyRange &q, int ti_bytes, bool fill, hipStream_t st)
+{
+    if (q.n <= 0) return;
+    const dim3 grid((unsigned)((q.n + kWavesPerPairsBlock - 1) / kWavesPerPairsBlock)), block(kPairsBlock);
+    if (ti_bytes == 8) {
+        if (fill) hipLaunchKernelGGL((lazy_range_kernel<int64_t, true>), grid, block, 0, st, q);
+        else hipLaunchKernelGGL((lazy_range_kernel<int64_t, false>), grid, block, 0, st, q);
+    } else {
+        if (fill) hipLaunchKernelGGL((lazy_range_kernel<int32_t, true>), grid, block, 0, st, q);
+        else hipLaunchKernelGGL((lazy_range_kernel<int32_t, false>), grid, block, 0, st, q);
     }
 }
 
