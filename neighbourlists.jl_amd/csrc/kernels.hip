@@ -64,17 +64,25 @@ __global__ __launch_bounds__(256) void bin_kernel(const double *__restrict__ X, 
 // ---------------------------------------------------------------------------
 //
 // Up to kLookbackTiles tiles of kScanTile items a scan is one kernel with a
-// decoupled look-back (one look-back step reaches tile 0); beyond that it is
-// reduce -> scan of the tile sums -> downsweep, three kernels, where a long
-// chain of look-back steps measured slower (1M pair counts: 51 us single pass
-// against 42 us).  The downsweep kernels serve both.
+// decoupled look-back; beyond that it is reduce -> scan of the tile sums ->
+// downsweep, three kernels.  The downsweep kernels serve both.  Pair counts,
+// single pass against the three kernels with their two launch gaps of about
+// 3 us (MI355X): 200k atoms 7.3 / 21 us, 1M 17 / 27, 4M 46 / 49, 8M 79 / 66.
 //
 // Look-back: desc[0] is a ticket, desc[1 + t] the descriptor of tile t: a state in the
 // top two bits (0 not yet published, 1 the tile's aggregate, 2 its inclusive
-// prefix) and the value below.  A block takes its tile from the ticket, so
-// every tile it waits for belongs to a block that started before it and is
-// running or done.  The descriptors are zero before a launch (cleared with
-// the status at the start of a build, or by clear_lookback before a repeated
+// prefix) and the value below.  A descriptor carries all that its reader
+// needs, so it is read and written with relaxed device-scope atomics: with
+// acquire and release each access also wrote back and invalidated the L2
+// (bucket counts of 1M atoms, 118 tiles: 8.5 -> 4.4 us).
+//
+// A block takes its tile from the ticket, so every tile it waits for belongs
+// to a block that started before it and is running or done.  The tickets of
+// a launch are atomics on one address, about 8 ns each (1M atoms: 17 us with
+// them, 13 without), so a launch of up to kOrderlessTiles blocks goes without:
+// that many blocks are on the device together, and whichever starts last
+// starts.  The descriptors are zero before a launch (cleared with the
+// status at the start of a build, or by clear_lookback before a repeated
 // pair scan).
 
 constexpr uint64_t kDescAgg = 1ull << 62, kDescInc = 2ull << 62, kDescVal = kDescAgg - 1;
@@ -97,7 +105,7 @@ __device__ __forceinline__ void load_tile(const int32_t *__restrict__ in, int64_
     }
 }
 
-// This block's tile, in launch order of the blocks; -1 (and scan_error)
+// A block's tile, in launch order of the blocks; -1 (and scan_error)
 // when the ticket was not zero at the launch, so no descriptor past the grid
 // is ever touched.
 __device__ __forceinline__ int64_t scan_ticket(uint64_t *__restrict__ desc, Status *__restrict__ status)
@@ -147,23 +155,23 @@ __global__ __launch_bounds__(kScanThreads) void scan_partials_kernel(int64_t *__
     }
 }
 
-// The tile of this block and the sum of the tiles before it: from the tile
-// sums when given (three-kernel scan), else by ticket and look-back.
-// Returns -1 for a block with no tile (see scan_ticket).
+// The tile of this block: its index when no block waits for another (tile
+// sums given: three-kernel scan) or all of them are on the device together,
+// else by ticket.  Returns -1 for a block with no tile (see scan_ticket).
 __device__ __forceinline__ int64_t scan_tile_begin(uint64_t *__restrict__ desc, const int64_t *__restrict__ partials,
                                                    Status *__restrict__ status)
 {
-    return partials ? (int64_t)blockIdx.x : scan_ticket(desc, status);
+    return partials || gridDim.x <= kOrderlessTiles ? (int64_t)blockIdx.x : scan_ticket(desc, status);
 }
 
 __device__ __forceinline__ uint64_t desc_load(const uint64_t *p)
 {
-    return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __device__ __forceinline__ void desc_store(uint64_t *p, uint64_t v)
 {
-    __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __device__ __forceinline__ int64_t wave_sum64(int64_t v)
@@ -173,58 +181,65 @@ __device__ __forceinline__ int64_t wave_sum64(int64_t v)
     return v;
 }
 
-// Exclusive prefix of tile `tile` whose own sum is `agg`.  The block's first
-// wave publishes the aggregate, then reads the descriptors of the 64
-// preceding tiles at once (lane l: tile - 1 - l), waits until those up to the
-// nearest inclusive prefix are published, and adds their values, moving 64
-// tiles further back if none is an inclusive prefix; then it publishes its
-// own inclusive prefix.
+// Exclusive prefix of tile `tile` whose own sum is `agg`.  The block
+// publishes the aggregate, then reads the descriptors of the kScanThreads
+// preceding tiles at once (thread t: tile - 1 - t).  Each wave waits until
+// its 64, up to its nearest inclusive prefix, are published and adds them;
+// the waves' sums count up to the first wave that met an inclusive prefix,
+// and the block moves kScanThreads tiles further back if none did.  Then it
+// publishes its own inclusive prefix.  (One wave looking back 64 tiles at a
+// time took eight dependent steps for the last of 489 tiles.)
 // Waits are bounded: a wave that waits too long sets status->scan_error (the
 // host reports it) rather than spin for ever.
 __device__ __forceinline__ int64_t scan_lookback(uint64_t *__restrict__ desc, int64_t tile, int64_t agg,
                                                  Status *__restrict__ status)
 {
-    __shared__ int64_t prefix;
+    constexpr int kW = kScanThreads / kWave;
+    __shared__ int64_t wsum[kW];
+    __shared__ int32_t winc[kW];
     uint64_t *d = desc + 1;
-    if (threadIdx.x < kWave) {
-        const int lane = (int)threadIdx.x;
-        if (tile > 0 && lane == 0) desc_store(d + tile, kDescAgg | (uint64_t)agg);
-        int64_t ex = 0;
-        int spins = 0;
-        for (int64_t top = tile - 1; top >= 0; top -= kWave) {
-            const int64_t idx = top - lane;
-            // before tile 0: an inclusive prefix of zero
-            uint64_t v = idx >= 0 ? desc_load(d + idx) : kDescInc;
-            for (;;) {
-                const bool pending = (v >> 62) == 0;
-                // only the lanes before the nearest inclusive prefix matter
-                const uint64_t inc = __builtin_amdgcn_ballot_w64((v >> 62) == 2);
-                const uint64_t need = inc ? (inc & (~inc + 1)) - 1 : ~0ull;
-                if ((__builtin_amdgcn_ballot_w64(pending) & need) == 0) break;
-                if (++spins > kLookbackSpins) {
-                    if (lane == 0) status->scan_error = 1;
-                    if (pending) v = kDescInc;   // give up on it: an inclusive zero
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
-                if (pending) v = desc_load(d + idx);
-            }
-            const uint64_t inc = __builtin_amdgcn_ballot_w64((v >> 62) == 2);
-            const int64_t val = (int64_t)(v & kDescVal);
-            if (inc != 0) {
-                const int k = __builtin_ctzll(inc);   // the nearest inclusive prefix
-                ex += wave_sum64(lane <= k ? val : 0);
+    const int lane = lane_id(), wv = (int)threadIdx.x / kWave;
+    if (tile > 0 && threadIdx.x == 0) desc_store(d + tile, kDescAgg | (uint64_t)agg);
+    int64_t ex = 0;
+    int spins = 0;
+    for (int64_t top = tile - 1; top >= 0; top -= kScanThreads) {   // uniform over the block
+        const int64_t idx = top - (int64_t)threadIdx.x;
+        // before tile 0: an inclusive prefix of zero
+        uint64_t v = idx >= 0 ? desc_load(d + idx) : kDescInc;
+        uint64_t inc;
+        for (;;) {
+            const bool pending = (v >> 62) == 0;
+            // only the lanes before the nearest inclusive prefix matter
+            inc = __builtin_amdgcn_ballot_w64((v >> 62) == 2);
+            const uint64_t need = inc ? (inc & (~inc + 1)) - 1 : ~0ull;
+            if ((__builtin_amdgcn_ballot_w64(pending) & need) == 0) break;
+            if (++spins > kLookbackSpins) {
+                if (lane == 0) status->scan_error = 1;
+                if (pending) v = kDescInc;   // give up on it: an inclusive zero
+                inc = __builtin_amdgcn_ballot_w64((v >> 62) == 2);
                 break;
             }
-            ex += wave_sum64(val);
+            __builtin_amdgcn_s_sleep(1);
+            if (pending) v = desc_load(d + idx);
         }
+        const int k = inc ? __builtin_ctzll(inc) : kWave;   // the nearest inclusive prefix
+        const int64_t s = wave_sum64(lane <= k ? (int64_t)(v & kDescVal) : 0);
         if (lane == 0) {
-            desc_store(d + tile, kDescInc | (uint64_t)(ex + agg));
-            prefix = ex;
+            wsum[wv] = s;
+            winc[wv] = inc != 0;
         }
+        __syncthreads();
+        bool done = false;
+#pragma unroll
+        for (int w = 0; w < kW; ++w) {
+            ex += done ? 0 : wsum[w];
+            done = done || winc[w];
+        }
+        __syncthreads();   // read before the next turn writes
+        if (done) break;
     }
-    __syncthreads();
-    return prefix;
+    if (threadIdx.x == 0) desc_store(d + tile, kDescInc | (uint64_t)(ex + agg));
+    return ex;
 }
 
 // A tile's exclusive prefixes and counts pass through LDS: written blocked
@@ -533,15 +548,14 @@ __global__ __launch_bounds__(kBinThreads) void bucket_count_kernel(
     for (int b = threadIdx.x; b < P.nb; b += kBinThreads) bmat[(int64_t)b * P.na + lb] = hist[b];
 }
 
-// Exclusive scan of n counts in place (the bucket counts); tile prefixes
-// by look-back, or from the tile sums of the three-kernel form.
+// Exclusive scan of n counts in place (the bucket counts, at most
+// kSortLookbackTiles tiles: sort_plan); tile prefixes by look-back.
 __global__ __launch_bounds__(kScanThreads) void scan_inplace_kernel(int32_t *__restrict__ a, int64_t n,
                                                                     uint64_t *__restrict__ desc,
-                                                                    const int64_t *__restrict__ partials,
                                                                     Status *__restrict__ status)
 {
-    const int64_t tile = scan_tile_begin(desc, partials, status);
-    if (tile < 0) return;
+    static_assert(kSortLookbackTiles <= kOrderlessTiles, "the tiles are on the device together");
+    const int64_t tile = blockIdx.x;
     int32_t v[kScanItems];
     const int64_t base = tile * kScanTile;
     load_tile(a, n, base, v);
@@ -550,7 +564,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_inplace_kernel(int32_t *__r
     for (int q = 0; q < kScanItems; ++q) s += v[q];
     int64_t tot;
     const int64_t ex = block_excl_scan(s, tot);
-    int64_t run = ex + (partials ? partials[tile] : scan_lookback(desc, tile, tot, status));
+    int64_t run = ex + scan_lookback(desc, tile, tot, status);
     const int64_t b = base + (int64_t)threadIdx.x * kScanItems;
     int32_t o[kScanItems];
 #pragma unroll
@@ -819,17 +833,8 @@ static void launch_bucket_sort(const PipelineBufs &b, hipStream_t st)
     const SortPlan &P = b.sort;
     hipLaunchKernelGGL(bucket_count_kernel, dim3((unsigned)P.na), dim3(kBinThreads), (size_t)P.nb * 4, st, b.X, b.sys,
                        b.atom_sys, b.nsys, b.nat, P, b.key, b.slot, b.bmat, b.status);
-    const int64_t nt = scan_tiles(P.n_sort);
-    int64_t *part = nullptr;   // three-kernel scan: tile sums in the (then unused) descriptor slots
-    if (nt > kSortLookbackTiles) {
-        part = reinterpret_cast<int64_t *>(b.lookback);
-        hipLaunchKernelGGL(scan_reduce_kernel, dim3((unsigned)nt), dim3(kScanThreads), 0, st, b.bmat, P.n_sort, part,
-                           (int32_t)-1);
-        hipLaunchKernelGGL(scan_partials_kernel, dim3(1), dim3(kScanThreads), 0, st, part, (int)nt, (Status *)nullptr,
-                           (int64_t)0);
-    }
-    hipLaunchKernelGGL(scan_inplace_kernel, dim3((unsigned)nt), dim3(kScanThreads), 0, st, b.bmat, P.n_sort,
-                       b.lookback, part, b.status);
+    hipLaunchKernelGGL(scan_inplace_kernel, dim3((unsigned)scan_tiles(P.n_sort)), dim3(kScanThreads), 0, st, b.bmat,
+                       P.n_sort, b.lookback, b.status);
     hipLaunchKernelGGL(bucket_scatter_kernel, dim3((unsigned)P.na), dim3(kBinThreads), 0, st, b.nat, P, b.key, b.slot,
                        b.bmat, b.bke);
     NLH_TI_DISPATCH(b.ti_bytes,

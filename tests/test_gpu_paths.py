@@ -1,5 +1,5 @@
 """Size edges of the launch paths, each against the oracle bit for bit:
-lazy range queries.
+lazy range queries, scans.
 """
 import numpy as np
 import pytest
@@ -35,3 +35,16 @@ def test_lazy_range_sizes(int_type, bits, wind):
         assert np.array_equal(offs, ref.first[first - 1:first + n] - ref.first[first - 1])
         assert np.array_equal(j, ref.j[a:b]) and np.array_equal(S, ref.S[a:b])
         assert np.array_equal(_bits(R), _bits(ref.R[a:b]))
+
+
+@pytest.mark.parametrize("n,rc", [(2047, 1.0), (2049, 1.0), (256 * 2048, 1.0), (256 * 2048 + 1, 1.0),
+                                  (2048 * 2048 + 3, 1.0)])
+def test_pair_scan_forms(n, rc):
+    """Pair counts of 1 and 2 tiles, of 256 tiles (single pass in block order)
+    and one more (by ticket), and of 2049 tiles (three kernels)."""
+    s = workloads.random_cubic(n, density=0.8, seed=7, cutoff=rc)
+    print(f"pair scan {n}", flush=True)
+    ref = oracle.neighbour_list(s.X, rc, s.cell, s.pbc, nthreads=8)
+    nl = nlhip.neighbour_list(s.X, rc, s.cell, s.pbc)
+    assert np.array_equal(nl.first, ref.first)
+    assert np.array_equal(nl.i, ref.i) and np.array_equal(nl.j, ref.j) and np.array_equal(nl.S, ref.S)
