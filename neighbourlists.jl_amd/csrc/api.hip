@@ -176,6 +176,7 @@ struct nlh_handle {
     std::vector<int32_t> cell_base_host;
     std::vector<int32_t> brick_base_host;
     int64_t nbricks = 0;
+    int32_t brick_copies = 1;
     std::vector<nlh_geometry> geoms;
     std::vector<int64_t> pair_offsets_host;
     // per-phase timing (nlh_set_profiling): events on the handle's stream
@@ -211,6 +212,7 @@ struct nlh_handle {
         b.sys_cell_base = cell_base_d;
         b.sys_brick_base = brick_base_d;
         b.nbricks = nbricks;
+        b.brick_copies = brick_copies;
         b.nsys = nsys;
         b.nat = nat;
         b.M = M;
@@ -431,9 +433,13 @@ void drop_graph(nlh_handle *h)
 
 // Pair-search brick of a system: the largest of a fixed ladder of shapes
 // whose halo atoms, expected at this system's mean atom density per cell,
-// stay within the budget (clipped to the cell grid).
-void choose_brick(const nlh_geometry &g, int64_t nat, int32_t budget, int32_t halo_max, int32_t out[3],
-                  int64_t min_bricks = 0)
+// stay within the budget (clipped to the cell grid), or, where the grid is
+// too coarse for that to fill the device, the smallest whose bricks still
+// run together (`slots` of them).  Count kernel on MI355X, event timed: 1k
+// atoms, 125 bricks of one cell against 27 of 2 x 2 x 2, 10.4 / 18.2 us; 10k,
+// 2 x 1 x 1 (666 bricks) 13.0 us, 1 x 1 x 1 (1331, two rounds) 17.2, 2 x 2 x 2
+// 17.5; 100k, 4 x 2 x 2 (1183) 31.6, 2 x 2 x 2 (2197) 32.6.
+void choose_brick(const nlh_geometry &g, int64_t nat, int32_t budget, int32_t halo_max, int64_t slots, int32_t out[3])
 {
     static const int32_t ladder[][3] = {{4, 4, 4}, {4, 4, 2}, {4, 2, 2}, {2, 2, 2}, {2, 2, 1}, {2, 1, 1}, {1, 1, 1}};
     const double per_cell = g.ncells_total > 0 ? (double)nat / (double)g.ncells_total : 0.0;
@@ -447,12 +453,10 @@ void choose_brick(const nlh_geometry &g, int64_t nat, int32_t budget, int32_t ha
             halo *= (double)(d[k] + 2);
             nb *= (g.ncells[k] + d[k] - 1) / d[k];
         }
+        if (found && nb > slots) return;
         if (halo * per_cell <= (double)budget && halo <= (double)halo_max) {
-            // the first shape that fits; a smaller one while the grid is too
-            // coarse to fill the device, down to one home cell per wave
             std::memcpy(out, d, sizeof d);
             found = true;
-            if (nb >= min_bricks || (int64_t)d[0] * d[1] * d[2] <= 8) return;
         }
     }
     if (!found) out[0] = out[1] = out[2] = 1;
@@ -501,6 +505,89 @@ constexpr int64_t kReplayMaxAtoms = 12288;
 // counted from global memory instead).
 constexpr double kHaloFill = 0.9;
 
+// Bounds of the 32-bit distance filter (SysDev; tile_kernel in pairs.hip).
+// With u = 2^-24, c the centre of a run of home cells, |p_i - c| <= H for
+// its home atoms and |p_j - c| <= H + rc for any candidate within the cutoff,
+// the computed 2 D = r^2 - rc^2 is off by at most
+//   10 u ((2 H + rc)^2 + rc^2)   five fused multiply-adds over partial sums
+//                                of at most (|p_i| + |p_j|)^2 + rc^2, doubled
+//   7 u (H + rc)^2 + 4 u rc^2    |p_j - c|^2, |p_i - c|^2 - rc^2, rc^2 itself
+//   7.2 u (P + 2 H + rc) rc      positions rounded to 32 bits, |p| <= P, then
+//                                taken from c
+//   1.6e-11 rc (|a1| + |a2| + |a3|)   the 64-bit roundings on both sides, for
+//                                windings within +-128 (nine times their bound)
+// and by less than its distance from zero for candidates further away.  A
+// quarter is added for what the line above leaves out (second-order terms).
+void filter_bounds(nlh::SysDev &sd, const nlh_geometry &g)
+{
+    constexpr double u = 1.0 / (1 << 24);
+    const double rc = g.cutoff;
+    double step[3][3], len[3], sum = 0.0, P = rc;
+    for (int k = 0; k < 3; ++k) {
+        double l2 = 0.0;
+        for (int m = 0; m < 3; ++m) {
+            step[k][m] = g.cell[k + 3 * m] / (double)sd.n[k];   // a cell's edge along lattice vector k
+            l2 += step[k][m] * step[k][m];
+        }
+        len[k] = std::sqrt(l2);
+        sum += len[k] * sd.n[k];
+        P += (sd.brick[k] / 2 + 2.5) * len[k];   // halo atom to an atom of the middle home cell
+    }
+    for (int m = 0; m < 3; ++m) step[0][m] *= sd.run;
+    double diag2 = 0.0;   // the longest diagonal of a run of home cells
+    for (int q = 0; q < 4; ++q) {
+        double d2 = 0.0;
+        for (int m = 0; m < 3; ++m) {
+            const double d = step[0][m] + (q & 1 ? -1 : 1) * step[1][m] + (q & 2 ? -1 : 1) * step[2][m];
+            d2 += d * d;
+        }
+        diag2 = std::max(diag2, d2);
+    }
+    const double H = 0.505 * std::sqrt(diag2) + 0.25 * rc;
+    const double tol = 1.25 * u * (10 * ((2 * H + rc) * (2 * H + rc) + rc * rc) + 7 * (H + rc) * (H + rc) +
+                                   4 * rc * rc + 7.2 * (P + 2 * H + rc) * rc) + 1.6e-11 * rc * sum;
+    const bool ok = H < 1000 * rc && P < 1e6 * rc && rc > 1e-9 && rc < 1e9;
+    sd.rc2half = (float)(0.5 * g.cutoff_sq);
+    sd.tol = (float)(0.505 * tol);
+    sd.h2half = (float)(0.499 * H * H);
+    sd.pmax2 = ok ? (float)(0.999 * P * P) : -1.0f;
+}
+
+// How a system's pair search is cut up: its brick, the run of home cells that
+// shares a candidate list, the split of a run's home atoms, and the number of
+// workgroups that share each brick (returned; 1 within a batch).
+//
+// A run of two cells halves the work per run but tests 36 cells' atoms per
+// home atom instead of 27: it pays below about 8 atoms per cell (6.4, 1M
+// atoms: 153 against 162 us; 10.9, FCC slab: 236 both), and only where the
+// bricks fill the device more than once, as it makes the longest brick longer
+// (100k atoms, one round: 35 against 32 us).  A brick of one or two cells splits
+// them over its four waves, and a system whose bricks leave most of the
+// device idle is split further, down to two or three home atoms per wave
+// (96-atom crystal, four cells of 24 atoms: 48 us unsplit, 15.6 over four waves
+// each, 13.6 over eight).
+int32_t plan_search(nlh::SysDev &sd, const nlh_geometry &g, bool single, int cus, int32_t brick_atoms, int bt)
+{
+    // five 256-thread bricks (28 KB of LDS each, 20 waves) or two 512-thread
+    // ones run on a CU; the LDS of a BT-thread brick holds 4 BT halo atoms
+    // and BT halo cells
+    const int64_t slots = single ? (int64_t)cus * (bt == 256 ? 5 : 2) : 0;
+    choose_brick(g, sd.nat, std::min(brick_atoms, (int32_t)(kHaloFill * 4 * bt)), bt, slots, sd.brick);
+    const double per_cell = (double)sd.nat / std::max(sd.M, 1);
+    int64_t bricks = 1;
+    for (int k = 0; k < 3; ++k) bricks *= (sd.n[k] + sd.brick[k] - 1) / sd.brick[k];
+    const int cells = sd.brick[0] * sd.brick[1] * sd.brick[2];
+    sd.run = sd.brick[0] > 1 && per_cell <= 8.0 && bricks > 2 * slots ? 2 : 1;
+    sd.split = cells == 1 ? 2 : (cells == 2 ? 1 : 0);
+    int32_t copies = 1;
+    while (single && sd.split > 0 && sd.split < 6 && per_cell >= 4 << sd.split && bricks * copies * 2 <= slots) {
+        ++sd.split;
+        copies *= 2;
+    }
+    filter_bounds(sd, g);
+    return copies;
+}
+
 // Pair-search bricks of every system for the current brick budget: brick
 // shape per system and the first brick of each system (host tables; the
 // caller uploads them).
@@ -511,15 +598,7 @@ void assign_bricks(nlh_handle *h)
     h->brick_base_host.resize(nsys + 1);
     for (int s = 0; s < nsys; ++s) {
         nlh::SysDev &sd = h->sys_host[s];
-        // a single system takes the largest brick that still fills the
-        // device once: four 256-thread bricks (39 KB of LDS each) or two
-        // 512-thread bricks fit a CU, and the largest-first launch order
-        // fills the end of the launch with the short partial bricks
-        // the LDS of a BT-thread brick holds 4 BT halo atoms and BT halo cells
-        const int bt = h->count_block();
-        const int64_t min_bricks = nsys == 1 ? (int64_t)h->cus * (bt == 256 ? 4 : 2) : 0;
-        choose_brick(h->geoms[s], sd.nat, std::min(h->tune.brick_atoms, (int32_t)(kHaloFill * 4 * bt)), bt,
-                     sd.brick, min_bricks);
+        h->brick_copies = plan_search(sd, h->geoms[s], nsys == 1, h->cus, h->tune.brick_atoms, h->count_block());
         sd.brick_base = (int32_t)bricks;
         h->brick_base_host[s] = (int32_t)bricks;
         bricks += brick_classes(sd);
@@ -837,7 +916,7 @@ void ensure_slots(nlh_handle *h, int32_t cap, bool want_R)
 {
     h->slot_cap = std::max(h->slot_cap, cap);
     const size_t n1 = (size_t)std::max<int64_t>(h->nat, 1) * (size_t)h->slot_cap;
-    h->slots.ensure(h->stream, n1 * (h->wide ? 16 : 8));
+    h->slots.ensure(h->stream, n1 * (h->wide ? 16 : 8) + nlh::kSlotSlack);
     if (want_R) h->slotsR.ensure(h->stream, n1 * 24);
 }
 
@@ -953,7 +1032,7 @@ void check_pair_buffers(const nlh_handle *h, bool want_R)
     const size_t n1 = (size_t)std::max<int64_t>(h->nat, 1);
     const size_t ent = (size_t)h->slot_cap * n1;
     const size_t ti = (size_t)h->ti_bytes, cap = (size_t)std::max<int64_t>(h->pair_capacity, 0);
-    bool ok = h->slot_cap > 0 && h->slots.p && h->slots.cap >= ent * (h->wide ? 16 : 8);
+    bool ok = h->slot_cap > 0 && h->slots.p && h->slots.cap >= ent * (h->wide ? 16 : 8) + nlh::kSlotSlack;
     ok = ok && h->pair_count.cap >= n1 * 4 && h->pair_off.cap >= (n1 + 1) * 8;
     ok = ok && h->first.cap >= (n1 + h->nsys) * ti && h->sys_pair_base.cap >= (size_t)(h->nsys + 1) * 8;
     ok = ok && h->i.cap >= cap * ti && h->j.cap >= cap * ti && h->S.cap >= cap * 3 * ti;
@@ -1317,6 +1396,7 @@ struct NoAllocPlan {
     int32_t cell_base[2];
     int32_t brick_base[2];
     int64_t nbricks;
+    int32_t brick_copies;
     nlh::SortPlan sort;
 };
 
@@ -1339,6 +1419,7 @@ size_t carve_noalloc(char *base, const NoAllocPlan &P, int ti, int32_t cap, bool
     b.nsys = 1;
     b.atom_sys = nullptr;
     b.nbricks = P.nbricks;
+    b.brick_copies = P.brick_copies;
     b.nat = P.sd.nat;
     b.M = P.sd.M;
     b.sort = P.sort;
@@ -1365,7 +1446,7 @@ size_t carve_noalloc(char *base, const NoAllocPlan &P, int ti, int32_t cap, bool
     // the tail: slot rows (the bucketed sort's (cell, index) scratch lives
     // at their start until the count pass rewrites them), then their R
     const size_t rows = n1 * (size_t)cap;
-    b.slots = c.take<void>(std::max(rows * (wide ? 16 : 8), n1 * nlh::kBucketBytes));
+    b.slots = c.take<void>(std::max(rows * (wide ? 16 : 8) + nlh::kSlotSlack, n1 * nlh::kBucketBytes));
     b.bke = reinterpret_cast<int2 *>(b.slots);
     b.slot_cap = cap;
     b.slotsR = want_R ? c.take<double>(rows * 24) : nullptr;
@@ -1442,8 +1523,7 @@ void neighbour_list_noalloc(hipStream_t st, const double *X, int64_t nat, const 
     NoAllocPlan P{};
     P.sd = make_sys(g, nat, 0, 0, 0);
     const int cus = g_scratch_cus[dev];
-    choose_brick(g, nat, std::min<int32_t>(920, (int32_t)(kHaloFill * 4 * 256)), 256, P.sd.brick,
-                 (int64_t)cus * 4);
+    P.brick_copies = plan_search(P.sd, g, true, cus, 920, 256);
     P.sd.brick_base = 0;
     P.nbricks = brick_classes(P.sd);
     P.atom_base[0] = 0;

@@ -96,6 +96,26 @@ __device__ __forceinline__ int64_t block_excl_scan_n(int64_t v, int64_t &total)
     return before + inc - v;
 }
 
+// The same for 32-bit values.
+template <int NT>
+__device__ __forceinline__ int block_excl_scan32(int v, int &total)
+{
+    __shared__ int wsum[NT / kWave];
+    const int lane = lane_id(), wv = threadIdx.x / kWave;
+    const int inc = wave_incl_scan(v);
+    if (lane == kWave - 1) wsum[wv] = inc;
+    __syncthreads();
+    int before = 0, tot = 0;
+#pragma unroll
+    for (int w = 0; w < NT / kWave; ++w) {
+        const int s = wsum[w];
+        if (w < wv) before += s;
+        tot += s;
+    }
+    total = __builtin_amdgcn_readfirstlane(tot);
+    return before + inc - v;
+}
+
 __device__ __forceinline__ int64_t block_excl_scan(int64_t v, int64_t &total)
 {
     return block_excl_scan_n<kScanThreads>(v, total);

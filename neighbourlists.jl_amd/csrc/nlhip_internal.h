@@ -103,6 +103,14 @@ struct SysDev {
     int32_t bfull[3];      // full bricks along each axis (n / brick)
     int32_t cls_first[9];
     int32_t cls_mask[8];   // bit k set: the class's bricks are the partial last brick along axis k
+    // Bounds of the 32-bit distance filter (tile_kernel; set by filter_bounds):
+    // with every brick atom within sqrt(pmax2) of the brick's origin and every
+    // home atom within sqrt(2 h2half) of its group's, the filter's value of
+    // (r^2 - rc^2) / 2 has the sign of the 64-bit test wherever it is at least
+    // tol away from zero.  pmax2 < 0: the system does not use the filter.
+    float rc2half, tol, h2half, pmax2;
+    int32_t run;           // home cells along x that share a candidate list (tile_kernel): 1 or 2
+    int32_t split;         // log2 of the work items a run's home atoms are split into
 };
 
 // Sorted atom record: position, original (system-local, 0-based) index and
@@ -121,6 +129,10 @@ constexpr uint32_t kWindBig = 0x80000000u;
 // set = 8-byte entries (j | packed S << 32).
 constexpr int32_t kRow8Bit = 1 << 30;
 constexpr int32_t kCountMask = kRow8Bit - 1;
+// Bytes after the last slot row that the count kernels may write when a row
+// overflows: a row takes at most the candidates of a brick's or a unit's LDS
+// (2048), 8 bytes each.
+constexpr size_t kSlotSlack = 2048 * 8;
 constexpr int32_t kNarrowMaxAtoms = 1 << 26;
 
 // 2-bit code of a shift component in {-1, 0, 1} and back
@@ -239,6 +251,7 @@ struct PipelineBufs {
     int32_t nsys;
     int32_t *atom_sys;          // batches: system of each atom (nat), then of each cell (M); else null
     int64_t nbricks;            // total pair-search bricks
+    int32_t brick_copies;       // workgroups sharing each brick (tile_kernel)
     int64_t nat;                // total atoms
     int32_t M;                  // total cells
     // build

@@ -3,22 +3,24 @@
 // (src/gpu_kernels.jl:132-180) around the inner loop _for_each_neighbor_pair
 // (src/gpu_kernels.jl:58-101).
 //
-// count_kernel -- work unit: a brick of up to 4x4x4 home cells per 256-thread
-// (or 512-thread) workgroup, the bricks launched largest first.  The brick
-// and its one-cell halo are staged in LDS in one load phase (every global
-// load of the phase in flight together), then the waves take home cells from
-// a workgroup counter and test candidates from LDS only:
+// tile_kernel (count_kernel when R is wanted or shifts are wide) -- work
+// unit: a brick of up to 4x4x4 home cells per 256-thread (or 512-thread)
+// workgroup, the bricks launched largest first.  The brick and its one-cell
+// halo are staged in LDS in one load phase (every global load of the phase in
+// flight together), then the waves take work items (one or two home cells, or
+// a part of one) from a workgroup counter and test candidates from LDS only:
 //   - the candidates of a home cell are its 27 neighbour cells flattened in
 //     the reference order (dz, dy, dx; gpu_kernels.jl:69-71) -- nine
 //     contiguous LDS rows -- cut into 64-candidate chunks, one per lane;
-//   - the home atoms stream through the wave as uniform values, two at a
-//     time; each (home atom, chunk) test is one ballot, and the hit lanes
-//     append their (j, S) to the home atom's slot row at its running count,
-//     so every row holds the atom's neighbours in exactly the reference
-//     traversal order.
-// Bricks whose neighbour reach exceeds one cell, whose halo does not fit
-// LDS, or whose windings do not pack take a per-wave path that reads global
-// memory (one home cell per wave) with the same enumeration and output.
+//   - the home atoms stream through the wave as uniform values; each (home
+//     atom, chunk) test is one ballot, and the hit lanes append their (j, S)
+//     to the home atom's slot row at its running count, so every row holds
+//     the atom's neighbours in exactly the reference traversal order.
+// tile_kernel tests 32-bit positions and decides what lies within their error
+// of the cutoff by the 64-bit test.  Bricks whose neighbour reach exceeds one
+// cell, whose halo does not fit LDS, or whose windings do not pack take a
+// per-wave path that reads global memory (one home cell per wave) with the
+// same enumeration and output.
 //
 // fill_kernel -- one wave per tile of consecutive output pairs, one lane per
 // pair: the tile's first atom comes from the pair scan's tile table, and
@@ -81,7 +83,7 @@ __device__ __forceinline__ void rec_winding(const Rec &r, const int32_t *__restr
     }
 }
 
-constexpr int kChunksPerPass = 4;   // candidate chunks a lane holds at once
+constexpr int kChunksPerPass = 2;   // candidate chunks a lane holds at once (per-wave path)
 constexpr double kFar = 1.0e200;    // invalid candidate: r^2 overflows to +inf, never a hit
 
 struct PairsArgs {
@@ -692,8 +694,8 @@ struct HomeRows {
     int self0;       // candidate index of home atom 0 (uniform)
 };
 
-template <int BT>
-__device__ __forceinline__ HomeRows brick_home(const Brick &B, const BrickLDS<BT> &L, int hc)
+template <typename LDS>
+__device__ __forceinline__ HomeRows brick_home(const Brick &B, const LDS &L, int hc)
 {
     HomeRows R;
     const int q0 = small_quot(hc, B.dnh0), iz = small_quot(q0, B.dnh1);
@@ -738,8 +740,8 @@ struct RowMap {
 
 // Publish the row offsets of a home cell; returns this lane's rank among the
 // non-empty rows (meaningful on the lanes of non-empty rows, `ne`).
-template <int BT>
-__device__ __forceinline__ int row_publish(const HomeRows &R, BrickLDS<BT> &L, int wv, bool &ne)
+template <typename LDS>
+__device__ __forceinline__ int row_publish(const HomeRows &R, LDS &L, int wv, bool &ne)
 {
     const int lane = lane_id();
     ne = lane < 9 && R.len > 0;
@@ -748,8 +750,8 @@ __device__ __forceinline__ int row_publish(const HomeRows &R, BrickLDS<BT> &L, i
     return q;
 }
 
-template <int BT>
-__device__ __forceinline__ RowMap row_map(const HomeRows &R, BrickLDS<BT> &L, int wv, int k0, int q, bool ne)
+template <typename LDS>
+__device__ __forceinline__ RowMap row_map(const HomeRows &R, LDS &L, int wv, int k0, int q, bool ne)
 {
     const int lane = lane_id();
     uint8_t *fl = reinterpret_cast<uint8_t *>(L.rowflag[wv]);
@@ -768,8 +770,8 @@ __device__ __forceinline__ RowMap row_map(const HomeRows &R, BrickLDS<BT> &L, in
     return M;
 }
 
-template <int BT>
-__device__ __forceinline__ int row_index(const RowMap &M, const BrickLDS<BT> &L, int wv, int g, int k)
+template <typename LDS>
+__device__ __forceinline__ int row_index(const RowMap &M, const LDS &L, int wv, int g, int k)
 {
     const int q = M.base[g] + (int)mbcnt64(M.sh[g]);
     return k + L.rowdl[wv][q];
@@ -801,7 +803,7 @@ constexpr uint32_t kDropOffset = 0x40800000u;
 static_assert(__builtin_bit_cast(uint32_t, 4.0f) == kDropOffset, "the select below writes the offset as 4.0");
 constexpr int32_t kRawBufferWord3 = 0x00020000; // raw 32-bit buffer access (GFX9 family)
 
-template <bool NARROW, bool WZERO, bool WANT_R, bool WIDE, bool DENSE = false>
+template <bool NARROW, bool WZERO, bool WANT_R, bool WIDE>
 __device__ __forceinline__ void emit_row(void *__restrict__ row, double *__restrict__ rrow, uint32_t cap,
                                          Status *__restrict__ status, uint64_t m, int32_t &ca, uint64_t ent,
                                          int32_t wix, int32_t wiy, int32_t wiz, double Rx, double Ry, double Rz)
@@ -811,7 +813,7 @@ __device__ __forceinline__ void emit_row(void *__restrict__ row, double *__restr
         // every lane stores, each lane without a hit at an offset past the
         // resource's end (a select on the ballot, not an exec-mask region);
         // an empty ballot skips it
-        if (!DENSE && n == 0) return;
+        if (n == 0) return;
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(row, 0, (int)(cap * 4u), kRawBufferWord3);
         const uint32_t rk = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
         uint32_t off;
@@ -913,7 +915,7 @@ __device__ __forceinline__ void test_home_atom(int nch, const double *cx, const 
 // same shifts) against the same chunks: both distance tests of a chunk come
 // before both emissions, two independent chains the scheduler interleaves.
 // Atom 1's self candidate follows atom 0's.
-template <bool WANT_R, bool WIDE, bool DENSE>
+template <bool WANT_R, bool WIDE>
 __device__ __forceinline__ void test_home_pair(int nch, const double *cx, const double *cy, const double *cz,
                                                const double *sx, const double *sy, const double *sz, const uint64_t *csh,
                                                const uint64_t *ent, double h0x, double h0y, double h0z, double h1x,
@@ -943,84 +945,9 @@ __device__ __forceinline__ void test_home_pair(int nch, const double *cx, const 
             const bool in1 = (R1x * R1x + R1y * R1y) + R1z * R1z < rc2;
             const uint64_t m0 = __builtin_amdgcn_ballot_w64(in0) & (g == gs0 ? nself0 : ~0ull);
             const uint64_t m1 = __builtin_amdgcn_ballot_w64(in1) & (g == gs1 ? nself1 : ~0ull);
-            emit_row<true, true, WANT_R, WIDE, DENSE>(row0, rrow0, cap, status, m0, ca0, ent[g], 0, 0, 0, R0x, R0y, R0z);
-            emit_row<true, true, WANT_R, WIDE, DENSE>(row1, rrow1, cap, status, m1, ca1, ent[g], 0, 0, 0, R1x, R1y, R1z);
+            emit_row<true, true, WANT_R, WIDE>(row0, rrow0, cap, status, m0, ca0, ent[g], 0, 0, 0, R0x, R0y, R0z);
+            emit_row<true, true, WANT_R, WIDE>(row1, rrow1, cap, status, m1, ca1, ent[g], 0, 0, 0, R1x, R1y, R1z);
         }
-    }
-}
-
-// test_home_pair for three full chunks with no shift and 4-byte rows without
-// R: the six distance tests of the pair, then its six emissions (every lane
-// stores, lanes without a hit at the dropped offset), one branch-free block.
-// G: the chunk that holds both self candidates (known for a whole group of
-// home atoms: one mask per atom), kBrickChunks when neither lies in the
-// pass, or -1 when the chunk is found per atom.
-template <int G>
-__device__ __forceinline__ void test_pair_plain(const double *cx, const double *cy, const double *cz,
-                                                const uint64_t *ent, double h0x, double h0y, double h0z, double h1x,
-                                                double h1y, double h1z, double rc2, int ks0, void *__restrict__ row0,
-                                                void *__restrict__ row1, uint32_t cap, int32_t &ca0, int32_t &ca1)
-{
-    const int gs0 = G < 0 ? ks0 >> 6 : G, gs1 = G < 0 ? (ks0 + 1) >> 6 : G;
-    const uint64_t nself0 = ~(1ull << (ks0 & (kWave - 1))), nself1 = ~(1ull << ((ks0 + 1) & (kWave - 1)));
-    uint64_t m0[kBrickChunks], m1[kBrickChunks];
-#pragma unroll
-    for (int g = 0; g < kBrickChunks; ++g) {
-        // R = xj - xi (shift zero) ; r^2 = dot(R, R)  (gpu_kernels.jl:89-92)
-        const double R0x = cx[g] - h0x, R0y = cy[g] - h0y, R0z = cz[g] - h0z;
-        const double R1x = cx[g] - h1x, R1y = cy[g] - h1y, R1z = cz[g] - h1z;
-        const bool in0 = (R0x * R0x + R0y * R0y) + R0z * R0z < rc2;
-        const bool in1 = (R1x * R1x + R1y * R1y) + R1z * R1z < rc2;
-        m0[g] = __builtin_amdgcn_ballot_w64(in0) & (g == gs0 ? nself0 : ~0ull);
-        m1[g] = __builtin_amdgcn_ballot_w64(in1) & (g == gs1 ? nself1 : ~0ull);
-    }
-#pragma unroll
-    for (int g = 0; g < kBrickChunks; ++g) {
-        emit_row<true, true, false, false, true>(row0, nullptr, cap, nullptr, m0[g], ca0, ent[g], 0, 0, 0, 0.0, 0.0, 0.0);
-        emit_row<true, true, false, false, true>(row1, nullptr, cap, nullptr, m1[g], ca1, ent[g], 0, 0, 0, 0.0, 0.0, 0.0);
-    }
-}
-
-// One home atom against three full chunks with no shift, 4-byte rows
-// without R (the odd atom of a pass through test_pair_plain).
-__device__ __forceinline__ void test_atom_plain(const double *cx, const double *cy, const double *cz,
-                                                const uint64_t *ent, double hx, double hy, double hz, double rc2,
-                                                int ks, void *__restrict__ row, uint32_t cap, int32_t &ca)
-{
-    const int gs = ks >> 6;
-    const uint64_t nself = ~(1ull << (ks & (kWave - 1)));
-    uint64_t m[kBrickChunks];
-#pragma unroll
-    for (int g = 0; g < kBrickChunks; ++g) {
-        // R = xj - xi (shift zero) ; r^2 = dot(R, R)  (gpu_kernels.jl:89-92)
-        const double Rx = cx[g] - hx, Ry = cy[g] - hy, Rz = cz[g] - hz;
-        m[g] = __builtin_amdgcn_ballot_w64((Rx * Rx + Ry * Ry) + Rz * Rz < rc2) & (g == gs ? nself : ~0ull);
-    }
-#pragma unroll
-    for (int g = 0; g < kBrickChunks; ++g)
-        emit_row<true, true, false, false, true>(row, nullptr, cap, nullptr, m[g], ca, ent[g], 0, 0, 0, 0.0, 0.0, 0.0);
-}
-
-// The home atoms of a pass through test_pair_plain<G>, two at a time from
-// home atom a (left at the first atom not done).  FRESH: the group's first
-// pass, every running count still zero.
-template <int G, bool FRESH = false>
-__device__ __forceinline__ void plain_pairs(const double *cx, const double *cy, const double *cz, const uint64_t *ent,
-                                            const LAtom *home, int nh, int32_t hj_l, int kpass, double rc2,
-                                            int64_t atom_base, void *__restrict__ slots, int32_t cap, int32_t &cnt_l,
-                                            int &a)
-{
-    for (; a + 1 < nh; a += 2) {
-        const LAtom h0 = home[a], h1 = home[a + 1];
-        int32_t ca0 = FRESH ? 0 : __builtin_amdgcn_readlane(cnt_l, a);
-        int32_t ca1 = FRESH ? 0 : __builtin_amdgcn_readlane(cnt_l, a + 1);
-        const int64_t srow0 = slot_row(atom_base + __builtin_amdgcn_readlane(hj_l, a), cap);
-        const int64_t srow1 = slot_row(atom_base + __builtin_amdgcn_readlane(hj_l, a + 1), cap);
-        test_pair_plain<G>(cx, cy, cz, ent, h0.x, h0.y, h0.z, h1.x, h1.y, h1.z, rc2, kpass + a,
-                           reinterpret_cast<uint64_t *>(slots) + srow0, reinterpret_cast<uint64_t *>(slots) + srow1,
-                           (uint32_t)cap, ca0, ca1);
-        cnt_l = write_lane(ca0, a, cnt_l);
-        cnt_l = write_lane(ca1, a + 1, cnt_l);
     }
 }
 
@@ -1030,10 +957,9 @@ __device__ __forceinline__ void plain_pairs(const double *cx, const double *cy, 
 // appended to its slot row at its running count (lane a of cnt_l for home
 // atom a).  home: the nh home atoms in LDS; ht_l, hj_l: lane a holds
 // pack(-w_i) and j of home atom a; kpass: the self candidate of home atom 0
-// in this pass (home atom a's is kpass + a); Cm: the cell matrix; fresh:
-// the first pass of the home atoms (every running count zero).
-template <bool WANT_R, bool WIDE, bool DENSE>
-__device__ __forceinline__ void pass_home_atoms(bool narrow, bool fresh, int nch, const double *cx, const double *cy,
+// in this pass (home atom a's is kpass + a); Cm: the cell matrix.
+template <bool WANT_R, bool WIDE>
+__device__ __forceinline__ void pass_home_atoms(bool narrow, int nch, const double *cx, const double *cy,
                                                 const double *cz, const uint64_t *ent, const LAtom *home, int nh,
                                                 uint32_t ht_l, int32_t hj_l, int kpass, const double *Cm, double rc2,
                                                 int64_t atom_base, void *__restrict__ slots, double *__restrict__ slotsR,
@@ -1052,36 +978,6 @@ __device__ __forceinline__ void pass_home_atoms(bool narrow, bool fresh, int nch
 #pragma unroll
         for (int g = 0; g < kBrickChunks; ++g)
             csh[g] = g < nch ? __builtin_amdgcn_ballot_w64((uint32_t)(ent[g] >> 32) != kPackZero) : 0;
-        if (DENSE && !WANT_R && !WIDE && nch == kBrickChunks && (csh[0] | csh[1] | csh[2]) == 0) {
-            // the self candidates kpass .. kpass + nh - 1 of the group: in one
-            // chunk (nearly always), in none, or across two
-            const int g0 = kpass >> 6, g1 = (kpass + nh - 1) >> 6;
-            if (g1 < 0 || g0 >= kBrickChunks)
-                plain_pairs<kBrickChunks>(cx, cy, cz, ent, home, nh, hj_l, kpass, rc2, atom_base, slots, cap, cnt_l, a);
-            else if (g0 == g1 && g0 == 0 && fresh)
-                plain_pairs<0, true>(cx, cy, cz, ent, home, nh, hj_l, kpass, rc2, atom_base, slots, cap, cnt_l, a);
-            else if (g0 == g1 && g0 == 1 && fresh)
-                plain_pairs<1, true>(cx, cy, cz, ent, home, nh, hj_l, kpass, rc2, atom_base, slots, cap, cnt_l, a);
-            else if (g0 == g1 && g0 == 2 && fresh)
-                plain_pairs<2, true>(cx, cy, cz, ent, home, nh, hj_l, kpass, rc2, atom_base, slots, cap, cnt_l, a);
-            else if (g0 == g1 && g0 == 0)
-                plain_pairs<0>(cx, cy, cz, ent, home, nh, hj_l, kpass, rc2, atom_base, slots, cap, cnt_l, a);
-            else if (g0 == g1 && g0 == 1)
-                plain_pairs<1>(cx, cy, cz, ent, home, nh, hj_l, kpass, rc2, atom_base, slots, cap, cnt_l, a);
-            else if (g0 == g1 && g0 == 2)
-                plain_pairs<2>(cx, cy, cz, ent, home, nh, hj_l, kpass, rc2, atom_base, slots, cap, cnt_l, a);
-            else
-                plain_pairs<-1>(cx, cy, cz, ent, home, nh, hj_l, kpass, rc2, atom_base, slots, cap, cnt_l, a);
-            if (a < nh) {   // the odd home atom
-                const LAtom hm = home[a];
-                int32_t ca = __builtin_amdgcn_readlane(cnt_l, a);
-                const int64_t srow = slot_row(atom_base + __builtin_amdgcn_readlane(hj_l, a), cap);
-                test_atom_plain(cx, cy, cz, ent, hm.x, hm.y, hm.z, rc2, kpass + a,
-                                reinterpret_cast<uint64_t *>(slots) + srow, (uint32_t)cap, ca);
-                cnt_l = write_lane(ca, a, cnt_l);
-            }
-            return;   // the shifts are never needed
-        }
 #pragma unroll
         for (int g = 0; g < kBrickChunks; ++g) {
             if (g < nch && (WANT_R || csh[g] != 0)) {
@@ -1105,8 +1001,8 @@ __device__ __forceinline__ void pass_home_atoms(bool narrow, bool fresh, int nch
                               : (void *)(reinterpret_cast<uint64_t *>(slots) + srow1);
             double *rrow0 = WANT_R ? slotsR + 3 * srow0 : nullptr;
             double *rrow1 = WANT_R ? slotsR + 3 * srow1 : nullptr;
-            test_home_pair<WANT_R, WIDE, DENSE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, h0x, h0y, h0z, h1x, h1y,
-                                         h1z, rc2, kpass + a, row0, row1, rrow0, rrow1,
+            test_home_pair<WANT_R, WIDE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, h0x, h0y, h0z, h1x, h1y, h1z,
+                                         rc2, kpass + a, row0, row1, rrow0, rrow1,
                                          (uint32_t)cap, status, ca0, ca1);
             cnt_l = write_lane(ca0, a, cnt_l);
             cnt_l = write_lane(ca1, a + 1, cnt_l);
@@ -1226,11 +1122,501 @@ __global__ __launch_bounds__(BT) void count_kernel(
                     cz[g] = c.z;
                     ent[g] = (uint64_t)((uint32_t)c.j & jmask) | ((uint64_t)c.t << 32);
                 }
-                pass_home_atoms<WANT_R, WIDE, true>(narrow, k0 == 0, nch, cx, cy, cz, ent, L.a + hb, nh, ht_l, hj_l,
+                pass_home_atoms<WANT_R, WIDE>(narrow, nch, cx, cy, cz, ent, L.a + hb, nh, ht_l, hj_l,
                                                     kself - k0, Csh, rc2, sd.atom_base, slots, slotsR, cap, status,
                                                     cnt_l);
             }
             if (lane < nh) pair_count[sd.atom_base + hj_l] = cnt_l | (narrow ? 0 : kRow8Bit);
+        }
+    }
+}
+
+// Append one chunk's hits (m) to a home atom's slot row: 4-byte entries (lo),
+// or 8-byte ones (lo, hi).  rs is a structured buffer over the row, so the
+// byte offset of its filled part.  The hit mask is the exec mask of the store
+// and a lane's rank among the hits its index.  The kernel is bound by how
+// many instructions its waves issue, scalar ones included: this is six of
+// them and the store, where a raw buffer store of every lane (at rank and
+// count shifted to a byte offset, or past the row's end) took nine.
+//
+// A row that overflows runs on into the next ones (kSlotSlack bytes after
+// the last row take the last ones' overflow): the host sees the count, and
+// the rows are grown and counted again before anything reads them.
+//
+// The assembler knows no hazards here, so the block keeps them itself: rs
+// comes from v_readlane, and a vector write of a scalar register wants five
+// wait states before a buffer instruction reads it.
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+
+template <bool NARROW>
+__device__ __forceinline__ void emit_chunk(v4u rs, uint64_t m, int32_t &so, uint32_t lo, uint32_t hi)
+{
+    uint32_t ix;
+    int32_t n, next;
+#define NLH_EMIT(shift, store)                   \
+    "s_mov_b64 exec, %4\n\t"                     \
+    "s_bcnt1_i32_b64 %1, %4\n\t"                 \
+    shift " %2, %1, %3\n\t"                      \
+    "v_mbcnt_lo_u32_b32 %0, exec_lo, 0\n\t"      \
+    "v_mbcnt_hi_u32_b32 %0, exec_hi, %0\n\t"     \
+    store " %5, %0, %6, %3 idxen\n\t"            \
+    "s_mov_b64 exec, -1"
+    if constexpr (NARROW)
+        __asm__ volatile(NLH_EMIT("s_lshl2_add_u32", "buffer_store_dword")
+                         : "=&v"(ix), "=&s"(n), "=&s"(next)
+                         : "s"(so), "s"(m), "v"(lo), "s"(rs)
+                         : "scc");
+    else
+        __asm__ volatile(NLH_EMIT("s_lshl3_add_u32", "buffer_store_dwordx2")
+                         : "=&v"(ix), "=&s"(n), "=&s"(next)
+                         : "s"(so), "s"(m), "v"((uint64_t)lo | (uint64_t)hi << 32), "s"(rs)
+                         : "scc");
+#undef NLH_EMIT
+    so = next;
+}
+
+// ---------------------------------------------------------------------------
+// the brick count with 32-bit positions
+// ---------------------------------------------------------------------------
+
+// A halo atom of tile_kernel: its position as the brick sees it (cell shift
+// and winding applied, relative to the brick's origin) in 32 bits, and j, or
+// j | S code << 26 when every j fits in 26 bits.  One 16-byte read.
+struct __attribute__((aligned(16))) TAtom {
+    float x, y, z;
+    int32_t j;
+};
+
+constexpr int kTileChunks = 4;                       // candidate chunks a lane holds in a pass
+constexpr int kTileCands = kTileChunks * kWave;
+constexpr int kTileHome = 64;                        // home cells of a brick at most (choose_brick)
+
+template <int BT>
+struct TileLDS {
+    using Sh = BrickShape<BT>;
+    // entry cap is a far-away atom that lanes past the last candidate read
+    TAtom a[Sh::cap + 1];
+    uint32_t t[Sh::cap + 1];        // pack(t' = s - w - (s - w) of the origin atom); S = t'_j - t'_i
+    int32_t hoff[Sh::halo + 1];     // LDS offset of each halo cell's atoms
+    int32_t hstart[Sh::halo];       // first sorted index of each halo cell
+    uint32_t hshift[Sh::halo];      // packed cell shift of each halo cell | kHomeCell
+    // per wave, for its current run of home cells (as in BrickLDS): row
+    // offsets, and one byte per candidate of a pass where a row starts
+    int32_t rowdl[Sh::waves][16];
+    uint32_t rowflag[Sh::waves][kTileCands / 4];
+    uint16_t owner[Sh::cap];        // halo cell of each LDS atom slot
+    float ctr[kTileHome][3];        // centre of each run of home cells
+    int32_t next_item;              // the next work item a wave takes
+    int32_t total, flag;
+    int32_t row8;                   // some shift needs 8-byte slot entries
+};
+
+constexpr float kFar32 = 1.0e18f;   // sentinel position: |p|^2 / 2 = 5e35, never a hit
+constexpr uint32_t kFieldsLow = 1u | (1u << 10) | (1u << 20);
+
+// The runs of a brick: sd.run home cells next to each other along x, the last
+// of a row possibly shorter.
+struct TileRuns {
+    int w, nx, n;          // cells of a run, runs of a row, runs
+    SmallDiv dnx;          // divisor nx
+};
+
+__device__ __forceinline__ TileRuns tile_runs(const Brick &B)
+{
+    TileRuns T;
+    T.w = B.sd->run;
+    T.nx = T.w == 1 ? B.nh[0] : (B.nh[0] + 1) >> 1;
+    T.n = T.nx * B.nh[1] * B.nh[2];
+    T.dnx = small_div(T.nx);
+    return T;
+}
+
+// First home cell (0-based in the brick) and cells of run r.
+__device__ __forceinline__ void tile_run(const Brick &B, const TileRuns &T, int r, int &ix, int &iy, int &iz, int &w)
+{
+    const int q0 = small_quot(r, T.dnx);
+    iz = small_quot(q0, B.dnh1);
+    iy = q0 - iz * B.nh[1];
+    ix = (r - q0 * T.nx) * T.w;
+    w = min(T.w, B.nh[0] - ix);
+}
+
+// Stage the brick and its halo in LDS.  Returns false (for every thread of
+// the block) when the brick must take the global-memory path: more halo
+// atoms than the LDS holds, windings beyond +-128, or atoms further out than
+// the filter's bounds allow (clamped into the grid from far outside).
+template <int BT>
+__device__ bool tile_load(const PairsArgs &A, const Brick &B, const TileRuns &T, TileLDS<BT> &L, const double *Csh)
+{
+    using Sh = BrickShape<BT>;
+    const SysDev &sd = *B.sd;
+    const int tid = threadIdx.x;
+    const bool p[3] = {(sd.pbc & 1) != 0, (sd.pbc & 2) != 0, (sd.pbc & 4) != 0};
+    // halo cell table: thread tid owns halo cell tid
+    int cnt = 0;
+    if (tid < B.nhalo) {
+        const int q0 = small_quot(tid, B.dhd0), uz = small_quot(q0, B.dhd1);
+        const int ux = tid - q0 * B.hd[0], uy = q0 - uz * B.hd[1];
+        const int a[3] = {B.b0[0] - 1 + ux, B.b0[1] - 1 + uy, B.b0[2] - 1 + uz};
+        bool inb = true;
+        for (int k = 0; k < 3; ++k) inb = inb && (p[k] || (a[k] >= 1 && a[k] <= sd.n[k]));
+        int st = 0;
+        uint32_t sh = kPackZero;
+        if (inb) {   // _is_cell_in_bounds / _get_neighbor_cell (gpu_kernels.jl:20-47)
+            int32_t c[3], sft[3];
+            for (int k = 0; k < 3; ++k) wrap_near(a[k], sd.n[k], c[k], sft[k]);
+            const int gc = sd.cell_base + (c[0] - 1) + (c[1] - 1) * sd.n[0] + (c[2] - 1) * sd.n[0] * sd.n[1];
+            st = A.cell_start[gc];
+            cnt = A.cell_start[gc + 1] - st;
+            sh = pack_wind(sft[0], sft[1], sft[2]);
+        }
+        const bool home = ux >= 1 && ux <= B.nh[0] && uy >= 1 && uy <= B.nh[1] && uz >= 1 && uz <= B.nh[2];
+        L.hstart[tid] = st;
+        L.hshift[tid] = sh | (home ? kHomeCell : 0u);
+    }
+    int tot;
+    const int run = block_excl_scan32<BT>(cnt, tot);
+    if (tid < B.nhalo) {
+        L.hoff[tid] = run;
+        // the cell's atom slots name their cell (a brick whose halo
+        // overflows the LDS takes the global-memory path)
+        const int e = min(run + cnt, Sh::cap);
+        for (int q = run; q < e; ++q) L.owner[q] = (uint16_t)tid;
+    }
+    if (tid == 0) {
+        L.hoff[B.nhalo] = tot;
+        L.next_item = Sh::waves;
+        L.flag = 0;
+        L.row8 = sd.nat > kNarrowMaxAtoms ? 1 : 0;
+        L.a[Sh::cap] = TAtom{kFar32, 0.0f, 0.0f, 0};
+        L.t[Sh::cap] = kPackZero;
+    }
+    __syncthreads();
+    const int total = tot;   // uniform
+    if (total > Sh::cap || sd.pmax2 < 0.0f) return false;
+    if (total == 0) return true;
+    // the origin: the first atom at or after the middle home cell
+    const int hm = (B.nh[0] / 2 + 1) + B.hd[0] * ((B.nh[1] / 2 + 1) + B.hd[1] * (B.nh[2] / 2 + 1));
+    const int im = min(L.hoff[hm], total - 1), ho = L.owner[im];
+    const int po = sgpr(L.hstart[ho] + (im - L.hoff[ho]));
+    const Rec ro = A.rec[po];
+    const double ox = ro.x, oy = ro.y, oz = ro.z;
+    // pack(t') of an atom = its cell shift's pack - its winding's + tb (no
+    // field leaves its 10 bits while every winding is within +-128)
+    const uint32_t to = (L.hshift[ho] & ~kHomeCell) - ro.w, tb = kPackZero - to;
+    // halo atoms: all loads of a thread in flight together
+    int pg[Sh::unroll];
+    uint32_t hs[Sh::unroll];
+#pragma unroll
+    for (int u = 0; u < Sh::unroll; ++u) {
+        const int idx = tid + u * BT;
+        pg[u] = po;
+        hs[u] = kPackZero;
+        if (idx < total) {
+            const int h = L.owner[idx];
+            pg[u] = L.hstart[h] + (idx - L.hoff[h]);
+            hs[u] = L.hshift[h];
+        }
+    }
+    Rec r[Sh::unroll];
+#pragma unroll
+    for (int u = 0; u < Sh::unroll; ++u)
+        if (tid + u * BT < total) r[u] = A.rec[pg[u]];
+    // winding fields (biased by 512) within [384, 639]: bits 9 and 8 differ,
+    // bits 8 and 7 do not
+    constexpr uint32_t kWindMask = (kFieldsLow << 9) | (kFieldsLow << 8) | kWindBig, kWindOk = kFieldsLow << 9;
+    bool bad = ((ro.w ^ ((ro.w & ~kWindBig) << 1)) & kWindMask) != kWindOk;
+#pragma unroll
+    for (int u = 0; u < Sh::unroll; ++u) {
+        const int idx = tid + u * BT;
+        if (idx < total) {
+            const uint32_t w = r[u].w;
+            bad |= ((w ^ ((w & ~kWindBig) << 1)) & kWindMask) != kWindOk;
+            const uint32_t t = (hs[u] & ~kHomeCell) - w + tb;
+            double dx = r[u].x - ox, dy = r[u].y - oy, dz = r[u].z - oz;
+            if (t != kPackZero) {
+                int32_t tx, ty, tz;
+                unpack_wind(t, tx, ty, tz);
+                double cx, cy, cz;
+                cell_shift(Csh, tx, ty, tz, cx, cy, cz);
+                dx += cx;
+                dy += cy;
+                dz += cz;
+            }
+            const float fx = (float)dx, fy = (float)dy, fz = (float)dz;
+            bad |= !(fx * fx + fy * fy + fz * fz <= sd.pmax2);
+            // 4-byte slot entries need every S = t'_j - t'_i within [-1, 1]^3: home
+            // atoms with t' = 0 and halo atoms with |t'_k| <= 1
+            const uint32_t c = t - 511u * kFieldsLow;   // fields 0, 1, 2 then
+            const bool near = (c & ~(3u * kFieldsLow)) == 0 && (c & (c >> 1) & kFieldsLow) == 0;
+            if (!((hs[u] & kHomeCell) ? t == kPackZero : near)) L.row8 = 1;
+            // the low 2 bits of the fields are the S codes of a 4-byte entry
+            const uint32_t code = (t & 3u) | ((t >> 8) & 12u) | ((t >> 16) & 48u);
+            L.a[idx] = TAtom{fx, fy, fz,
+                             sd.nat <= kNarrowMaxAtoms ? (int32_t)((uint32_t)r[u].j | code << 26) : r[u].j};
+            L.t[idx] = t;
+        }
+    }
+    if (tid < T.n) {   // centre of run tid, from the brick's origin
+        int ix, iy, iz, w;
+        tile_run(B, T, tid, ix, iy, iz, w);
+        const double f0 = (B.b0[0] - 1 + ix + 0.5 * w) / sd.n[0], f1 = (B.b0[1] - 0.5 + iy) / sd.n[1],
+                     f2 = (B.b0[2] - 0.5 + iz) / sd.n[2];
+        int32_t tx, ty, tz;
+        unpack_wind(to + kPackZero, tx, ty, tz);
+        for (int k = 0; k < 3; ++k)
+            L.ctr[tid][k] = (float)(((Csh[3 * k] * (f0 - tx) + Csh[3 * k + 1] * (f1 - ty)) +
+                                     Csh[3 * k + 2] * (f2 - tz)) - (k == 0 ? ox : k == 1 ? oy : oz));
+    }
+    if (bad) L.flag = 1;
+    __syncthreads();
+    return L.flag == 0;
+}
+
+// The 64-bit test of home atom hl (LDS index) against candidate li: -1 for
+// a hit, 1 otherwise.  A candidate more than one cell along x from the home
+// atom (a run of two cells shares its list) is none of the reference's.
+// Called for the few values the filter cannot decide, out of line and one
+// component at a time: the registers it uses are lost to the pass around it.
+template <int BT>
+__device__ __attribute__((noinline)) float tile_exact(const Rec *rec, const TileLDS<BT> *L, const double *Csh, double rc2,
+                                                      int hd0, int hl, int li)
+{
+    if (li == BrickShape<BT>::cap) return 1.0f;
+    const int oc = L->owner[li], oh = L->owner[hl];
+    if ((unsigned)(oc % hd0 - oh % hd0 + 1) > 2u) return 1.0f;
+    const double *c = &rec[L->hstart[oc] + (li - L->hoff[oc])].x, *h = &rec[L->hstart[oh] + (hl - L->hoff[oh])].x;
+    const uint32_t t = L->t[li] - L->t[hl] + kPackZero;   // pack(S)
+    double r2 = 0.0;
+#pragma unroll 1
+    for (int k = 0; k < 3; ++k) {
+        // R = xj - xi + C' * S ; r^2 = dot(R, R)  (gpu_kernels.jl:89-92)
+        int32_t Sx, Sy, Sz;
+        unpack_wind(t, Sx, Sy, Sz);
+        const double *C = Csh + 3 * k;
+        const double R = (c[k] - h[k]) + ((C[0] * (double)Sx + C[1] * (double)Sy) + C[2] * (double)Sz);
+        r2 = k == 0 ? R * R : r2 + R * R;
+    }
+    return r2 < rc2 ? -1.0f : 1.0f;
+}
+
+// What a pass over a run's candidates reads: NCH chunks, one candidate per
+// lane (b*: position from the run's centre, bq: half its square, ent: low word
+// of the slot entry, ct: the high word for t'_i = 0, li: LDS index).
+struct TileCands {
+    float bx[kTileChunks], by[kTileChunks], bz[kTileChunks], bq[kTileChunks];
+    int ent[kTileChunks], li[kTileChunks];
+    uint32_t ct[kTileChunks];
+};
+
+// ... and its home atoms, one per lane: minus the position from the run's
+// centre, (|p|^2 - rc^2) / 2, the buffer over the slot row (address and entry
+// size), t', and the bytes filled of the row.
+struct TileHomes {
+    float nx, ny, nz, ai;
+    uint64_t row;
+    uint32_t t;
+    int32_t fill;
+};
+
+__device__ __forceinline__ float readlane_f32(float v, int l)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
+
+// Home atoms a0 .. a1 - 1 against NCH chunks.  D = bq + ai - p_i . p_j is half
+// of r^2 - rc^2.  G: the chunk that holds the home atoms' own candidates
+// (kpass + a; -1: none does).
+template <int BT, int NCH, bool NARROW, int G>
+__device__ __forceinline__ void tile_rows(const Rec *rec, const TileLDS<BT> &L, const double *Csh, double rc2, int hd0,
+                                          float tol, const TileCands &C, int hb, int a0, int a1, int kpass, TileHomes &H)
+{
+    for (int a = a0; a < a1; ++a) {
+        const float sx = readlane_f32(H.nx, a), sy = readlane_f32(H.ny, a), sz = readlane_f32(H.nz, a),
+                    sa = readlane_f32(H.ai, a);
+        float D[NCH];
+        float mn = kFar32;
+#pragma unroll
+        for (int g = 0; g < NCH; ++g)
+            D[g] = __builtin_fmaf(sz, C.bz[g], __builtin_fmaf(sy, C.by[g], __builtin_fmaf(sx, C.bx[g], C.bq[g] + sa)));
+#pragma unroll
+        for (int g = 0; g + 1 < NCH; g += 2)
+            mn = __builtin_fminf(__builtin_fminf(mn, __builtin_fabsf(D[g])), __builtin_fabsf(D[g + 1]));
+        if (NCH & 1) mn = __builtin_fminf(mn, __builtin_fabsf(D[NCH - 1]));
+        // a value within the filter's error of zero: the 64-bit test
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(mn < tol) != 0, 0)) {
+#pragma unroll
+            for (int g = 0; g < NCH; ++g)
+                if (__builtin_amdgcn_ballot_w64(__builtin_fabsf(D[g]) < tol) != 0)
+                    D[g] = tile_exact<BT>(rec, &L, Csh, rc2, hd0, hb + a, C.li[g]);
+        }
+        int32_t so = __builtin_amdgcn_readlane(H.fill, a);
+        const v4u rs = {(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)H.row, a),
+                        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(H.row >> 32), a), (uint32_t)kWave,
+                        (uint32_t)kRawBufferWord3};
+        const uint32_t dt = NARROW ? 0u : (uint32_t)__builtin_amdgcn_readlane((int)H.t, a);
+#pragma unroll
+        for (int g = 0; g < NCH; ++g) {
+            uint64_t m = __builtin_amdgcn_ballot_w64(D[g] < 0.0f);
+            if (g == G) m &= ~(1ull << ((kpass + a) & (kWave - 1)));   // j == i, s == 0 is no pair
+            emit_chunk<NARROW>(rs, m, so, (uint32_t)C.ent[g], NARROW ? 0u : C.ct[g] - dt);
+        }
+        H.fill = write_lane(so, a, H.fill);
+    }
+}
+
+// The run's nh home atoms against NCH chunks: their own candidates are
+// consecutive, in one chunk or across two.
+template <int BT, int NCH, bool NARROW>
+__device__ __forceinline__ void tile_pass(const Rec *rec, const TileLDS<BT> &L, const double *Csh, double rc2, int hd0,
+                                          float tol, const TileCands &C, int hb, int nh, int kpass, TileHomes &H)
+{
+    int a = 0;
+    while (a < nh) {
+        const int g = (kpass + a) >> 6;   // negative: before this pass
+        const int e = g >= NCH ? nh : min(nh, g < 0 ? -kpass : (g + 1) * kWave - kpass);
+        if (NCH > 0 && g == 0) tile_rows<BT, NCH, NARROW, 0>(rec, L, Csh, rc2, hd0, tol, C, hb, a, e, kpass, H);
+        else if (NCH > 1 && g == 1) tile_rows<BT, NCH, NARROW, 1>(rec, L, Csh, rc2, hd0, tol, C, hb, a, e, kpass, H);
+        else if (NCH > 2 && g == 2) tile_rows<BT, NCH, NARROW, 2>(rec, L, Csh, rc2, hd0, tol, C, hb, a, e, kpass, H);
+        else if (NCH > 3 && g == 3) tile_rows<BT, NCH, NARROW, 3>(rec, L, Csh, rc2, hd0, tol, C, hb, a, e, kpass, H);
+        else tile_rows<BT, NCH, NARROW, -1>(rec, L, Csh, rc2, hd0, tol, C, hb, a, e, kpass, H);
+        a = e;
+    }
+}
+
+// Brick pass of the count (no R, no 16-byte entries): the distance tests run
+// on 32-bit positions, exact to a known bound (filter_bounds), and every value
+// within that bound of the cutoff is decided again by the 64-bit test, so the
+// pairs are those of the 64-bit kernel.
+//
+// Bound by instruction issue: a home atom against four chunks is 39 vector and
+// 30 scalar instructions; at 1M atoms the vector unit issues for 73% of the
+// time (61.5 instructions per home atom, 45 scalar; 73.9 and 64 in the 64-bit
+// kernel, whose 32-byte atoms also held a CU to four bricks, now five).  The
+// tests as matrix instructions (4 x 4 x 1 in 32 bits, 16 blocks: four home atoms
+// by 64 candidates) took 12 cycles of the wave's SIMD each, more than the
+// vector instructions they replaced: 157 against 151 us.  Kernel times before
+// and after (MI355X): 96-atom crystal 66 / 12 us, 1k atoms 17.2 / 7.8, 100k 33 /
+// 28, 1M 193 / 151, 1M FCC slab 368 / 234 (there most bricks of atoms outside
+// the cell wrote 8-byte rows; windings now count from the brick's own).
+//
+// A run of two home cells shares one candidate list, their nine rows of four
+// cells: a pair of cells two apart along x that a home cell's own 27 cells
+// would not hold is at least one cell height (>= rc) apart, so it is no hit
+// beyond the filter's error, and within it tile_exact leaves it out.
+template <int BT>
+__global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(5))) void tile_kernel(
+    const SysDev *__restrict__ sys, const int32_t *__restrict__ sys_cell_base, const int32_t *__restrict__ sys_brick_base,
+    int nsys, int copies, int32_t M, int64_t nat, const int32_t *__restrict__ cell_start,
+    const Rec *__restrict__ rec, const int32_t *__restrict__ wbig, int32_t *__restrict__ pair_count,
+    void *__restrict__ slots, int32_t cap, Status *__restrict__ status)
+{
+    __shared__ TileLDS<BT> L;
+    __shared__ double Csh[9];
+    const PairsArgs A{sys, sys_cell_base, nsys, M, nat, cell_start, rec, wbig};
+    Brick B;
+    const int copy = copies == 1 ? 0 : (int)(blockIdx.x % (unsigned)copies);
+    brick_locate(A, sys_brick_base, copies == 1 ? (int)blockIdx.x : (int)(blockIdx.x / (unsigned)copies),
+                 BrickShape<BT>::halo, B);
+    const TileRuns T = tile_runs(B);
+    if (threadIdx.x < 9) Csh[threadIdx.x] = B.sd->C[threadIdx.x];   // visible after tile_load's first barrier
+    const bool lds = B.fast && tile_load(A, B, T, L, Csh);
+    const int lane = lane_id();
+    const int wv = sgpr((int)(threadIdx.x >> 6));
+    if (!lds) {
+        const SlotArgs O{slots, nullptr, cap, status};
+        for (int hc = copy + copies * wv; hc < B.nhome; hc += copies * BrickShape<BT>::waves)
+            count_cell<false, false>(A, *B.sd, brick_cell_id(B, hc), pair_count, O);
+        return;
+    }
+    const SysDev &sd = *B.sd;
+    const bool narrow = sgpr(L.row8) == 0;   // the brick writes 4-byte slot entries
+    // L.a[].j holds j | S code << 26 whenever every j fits in 26 bits
+    const uint32_t hjmask = sd.nat <= kNarrowMaxAtoms ? (uint32_t)(kNarrowMaxAtoms - 1) : 0xffffffffu;
+    const uint32_t jmask = narrow ? 0xffffffffu : hjmask;   // entry low word: j | code << 26, or j
+    // halo cell of row lane < 9, (dz, dy) = (lane / 3 - 1, lane % 3 - 1), from the run's own
+    const int roff = lane < 9 ? B.hd[0] * ((lane % 3 - 1) + B.hd[1] * (lane / 3 - 1)) : 0;
+    uint8_t *fl = reinterpret_cast<uint8_t *>(L.rowflag[wv]);
+    // items: the home atoms of a run in 2^split parts, those of the brick
+    // dealt to its copies, then to their waves
+    const int split = sd.split, items = T.n << split;
+    for (int it = copy + copies * wv; it < items; it = copy + copies * take_next(&L.next_item)) {
+        const int rn = it >> split, part = it & ((1 << split) - 1);
+        int ix, iy, iz, w;
+        tile_run(B, T, rn, ix, iy, iz, w);
+        const int hc = ix + B.hd[0] * ((iy + 1) + B.hd[1] * (iz + 1));   // halo cell before the run's first
+        const int h0 = sgpr(L.hoff[hc + 1]), nha = sgpr(L.hoff[hc + 1 + w]) - h0;
+        if (nha <= 0) continue;
+        const float ox = L.ctr[rn][0], oy = L.ctr[rn][1], oz = L.ctr[rn][2];
+        // candidates: nine rows of w + 2 cells, each contiguous in LDS
+        const int rst = L.hoff[hc + roff];
+        const int len = lane < 9 ? L.hoff[hc + roff + w + 2] - rst : 0;
+        const int incl = row16_incl_scan(len);
+        const int rex = incl - len;
+        const int total = __builtin_amdgcn_readlane(incl, 8);
+        // row 4 is (dz, dy) = (0, 0); the run starts at its second cell
+        const int self0 = __builtin_amdgcn_readlane(rex, 4) + (h0 - __builtin_amdgcn_readlane(rst, 4));
+        // LDS index less candidate index of the non-empty rows, in row order
+        const uint64_t bne = __builtin_amdgcn_ballot_w64(len > 0);
+        const int rq = (int)mbcnt64(bne);
+        if (len > 0) L.rowdl[wv][rq] = rst - rex;
+        const int r1 = nha * (part + 1) >> split;
+        for (int hg = nha * part >> split; hg < r1; hg += kWave) {
+            const int nh = sgpr(min(kWave, r1 - hg));
+            const int hb = h0 + hg;          // LDS index of home atom hg (uniform)
+            const int hl = hb + (lane < nh ? lane : 0);
+            const TAtom h = L.a[hl];
+            const int32_t hj_l = (int32_t)((uint32_t)h.j & hjmask);
+            TileHomes H;
+            H.nx = ox - h.x;
+            H.ny = oy - h.y;
+            H.nz = oz - h.z;
+            const float hq = 0.5f * __builtin_fmaf(H.nz, H.nz, __builtin_fmaf(H.ny, H.ny, H.nx * H.nx));
+            H.ai = hq - sd.rc2half;
+            H.row = (reinterpret_cast<uint64_t>(slots) + 8ull * (uint64_t)slot_row(sd.atom_base + hj_l, cap)) |
+                    (uint64_t)(narrow ? 4 : 8) << 48;
+            H.t = L.t[hl];
+            H.fill = 0;
+            // a home atom further from the run's centre than the bounds assume
+            // (clamped into its cell): 64-bit tests for all
+            const float tol = __builtin_amdgcn_ballot_w64(!(hq <= sd.h2half)) != 0 ? kFar32 * kFar32 : sd.tol;
+            for (int k0 = 0; k0 < total; k0 += kTileCands) {
+                const int nch = sgpr(min(kTileChunks, (total - k0 + kWave - 1) / kWave));
+                // marks where a non-empty row other than the first starts (see row_map)
+                L.rowflag[wv][lane] = 0u;
+                const int p = rex - k0;
+                if (len > 0 && rq > 0 && p > 0 && p < kTileCands) fl[p] = 1;
+                int acc = k0 == 0 ? 0 : (int)__popcll(bne & __builtin_amdgcn_ballot_w64(rq > 0) & __builtin_amdgcn_ballot_w64(p <= 0));
+                TileCands C;
+#pragma unroll
+                for (int g = 0; g < kTileChunks; ++g) {
+                    const uint64_t bm = __builtin_amdgcn_ballot_w64(fl[g * kWave + lane] != 0);
+                    const int q = acc + (int)(bm & 1u) + (int)mbcnt64(bm >> 1);
+                    acc += (int)__popcll(bm);
+                    const int k = k0 + g * kWave + lane;
+                    C.li[g] = k < total ? k + L.rowdl[wv][q] : BrickShape<BT>::cap;   // else the far sentinel
+                    const TAtom c = L.a[C.li[g]];
+                    C.bx[g] = c.x - ox;
+                    C.by[g] = c.y - oy;
+                    C.bz[g] = c.z - oz;
+                    C.bq[g] = 0.5f * __builtin_fmaf(C.bz[g], C.bz[g], __builtin_fmaf(C.by[g], C.by[g], C.bx[g] * C.bx[g]));
+                    C.ent[g] = (int)((uint32_t)c.j & jmask);
+                    if (!narrow) C.ct[g] = L.t[C.li[g]] + kPackZero;
+                }
+                const int kp = self0 + hg - k0;   // home atom hg + a is candidate kp + a of this pass
+#define NLH_TILE_PASS(N, W) tile_pass<BT, N, W>(rec, L, Csh, sd.rc2, B.hd[0], tol, C, hb, nh, kp, H)
+                if (narrow) {
+                    if (nch == 4) NLH_TILE_PASS(4, true);
+                    else if (nch == 3) NLH_TILE_PASS(3, true);
+                    else NLH_TILE_PASS(2, true);
+                } else {
+                    if (nch == 4) NLH_TILE_PASS(4, false);
+                    else if (nch == 3) NLH_TILE_PASS(3, false);
+                    else NLH_TILE_PASS(2, false);
+                }
+#undef NLH_TILE_PASS
+            }
+            if (lane < nh) pair_count[sd.atom_base + hj_l] = narrow ? H.fill >> 2 : (H.fill >> 3) | kRow8Bit;
         }
     }
 }
@@ -1561,7 +1947,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
                         const uint32_t lo = narrow ? ((uint32_t)c.j | code << 26) : (uint32_t)c.j;
                         ent[g] = (uint64_t)lo | ((uint64_t)t << 32);
                     }
-                    pass_home_atoms<WANT_R, false, false>(narrow, false, nch, cx, cy, cz, ent, L.a + hb, nh, ht_l, hj_l,
+                    pass_home_atoms<WANT_R, false>(narrow, nch, cx, cy, cz, ent, L.a + hb, nh, ht_l, hj_l,
                                                    self0 + hg - k0, sd.C, sd.rc2, sd.atom_base, A.slots, A.slotsR,
                                                    A.cap, A.status, cnt_l);
                 }
@@ -1833,6 +2219,18 @@ static void count_launch(const PipelineBufs &b, hipStream_t st)
                            b.pair_count, b.slots, b.slotsR, b.slot_cap, b.status);
 }
 
+static void tile_launch(const PipelineBufs &b, hipStream_t st)
+{
+    if (b.count_block == 256)
+        hipLaunchKernelGGL(tile_kernel<256>, dim3((unsigned)(b.nbricks * b.brick_copies)), dim3(256), 0, st, b.sys,
+                           b.sys_cell_base, b.sys_brick_base, b.nsys, b.brick_copies, b.M, b.nat, b.cell_start, b.rec, b.wbig, b.pair_count, b.slots,
+                           b.slot_cap, b.status);
+    else
+        hipLaunchKernelGGL(tile_kernel<512>, dim3((unsigned)(b.nbricks * b.brick_copies)), dim3(512), 0, st, b.sys,
+                           b.sys_cell_base, b.sys_brick_base, b.nsys, b.brick_copies, b.M, b.nat, b.cell_start, b.rec, b.wbig, b.pair_count, b.slots,
+                           b.slot_cap, b.status);
+}
+
 void launch_count(const PipelineBufs &b, bool want_R, bool wide, hipStream_t st)
 {
     if (b.nunits > 0) {   // cell list, counts and slot rows of every unit of small systems
@@ -1845,7 +2243,7 @@ void launch_count(const PipelineBufs &b, bool want_R, bool wide, hipStream_t st)
         else count_launch<true, false>(b, st);
     } else {
         if (wide) count_launch<false, true>(b, st);
-        else count_launch<false, false>(b, st);
+        else tile_launch(b, st);
     }
 }
 

@@ -1,5 +1,5 @@
 """Size edges of the launch paths, each against the oracle bit for bit:
-lazy range queries, scans.
+lazy range queries, scans, the pair search.
 """
 import numpy as np
 import pytest
@@ -48,3 +48,66 @@ def test_pair_scan_forms(n, rc):
     nl = nlhip.neighbour_list(s.X, rc, s.cell, s.pbc)
     assert np.array_equal(nl.first, ref.first)
     assert np.array_equal(nl.i, ref.i) and np.array_equal(nl.j, ref.j) and np.array_equal(nl.S, ref.S)
+
+
+def _check(X, rc, cell, pbc, int_type=np.int32):
+    bits = 32 if int_type == np.int32 else 64
+    ref = oracle.neighbour_list(X, rc, cell, pbc, ti_bits=bits, nthreads=8)
+    nl = nlhip.neighbour_list(X, rc, cell, pbc, int_type=int_type)
+    assert np.array_equal(nl.first, ref.first)
+    assert np.array_equal(nl.i, ref.i) and np.array_equal(nl.j, ref.j) and np.array_equal(nl.S, ref.S)
+
+
+@pytest.mark.parametrize("reps", [(2, 2, 2), (3, 5, 4), (12, 11, 13)])
+@pytest.mark.parametrize("shell", [0.5, 1.0, 1.5, 2.0])
+@pytest.mark.parametrize("eps", [0.0, 3e-16, -3e-16, 1e-7, -1e-7])
+def test_cutoff_on_a_shell(reps, shell, eps):
+    """A perfect crystal with the cutoff at a neighbour distance, to the last
+    bit and to about the 32-bit filter's error: every pair of that shell is
+    decided by the 64-bit test."""
+    X, cell = workloads.fcc(3.61, reps)
+    rc = 3.61 * np.sqrt(shell) * (1.0 + eps)
+    print(f"shell {reps} {shell} {eps}", flush=True)
+    _check(X + 0.1, rc, cell, (True, True, True))
+
+
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 700, 3000, 30000])
+@pytest.mark.parametrize("spread", [0, 1, 120, 140])
+@pytest.mark.parametrize("pbc", [(True, True, True), (True, False, True), (False, False, False)])
+def test_unwrapped_positions(n, spread, pbc):
+    """Atoms each moved by its own lattice vector (up to `spread` cells, past
+    the packed range of a brick at 140) or, along open axes, far outside the
+    grid: 4-byte rows, 8-byte rows and the per-wave path."""
+    s = workloads.random_in_cell(n, np.array([[1.0, 0.1, 0.0], [0.2, 1.1, 0.1], [0.0, 0.1, 0.9]]) * (n / 0.06) ** (1 / 3),
+                                 seed=n, cutoff=4.0, pbc=pbc)
+    rng = np.random.default_rng(n + spread)
+    X = s.X + rng.integers(-spread, spread + 1, (n, 3)).astype(float) @ s.cell * (rng.random((n, 1)) < 0.3)
+    print(f"unwrapped {n} {spread} {pbc}", flush=True)
+    _check(X, 4.0, s.cell, pbc)
+
+
+@pytest.mark.parametrize("ncells", [(1, 1, 1), (2, 1, 3), (3, 2, 1), (2, 2, 2), (4, 3, 5), (5, 5, 1), (7, 1, 2)])
+@pytest.mark.parametrize("per_cell", [1, 6, 24, 70])
+def test_small_grids_and_dense_cells(ncells, per_cell):
+    """Grids of a few cells, each its own neighbour along the short axes, from
+    one atom per cell to more than a wave of home atoms and several passes of
+    candidates; the search split over the waves and over several workgroups."""
+    rc = 3.0
+    n = max(1, per_cell * int(np.prod(ncells)))
+    cell = np.diag([(k + 0.2) * rc for k in ncells])
+    s = workloads.random_in_cell(n, cell, seed=n, cutoff=rc)
+    for pbc in [(True, True, True), (False, True, False)]:
+        print(f"grid {ncells} {per_cell} {pbc}", flush=True)
+        _check(s.X, rc, cell, pbc, np.int64)
+
+
+@pytest.mark.parametrize("n", [40000, 1000000])
+def test_rows_that_overflow(n):
+    """A dense cluster whose atoms outgrow the estimated slot rows, among them
+    the last rows of the buffer (the build grows them and counts again)."""
+    s = workloads.random_cubic(n, density=0.02, seed=3, cutoff=5.0)
+    X = s.X.copy()
+    rng = np.random.default_rng(1)
+    X[-40:] = X[100] + 0.9 * rng.random((40, 3))
+    X[5000:5040] = X[4000] + 0.9 * rng.random((40, 3))
+    _check(X, 5.0, s.cell, s.pbc)
