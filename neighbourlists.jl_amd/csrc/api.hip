@@ -124,7 +124,7 @@ struct nlh_handle {
     int device = 0;
     hipStream_t stream = nullptr;
     DevBuf X, tables, key, slot, cell_count, bmat, recb, cell_start, tmp, rec, wbig, perm, cell_id,
-        cell_offsets, pair_count, slots, slotsR, pair_off, tiles, lookback, sysmap, sys_pair_base, first, i, j, S, R, status, Xsorted, nb_j, nb_R,
+        cell_offsets, pair_count, slots, Xr, pair_off, tiles, lookback, sysmap, sys_pair_base, first, i, j, S, R, status, Xsorted, nb_j, nb_R,
         nb_S, nb_count, nr_count, nr_off, nr_j, nr_R, nr_S;
     // lazy queries over a range of atoms (nlh_neighbours_range): the last
     // range's results stay on the device, keyed by the build they came from
@@ -237,7 +237,7 @@ struct nlh_handle {
         b.cell_offsets_out = cell_offsets.p;
         b.pair_count = pair_count.as<int32_t>();
         b.slots = slots.p;
-        b.slotsR = slotsR.as<double>();
+        b.Xr = X_dev == X.as<double>() ? X.as<double>() : Xr.as<double>();
         b.slot_cap = slot_cap;
         b.pair_off = pair_off.as<int64_t>();
         b.tile_atom = tiles.as<int32_t>();
@@ -912,12 +912,11 @@ int32_t estimate_slot_cap(const nlh_handle *h)
     return round_slot_cap(c);
 }
 
-void ensure_slots(nlh_handle *h, int32_t cap, bool want_R)
+void ensure_slots(nlh_handle *h, int32_t cap)
 {
     h->slot_cap = std::max(h->slot_cap, cap);
     const size_t n1 = (size_t)std::max<int64_t>(h->nat, 1) * (size_t)h->slot_cap;
     h->slots.ensure(h->stream, n1 * (h->wide ? 16 : 8) + nlh::kSlotSlack);
-    if (want_R) h->slotsR.ensure(h->stream, n1 * 24);
 }
 
 void ensure_pair_outputs(nlh_handle *h, int64_t cap, bool want_R)
@@ -927,6 +926,10 @@ void ensure_pair_outputs(nlh_handle *h, int64_t cap, bool want_R)
     h->j.ensure(h->stream, (size_t)cap * ti);
     h->S.ensure(h->stream, (size_t)cap * 3 * ti);
     if (want_R) h->R.ensure(h->stream, (size_t)cap * 24);
+    // positions in the caller's memory are copied for the fill, which may run
+    // after the call
+    if (want_R && h->X_dev != h->X.as<double>())
+        h->Xr.ensure(h->stream, (size_t)std::max<int64_t>(h->nat, 1) * 24);
     int64_t c = (int64_t)(h->i.cap / ti);
     c = std::min<int64_t>(c, (int64_t)(h->j.cap / ti));
     c = std::min<int64_t>(c, (int64_t)(h->S.cap / (3 * ti)));
@@ -1024,7 +1027,7 @@ void check_positions(nlh_handle *h)
 void finish_pairs(nlh_handle *h, bool want_R);
 
 // Host-side bounds check of everything the count and fill kernels write:
-// slots of slot_cap entries per atom (and their R), pair outputs of
+// slots of slot_cap entries per atom, pair outputs of
 // pair_capacity entries (the fill skips itself beyond that), per-atom
 // counts and offsets.
 void check_pair_buffers(const nlh_handle *h, bool want_R)
@@ -1037,7 +1040,8 @@ void check_pair_buffers(const nlh_handle *h, bool want_R)
     ok = ok && h->first.cap >= (n1 + h->nsys) * ti && h->sys_pair_base.cap >= (size_t)(h->nsys + 1) * 8;
     ok = ok && h->i.cap >= cap * ti && h->j.cap >= cap * ti && h->S.cap >= cap * 3 * ti;
     ok = ok && h->tiles.cap >= (cap / nlh::kMinFillPairs + 2) * 8;
-    if (want_R) ok = ok && h->slotsR.p && h->slotsR.cap >= ent * 24 && h->R.p && h->R.cap >= cap * 24;
+    if (want_R)
+        ok = ok && h->R.p && h->R.cap >= cap * 24 && (h->X_dev == h->X.as<double>() ? h->X : h->Xr).cap >= n1 * 24;
     if (!ok) throw Error(NLH_EDEVICE, "internal: pair-stage buffers are smaller than the launch needs");
 }
 
@@ -1066,7 +1070,7 @@ void materialize(nlh_handle *h, uint32_t flags)
         return;
     }
     ensure_pair_outputs(h, std::max(h->pair_capacity, estimate_pairs(h)), want_R);
-    ensure_slots(h, std::max(h->slot_cap, estimate_slot_cap(h)), want_R);
+    ensure_slots(h, std::max(h->slot_cap, estimate_slot_cap(h)));
     check_pair_buffers(h, want_R);
     nlh::PipelineBufs b = h->bufs();
     mark(h, 1);
@@ -1099,7 +1103,7 @@ void materialize(nlh_handle *h, uint32_t flags)
         if (st.wide) h->wide = true;
         ensure_pair_outputs(h, std::max<int64_t>(st.npairs, 1), want_R);
         h->slots.release(h->stream);
-        ensure_slots(h, round_slot_cap(std::max(st.max_count, 1)), want_R);
+        ensure_slots(h, round_slot_cap(std::max(st.max_count, 1)));
         check_pair_buffers(h, want_R);
         b = h->bufs();
         nlh::launch_count(b, want_R, h->wide, h->stream);
@@ -1181,7 +1185,7 @@ bool rebuild_graph(nlh_handle *h, bool want_R)
     // and not at the build that sized them)
     ensure_pair_buffers(h);
     ensure_pair_outputs(h, std::max(h->pair_capacity, estimate_pairs(h)), want_R);
-    ensure_slots(h, std::max(h->slot_cap, estimate_slot_cap(h)), want_R);
+    ensure_slots(h, std::max(h->slot_cap, estimate_slot_cap(h)));
     check_pair_buffers(h, want_R);
     const nlh::PipelineBufs b = h->bufs();
     // the slot-entry width is baked into the captured count and fill: a build
@@ -1349,7 +1353,7 @@ void neighbours_range(nlh_handle *h, int32_t sys, int64_t i_first, int64_t n)
 // ---------------------------------------------------------------------------
 
 constexpr size_t kScratchBytes = (size_t)128 << 20;   // 128 MiB per device
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kScratchBytes + nlh::kSlotSlack];
 
 namespace {
 
@@ -1444,12 +1448,16 @@ size_t carve_noalloc(char *base, const NoAllocPlan &P, int ti, int32_t cap, bool
     b.tile_atom = c.take<int32_t>((size_t)b.tile_cap * 8);
     b.sys_pair_base = c.take<int64_t>(16);
     // the tail: slot rows (the bucketed sort's (cell, index) scratch lives
-    // at their start until the count pass rewrites them), then their R
+    // at their start until the count pass rewrites them); the array's
+    // last kSlotSlack bytes, beyond the limit, take what overflows them.  A
+    // build with R counts 24 more bytes per entry against the limit, whose
+    // atom counts are part of the interface.
     const size_t rows = n1 * (size_t)cap;
-    b.slots = c.take<void>(std::max(rows * (wide ? 16 : 8) + nlh::kSlotSlack, n1 * nlh::kBucketBytes));
+    b.slots = c.take<void>(std::max(rows * (wide ? 16 : 8), n1 * nlh::kBucketBytes));
     b.bke = reinterpret_cast<int2 *>(b.slots);
     b.slot_cap = cap;
-    b.slotsR = want_R ? c.take<double>(rows * 24) : nullptr;
+    if (want_R) c.take<void>(rows * 24);
+    b.Xr = const_cast<double *>(X);   // the call ends after its fill
     b.first_out = first_out;
     b.i_out = i_out;
     b.j_out = j_out;
@@ -1691,7 +1699,7 @@ int nlh_destroy(nlh_handle *h)
         });
         DevBuf *bufs[] = {&h->X,        &h->tables,    &h->key,    &h->slot,
                           &h->cell_count, &h->bmat,     &h->recb,       &h->cell_start, &h->tmp,    &h->rec,
-                          &h->wbig,     &h->perm,       &h->cell_id,  &h->cell_offsets, &h->pair_count, &h->slots, &h->slotsR, &h->pair_off,   &h->tiles, &h->lookback, &h->sysmap,
+                          &h->wbig,     &h->perm,       &h->cell_id,  &h->cell_offsets, &h->pair_count, &h->slots, &h->Xr, &h->pair_off,   &h->tiles, &h->lookback, &h->sysmap,
                           &h->sys_pair_base, &h->first, &h->i,          &h->j,            &h->S,      &h->R,
                           &h->status,   &h->Xsorted,   &h->nb_j,       &h->nb_R,         &h->nb_S,   &h->nb_count,
                           &h->nr_count, &h->nr_off,    &h->nr_j,       &h->nr_R,         &h->nr_S};

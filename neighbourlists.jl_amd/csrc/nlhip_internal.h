@@ -270,8 +270,8 @@ struct PipelineBufs {
     void *cell_offsets_out;     // M + nsys, TI, 1-based per system
     // pairs
     int32_t *pair_count;
+    double *Xr;                 // 3 * nat (R requested): positions the fill reads; X itself, or a copy out of rec
     void *slots;                // nat * slot_cap slot entries
-    double *slotsR;             // 3 * nat * slot_cap (R requested)
     int32_t slot_cap;
     int64_t *pair_off;          // nat + 1
     int32_t *tile_atom;         // 2 tile_cap: atom owning pair t * fill_pairs, its pairs before it
@@ -340,6 +340,5 @@ constexpr int kUnitCells = 2048;      // cells of one unit at most
 constexpr int kUnitSystems = 256;     // systems of one unit at most
 constexpr int kUnitMaxReach = 3;      // neighbour-cell reach per axis at most
 constexpr int kUnitMaxAxisCells = 256;   // cells per axis of one system at most
-void launch_small(const PipelineBufs &b, bool want_R, hipStream_t st);
 
 }  // namespace nlh

@@ -127,7 +127,6 @@ struct SlotEntry<true> {
 
 struct SlotArgs {
     void *__restrict__ slots;
-    double *__restrict__ slotsR;     // 3 doubles per entry (NLH_WANT_R)
     int32_t cap;
     Status *__restrict__ status;
 };
@@ -136,10 +135,10 @@ struct SlotArgs {
 // sbase = sorted index of the home atom * cap; ca = its running count
 // (wave-uniform).  t_pk: this lane's packed s - w_j (valid when tfits);
 // (tx, ty, tz) the same unpacked; w_i the home atom's winding, wzero when 0.
-template <bool WANT_R, bool WIDE>
+template <bool WIDE>
 __device__ __forceinline__ void emit_hits(const SlotArgs &O, uint64_t mask, int64_t sbase, int32_t &ca, int32_t cj,
                                           uint32_t t_pk, int32_t tx, int32_t ty, int32_t tz, int32_t wix, int32_t wiy,
-                                          int32_t wiz, bool wzero, double Rx, double Ry, double Rz)
+                                          int32_t wiz, bool wzero)
 {
     if (mask == 0) return;   // wave-uniform
     const int lane = lane_id();
@@ -153,12 +152,6 @@ __device__ __forceinline__ void emit_hits(const SlotArgs &O, uint64_t mask, int6
             const uint32_t spk = wzero ? t_pk : pack_wind(tx + wix, ty + wiy, tz + wiz);
             if (spk & kWindBig) O.status->wide = 1;
             reinterpret_cast<uint64_t *>(O.slots)[sidx] = (uint64_t)(uint32_t)cj | ((uint64_t)spk << 32);
-        }
-        if (WANT_R) {
-            double *R = O.slotsR + 3 * sidx;
-            R[0] = Rx;
-            R[1] = Ry;
-            R[2] = Rz;
         }
     }
     ca += __popcll(mask);
@@ -279,7 +272,7 @@ __device__ __forceinline__ Cand load_candidate(const PairsArgs &A, int k, int to
 // Per-wave count of one home cell from global memory: test every (home
 // atom, chunk) and append hits to the slots (the brick path's fallback, and
 // the path for neighbour reach beyond one cell).
-template <bool WANT_R, bool WIDE>
+template <bool WIDE>
 __device__ __forceinline__ void count_cell(const PairsArgs &A, const SysDev &sd, int cell, int32_t *__restrict__ pair_count,
                                         const SlotArgs &O)
 {
@@ -343,8 +336,8 @@ __device__ __forceinline__ void count_cell(const PairsArgs &A, const SysDev &sd,
                             const double Rz = (c[g].z - h.z) + cz[g];
                             const double r2 = (Rx * Rx + Ry * Ry) + Rz * Rz;
                             const uint64_t mask = __ballot((r2 < rc2) & (key[g] != h.j));
-                            emit_hits<WANT_R, WIDE>(O, mask, sbase, ca, c[g].j, tpk[g], c[g].tx, c[g].ty, c[g].tz, wix,
-                                                    wiy, wiz, wzero, Rx, Ry, Rz);
+                            emit_hits<WIDE>(O, mask, sbase, ca, c[g].j, tpk[g], c[g].tx, c[g].ty, c[g].tz, wix, wiy, wiz,
+                                            wzero);
                         }
                     }
                     cnt_lane = lane == a ? ca : cnt_lane;
@@ -561,7 +554,6 @@ struct BrickLDS {
     uint16_t owner[Sh::cap];        // halo cell of each LDS atom slot (while loading)
     int32_t next_cell;              // the next home cell a wave takes
     int32_t total, flag;
-    int32_t row8;                   // some shift needs 8-byte slot entries
 };
 
 constexpr uint32_t kHomeCell = 1u << 30;   // halo-table mark of the brick's own cells
@@ -625,7 +617,6 @@ __device__ bool brick_load(const PairsArgs &A, const Brick &B, BrickLDS<BT> &L)
         L.total = (int32_t)tot;
         L.next_cell = Sh::waves;
         L.flag = 0;
-        L.row8 = sd.nat > kNarrowMaxAtoms ? 1 : 0;
         L.a[Sh::cap].x = L.a[Sh::cap].y = L.a[Sh::cap].z = kFar;
         L.a[Sh::cap].j = 0;
         L.a[Sh::cap].t = kPackZero;
@@ -658,23 +649,13 @@ __device__ bool brick_load(const PairsArgs &A, const Brick &B, BrickLDS<BT> &L)
             int32_t wx, wy, wz, sx, sy, sz;
             rec_winding(r[u], A.wbig, pg[u], wx, wy, wz);
             unpack_wind(hs[u] & ~kHomeCell, sx, sy, sz);
-            const int32_t tx = sx - wx, ty = sy - wy, tz = sz - wz;
-            const uint32_t t = pack_wind(tx, ty, tz);
+            const uint32_t t = pack_wind(sx - wx, sy - wy, sz - wz);
             if (t & kWindBig) L.flag = 1;
-            // 4-byte slot entries need every S = t + w_i within [-1, 1]^3: home
-            // atoms inside the cell (w_i = 0) and halo atoms with |t_k| <= 1
-            const bool ok = (hs[u] & kHomeCell) ? (tx | ty | tz) == 0
-                                                : ((unsigned)(tx + 1) <= 2u && (unsigned)(ty + 1) <= 2u &&
-                                                   (unsigned)(tz + 1) <= 2u);
-            if (!ok) L.row8 = 1;
-            // the 10-bit biased fields of t carry the S codes of a 4-byte entry in
-            // their low 2 bits (meaningful only when the brick stays 4-byte)
-            const uint32_t code = (t & 3u) | ((t >> 8) & 12u) | ((t >> 16) & 48u);
             LAtom la;
             la.x = r[u].x;
             la.y = r[u].y;
             la.z = r[u].z;
-            la.j = sd.nat <= kNarrowMaxAtoms ? (int32_t)((uint32_t)r[u].j | code << 26) : r[u].j;
+            la.j = r[u].j;
             la.t = t;
             L.a[idx] = la;
         }
@@ -803,13 +784,12 @@ constexpr uint32_t kDropOffset = 0x40800000u;
 static_assert(__builtin_bit_cast(uint32_t, 4.0f) == kDropOffset, "the select below writes the offset as 4.0");
 constexpr int32_t kRawBufferWord3 = 0x00020000; // raw 32-bit buffer access (GFX9 family)
 
-template <bool NARROW, bool WZERO, bool WANT_R, bool WIDE>
-__device__ __forceinline__ void emit_row(void *__restrict__ row, double *__restrict__ rrow, uint32_t cap,
-                                         Status *__restrict__ status, uint64_t m, int32_t &ca, uint64_t ent,
-                                         int32_t wix, int32_t wiy, int32_t wiz, double Rx, double Ry, double Rz)
+template <bool NARROW, bool WZERO, bool WIDE>
+__device__ __forceinline__ void emit_row(void *__restrict__ row, uint32_t cap, Status *__restrict__ status, uint64_t m,
+                                         int32_t &ca, uint64_t ent, int32_t wix, int32_t wiy, int32_t wiz)
 {
     const uint32_t n = (uint32_t)__popcll(m);
-    if (NARROW && !WANT_R) {
+    if (NARROW) {
         // every lane stores, each lane without a hit at an offset past the
         // resource's end (a select on the ballot, not an exec-mask region);
         // an empty ballot skips it
@@ -832,10 +812,7 @@ __device__ __forceinline__ void emit_row(void *__restrict__ row, double *__restr
             st &= __builtin_amdgcn_ballot_w64((int32_t)rk < (int32_t)cap - ca);
         const uint32_t r = rk + (uint32_t)ca;
         if (__builtin_amdgcn_inverse_ballot_w64(st)) {
-            if (NARROW) {
-                // j | S code << 26 (w_i = 0 in a 4-byte brick)
-                *reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(row) + (r << 2)) = (uint32_t)ent;
-            } else if (WIDE) {
+            if (WIDE) {
                 int32_t tx, ty, tz;
                 unpack_wind((uint32_t)(ent >> 32), tx, ty, tz);
                 reinterpret_cast<int4 *>(row)[r] = make_int4((int32_t)(uint32_t)ent, tx + wix, ty + wiy, tz + wiz);
@@ -849,25 +826,19 @@ __device__ __forceinline__ void emit_row(void *__restrict__ row, double *__restr
                 if (spk & kWindBig) status->wide = 1;
                 reinterpret_cast<uint64_t *>(row)[r] = (ent & 0xffffffffull) | ((uint64_t)spk << 32);
             }
-            if (WANT_R) {
-                double *Rd = rrow + 3 * r;
-                Rd[0] = Rx;
-                Rd[1] = Ry;
-                Rd[2] = Rz;
-            }
         }
         ca += (int32_t)n;
     }
 }
 
 // One (home atom, chunk) test of the brick pass.  SHIFT: add the candidate's
-// cell shift C' S (left out when every lane's shift is zero and R is not
-// written: r^2 is then the same).  `self` clears the home atom's own
+// cell shift C' S (left out when every lane's shift is zero: r^2 is then the
+// same).  `self` clears the home atom's own
 // (j == i, s == 0) candidate from the ballot when it lies in this chunk.
-template <bool NARROW, bool SHIFT, bool WZERO, bool WANT_R, bool WIDE>
+template <bool NARROW, bool SHIFT, bool WZERO, bool WIDE>
 __device__ __forceinline__ void test_chunk(double cx, double cy, double cz, double sx, double sy, double sz, double hx,
                                            double hy, double hz, double rc2, uint64_t self, void *__restrict__ row,
-                                           double *__restrict__ rrow, uint32_t cap, Status *__restrict__ status,
+                                           uint32_t cap, Status *__restrict__ status,
                                            int32_t &ca, uint64_t ent, int32_t wix, int32_t wiy, int32_t wiz)
 {
     // R = xj - xi + C' * S ; r^2 = dot(R, R)  (gpu_kernels.jl:89-92)
@@ -880,17 +851,16 @@ __device__ __forceinline__ void test_chunk(double cx, double cy, double cz, doub
     const double r2 = (Rx * Rx + Ry * Ry) + Rz * Rz;
     const bool in = r2 < rc2;
     const uint64_t m = __builtin_amdgcn_ballot_w64(in) & self;
-    emit_row<NARROW, WZERO, WANT_R, WIDE>(row, rrow, cap, status, m, ca, ent, wix, wiy, wiz, Rx, Ry, Rz);
+    emit_row<NARROW, WZERO, WIDE>(row, cap, status, m, ca, ent, wix, wiy, wiz);
 }
 
 // All chunks of one home atom.
-template <bool NARROW, bool WZERO, bool WANT_R, bool WIDE>
+template <bool NARROW, bool WZERO, bool WIDE>
 __device__ __forceinline__ void test_home_atom(int nch, const double *cx, const double *cy, const double *cz,
                                                const double *sx, const double *sy, const double *sz, const uint64_t *csh,
                                                const uint64_t *ent, double hx, double hy, double hz, double rc2,
-                                               int ks, void *__restrict__ row, double *__restrict__ rrow, uint32_t cap,
-                                               Status *__restrict__ status, int32_t &ca, int32_t wix, int32_t wiy,
-                                               int32_t wiz)
+                                               int ks, void *__restrict__ row, uint32_t cap, Status *__restrict__ status,
+                                               int32_t &ca, int32_t wix, int32_t wiy, int32_t wiz)
 {
     // _is_self_interaction: j == i with no cell shift is the home atom's own
     // slot in the home cell, candidate ks of this pass: chunk ks >> 6 (none
@@ -901,12 +871,12 @@ __device__ __forceinline__ void test_home_atom(int nch, const double *cx, const 
     for (int g = 0; g < kBrickChunks; ++g) {
         if (g < nch) {
             const uint64_t self = g == gs ? nself : ~0ull;
-            if (WANT_R || csh[g] != 0)
-                test_chunk<NARROW, true, WZERO, WANT_R, WIDE>(cx[g], cy[g], cz[g], sx[g], sy[g], sz[g], hx, hy, hz, rc2,
-                                                              self, row, rrow, cap, status, ca, ent[g], wix, wiy, wiz);
+            if (csh[g] != 0)
+                test_chunk<NARROW, true, WZERO, WIDE>(cx[g], cy[g], cz[g], sx[g], sy[g], sz[g], hx, hy, hz, rc2, self,
+                                                      row, cap, status, ca, ent[g], wix, wiy, wiz);
             else
-                test_chunk<NARROW, false, WZERO, WANT_R, WIDE>(cx[g], cy[g], cz[g], sx[g], sy[g], sz[g], hx, hy, hz, rc2,
-                                                               self, row, rrow, cap, status, ca, ent[g], wix, wiy, wiz);
+                test_chunk<NARROW, false, WZERO, WIDE>(cx[g], cy[g], cz[g], sx[g], sy[g], sz[g], hx, hy, hz, rc2, self,
+                                                       row, cap, status, ca, ent[g], wix, wiy, wiz);
         }
     }
 }
@@ -915,13 +885,12 @@ __device__ __forceinline__ void test_home_atom(int nch, const double *cx, const 
 // same shifts) against the same chunks: both distance tests of a chunk come
 // before both emissions, two independent chains the scheduler interleaves.
 // Atom 1's self candidate follows atom 0's.
-template <bool WANT_R, bool WIDE>
+template <bool WIDE>
 __device__ __forceinline__ void test_home_pair(int nch, const double *cx, const double *cy, const double *cz,
                                                const double *sx, const double *sy, const double *sz, const uint64_t *csh,
                                                const uint64_t *ent, double h0x, double h0y, double h0z, double h1x,
                                                double h1y, double h1z, double rc2, int ks0, void *__restrict__ row0,
-                                               void *__restrict__ row1, double *__restrict__ rrow0,
-                                               double *__restrict__ rrow1, uint32_t cap, Status *__restrict__ status,
+                                               void *__restrict__ row1, uint32_t cap, Status *__restrict__ status,
                                                int32_t &ca0, int32_t &ca1)
 {
     // self candidates (as in test_home_atom): ks0 for atom 0, ks0 + 1 for atom 1
@@ -933,7 +902,7 @@ __device__ __forceinline__ void test_home_pair(int nch, const double *cx, const 
             // R = xj - xi + C' * S ; r^2 = dot(R, R)  (gpu_kernels.jl:89-92)
             double R0x = cx[g] - h0x, R0y = cy[g] - h0y, R0z = cz[g] - h0z;
             double R1x = cx[g] - h1x, R1y = cy[g] - h1y, R1z = cz[g] - h1z;
-            if (WANT_R || csh[g] != 0) {
+            if (csh[g] != 0) {
                 R0x = R0x + sx[g];
                 R0y = R0y + sy[g];
                 R0z = R0z + sz[g];
@@ -945,8 +914,8 @@ __device__ __forceinline__ void test_home_pair(int nch, const double *cx, const 
             const bool in1 = (R1x * R1x + R1y * R1y) + R1z * R1z < rc2;
             const uint64_t m0 = __builtin_amdgcn_ballot_w64(in0) & (g == gs0 ? nself0 : ~0ull);
             const uint64_t m1 = __builtin_amdgcn_ballot_w64(in1) & (g == gs1 ? nself1 : ~0ull);
-            emit_row<true, true, WANT_R, WIDE>(row0, rrow0, cap, status, m0, ca0, ent[g], 0, 0, 0, R0x, R0y, R0z);
-            emit_row<true, true, WANT_R, WIDE>(row1, rrow1, cap, status, m1, ca1, ent[g], 0, 0, 0, R1x, R1y, R1z);
+            emit_row<true, true, WIDE>(row0, cap, status, m0, ca0, ent[g], 0, 0, 0);
+            emit_row<true, true, WIDE>(row1, cap, status, m1, ca1, ent[g], 0, 0, 0);
         }
     }
 }
@@ -958,18 +927,18 @@ __device__ __forceinline__ void test_home_pair(int nch, const double *cx, const 
 // atom a).  home: the nh home atoms in LDS; ht_l, hj_l: lane a holds
 // pack(-w_i) and j of home atom a; kpass: the self candidate of home atom 0
 // in this pass (home atom a's is kpass + a); Cm: the cell matrix.
-template <bool WANT_R, bool WIDE>
+template <bool WIDE>
 __device__ __forceinline__ void pass_home_atoms(bool narrow, int nch, const double *cx, const double *cy,
                                                 const double *cz, const uint64_t *ent, const LAtom *home, int nh,
                                                 uint32_t ht_l, int32_t hj_l, int kpass, const double *Cm, double rc2,
-                                                int64_t atom_base, void *__restrict__ slots, double *__restrict__ slotsR,
-                                                int32_t cap, Status *__restrict__ status, int32_t &cnt_l)
+                                                int64_t atom_base, void *__restrict__ slots, int32_t cap,
+                                                Status *__restrict__ status, int32_t &cnt_l)
 {
     double sx[kBrickChunks], sy[kBrickChunks], sz[kBrickChunks];
     uint32_t wcur = 0xffffffffu;   // home winding the shifts were computed for
     int32_t wix = 0, wiy = 0, wiz = 0;
     // wave-uniform, per chunk: the lanes whose shift is nonzero (the
-    // shifts sx, sy, sz are set only where this is nonzero or R is written)
+    // shifts sx, sy, sz are set only where this is nonzero)
     uint64_t csh[kBrickChunks];
     int a = 0;
     if (narrow && nh >= 2) {
@@ -980,7 +949,7 @@ __device__ __forceinline__ void pass_home_atoms(bool narrow, int nch, const doub
             csh[g] = g < nch ? __builtin_amdgcn_ballot_w64((uint32_t)(ent[g] >> 32) != kPackZero) : 0;
 #pragma unroll
         for (int g = 0; g < kBrickChunks; ++g) {
-            if (g < nch && (WANT_R || csh[g] != 0)) {
+            if (g < nch && (csh[g] != 0)) {
                 int32_t cx_, cy_, cz_;
                 unpack_wind((uint32_t)(ent[g] >> 32), cx_, cy_, cz_);
                 cell_shift(Cm, cx_, cy_, cz_, sx[g], sy[g], sz[g]);
@@ -999,11 +968,8 @@ __device__ __forceinline__ void pass_home_atoms(bool narrow, int nch, const doub
                               : (void *)(reinterpret_cast<uint64_t *>(slots) + srow0);
             void *row1 = WIDE ? (void *)(reinterpret_cast<int4 *>(slots) + srow1)
                               : (void *)(reinterpret_cast<uint64_t *>(slots) + srow1);
-            double *rrow0 = WANT_R ? slotsR + 3 * srow0 : nullptr;
-            double *rrow1 = WANT_R ? slotsR + 3 * srow1 : nullptr;
-            test_home_pair<WANT_R, WIDE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, h0x, h0y, h0z, h1x, h1y, h1z,
-                                         rc2, kpass + a, row0, row1, rrow0, rrow1,
-                                         (uint32_t)cap, status, ca0, ca1);
+            test_home_pair<WIDE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, h0x, h0y, h0z, h1x, h1y, h1z, rc2, kpass + a,
+                                 row0, row1, (uint32_t)cap, status, ca0, ca1);
             cnt_l = write_lane(ca0, a, cnt_l);
             cnt_l = write_lane(ca1, a + 1, cnt_l);
         }
@@ -1024,7 +990,7 @@ __device__ __forceinline__ void pass_home_atoms(bool narrow, int nch, const doub
                     unpack_wind((uint32_t)(ent[g] >> 32), cx_, cy_, cz_);
                     cx_ += wix; cy_ += wiy; cz_ += wiz;
                     csh[g] = __builtin_amdgcn_ballot_w64((cx_ | cy_ | cz_) != 0);
-                    if (WANT_R || csh[g] != 0) cell_shift(Cm, cx_, cy_, cz_, sx[g], sy[g], sz[g]);
+                    if (csh[g] != 0) cell_shift(Cm, cx_, cy_, cz_, sx[g], sy[g], sz[g]);
                 }
             }
             wcur = ht;
@@ -1035,36 +1001,32 @@ __device__ __forceinline__ void pass_home_atoms(bool narrow, int nch, const doub
         const int64_t srow = slot_row(atom_base + __builtin_amdgcn_readlane(hj_l, a), cap);
         void *row = WIDE ? (void *)(reinterpret_cast<int4 *>(slots) + srow)
                          : (void *)(reinterpret_cast<uint64_t *>(slots) + srow);
-        double *rrow = WANT_R ? slotsR + 3 * srow : nullptr;
         const int ks = kpass + a;   // the self candidate's place in this pass
         if (narrow)   // every home atom of a 4-byte brick has w_i = 0
-            test_home_atom<true, true, WANT_R, WIDE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, hx, hy, hz, rc2,
-                                                     ks, row, rrow, (uint32_t)cap, status, ca, wix, wiy,
-                                                     wiz);
+            test_home_atom<true, true, WIDE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, hx, hy, hz, rc2, ks, row,
+                                             (uint32_t)cap, status, ca, wix, wiy, wiz);
         else if (wzero)
-            test_home_atom<false, true, WANT_R, WIDE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, hx, hy, hz, rc2,
-                                                      ks, row, rrow, (uint32_t)cap, status, ca, wix, wiy,
-                                                      wiz);
+            test_home_atom<false, true, WIDE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, hx, hy, hz, rc2, ks, row,
+                                              (uint32_t)cap, status, ca, wix, wiy, wiz);
         else
-            test_home_atom<false, false, WANT_R, WIDE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, hx, hy, hz,
-                                                       rc2, ks, row, rrow, (uint32_t)cap, status, ca, wix,
-                                                       wiy, wiz);
+            test_home_atom<false, false, WIDE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, hx, hy, hz, rc2, ks, row,
+                                               (uint32_t)cap, status, ca, wix, wiy, wiz);
         cnt_l = write_lane(ca, a, cnt_l);
     }
 }
 
-// Brick pass of the count: home atoms stream through the wave as scalars
+// Brick pass of the count with 16-byte slot entries: home atoms stream through the wave as scalars
 // (read out of one-per-lane registers), candidates sit one per lane in
 // registers, chunk by chunk; each (home atom, chunk) is one FP64 distance
 // test and one ballot.  Bricks that cannot take this path (reach beyond one
 // cell, halo over the LDS, windings beyond the packed range) are counted
 // from global memory, one home cell per wave.
-template <bool WANT_R, bool WIDE, int BT>
+template <int BT>
 __global__ __launch_bounds__(BT) void count_kernel(
     const SysDev *__restrict__ sys, const int32_t *__restrict__ sys_cell_base, const int32_t *__restrict__ sys_brick_base,
     int nsys, int32_t M, int64_t nat, const int32_t *__restrict__ cell_start, const Rec *__restrict__ rec,
     const int32_t *__restrict__ wbig, int32_t *__restrict__ pair_count, void *__restrict__ slots,
-    double *__restrict__ slotsR, int32_t cap, Status *__restrict__ status)
+    int32_t cap, Status *__restrict__ status)
 {
     __shared__ BrickLDS<BT> L;
     __shared__ double Csh[9];
@@ -1074,20 +1036,16 @@ __global__ __launch_bounds__(BT) void count_kernel(
     if (threadIdx.x < 9) Csh[threadIdx.x] = B.sd->C[threadIdx.x];   // visible after brick_load's barrier
     const bool lds = B.fast && brick_load(A, B, L);
     if (!lds) {
-        const SlotArgs O{slots, slotsR, cap, status};
+        const SlotArgs O{slots, cap, status};
         const int wv0 = sgpr((int)(threadIdx.x >> 6));
         for (int hc = wv0; hc < B.nhome; hc += BrickShape<BT>::waves)
-            count_cell<WANT_R, WIDE>(A, *B.sd, brick_cell_id(B, hc), pair_count, O);
+            count_cell<true>(A, *B.sd, brick_cell_id(B, hc), pair_count, O);
         return;
     }
     const SysDev &sd = *B.sd;
     const double rc2 = sd.rc2;
     const int lane = lane_id();
     const int wv = sgpr((int)(threadIdx.x >> 6));
-    const bool narrow = !WIDE && sgpr(L.row8) == 0;   // the brick writes 4-byte slot entries
-    // L.j holds j | S code << 26 whenever every j fits in 26 bits
-    const uint32_t hjmask = sd.nat <= kNarrowMaxAtoms ? (uint32_t)(kNarrowMaxAtoms - 1) : 0xffffffffu;
-    const uint32_t jmask = narrow ? 0xffffffffu : hjmask;   // entry low word: j | code << 26, or j
     // home cells: one per wave, then the next one not taken (a wave that
     // ends its cell early takes the next at once)
     for (int hc = wv; hc < B.nhome; hc = take_next(&L.next_cell)) {
@@ -1100,7 +1058,7 @@ __global__ __launch_bounds__(BT) void count_kernel(
             const int hb = R.h0 + hg;        // LDS index of home atom hg (uniform)
             const int hl = hb + (lane < nh ? lane : 0);
             const uint32_t ht_l = L.a[hl].t;   // pack(-w_i): a home cell's own shift is zero
-            const int32_t hj_l = (int32_t)((uint32_t)L.a[hl].j & hjmask);
+            const int32_t hj_l = L.a[hl].j;
             const int kself = R.self0 + hg;  // candidate index of home atom hg + a is kself + a
             int32_t cnt_l = 0;                // lane a: running count of home atom hg + a
             for (int k0 = 0; k0 < R.total; k0 += kBrickChunks * kWave) {
@@ -1120,13 +1078,12 @@ __global__ __launch_bounds__(BT) void count_kernel(
                     cx[g] = c.x;
                     cy[g] = c.y;
                     cz[g] = c.z;
-                    ent[g] = (uint64_t)((uint32_t)c.j & jmask) | ((uint64_t)c.t << 32);
+                    ent[g] = (uint64_t)(uint32_t)c.j | ((uint64_t)c.t << 32);
                 }
-                pass_home_atoms<WANT_R, WIDE>(narrow, nch, cx, cy, cz, ent, L.a + hb, nh, ht_l, hj_l,
-                                                    kself - k0, Csh, rc2, sd.atom_base, slots, slotsR, cap, status,
-                                                    cnt_l);
+                pass_home_atoms<true>(false, nch, cx, cy, cz, ent, L.a + hb, nh, ht_l, hj_l, kself - k0, Csh, rc2,
+                                      sd.atom_base, slots, cap, status, cnt_l);
             }
-            if (lane < nh) pair_count[sd.atom_base + hj_l] = cnt_l | (narrow ? 0 : kRow8Bit);
+            if (lane < nh) pair_count[sd.atom_base + hj_l] = cnt_l | kRow8Bit;
         }
     }
 }
@@ -1484,7 +1441,7 @@ __device__ __forceinline__ void tile_pass(const Rec *rec, const TileLDS<BT> &L, 
     }
 }
 
-// Brick pass of the count (no R, no 16-byte entries): the distance tests run
+// Brick pass of the count (no 16-byte entries): the distance tests run
 // on 32-bit positions, exact to a known bound (filter_bounds), and every value
 // within that bound of the cutoff is decided again by the 64-bit test, so the
 // pairs are those of the 64-bit kernel.
@@ -1524,9 +1481,9 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(5))) void ti
     const int lane = lane_id();
     const int wv = sgpr((int)(threadIdx.x >> 6));
     if (!lds) {
-        const SlotArgs O{slots, nullptr, cap, status};
+        const SlotArgs O{slots, cap, status};
         for (int hc = copy + copies * wv; hc < B.nhome; hc += copies * BrickShape<BT>::waves)
-            count_cell<false, false>(A, *B.sd, brick_cell_id(B, hc), pair_count, O);
+            count_cell<false>(A, *B.sd, brick_cell_id(B, hc), pair_count, O);
         return;
     }
     const SysDev &sd = *B.sd;
@@ -1692,7 +1649,6 @@ struct SmallArgs {
     void *__restrict__ cell_offsets_out;
     int32_t *__restrict__ pair_count;
     void *__restrict__ slots;
-    double *__restrict__ slotsR;
     int32_t cap;
     Status *__restrict__ status;
 };
@@ -1713,7 +1669,7 @@ __device__ __forceinline__ void wrap_small(int32_t a, int32_t n, float rn, bool 
     s = q;
 }
 
-template <bool WANT_R, typename TI>
+template <typename TI>
 __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
 {
     __shared__ SmallLDS L;
@@ -1947,9 +1903,8 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
                         const uint32_t lo = narrow ? ((uint32_t)c.j | code << 26) : (uint32_t)c.j;
                         ent[g] = (uint64_t)lo | ((uint64_t)t << 32);
                     }
-                    pass_home_atoms<WANT_R, false>(narrow, nch, cx, cy, cz, ent, L.a + hb, nh, ht_l, hj_l,
-                                                   self0 + hg - k0, sd.C, sd.rc2, sd.atom_base, A.slots, A.slotsR,
-                                                   A.cap, A.status, cnt_l);
+                    pass_home_atoms<false>(narrow, nch, cx, cy, cz, ent, L.a + hb, nh, ht_l, hj_l, self0 + hg - k0,
+                                           sd.C, sd.rc2, sd.atom_base, A.slots, A.cap, A.status, cnt_l);
                 }
             }
             if (lane < nh) A.pair_count[sd.atom_base + hj_l] = cnt_l | (narrow ? 0 : kRow8Bit);
@@ -1957,25 +1912,20 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
     }
 }
 
-template <bool R, typename TI>
+template <typename TI>
 static void small_launch(const PipelineBufs &b, hipStream_t st)
 {
     SmallArgs A{b.X,          b.sys,     b.sys_atom_base, b.sys_cell_base, b.units,  b.unit_order,
                 b.atom_sys,   b.rec,     b.perm_out,      b.cell_id_out,   b.cell_offsets_out,
-                b.pair_count, b.slots,   b.slotsR,        b.slot_cap,      b.status};
-    hipLaunchKernelGGL((small_kernel<R, TI>), dim3((unsigned)b.nitems), dim3(kSmallThreads), 0, st, A);
+                b.pair_count, b.slots,   b.slot_cap,      b.status};
+    hipLaunchKernelGGL((small_kernel<TI>), dim3((unsigned)b.nitems), dim3(kSmallThreads), 0, st, A);
 }
 
-void launch_small(const PipelineBufs &b, bool want_R, hipStream_t st)
+static void launch_small(const PipelineBufs &b, hipStream_t st)
 {
-    if (b.nunits <= 0 || b.nitems <= 0) return;
-    if (b.ti_bytes == 8) {
-        if (want_R) small_launch<true, int64_t>(b, st);
-        else small_launch<false, int64_t>(b, st);
-    } else {
-        if (want_R) small_launch<true, int32_t>(b, st);
-        else small_launch<false, int32_t>(b, st);
-    }
+    if (b.nitems <= 0) return;
+    if (b.ti_bytes == 8) small_launch<int64_t>(b, st);
+    else small_launch<int32_t>(b, st);
 }
 
 // Fill pass (fill_pairs_kernel!, gpu_kernels.jl:159-180): one wave per tile
@@ -1984,6 +1934,12 @@ void launch_small(const PipelineBufs &b, bool want_R, hipStream_t st)
 // block of i, j, S (and R): the stores write whole cache lines, and lines
 // shared between waves occur only at tile edges.  A wave issues the slot
 // loads of all its TW blocks before its first store.
+//
+// R is computed here, from the positions (24 bytes gathered per pair, cached),
+// by the expression of the 64-bit distance test: keeping it in rows beside the
+// slots wrote and read 24 more bytes per pair through memory and held the
+// count pass to its 64-bit form (count and fill with R, 20k atoms 47 / 30 us,
+// 100k 93 / 66, 200k 162 / 123).
 //
 // The pair scan writes, per tile t, the atom A0 owning pair t TP and how
 // many of its pairs come before that one; the next tile's entry bounds the
@@ -2041,45 +1997,86 @@ __device__ __forceinline__ void decode_entry(const RawEntry<WIDE> &x, int32_t &j
     }
 }
 
-// Decode and store one pair at output position pos.  The stores are
-// non-temporal: the output streams past the caches, which keep holding the
-// slot rows the count pass wrote and the fill reads (with cached stores the
-// 1M-atom fill ran at 147 us, with these at 103 us).
-template <bool WANT_R, bool WIDE, typename TI>
-__device__ __forceinline__ void fill_store_one(const RawEntry<WIDE> &e, int32_t is, int64_t ridx, int64_t pos,
-                                               bool live, const double *__restrict__ slotsR, TI *__restrict__ i_out,
-                                               TI *__restrict__ j_out, TI *__restrict__ S_out,
-                                               double *__restrict__ R_out)
+// The stores are non-temporal: the output streams past the caches, which
+// keep holding the slot rows the count pass wrote and the fill reads (with
+// cached stores the 1M-atom fill ran at 147 us, with these at 103 us; 200k
+// atoms with R 87 against 79).
+//
+// Bound by the bytes written.  Three 8-byte components per pair (R, and S
+// in 64 bits) go through the wave's LDS: stored straight from the lanes, 24
+// bytes apart, the Int64 fill of 1M atoms (1.05 GB) took 295 us, in whole lines
+// 164 (6.4 TB/s); 200k atoms Int64 62 / 37 us, with R 99 / 80.  4-byte
+// components (12 bytes apart) write as fast as they are (5.7 TB/s at 1M).
+//
+// Components v0, v1, v2 of pair `lane` to out[3 lane ..], for the first n
+// pairs (wave-uniform n; lds: 3 kWave values of the wave's own).
+template <typename T>
+__device__ __forceinline__ void store_triples(T v0, T v1, T v2, T *__restrict__ out, int n, T *lds)
 {
-    int32_t j, Sx, Sy, Sz;
-    decode_entry<WIDE>(e, j, Sx, Sy, Sz);   // outside the branch: it covers the stores only
-    if (live) {
-        __builtin_nontemporal_store((TI)is, i_out + pos);
-        __builtin_nontemporal_store((TI)(j + 1), j_out + pos);
-        TI *S = S_out + 3 * pos;
-        __builtin_nontemporal_store((TI)Sx, S);
-        __builtin_nontemporal_store((TI)Sy, S + 1);
-        __builtin_nontemporal_store((TI)Sz, S + 2);
-        if (WANT_R) {
-            const double *Rs = slotsR + 3 * ridx;
-            double *Rd = R_out + 3 * pos;
-            __builtin_nontemporal_store(Rs[0], Rd);
-            __builtin_nontemporal_store(Rs[1], Rd + 1);
-            __builtin_nontemporal_store(Rs[2], Rd + 2);
+    const int lane = lane_id();
+    lds[3 * lane] = v0;
+    lds[3 * lane + 1] = v1;
+    lds[3 * lane + 2] = v2;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    T w[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) w[k] = lds[k * kWave + lane];
+    __builtin_amdgcn_wave_barrier();   // read before the next triples are written
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        if (k * kWave + lane < 3 * n) __builtin_nontemporal_store(w[k], out + k * kWave + lane);
+}
+
+// Store the pairs of one block of 64 output positions from pos0 on, the first
+// n of them live.
+template <typename TI>
+__device__ __forceinline__ void fill_store_pairs(int32_t is, int32_t j, int32_t Sx, int32_t Sy, int32_t Sz, int64_t pos0,
+                                                 int n, TI *__restrict__ i_out, TI *__restrict__ j_out,
+                                                 TI *__restrict__ S_out, void *lds)
+{
+    const int lane = lane_id();
+    if (lane < n) {
+        __builtin_nontemporal_store((TI)is, i_out + pos0 + lane);
+        __builtin_nontemporal_store((TI)(j + 1), j_out + pos0 + lane);
+        if (sizeof(TI) == 4) {
+            TI *S = S_out + 3 * (pos0 + lane);
+            __builtin_nontemporal_store((TI)Sx, S);
+            __builtin_nontemporal_store((TI)Sy, S + 1);
+            __builtin_nontemporal_store((TI)Sz, S + 2);
         }
     }
+    if (sizeof(TI) == 8) store_triples<TI>((TI)Sx, (TI)Sy, (TI)Sz, S_out + 3 * pos0, n, static_cast<TI *>(lds));
 }
+
+// R = xj - xi + C' * S  (gpu_kernels.jl:89)
+__device__ __forceinline__ void pair_vector(const double *__restrict__ C, const double xi[3], const double xj[3],
+                                            int32_t Sx, int32_t Sy, int32_t Sz, double R[3])
+{
+    double cx, cy, cz;
+    cell_shift(C, Sx, Sy, Sz, cx, cy, cz);
+    R[0] = (xj[0] - xi[0]) + cx;
+    R[1] = (xj[1] - xi[1]) + cy;
+    R[2] = (xj[2] - xi[2]) + cz;
+}
+
+// LDS of a fill block: one buffer of triples per wave when 8-byte
+// components pass through it.
+constexpr size_t kTripleBytes = 3 * kWave * 8;
 
 template <bool WANT_R, bool WIDE, typename TI, int TW>
 __global__ __launch_bounds__(1024) void fill_kernel(
-    const int64_t *__restrict__ sys_atom_base, const int32_t *__restrict__ atom_sys, int nsys, int64_t nat, const int32_t *__restrict__ pair_count,
+    const double *__restrict__ X, const SysDev *__restrict__ sys, const int64_t *__restrict__ sys_atom_base,
+    const int32_t *__restrict__ atom_sys, int nsys, int64_t nat, const int32_t *__restrict__ pair_count,
     const int64_t *__restrict__ pair_off, const int32_t *__restrict__ tile_atom, int64_t tile_cap,
-    const void *__restrict__ slots, const double *__restrict__ slotsR, const Status *__restrict__ status,
+    const void *__restrict__ slots, const Status *__restrict__ status,
     Status *__restrict__ status_pub, int32_t cap, int64_t pair_capacity, TI *__restrict__ i_out,
     TI *__restrict__ j_out, TI *__restrict__ S_out, double *__restrict__ R_out)
 {
     constexpr int TP = TW * kWave;
     constexpr int32_t kBeyond = 1 << 30;   // window position past every pair of the tile
+    extern __shared__ double fill_lds[];
+    void *lds = fill_lds + 3 * kWave * (threadIdx.x / kWave);   // the wave's triples
     const int lane = lane_id();
     // tiles in block order: the waves in flight write one advancing front of
     // the output (an XCD-contiguous block order measured much slower)
@@ -2155,7 +2152,6 @@ __global__ __launch_bounds__(1024) void fill_kernel(
         }
         RawEntry<WIDE> e[TW];
         int32_t is[TW];
-        int64_t ridx[TW];   // used only with R
 #pragma unroll
         for (int u = 0; u < TW; ++u) {
             const int q = u * kWave + lane;
@@ -2166,14 +2162,43 @@ __global__ __launch_bounds__(1024) void fill_kernel(
             const int64_t rs = live ? (A0 + s[u]) * (int64_t)cap : 0;
             const bool w8 = ((row8 >> s[u]) & 1) != 0;
             is[u] = batch ? __shfl(il, s[u], kWave) : (int32_t)(A0 + s[u] + 1);
-            ridx[u] = rs + r;
             e[u] = load_entry<WIDE>(slots, rs, r, w8);
         }
+        if constexpr (!WANT_R) {
 #pragma unroll
-        for (int u = 0; u < TW; ++u) {
-            const int q = u * kWave + lane;
-            fill_store_one<WANT_R, WIDE, TI>(e[u], is[u], ridx[u], Q0 + q, q < nlive, slotsR, i_out,
-                                             j_out, S_out, R_out);
+            for (int u = 0; u < TW; ++u) {
+                int32_t j, Sx, Sy, Sz;
+                decode_entry<WIDE>(e[u], j, Sx, Sy, Sz);   // outside the branch: it covers the stores only
+                fill_store_pairs<TI>(is[u], j, Sx, Sy, Sz, Q0 + u * kWave, nlive - u * kWave, i_out, j_out, S_out, lds);
+            }
+        } else {
+            // R from the positions themselves: every gather of the tile before
+            // its first store
+            int32_t j[TW], S[TW][3];
+            double xi[TW][3], xj[TW][3];
+#pragma unroll
+            for (int u = 0; u < TW; ++u) {
+                decode_entry<WIDE>(e[u], j[u], S[u][0], S[u][1], S[u][2]);
+                const int64_t gi = A0 + s[u];
+                const int64_t gj = u * kWave + lane < nlive ? gi - is[u] + 1 + j[u] : gi;   // the system's atom j
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    xi[u][k] = X[3 * gi + k];
+                    xj[u][k] = X[3 * gj + k];
+                }
+            }
+            const int s0 = batch ? sgpr(atom_sys[A0]) : 0;
+            const bool one = !batch || s0 == sgpr(atom_sys[A1]);   // the whole tile in one system
+#pragma unroll
+            for (int u = 0; u < TW; ++u) {
+                const int64_t pos0 = Q0 + u * kWave;
+                const int n = nlive - u * kWave;
+                fill_store_pairs<TI>(is[u], j[u], S[u][0], S[u][1], S[u][2], pos0, n, i_out, j_out, S_out, lds);
+                double R[3];
+                if (one) pair_vector(sys[s0].C, xi[u], xj[u], S[u][0], S[u][1], S[u][2], R);
+                else pair_vector(sys[atom_sys[A0 + s[u]]].C, xi[u], xj[u], S[u][0], S[u][1], S[u][2], R);
+                store_triples<double>(R[0], R[1], R[2], R_out + 3 * pos0, n, static_cast<double *>(lds));
+            }
         }
         return;
     }
@@ -2181,70 +2206,151 @@ __global__ __launch_bounds__(1024) void fill_kernel(
     // between A0 and A1 for the atom of its pair
     const int64_t hi0 = A1;
     for (int u = 0; u < TW; ++u) {
-        const int q = u * kWave + lane;
-        if (q < nlive) {
-            const int64_t P = Q0 + q;
-            int64_t lo = A0, hi = hi0;   // largest atom in [lo, hi] whose run starts at or before P
-            while (lo < hi) {
-                const int64_t mid = (lo + hi + 1) >> 1;
-                if (pair_off[mid] <= P) lo = mid;
-                else hi = mid - 1;
-            }
-            const int32_t pc = pair_count[lo];
-            const int r = (int)(P - pair_off[lo]);
-            const int64_t rs = lo * (int64_t)cap;
-            int32_t isv = (int32_t)(lo + 1);
-            if (nsys > 1) isv = (int32_t)(lo - sys_atom_base[atom_sys[lo]] + 1);
-            const RawEntry<WIDE> e = load_entry<WIDE>(slots, rs, r, (pc & kRow8Bit) != 0);
-            fill_store_one<WANT_R, WIDE, TI>(e, isv, rs + r, P, true, slotsR, i_out, j_out, S_out, R_out);
+        const int64_t pos0 = Q0 + u * kWave;
+        const int n = nlive - u * kWave;   // may be none
+        int64_t lo = A0, hi = hi0;   // largest atom in [lo, hi] whose run starts at or before the lane's pair
+        const int64_t P = lane < n ? pos0 + lane : Q0;
+        while (lo < hi) {
+            const int64_t mid = (lo + hi + 1) >> 1;
+            if (pair_off[mid] <= P) lo = mid;
+            else hi = mid - 1;
+        }
+        const int r = (int)(P - pair_off[lo]);
+        const int ls = nsys > 1 ? atom_sys[lo] : 0;
+        const int32_t isv = (int32_t)(lo - (nsys > 1 ? sys_atom_base[ls] : 0) + 1);
+        const RawEntry<WIDE> e = load_entry<WIDE>(slots, lo * (int64_t)cap, r, (pair_count[lo] & kRow8Bit) != 0);
+        int32_t j, Sx, Sy, Sz;
+        decode_entry<WIDE>(e, j, Sx, Sy, Sz);
+        fill_store_pairs<TI>(isv, j, Sx, Sy, Sz, pos0, n, i_out, j_out, S_out, lds);
+        if constexpr (WANT_R) {
+            const int64_t gj = lo - isv + 1 + j;
+            const double xi[3] = {X[3 * lo], X[3 * lo + 1], X[3 * lo + 2]};
+            const double xj[3] = {X[3 * gj], X[3 * gj + 1], X[3 * gj + 2]};
+            double R[3];
+            pair_vector(sys[ls].C, xi, xj, Sx, Sy, Sz, R);
+            store_triples<double>(R[0], R[1], R[2], R_out + 3 * pos0, n, static_cast<double *>(lds));
         }
     }
 }
 
+// R of every pair of one large system in cell order: a wave takes kRAtoms
+// consecutive sorted atoms, one lane per pair.  Atoms near one another in that
+// order share neighbours, so the position gathers hit the L2; the
+// fill's own, in atom order, do not once the positions outgrow it.  The
+// price: every atom's run of R (37 pairs, 888 bytes) is written on its own, at
+// 1.7 TB/s (cached stores: 20% slower).
+constexpr int kRAtoms = 16;
+// Atoms above which that pays: 24 bytes each against 4 MB of L2 (fill with R
+// in cell order / in atom order: 200k atoms 85 / 70 us, 400k 168 / 204, 1M
+// 487 / 646).
+constexpr int64_t kRCellOrder = 262144;
+__global__ __launch_bounds__(256) void fill_R_kernel(const double *__restrict__ X, const SysDev *__restrict__ sys,
+                                                     int64_t nat, const Rec *__restrict__ rec,
+                                                     const int32_t *__restrict__ pair_count,
+                                                     const int64_t *__restrict__ pair_off, const void *__restrict__ slots,
+                                                     const Status *__restrict__ status, int32_t cap,
+                                                     int64_t pair_capacity, double *__restrict__ R_out)
+{
+    __shared__ double lds[4][3 * kWave];
+    __shared__ int64_t at[4][kWave];   // output position of each lane's pair
+    const Status st = *status;
+    if ((st.npairs > pair_capacity) | (st.max_count > cap) | (st.wide != 0)) return;
+    const int lane = lane_id(), wv = (int)(threadIdx.x / kWave);
+    const int64_t p0 = ((int64_t)blockIdx.x * 4 + sgpr((int)(threadIdx.x / kWave))) * kRAtoms;
+    if (p0 >= nat) return;
+    const int na = (int)(nat - p0 < kRAtoms ? nat - p0 : kRAtoms);
+    Rec h{};
+    int32_t pc = 0;
+    int64_t gi = 0, off = 0;
+    if (lane < na) {
+        h = rec[p0 + lane];
+        gi = h.j;   // single system
+        pc = pair_count[gi];
+        off = pair_off[gi];
+    }
+    const int cnt = pc & kCountMask;
+    const int incl = wave_incl_scan(cnt);
+    const int fo = lane < na ? incl - cnt : 1 << 30;
+    const int total = sgpr(__shfl(incl, kWave - 1, kWave));
+    const uint64_t row8 = __ballot((pc & kRow8Bit) != 0);
+    for (int q0 = 0; q0 < total; q0 += kWave) {
+        const int q = q0 + lane;
+        int s = 0;
+#pragma unroll
+        for (int step = kRAtoms / 2; step >= 1; step >>= 1)
+            if (__shfl(fo, s + step, kWave) <= q) s += step;
+        const bool live = q < total;
+        const int fs = __shfl(fo, s, kWave);   // read by every lane: the source may be a lane past the last pair
+        const int r = live ? q - fs : 0;
+        const int64_t ga = (int64_t)(int)__shfl((int)gi, s, kWave);
+        const int64_t o = (int64_t)shfl64((uint64_t)off, s) + r;
+        const RawEntry<false> e = load_entry<false>(slots, live ? ga * cap : 0, r, (row8 >> s) & 1);
+        int32_t j, Sx, Sy, Sz;
+        decode_entry<false>(e, j, Sx, Sy, Sz);
+        const int64_t gj = live ? j : ga;
+        const double xi[3] = {X[3 * ga], X[3 * ga + 1], X[3 * ga + 2]};
+        const double xj[3] = {X[3 * gj], X[3 * gj + 1], X[3 * gj + 2]};
+        double R[3];
+        pair_vector(sys[0].C, xi, xj, Sx, Sy, Sz, R);
+        lds[wv][3 * lane] = R[0];
+        lds[wv][3 * lane + 1] = R[1];
+        lds[wv][3 * lane + 2] = R[2];
+        at[wv][lane] = o;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int e3 = k * kWave + lane, pr = e3 / 3;
+            const double v = lds[wv][e3];
+            const int64_t oo = at[wv][pr];
+            if (q0 + pr < total) __builtin_nontemporal_store(v, R_out + 3 * oo + (e3 - 3 * pr));
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// Positions back in atom order out of the records, for a fill with R when
+// they came in the caller's device memory: the fill may run after the call has
+// returned, when that memory is the caller's again.
+__global__ __launch_bounds__(256) void unsort_kernel(const Rec *__restrict__ rec, const int32_t *__restrict__ atom_sys,
+                                                     const int64_t *__restrict__ sys_atom_base, int64_t nat,
+                                                     double *__restrict__ Xr)
+{
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p >= nat) return;
+    const Rec h = rec[p];
+    const int64_t g = (atom_sys ? sys_atom_base[atom_sys[p]] : 0) + h.j;   // a system's atoms stay in its range
+    Xr[3 * g] = h.x;
+    Xr[3 * g + 1] = h.y;
+    Xr[3 * g + 2] = h.z;
+}
 
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
 
-template <bool R, bool W>
-static void count_launch(const PipelineBufs &b, hipStream_t st)
+template <int BT>
+static void count_launch(const PipelineBufs &b, bool wide, hipStream_t st)
 {
-    if (b.count_block == 256)
-        hipLaunchKernelGGL((count_kernel<R, W, 256>), dim3((unsigned)b.nbricks), dim3(256), 0, st, b.sys,
+    if (wide)
+        hipLaunchKernelGGL(count_kernel<BT>, dim3((unsigned)b.nbricks), dim3(BT), 0, st, b.sys,
                            b.sys_cell_base, b.sys_brick_base, b.nsys, b.M, b.nat, b.cell_start, b.rec, b.wbig,
-                           b.pair_count, b.slots, b.slotsR, b.slot_cap, b.status);
+                           b.pair_count, b.slots, b.slot_cap, b.status);
     else
-        hipLaunchKernelGGL((count_kernel<R, W, 512>), dim3((unsigned)b.nbricks), dim3(512), 0, st, b.sys,
-                           b.sys_cell_base, b.sys_brick_base, b.nsys, b.M, b.nat, b.cell_start, b.rec, b.wbig,
-                           b.pair_count, b.slots, b.slotsR, b.slot_cap, b.status);
-}
-
-static void tile_launch(const PipelineBufs &b, hipStream_t st)
-{
-    if (b.count_block == 256)
-        hipLaunchKernelGGL(tile_kernel<256>, dim3((unsigned)(b.nbricks * b.brick_copies)), dim3(256), 0, st, b.sys,
-                           b.sys_cell_base, b.sys_brick_base, b.nsys, b.brick_copies, b.M, b.nat, b.cell_start, b.rec, b.wbig, b.pair_count, b.slots,
-                           b.slot_cap, b.status);
-    else
-        hipLaunchKernelGGL(tile_kernel<512>, dim3((unsigned)(b.nbricks * b.brick_copies)), dim3(512), 0, st, b.sys,
-                           b.sys_cell_base, b.sys_brick_base, b.nsys, b.brick_copies, b.M, b.nat, b.cell_start, b.rec, b.wbig, b.pair_count, b.slots,
-                           b.slot_cap, b.status);
+        hipLaunchKernelGGL(tile_kernel<BT>, dim3((unsigned)(b.nbricks * b.brick_copies)), dim3(BT), 0, st, b.sys,
+                           b.sys_cell_base, b.sys_brick_base, b.nsys, b.brick_copies, b.M, b.nat, b.cell_start, b.rec,
+                           b.wbig, b.pair_count, b.slots, b.slot_cap, b.status);
 }
 
 void launch_count(const PipelineBufs &b, bool want_R, bool wide, hipStream_t st)
 {
-    if (b.nunits > 0) {   // cell list, counts and slot rows of every unit of small systems
-        launch_small(b, want_R, st);
-        return;
-    }
-    if (b.nat == 0 || b.nbricks == 0) return;
-    if (want_R) {
-        if (wide) count_launch<true, true>(b, st);
-        else count_launch<true, false>(b, st);
-    } else {
-        if (wide) count_launch<false, true>(b, st);
-        else tile_launch(b, st);
-    }
+    if (b.nunits > 0) launch_small(b, st);   // cell list, counts and slot rows of every unit of small systems
+    else if (b.nat == 0 || b.nbricks == 0) return;
+    else if (b.count_block == 256) count_launch<256>(b, wide, st);
+    else count_launch<512>(b, wide, st);
+    if (want_R && b.Xr != b.X)
+        hipLaunchKernelGGL(unsort_kernel, dim3((unsigned)((b.nat + 255) / 256)), dim3(256), 0, st, b.rec, b.atom_sys,
+                           b.sys_atom_base, b.nat, b.Xr);
 }
 
 template <bool R, bool W, typename TI, int TW>
@@ -2255,10 +2361,10 @@ static bool fill_launch(const PipelineBufs &b, hipStream_t st)
     const int64_t waves = (b.pair_capacity + TW * kWave - 1) / (TW * kWave);
     if (waves <= 0) return false;
     const unsigned nblk = (unsigned)((waves * kWave + bs - 1) / bs);
-    hipLaunchKernelGGL((fill_kernel<R, W, TI, TW>), dim3(nblk), dim3(bs), 0, st, b.sys_atom_base, b.atom_sys, b.nsys,
-                       b.nat,
-                       b.pair_count, b.pair_off, b.tile_atom, b.tile_cap, b.slots, b.slotsR, b.status, b.status_pub,
-                       b.slot_cap, b.pair_capacity, (TI *)b.i_out, (TI *)b.j_out, (TI *)b.S_out, b.R_out);
+    const size_t lds = R || sizeof(TI) == 8 ? bs / kWave * kTripleBytes : 0;
+    hipLaunchKernelGGL((fill_kernel<R, W, TI, TW>), dim3(nblk), dim3(bs), lds, st, b.Xr, b.sys, b.sys_atom_base,
+                       b.atom_sys, b.nsys, b.nat, b.pair_count, b.pair_off, b.tile_atom, b.tile_cap, b.slots, b.status,
+                       b.status_pub, b.slot_cap, b.pair_capacity, (TI *)b.i_out, (TI *)b.j_out, (TI *)b.S_out, b.R_out);
     return true;
 }
 
@@ -2273,6 +2379,13 @@ static bool fill_tiles(const PipelineBufs &b, hipStream_t st)
 template <typename TI>
 static bool fill_dispatch(const PipelineBufs &b, bool want_R, bool wide, hipStream_t st)
 {
+    if (want_R && b.nsys == 1 && !wide && b.nat > kRCellOrder) {
+        const bool launched = fill_tiles<false, false, TI>(b, st);
+        hipLaunchKernelGGL(fill_R_kernel, dim3((unsigned)((b.nat + 4 * kRAtoms - 1) / (4 * kRAtoms))), dim3(256), 0, st,
+                           b.Xr, b.sys, b.nat, b.rec, b.pair_count, b.pair_off, b.slots, b.status, b.slot_cap,
+                           b.pair_capacity, b.R_out);
+        return launched;
+    }
     if (want_R) return wide ? fill_tiles<true, true, TI>(b, st) : fill_tiles<true, false, TI>(b, st);
     return wide ? fill_tiles<false, true, TI>(b, st) : fill_tiles<false, false, TI>(b, st);
 }

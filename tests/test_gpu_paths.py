@@ -1,12 +1,16 @@
 """Size edges of the launch paths, each against the oracle bit for bit:
 lazy range queries, scans, the pair search.
 """
+import ctypes
+import dataclasses
+
 import numpy as np
 import pytest
+import torch
 
 import nlhip
 import oracle
-from nlhip import workloads
+from nlhip import _lib, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -111,3 +115,70 @@ def test_rows_that_overflow(n):
     X[-40:] = X[100] + 0.9 * rng.random((40, 3))
     X[5000:5040] = X[4000] + 0.9 * rng.random((40, 3))
     _check(X, 5.0, s.cell, s.pbc)
+
+
+def _same_R(nl, ref):
+    assert np.array_equal(nl.first, ref.first)
+    assert np.array_equal(nl.i, ref.i) and np.array_equal(nl.j, ref.j) and np.array_equal(nl.S, ref.S)
+    assert np.array_equal(_bits(nl.R), _bits(ref.R))
+
+
+@pytest.mark.parametrize("int_type,bits", [(np.int32, 32), (np.int64, 64)])
+@pytest.mark.parametrize("n,density,wind", [(1, 0.05, 0), (7, 0.5, 0), (300, 0.05, 2), (5000, 0.001, 0), (5000, 0.05, 700),
+                                            (262144, 0.004, 0), (262145, 0.004, 0), (262145, 0.004, 700)])
+def test_R_in_the_fill(int_type, bits, n, density, wind):
+    """R of lists with few pairs, of runs of atoms without any, of 4-byte,
+    8-byte and 16-byte rows, below and above the size from which R is
+    written in cell order."""
+    s = workloads.random_cubic(n, density=density, seed=n, cutoff=5.0)
+    X = s.X.copy()
+    X[::5] += wind * np.asarray(s.cell)[0]
+    print(f"R {n} {density} {wind}", flush=True)
+    ref = oracle.neighbour_list(X, 5.0, s.cell, s.pbc, ti_bits=bits, want_R=True, nthreads=8)
+    _same_R(nlhip.neighbour_list(X, 5.0, s.cell, s.pbc, int_type=int_type, want_R=True), ref)
+
+
+@pytest.mark.parametrize("int_type,bits", [(np.int32, 32), (np.int64, 64)])
+@pytest.mark.parametrize("sizes", [[3] * 300, [1, 0, 40, 2, 0, 0, 5] * 60, [700, 5000, 2]])
+def test_R_in_the_fill_of_batches(int_type, bits, sizes):
+    """Tiles of pairs that span several systems, each with its own cell."""
+    systems = []
+    for k, n in enumerate(sizes):
+        y = workloads.random_cubic(max(n, 1), density=0.05, seed=k, cutoff=4.0 + 0.01 * (k % 7))
+        systems.append(dataclasses.replace(y, X=y.X[:n]))
+    print(f"R batch {len(sizes)} {bits}", flush=True)
+    got = nlhip.BatchBuilder(int_type=int_type).run(systems, want_R=True)
+    for k, y in enumerate(systems):
+        ref = oracle.neighbour_list(y.X, y.cutoff, y.cell, y.pbc, ti_bits=bits, want_R=True)
+        _same_R(got.pairlist(k), ref)
+
+
+@pytest.mark.parametrize("n", [100, 20000, 300000])
+def test_R_after_the_positions_are_gone(n):
+    """Device positions belong to the caller again once a build has returned:
+    overwritten at once, and before a later materialisation, R is the same."""
+    s = workloads.random_cubic(n, density=0.02, seed=n, cutoff=4.0)
+    ref = nlhip.neighbour_list(s.X, 4.0, s.cell, s.pbc, want_R=True)
+    print(f"R after {n}", flush=True)
+    L = _lib.lib()
+    side = torch.cuda.Stream()
+    h = _lib.Handle()
+    geom = _lib.geometry(s.cell, 4.0, s.pbc, 4)
+    m = ctypes.c_int64()
+    for step in range(4):
+        X = torch.as_tensor(s.X).cuda()
+        torch.cuda.synchronize()
+        if step < 3:
+            _lib.check(L.nlh_neighbour_list(h.ptr, X.data_ptr(), n, ctypes.byref(geom),
+                                            _lib.NLH_X_DEVICE | _lib.NLH_WANT_R, ctypes.byref(m)))
+        else:
+            _lib.check(L.nlh_build_cell_list(h.ptr, X.data_ptr(), n, ctypes.byref(geom), _lib.NLH_X_DEVICE))
+            _lib.check(L.nlh_synchronize(h.ptr))
+        with torch.cuda.stream(side):
+            X.fill_(float("nan"))
+            side.synchronize()
+        if step == 3:
+            _lib.check(L.nlh_materialize(h.ptr, _lib.NLH_WANT_R, ctypes.byref(m)))
+        R = np.empty((m.value, 3))
+        _lib.check(L.nlh_copy_pairlist(h.ptr, None, None, None, None, R.ctypes.data))
+        assert m.value == ref.npairs() and np.array_equal(_bits(R), _bits(ref.R))
