@@ -143,7 +143,7 @@ struct nlh_handle {
     // system of each, then the end) and the work items in launch order
     // (unit, then part | parts << 16), in the tables
     std::vector<int32_t> units_host, order_host;
-    int32_t nunits = 0, nitems = 0;
+    int32_t nunits = 0, nitems = 0, item_tests = 0;
     int32_t *units_d = nullptr, *order_d = nullptr;
     bool small_ok = true;   // cleared when a fused build met a winding beyond +-511
     std::vector<char> tables_host;        // bytes of the last upload
@@ -259,6 +259,7 @@ struct nlh_handle {
         b.count_block = count_block();
         b.nunits = nunits;
         b.nitems = nitems;
+        b.item_tests = item_tests;
         b.units = units_d;
         b.unit_order = order_d;
         return b;
@@ -546,11 +547,35 @@ void filter_bounds(nlh::SysDev &sd, const nlh_geometry &g)
     const double H = 0.505 * std::sqrt(diag2) + 0.25 * rc;
     const double tol = 1.25 * u * (10 * ((2 * H + rc) * (2 * H + rc) + rc * rc) + 7 * (H + rc) * (H + rc) +
                                    4 * rc * rc + 7.2 * (P + 2 * H + rc) * rc) + 1.6e-11 * rc * sum;
-    const bool ok = H < 1000 * rc && P < 1e6 * rc && rc > 1e-9 && rc < 1e9;
+    const bool ok = H < 1000 * rc && P < 1e6 * rc && rc > 1e-14 && rc < 1e9;
     sd.rc2half = (float)(0.5 * g.cutoff_sq);
     sd.tol = (float)(0.505 * tol);
     sd.h2half = (float)(0.499 * H * H);
     sd.pmax2 = ok ? (float)(0.999 * P * P) : -1.0f;
+}
+
+// The same for a system of a fused build (small_kernel), whose positions are
+// kept in 32 bits from the system's centre, wrapped: with o the home cell's
+// centre, A the longest cell shift of a candidate, O = (|a1| + |a2| + |a3|) / 2 and
+// H as found for each group of home atoms, the positions' share is
+//   u rc (8 H + 4 rc + 10 (A + O))
+// (home atom u (|o| + 2 H); candidate u (2 (H + rc) + |s - o|) and, for s - o
+// itself, u (4 A + 3 |o|)); with 2 H rc <= H^2 + rc^2 the sum of all terms is at
+// most u (78 H^2 + 66 rc^2 + 10 (A + O) rc), of which the kernel adds the first.
+void small_bounds(nlh::SysDev &sd, const nlh_geometry &g)
+{
+    constexpr double u = 1.0 / (1 << 24);
+    const double rc = g.cutoff;
+    double sum = 0.0, A = 0.0;
+    for (int k = 0; k < 3; ++k) {
+        double l2 = 0.0;
+        for (int m = 0; m < 3; ++m) l2 += g.cell[k + 3 * m] * g.cell[k + 3 * m];
+        const double len = std::sqrt(l2);
+        sum += len;
+        if (sd.pbc >> k & 1) A += len * ((sd.nxyz[k] + sd.n[k] - 1) / sd.n[k]);
+    }
+    sd.small_tol = (float)(0.505 * (1.25 * u * (66 * rc * rc + 10 * (A + 0.5 * sum) * rc) + 1.6e-11 * rc * sum));
+    for (int k = 0; k < 9; ++k) sd.C32[k] = (float)sd.C[k];
 }
 
 // How a system's pair search is cut up: its brick, the run of home cells that
@@ -585,6 +610,7 @@ int32_t plan_search(nlh::SysDev &sd, const nlh_geometry &g, bool single, int cus
         copies *= 2;
     }
     filter_bounds(sd, g);
+    if (!single) small_bounds(sd, g);
     return copies;
 }
 
@@ -611,14 +637,24 @@ void assign_bricks(nlh_handle *h)
 // Fused build of small systems: a batch of at least kSmallMinSystems systems,
 // each within a unit's limits (atoms, cells, neighbour-cell reach), is cut
 // into units of consecutive systems, at most kUnitAtoms atoms, kUnitCells
-// cells and kUnitSystems systems each.  A unit whose estimated count work is
-// well above an even share of the batch is split into parts (each sorts the
-// whole unit and counts every parts-th home cell), and the work items are
-// launched largest first.  Otherwise (or when turned off, or after a winding
+// cells and kUnitSystems systems each, and no more atoms than spread the batch
+// over kUnitRounds units per workgroup place.  A unit whose estimated count work
+// is well above an even share of the batch is split into parts (each sorts the
+// whole unit and counts every parts-th group of home atoms), and the work items
+// are launched largest first.  Otherwise (or when turned off, or after a winding
 // beyond +-511 made a fused build fall back) no units: the general pipeline.
+//
+// small_kernel, event timed (us): full units / units over 1.6 rounds: 128
+// systems of 8 to 400 atoms 39 / 39, 4,096 of 8 to 2,048 354 / 330; parts by
+// cells alone / by atoms as well, for systems of one or two cells: 128 systems
+// 39 / 29, 500 52 / 46, 2,000 97 / 82; wave items of 512 / 256 / 128 tests, 64
+// systems 31 / 29 / 23, 128 31 / 29 / 25, 500 48 / 46 / 54, 4,096 330 / 335 / 358.
 constexpr int kSmallMinSystems = 64;
-constexpr int kMaxUnitParts = 16;       // parts of one unit at most (each at least 4 home cells)
-constexpr double kItemRounds = 2.0;     // work items per CU the split aims at
+constexpr int kMaxUnitParts = 16;       // parts of one unit at most (each at least 4 home cells or 32 atoms)
+constexpr int kUnitsPerCu = 2;          // workgroups of small_kernel on a CU
+constexpr double kUnitRounds = 1.6;     // units per such place that merging systems aims at
+constexpr double kItemRounds = 2.0;     // work items per place that splitting units aims at
+constexpr double kFewTests = 32;        // tests per wave of a full device up to which waves take smaller items
 
 // Estimated count work of a system in distance tests of 64 candidates: every
 // atom against the atoms of its (2 nxyz + 1)^3 neighbour cells, the cells
@@ -641,7 +677,7 @@ void plan_units(nlh_handle *h)
     int64_t total = 0;
     for (const nlh::SysDev &sd : h->sys_host) {
         total += sd.nat;
-        if (sd.nat > nlh::kUnitAtoms || sd.M > nlh::kUnitCells) return;
+        if (sd.nat > nlh::kUnitAtoms || sd.M > nlh::kUnitCells || sd.pmax2 < 0.0f) return;
         for (int k = 0; k < 3; ++k)
             if (sd.nxyz[k] > nlh::kUnitMaxReach || sd.n[k] > nlh::kUnitMaxAxisCells) return;
     }
@@ -649,12 +685,14 @@ void plan_units(nlh_handle *h)
     std::vector<double> work;
     std::vector<int64_t> atoms_u, cells_u;
     int s = 0;
+    const int64_t slots = (int64_t)kUnitsPerCu * std::max(h->cus, 1);
+    const int64_t target = std::min<int64_t>(nlh::kUnitAtoms, (int64_t)(total / (slots * kUnitRounds)));
     while (s < nsys) {
         const int first = s;
         int64_t atoms = 0, cells = 0;
         double w = 0.0;
-        while (s < nsys && s - first < nlh::kUnitSystems && atoms + h->sys_host[s].nat <= nlh::kUnitAtoms &&
-               cells + h->sys_host[s].M <= nlh::kUnitCells) {
+        while (s < nsys && s - first < nlh::kUnitSystems &&
+               (s == first || (atoms + h->sys_host[s].nat <= target && cells + h->sys_host[s].M <= nlh::kUnitCells))) {
             atoms += h->sys_host[s].nat;
             cells += h->sys_host[s].M;
             w += small_count_work(h->sys_host[s]);
@@ -667,30 +705,33 @@ void plan_units(nlh_handle *h)
     }
     h->units_host.push_back(nsys);
     h->nunits = (int32_t)work.size();
-    // A workgroup's time, fitted on MI355X (us): 14.4 + 0.0115 per atom of
-    // the unit (its sort, done by every part) + 0.0072 per estimated test +
-    // 0.154 per cell (the last two shared by the parts).
+    // A workgroup's time, fitted on MI355X (up to a factor): 14.4 + 0.0115 per
+    // atom of the unit (its sort, done by every part) + 0.0072 per estimated
+    // test + 0.154 per cell (the last two shared by the parts).
     std::vector<double> fixed(h->nunits), shared(h->nunits);
-    double time_total = 0.0;
+    double time_total = 0.0, work_total = 0.0;
     for (int u = 0; u < h->nunits; ++u) {
         fixed[u] = 14.4 + 0.0115 * atoms_u[u];
         shared[u] = 0.0072 * work[u] + 0.154 * cells_u[u];
         time_total += fixed[u] + shared[u];
+        work_total += work[u];
     }
-    const double share = std::max(1.0, time_total / (std::max(h->cus, 1) * kItemRounds));
+    const double share = std::max(1.0, time_total / (slots * kItemRounds));
     struct Item {
         double key;
         int32_t u, part, parts;
     };
     std::vector<Item> items;
     for (int u = 0; u < h->nunits; ++u) {
-        const int cap = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxUnitParts, cells_u[u] / 4));
+        const int cap = (int)std::clamp<int64_t>(std::max(cells_u[u] / 4, atoms_u[u] / 32), 1, kMaxUnitParts);
         const int parts = (int)std::max<double>(1.0, std::min<double>(cap, std::llround(shared[u] / share)));
         const double key = fixed[u] + shared[u] / parts;
         for (int p = 0; p < parts; ++p) items.push_back({key, u, p, parts});
     }
     std::stable_sort(items.begin(), items.end(), [](const Item &a, const Item &b) { return a.key > b.key; });
     h->nitems = (int32_t)items.size();
+    const double waves = (double)slots * (nlh::kSmallThreads / 64);
+    h->item_tests = work_total <= kFewTests * waves ? 128 : 256;
     h->order_host.resize(2 * items.size());
     for (size_t t = 0; t < items.size(); ++t) {
         h->order_host[2 * t] = items[t].u;

@@ -109,6 +109,8 @@ struct SysDev {
     // (r^2 - rc^2) / 2 has the sign of the 64-bit test wherever it is at least
     // tol away from zero.  pmax2 < 0: the system does not use the filter.
     float rc2half, tol, h2half, pmax2;
+    float small_tol;       // ... in small_kernel, less its home group's share (set by small_bounds)
+    float C32[9];          // C in 32 bits
     int32_t run;           // home cells along x that share a candidate list (tile_kernel): 1 or 2
     int32_t split;         // log2 of the work items a run's home atoms are split into
 };
@@ -289,6 +291,7 @@ struct PipelineBufs {
     // workgroup each): 0 units = the general pipeline
     int32_t nunits = 0;
     int32_t nitems = 0;                   // work items: parts of units, one workgroup each
+    int32_t item_tests = 0;               // distance tests of 64 candidates a wave takes at a time
     const int32_t *units = nullptr;       // nunits + 1: first system of each unit
     const int32_t *unit_order = nullptr;  // 2 nitems: unit, part | parts << 16 (launch order, largest first)
     int fill_block;          // threads per fill workgroup (multiple of 64)
@@ -334,7 +337,7 @@ void launch_range_scan(const LazyRange &q, hipStream_t st);
 // system, its pair counts and its slot rows, by one workgroup per work item
 // (a unit of consecutive systems or one part of one); launched by
 // launch_count, while launch_build launches nothing for such a batch.
-constexpr int kSmallThreads = 1024;
+constexpr int kSmallThreads = 512;
 constexpr int kUnitAtoms = 2048;      // atoms of one unit (and of one system) at most
 constexpr int kUnitCells = 2048;      // cells of one unit at most
 constexpr int kUnitSystems = 256;     // systems of one unit at most

@@ -62,8 +62,9 @@ __device__ __forceinline__ uint64_t shfl64(uint64_t v, int src)
 }
 
 // (C' * S)_k = sum_m C[m,k] S_m   (gpu_kernels.jl:89)
-__device__ __forceinline__ void cell_shift(const double *__restrict__ Cm, int32_t Sx, int32_t Sy, int32_t Sz, double &cx,
-                                           double &cy, double &cz)
+template <typename Mat>   // const double *, of any address space
+__device__ __forceinline__ void cell_shift(const Mat &Cm, int32_t Sx, int32_t Sy, int32_t Sz, double &cx, double &cy,
+                                           double &cz)
 {
     const double fx = (double)Sx, fy = (double)Sy, fz = (double)Sz;
     cx = (Cm[0] * fx + Cm[1] * fy) + Cm[2] * fz;
@@ -531,7 +532,7 @@ __device__ __forceinline__ int brick_cell_id(const Brick &B, int hc)
 // One halo atom in LDS, 32 bytes: a candidate is two 16-byte reads.
 struct __attribute__((aligned(16))) LAtom {
     double x, y, z;
-    int32_t j;                      // j, or j | S code << 26 when every j fits in 26 bits
+    int32_t j;
     uint32_t t;                     // pack(s_halo - w_j); home cells have s_halo = 0
 };
 
@@ -765,81 +766,18 @@ __device__ __forceinline__ int64_t slot_row(int64_t e, int32_t cap)
     return (int64_t)((uint64_t)(uint32_t)e * (uint32_t)cap);
 }
 
-// Append one ballot's hits to a home atom's slot row.  `row` and `rrow` are
-// the (wave-uniform) slot row and its R row; ca the atom's running count;
-// m the ballot of the hit lanes (the self pair already cleared), which also
-// serves as the store mask; ent = j | pack(s - w_j) << 32 is the candidate's
-// entry when w_i = 0.  Entry r of the row is written only while r < cap; the
-// per-lane bound is tested only when the row can overflow in this ballot.
-//
-// 4-byte rows without R go through a buffer resource spanning the row's cap
-// entries: every lane stores, lanes without a hit at an offset past the
-// resource's end, and the hardware's range check drops those stores and any
-// entry at r >= cap.  No exec-mask or bound branches.
-//
-// The offset of a lane without a hit: beyond any row resource (cap * 4 <
-// 2^30); the bit pattern of 4.0f, an inline constant, so the select that
-// applies it needs no literal.
-constexpr uint32_t kDropOffset = 0x40800000u;
-static_assert(__builtin_bit_cast(uint32_t, 4.0f) == kDropOffset, "the select below writes the offset as 4.0");
 constexpr int32_t kRawBufferWord3 = 0x00020000; // raw 32-bit buffer access (GFX9 family)
 
-template <bool NARROW, bool WZERO, bool WIDE>
-__device__ __forceinline__ void emit_row(void *__restrict__ row, uint32_t cap, Status *__restrict__ status, uint64_t m,
-                                         int32_t &ca, uint64_t ent, int32_t wix, int32_t wiy, int32_t wiz)
-{
-    const uint32_t n = (uint32_t)__popcll(m);
-    if (NARROW) {
-        // every lane stores, each lane without a hit at an offset past the
-        // resource's end (a select on the ballot, not an exec-mask region);
-        // an empty ballot skips it
-        if (n == 0) return;
-        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(row, 0, (int)(cap * 4u), kRawBufferWord3);
-        const uint32_t rk = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-        uint32_t off;
-        // a plain select on the 64-bit ballot (the compiler would otherwise
-        // open an exec-mask region around the offset computation)
-        __asm__("v_cndmask_b32_e64 %0, 4.0, %1, %2" : "=v"(off) : "v"((rk + (uint32_t)ca) << 2), "s"(m));
-        // j | S code << 26 (w_i = 0 in a 4-byte brick)
-        __builtin_amdgcn_raw_buffer_store_b32((uint32_t)ent, rs, (int)off, 0, 0);
-        ca += (int32_t)n;
-        return;
-    }
-    if (n != 0) {
-        const uint32_t rk = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-        uint64_t st = m;
-        if ((uint32_t)ca + n > cap)   // lanes whose entry would fall past the row's end store nothing
-            st &= __builtin_amdgcn_ballot_w64((int32_t)rk < (int32_t)cap - ca);
-        const uint32_t r = rk + (uint32_t)ca;
-        if (__builtin_amdgcn_inverse_ballot_w64(st)) {
-            if (WIDE) {
-                int32_t tx, ty, tz;
-                unpack_wind((uint32_t)(ent >> 32), tx, ty, tz);
-                reinterpret_cast<int4 *>(row)[r] = make_int4((int32_t)(uint32_t)ent, tx + wix, ty + wiy, tz + wiz);
-            } else if (WZERO) {
-                // S = s_loop + w_i - w_j = s_loop - w_j  (gpu_kernels.jl:88)
-                reinterpret_cast<uint64_t *>(row)[r] = ent;
-            } else {
-                int32_t tx, ty, tz;
-                unpack_wind((uint32_t)(ent >> 32), tx, ty, tz);
-                const uint32_t spk = pack_wind(tx + wix, ty + wiy, tz + wiz);
-                if (spk & kWindBig) status->wide = 1;
-                reinterpret_cast<uint64_t *>(row)[r] = (ent & 0xffffffffull) | ((uint64_t)spk << 32);
-            }
-        }
-        ca += (int32_t)n;
-    }
-}
-
-// One (home atom, chunk) test of the brick pass.  SHIFT: add the candidate's
-// cell shift C' S (left out when every lane's shift is zero: r^2 is then the
-// same).  `self` clears the home atom's own
-// (j == i, s == 0) candidate from the ballot when it lies in this chunk.
-template <bool NARROW, bool SHIFT, bool WZERO, bool WIDE>
+// One (home atom, chunk) test of the brick pass, its hits appended to the home
+// atom's row of 16-byte entries at its running count ca (wave-uniform).  SHIFT:
+// add the candidate's cell shift C' S (left out when every lane's shift is
+// zero: r^2 is then the same).  `self` clears the home atom's own (j == i, s ==
+// 0) candidate from the ballot when it lies in this chunk.  ent = j | pack(s -
+// w_j) << 32.
+template <bool SHIFT>
 __device__ __forceinline__ void test_chunk(double cx, double cy, double cz, double sx, double sy, double sz, double hx,
-                                           double hy, double hz, double rc2, uint64_t self, void *__restrict__ row,
-                                           uint32_t cap, Status *__restrict__ status,
-                                           int32_t &ca, uint64_t ent, int32_t wix, int32_t wiy, int32_t wiz)
+                                           double hy, double hz, double rc2, uint64_t self, int4 *__restrict__ row,
+                                           int32_t cap, int32_t &ca, uint64_t ent, int32_t wix, int32_t wiy, int32_t wiz)
 {
     // R = xj - xi + C' * S ; r^2 = dot(R, R)  (gpu_kernels.jl:89-92)
     double Rx = cx - hx, Ry = cy - hy, Rz = cz - hz;
@@ -849,90 +787,28 @@ __device__ __forceinline__ void test_chunk(double cx, double cy, double cz, doub
         Rz = Rz + sz;
     }
     const double r2 = (Rx * Rx + Ry * Ry) + Rz * Rz;
-    const bool in = r2 < rc2;
-    const uint64_t m = __builtin_amdgcn_ballot_w64(in) & self;
-    emit_row<NARROW, WZERO, WIDE>(row, cap, status, m, ca, ent, wix, wiy, wiz);
-}
-
-// All chunks of one home atom.
-template <bool NARROW, bool WZERO, bool WIDE>
-__device__ __forceinline__ void test_home_atom(int nch, const double *cx, const double *cy, const double *cz,
-                                               const double *sx, const double *sy, const double *sz, const uint64_t *csh,
-                                               const uint64_t *ent, double hx, double hy, double hz, double rc2,
-                                               int ks, void *__restrict__ row, uint32_t cap, Status *__restrict__ status,
-                                               int32_t &ca, int32_t wix, int32_t wiy, int32_t wiz)
-{
-    // _is_self_interaction: j == i with no cell shift is the home atom's own
-    // slot in the home cell, candidate ks of this pass: chunk ks >> 6 (none
-    // when ks is out of the pass), lane ks & 63
-    const int gs = ks >> 6;
-    const uint64_t nself = ~(1ull << (ks & (kWave - 1)));
-#pragma unroll
-    for (int g = 0; g < kBrickChunks; ++g) {
-        if (g < nch) {
-            const uint64_t self = g == gs ? nself : ~0ull;
-            if (csh[g] != 0)
-                test_chunk<NARROW, true, WZERO, WIDE>(cx[g], cy[g], cz[g], sx[g], sy[g], sz[g], hx, hy, hz, rc2, self,
-                                                      row, cap, status, ca, ent[g], wix, wiy, wiz);
-            else
-                test_chunk<NARROW, false, WZERO, WIDE>(cx[g], cy[g], cz[g], sx[g], sy[g], sz[g], hx, hy, hz, rc2, self,
-                                                       row, cap, status, ca, ent[g], wix, wiy, wiz);
-        }
+    const uint64_t m = __builtin_amdgcn_ballot_w64(r2 < rc2) & self;
+    if (m == 0) return;
+    const int32_t rank = ca + (int32_t)mbcnt64(m);
+    if (((m >> lane_id()) & 1) && rank < cap) {
+        // S = s_loop + w_i - w_j  (gpu_kernels.jl:88)
+        int32_t tx, ty, tz;
+        unpack_wind((uint32_t)(ent >> 32), tx, ty, tz);
+        row[rank] = make_int4((int32_t)(uint32_t)ent, tx + wix, ty + wiy, tz + wiz);
     }
-}
-
-// Two consecutive home atoms of a 4-byte brick (w_i = 0 for both, so the
-// same shifts) against the same chunks: both distance tests of a chunk come
-// before both emissions, two independent chains the scheduler interleaves.
-// Atom 1's self candidate follows atom 0's.
-template <bool WIDE>
-__device__ __forceinline__ void test_home_pair(int nch, const double *cx, const double *cy, const double *cz,
-                                               const double *sx, const double *sy, const double *sz, const uint64_t *csh,
-                                               const uint64_t *ent, double h0x, double h0y, double h0z, double h1x,
-                                               double h1y, double h1z, double rc2, int ks0, void *__restrict__ row0,
-                                               void *__restrict__ row1, uint32_t cap, Status *__restrict__ status,
-                                               int32_t &ca0, int32_t &ca1)
-{
-    // self candidates (as in test_home_atom): ks0 for atom 0, ks0 + 1 for atom 1
-    const int gs0 = ks0 >> 6, gs1 = (ks0 + 1) >> 6;
-    const uint64_t nself0 = ~(1ull << (ks0 & (kWave - 1))), nself1 = ~(1ull << ((ks0 + 1) & (kWave - 1)));
-#pragma unroll
-    for (int g = 0; g < kBrickChunks; ++g) {
-        if (g < nch) {
-            // R = xj - xi + C' * S ; r^2 = dot(R, R)  (gpu_kernels.jl:89-92)
-            double R0x = cx[g] - h0x, R0y = cy[g] - h0y, R0z = cz[g] - h0z;
-            double R1x = cx[g] - h1x, R1y = cy[g] - h1y, R1z = cz[g] - h1z;
-            if (csh[g] != 0) {
-                R0x = R0x + sx[g];
-                R0y = R0y + sy[g];
-                R0z = R0z + sz[g];
-                R1x = R1x + sx[g];
-                R1y = R1y + sy[g];
-                R1z = R1z + sz[g];
-            }
-            const bool in0 = (R0x * R0x + R0y * R0y) + R0z * R0z < rc2;
-            const bool in1 = (R1x * R1x + R1y * R1y) + R1z * R1z < rc2;
-            const uint64_t m0 = __builtin_amdgcn_ballot_w64(in0) & (g == gs0 ? nself0 : ~0ull);
-            const uint64_t m1 = __builtin_amdgcn_ballot_w64(in1) & (g == gs1 ? nself1 : ~0ull);
-            emit_row<true, true, WIDE>(row0, cap, status, m0, ca0, ent[g], 0, 0, 0);
-            emit_row<true, true, WIDE>(row1, cap, status, m1, ca1, ent[g], 0, 0, 0);
-        }
-    }
+    ca += (int32_t)__popcll(m);
 }
 
 // One pass of a home cell's atoms over loaded candidate chunks: every home
-// atom's distance tests against the nch chunks (cx, cy, cz, ent: j |
-// pack(s - w_j) << 32, or j | S code << 26 in a 4-byte brick), its hits
+// atom's distance tests against the nch chunks (cx, cy, cz, ent), its hits
 // appended to its slot row at its running count (lane a of cnt_l for home
 // atom a).  home: the nh home atoms in LDS; ht_l, hj_l: lane a holds
 // pack(-w_i) and j of home atom a; kpass: the self candidate of home atom 0
 // in this pass (home atom a's is kpass + a); Cm: the cell matrix.
-template <bool WIDE>
-__device__ __forceinline__ void pass_home_atoms(bool narrow, int nch, const double *cx, const double *cy,
-                                                const double *cz, const uint64_t *ent, const LAtom *home, int nh,
-                                                uint32_t ht_l, int32_t hj_l, int kpass, const double *Cm, double rc2,
-                                                int64_t atom_base, void *__restrict__ slots, int32_t cap,
-                                                Status *__restrict__ status, int32_t &cnt_l)
+__device__ __forceinline__ void pass_home_atoms(int nch, const double *cx, const double *cy, const double *cz,
+                                                const uint64_t *ent, const LAtom *home, int nh, uint32_t ht_l,
+                                                int32_t hj_l, int kpass, const double *Cm, double rc2,
+                                                int64_t atom_base, void *__restrict__ slots, int32_t cap, int32_t &cnt_l)
 {
     double sx[kBrickChunks], sy[kBrickChunks], sz[kBrickChunks];
     uint32_t wcur = 0xffffffffu;   // home winding the shifts were computed for
@@ -940,43 +816,8 @@ __device__ __forceinline__ void pass_home_atoms(bool narrow, int nch, const doub
     // wave-uniform, per chunk: the lanes whose shift is nonzero (the
     // shifts sx, sy, sz are set only where this is nonzero)
     uint64_t csh[kBrickChunks];
-    int a = 0;
-    if (narrow && nh >= 2) {
-        // every home atom of a 4-byte brick has w_i = 0: the shifts of
-        // the candidates are their own cell shifts
-#pragma unroll
-        for (int g = 0; g < kBrickChunks; ++g)
-            csh[g] = g < nch ? __builtin_amdgcn_ballot_w64((uint32_t)(ent[g] >> 32) != kPackZero) : 0;
-#pragma unroll
-        for (int g = 0; g < kBrickChunks; ++g) {
-            if (g < nch && (csh[g] != 0)) {
-                int32_t cx_, cy_, cz_;
-                unpack_wind((uint32_t)(ent[g] >> 32), cx_, cy_, cz_);
-                cell_shift(Cm, cx_, cy_, cz_, sx[g], sy[g], sz[g]);
-            }
-        }
-        wcur = kPackZero;
-        for (; a + 1 < nh; a += 2) {
-            // uniform LDS reads: every lane receives the home atom's coordinates
-            const LAtom h0 = home[a], h1 = home[a + 1];
-            const double h0x = h0.x, h0y = h0.y, h0z = h0.z;
-            const double h1x = h1.x, h1y = h1.y, h1z = h1.z;
-            int32_t ca0 = __builtin_amdgcn_readlane(cnt_l, a), ca1 = __builtin_amdgcn_readlane(cnt_l, a + 1);
-            const int64_t srow0 = slot_row(atom_base + __builtin_amdgcn_readlane(hj_l, a), cap);
-            const int64_t srow1 = slot_row(atom_base + __builtin_amdgcn_readlane(hj_l, a + 1), cap);
-            void *row0 = WIDE ? (void *)(reinterpret_cast<int4 *>(slots) + srow0)
-                              : (void *)(reinterpret_cast<uint64_t *>(slots) + srow0);
-            void *row1 = WIDE ? (void *)(reinterpret_cast<int4 *>(slots) + srow1)
-                              : (void *)(reinterpret_cast<uint64_t *>(slots) + srow1);
-            test_home_pair<WIDE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, h0x, h0y, h0z, h1x, h1y, h1z, rc2, kpass + a,
-                                 row0, row1, (uint32_t)cap, status, ca0, ca1);
-            cnt_l = write_lane(ca0, a, cnt_l);
-            cnt_l = write_lane(ca1, a + 1, cnt_l);
-        }
-    }
-    for (; a < nh; ++a) {
+    for (int a = 0; a < nh; ++a) {
         const LAtom hm = home[a];
-        const double hx = hm.x, hy = hm.y, hz = hm.z;
         const uint32_t ht = (uint32_t)__builtin_amdgcn_readlane((int)ht_l, a);
         if (ht != wcur) {   // first home atom, or a new home winding
             int32_t tx, ty, tz;
@@ -995,22 +836,26 @@ __device__ __forceinline__ void pass_home_atoms(bool narrow, int nch, const doub
             }
             wcur = ht;
         }
-        const bool wzero = ht == kPackZero;   // the home atom lies inside the cell
         int32_t ca = __builtin_amdgcn_readlane(cnt_l, a);
         // slot rows are indexed by original atom index, so the fill reads them in order
-        const int64_t srow = slot_row(atom_base + __builtin_amdgcn_readlane(hj_l, a), cap);
-        void *row = WIDE ? (void *)(reinterpret_cast<int4 *>(slots) + srow)
-                         : (void *)(reinterpret_cast<uint64_t *>(slots) + srow);
-        const int ks = kpass + a;   // the self candidate's place in this pass
-        if (narrow)   // every home atom of a 4-byte brick has w_i = 0
-            test_home_atom<true, true, WIDE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, hx, hy, hz, rc2, ks, row,
-                                             (uint32_t)cap, status, ca, wix, wiy, wiz);
-        else if (wzero)
-            test_home_atom<false, true, WIDE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, hx, hy, hz, rc2, ks, row,
-                                              (uint32_t)cap, status, ca, wix, wiy, wiz);
-        else
-            test_home_atom<false, false, WIDE>(nch, cx, cy, cz, sx, sy, sz, csh, ent, hx, hy, hz, rc2, ks, row,
-                                               (uint32_t)cap, status, ca, wix, wiy, wiz);
+        int4 *row = reinterpret_cast<int4 *>(slots) + slot_row(atom_base + __builtin_amdgcn_readlane(hj_l, a), cap);
+        // _is_self_interaction: j == i with no cell shift is the home atom's own
+        // slot in the home cell, candidate kpass + a: chunk gs (none when it
+        // is out of the pass)
+        const int gs = (kpass + a) >> 6;
+        const uint64_t nself = ~(1ull << ((kpass + a) & (kWave - 1)));
+#pragma unroll
+        for (int g = 0; g < kBrickChunks; ++g) {
+            if (g < nch) {
+                const uint64_t self = g == gs ? nself : ~0ull;
+                if (csh[g] != 0)
+                    test_chunk<true>(cx[g], cy[g], cz[g], sx[g], sy[g], sz[g], hm.x, hm.y, hm.z, rc2, self, row, cap, ca,
+                                     ent[g], wix, wiy, wiz);
+                else
+                    test_chunk<false>(cx[g], cy[g], cz[g], sx[g], sy[g], sz[g], hm.x, hm.y, hm.z, rc2, self, row, cap, ca,
+                                      ent[g], wix, wiy, wiz);
+            }
+        }
         cnt_l = write_lane(ca, a, cnt_l);
     }
 }
@@ -1080,8 +925,8 @@ __global__ __launch_bounds__(BT) void count_kernel(
                     cz[g] = c.z;
                     ent[g] = (uint64_t)(uint32_t)c.j | ((uint64_t)c.t << 32);
                 }
-                pass_home_atoms<true>(false, nch, cx, cy, cz, ent, L.a + hb, nh, ht_l, hj_l, kself - k0, Csh, rc2,
-                                      sd.atom_base, slots, cap, status, cnt_l);
+                pass_home_atoms(nch, cx, cy, cz, ent, L.a + hb, nh, ht_l, hj_l, kself - k0, Csh, rc2, sd.atom_base, slots,
+                                cap, cnt_l);
             }
             if (lane < nh) pair_count[sd.atom_base + hj_l] = cnt_l | kRow8Bit;
         }
@@ -1368,12 +1213,12 @@ struct TileCands {
 
 // ... and its home atoms, one per lane: minus the position from the run's
 // centre, (|p|^2 - rc^2) / 2, the buffer over the slot row (address and entry
-// size), t', and the bytes filled of the row.
+// size), t', the bytes filled of the row, and the entries a chunk may store.
 struct TileHomes {
     float nx, ny, nz, ai;
     uint64_t row;
     uint32_t t;
-    int32_t fill;
+    int32_t fill, left;
 };
 
 __device__ __forceinline__ float readlane_f32(float v, int l)
@@ -1381,12 +1226,16 @@ __device__ __forceinline__ float readlane_f32(float v, int l)
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
 
+// Slot entries of a pass: 4 or 8 bytes.
+enum { kEntry4, kEntry8 };
+
 // Home atoms a0 .. a1 - 1 against NCH chunks.  D = bq + ai - p_i . p_j is half
 // of r^2 - rc^2.  G: the chunk that holds the home atoms' own candidates
-// (kpass + a; -1: none does).
-template <int BT, int NCH, bool NARROW, int G>
-__device__ __forceinline__ void tile_rows(const Rec *rec, const TileLDS<BT> &L, const double *Csh, double rc2, int hd0,
-                                          float tol, const TileCands &C, int hb, int a0, int a1, int kpass, TileHomes &H)
+// (kpass + a; -1: none does).  E: the 64-bit test of home atom a against the
+// lane's candidate of chunk g, and whether stores stop at H.left entries.
+template <int NCH, int MODE, int G, typename Env>
+__device__ __forceinline__ void tile_rows(const Env &E, float tol, const TileCands &C, int a0, int a1, int kpass,
+                                          TileHomes &H)
 {
     for (int a = a0; a < a1; ++a) {
         const float sx = readlane_f32(H.nx, a), sy = readlane_f32(H.ny, a), sz = readlane_f32(H.nz, a),
@@ -1404,19 +1253,19 @@ __device__ __forceinline__ void tile_rows(const Rec *rec, const TileLDS<BT> &L, 
         if (__builtin_expect(__builtin_amdgcn_ballot_w64(mn < tol) != 0, 0)) {
 #pragma unroll
             for (int g = 0; g < NCH; ++g)
-                if (__builtin_amdgcn_ballot_w64(__builtin_fabsf(D[g]) < tol) != 0)
-                    D[g] = tile_exact<BT>(rec, &L, Csh, rc2, hd0, hb + a, C.li[g]);
+                if (__builtin_amdgcn_ballot_w64(__builtin_fabsf(D[g]) < tol) != 0) D[g] = E.template exact<MODE>(a, g);
         }
         int32_t so = __builtin_amdgcn_readlane(H.fill, a);
         const v4u rs = {(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)H.row, a),
-                        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(H.row >> 32), a), (uint32_t)kWave,
+                        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(H.row >> 32), a),
+                        Env::kLimit ? (uint32_t)__builtin_amdgcn_readlane(H.left, a) : (uint32_t)kWave,
                         (uint32_t)kRawBufferWord3};
-        const uint32_t dt = NARROW ? 0u : (uint32_t)__builtin_amdgcn_readlane((int)H.t, a);
+        const uint32_t dt = MODE == kEntry8 ? (uint32_t)__builtin_amdgcn_readlane((int)H.t, a) : 0u;
 #pragma unroll
         for (int g = 0; g < NCH; ++g) {
             uint64_t m = __builtin_amdgcn_ballot_w64(D[g] < 0.0f);
             if (g == G) m &= ~(1ull << ((kpass + a) & (kWave - 1)));   // j == i, s == 0 is no pair
-            emit_chunk<NARROW>(rs, m, so, (uint32_t)C.ent[g], NARROW ? 0u : C.ct[g] - dt);
+            emit_chunk<MODE == kEntry4>(rs, m, so, (uint32_t)C.ent[g], MODE == kEntry4 ? 0u : C.ct[g] - dt);
         }
         H.fill = write_lane(so, a, H.fill);
     }
@@ -1424,22 +1273,39 @@ __device__ __forceinline__ void tile_rows(const Rec *rec, const TileLDS<BT> &L, 
 
 // The run's nh home atoms against NCH chunks: their own candidates are
 // consecutive, in one chunk or across two.
-template <int BT, int NCH, bool NARROW>
-__device__ __forceinline__ void tile_pass(const Rec *rec, const TileLDS<BT> &L, const double *Csh, double rc2, int hd0,
-                                          float tol, const TileCands &C, int hb, int nh, int kpass, TileHomes &H)
+template <int NCH, int MODE, typename Env>
+__device__ __forceinline__ void tile_pass(const Env &E, float tol, const TileCands &C, int nh, int kpass, TileHomes &H)
 {
     int a = 0;
     while (a < nh) {
         const int g = (kpass + a) >> 6;   // negative: before this pass
         const int e = g >= NCH ? nh : min(nh, g < 0 ? -kpass : (g + 1) * kWave - kpass);
-        if (NCH > 0 && g == 0) tile_rows<BT, NCH, NARROW, 0>(rec, L, Csh, rc2, hd0, tol, C, hb, a, e, kpass, H);
-        else if (NCH > 1 && g == 1) tile_rows<BT, NCH, NARROW, 1>(rec, L, Csh, rc2, hd0, tol, C, hb, a, e, kpass, H);
-        else if (NCH > 2 && g == 2) tile_rows<BT, NCH, NARROW, 2>(rec, L, Csh, rc2, hd0, tol, C, hb, a, e, kpass, H);
-        else if (NCH > 3 && g == 3) tile_rows<BT, NCH, NARROW, 3>(rec, L, Csh, rc2, hd0, tol, C, hb, a, e, kpass, H);
-        else tile_rows<BT, NCH, NARROW, -1>(rec, L, Csh, rc2, hd0, tol, C, hb, a, e, kpass, H);
+        if (NCH > 0 && g == 0) tile_rows<NCH, MODE, 0>(E, tol, C, a, e, kpass, H);
+        else if (NCH > 1 && g == 1) tile_rows<NCH, MODE, 1>(E, tol, C, a, e, kpass, H);
+        else if (NCH > 2 && g == 2) tile_rows<NCH, MODE, 2>(E, tol, C, a, e, kpass, H);
+        else if (NCH > 3 && g == 3) tile_rows<NCH, MODE, 3>(E, tol, C, a, e, kpass, H);
+        else tile_rows<NCH, MODE, -1>(E, tol, C, a, e, kpass, H);
         a = e;
     }
 }
+
+// tile_kernel's side of tile_rows: hb, hd0 as in tile_exact; a row's stores
+// are not limited (kSlotSlack).
+template <int BT>
+struct TileEnv {
+    static constexpr bool kLimit = false;
+    const Rec *rec;
+    const TileLDS<BT> &L;
+    const double *Csh;
+    double rc2;
+    int hd0, hb;
+    const TileCands &C;
+    template <int MODE>
+    __device__ __forceinline__ float exact(int a, int g) const
+    {
+        return tile_exact<BT>(rec, &L, Csh, rc2, hd0, hb + a, C.li[g]);
+    }
+};
 
 // Brick pass of the count (no 16-byte entries): the distance tests run
 // on 32-bit positions, exact to a known bound (filter_bounds), and every value
@@ -1561,17 +1427,16 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(5))) void ti
                     if (!narrow) C.ct[g] = L.t[C.li[g]] + kPackZero;
                 }
                 const int kp = self0 + hg - k0;   // home atom hg + a is candidate kp + a of this pass
-#define NLH_TILE_PASS(N, W) tile_pass<BT, N, W>(rec, L, Csh, sd.rc2, B.hd[0], tol, C, hb, nh, kp, H)
+const TileEnv<BT> E{rec, L, Csh, sd.rc2, B.hd[0], hb, C};
                 if (narrow) {
-                    if (nch == 4) NLH_TILE_PASS(4, true);
-                    else if (nch == 3) NLH_TILE_PASS(3, true);
-                    else NLH_TILE_PASS(2, true);
+                    if (nch == 4) tile_pass<4, kEntry4>(E, tol, C, nh, kp, H);
+                    else if (nch == 3) tile_pass<3, kEntry4>(E, tol, C, nh, kp, H);
+                    else tile_pass<2, kEntry4>(E, tol, C, nh, kp, H);
                 } else {
-                    if (nch == 4) NLH_TILE_PASS(4, false);
-                    else if (nch == 3) NLH_TILE_PASS(3, false);
-                    else NLH_TILE_PASS(2, false);
+                    if (nch == 4) tile_pass<4, kEntry8>(E, tol, C, nh, kp, H);
+                    else if (nch == 3) tile_pass<3, kEntry8>(E, tol, C, nh, kp, H);
+                    else tile_pass<2, kEntry8>(E, tol, C, nh, kp, H);
                 }
-#undef NLH_TILE_PASS
             }
             if (lane < nh) pair_count[sd.atom_base + hj_l] = narrow ? H.fill >> 2 : (H.fill >> 3) | kRow8Bit;
         }
@@ -1589,20 +1454,29 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(5))) void ti
 // original index, Julia's stable sortperm), the cell-list outputs (written
 // by part 0), and the neighbour count and slot row of every home atom of
 // the part's count work items (items part, part + parts, ..., each a group
-// of home atoms of one cell), through the brick pass's tests and emission;
+// of home atoms of one cell), through tile_kernel's 32-bit tests and emission;
 // the waves take those items from a workgroup counter.  A home cell's
 // candidates are its (2 nxyz + 1)^3 neighbour cells in the reference order
 // (dz, dy, dx outer to inner, gpu_kernels.jl:69-71), each a segment of the
 // sorted atoms with its cell shift, taken 64 segments at a time.
 
+// Bound by instruction issue and, in what comes before the tests, by latency:
+// in a batch of 4,096 systems of 8 to 2,048 atoms (1.6M atoms) the vector unit
+// issues for 70% of the time, 68M of its 126M instructions in the tests, 29M
+// in the items' segments, 20M in loading candidates, 10M in the sort.  Two
+// workgroups share a CU (79 KB of LDS each), so that one counts while the other
+// sorts.  Before, with 32-byte atoms, 64-bit tests and one workgroup of 1,024
+// threads per CU, against now: that batch 485 / 335 us, 128 systems of 8 to 400
+// atoms 58 / 25.
+//
 // Count work items: a group of at most sys_group home atoms of one cell.
-// The group size of a system aims at kItemTests distance tests (chunks of 64
+// The group size of a system aims at item_tests distance tests (chunks of 64
 // candidates) per item, at least kMinGroup atoms: a cell whose candidates run
 // to thousands (a small periodic cell, its own 26 images) is shared by
 // several waves instead of holding one wave for all of it.
-constexpr int kItemTests = 512;
 constexpr int kMinGroup = 4;
 constexpr int kUnitItems = kUnitAtoms / kMinGroup + kUnitCells;   // items of one unit at most
+constexpr int kThreadCells = kUnitCells / kSmallThreads;          // cells per thread in the scans
 
 struct SmallSort {                 // LDS of the sort
     int16_t key[kUnitAtoms];       // unit cell of each atom
@@ -1611,29 +1485,51 @@ struct SmallSort {                 // LDS of the sort
     uint32_t wk[kUnitAtoms];       // packed winding of each atom
     uint8_t sy[kUnitAtoms];        // unit system of each atom
 };
-struct SmallRows {                 // LDS of one wave in the count
-    int32_t dl[kWave];             // LDS offset less candidate prefix of each non-empty segment
-    uint32_t sh[kWave];            // packed cell shift of each non-empty segment
-    uint32_t flag[kPassCands / 4]; // one byte per candidate of a pass: a segment starts there
+struct __attribute__((aligned(16))) SegShift {
+    float x, y, z;                 // cell shift of a segment, less the home group's centre
+    uint32_t s;                    // the shift packed, or in a 4-byte system its S code << 26
 };
-struct SmallLDS {
-    LAtom a[kUnitAtoms + 1];       // sorted atoms {x, y, z, system-local j, packed winding}; far sentinel last
-    int32_t cs[kUnitCells + 1];    // first sorted atom of each unit cell
-    int32_t sys_cell0[kUnitSystems + 1];
-    int32_t sys_atom0[kUnitSystems + 1];
-    int32_t sys_row8[kUnitSystems];   // 8-byte slot rows: some winding, or reach beyond one cell
-    int32_t next_item;                // the next count work item a wave takes
-    int32_t sys_group[kUnitSystems];  // home atoms per count work item of each system
+struct SmallRows {                 // LDS of one wave in the count
+    SegShift sv[kWave];            // each non-empty segment
+    int32_t dl[kWave];             // LDS offset less candidate prefix of each non-empty segment
+    uint32_t flag[kTileCands / 4]; // one byte per candidate of a pass: a segment starts there
+};
+struct SmallCount {                // LDS of the count
     uint32_t cell_info[kUnitCells];   // per unit cell: system | (c1 - 1) << 8 | (c2 - 1) << 16 | (c3 - 1) << 24
     int16_t item0[kUnitCells + 1];    // first count work item of each unit cell
     int16_t item_cell[kUnitItems];    // unit cell of each count work item
+    SmallRows r[kSmallThreads / kWave];
+};
+struct SmallLDS {
+    TAtom a[kUnitAtoms + 1];       // sorted atoms, wrapped, from the system's centre, and j; far sentinel last
+    uint32_t w[kUnitAtoms + 1];    // their packed windings
+    int16_t cs[kUnitCells + 1];    // first sorted atom of each unit cell
+    int16_t sys_cell0[kUnitSystems + 1];
+    int16_t sys_atom0[kUnitSystems + 1];
+    int32_t next_item;                // the next count work item a wave takes
+    uint32_t sys_geo[kUnitSystems];   // grid and periodicity: n0 | n1 << 9 | n2 << 18 | pbc << 27
+    uint8_t sys_reach[kUnitSystems];  // nxyz: x | y << 2 | z << 4
+    uint8_t sys_group[kUnitSystems];  // home atoms per count work item
+    uint8_t sys_row8[kUnitSystems];   // 8-byte slot rows: some winding, or reach beyond one cell
+    uint8_t sys_far[kUnitSystems];    // some winding beyond +-128
     union {
         SmallSort s;
-        SmallRows r[kSmallThreads / kWave];
+        SmallCount c;
     } u;
 };
+static_assert(sizeof(SmallLDS) <= 79 * 1024, "two workgroups share a compute unit's LDS");
 
-constexpr uint32_t kPackNeg = (1024u) | (1024u << 10) | (1024u << 20);   // pack(-w) = kPackNeg - pack(w)
+// The system of cell or atom v of a unit: the last one that starts at or before v.
+__device__ __forceinline__ int unit_sys(const int16_t *first, int n, int v)
+{
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (first[mid] <= v) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
 
 struct SmallArgs {
     const double *__restrict__ X;
@@ -1649,24 +1545,148 @@ struct SmallArgs {
     void *__restrict__ cell_offsets_out;
     int32_t *__restrict__ pair_count;
     void *__restrict__ slots;
-    int32_t cap;
+    int32_t cap, item_tests;
     Status *__restrict__ status;
 };
 
 // wrap_and_shift (cell_list.jl:105-120) of a neighbour cell index a within a
-// few cells of [1, n] on a periodic axis (rn = 1 / n as float: the floor
-// of (a - 1/2) / n is exact for |a| < 1024); on an open axis only in-bounds
+// few cells of [1, n] on a periodic axis (the floor of (a - 1/2) / n by a
+// reciprocal is exact for |a| < 1024); on an open axis only in-bounds
 // indices reach here.
-__device__ __forceinline__ void wrap_small(int32_t a, int32_t n, float rn, bool p, int32_t &w, int32_t &s)
+__device__ __forceinline__ void wrap_small(int32_t a, int32_t n, bool p, int32_t &w, int32_t &s)
 {
     if (!p) {
         w = a;
         s = 0;
         return;
     }
-    const int32_t q = (int32_t)floorf(((float)a - 0.5f) * rn);
+    const int32_t q = (int32_t)floorf(((float)a - 0.5f) * __builtin_amdgcn_rcpf((float)n));
     w = a - q * n;
     s = q;
+}
+
+// pack_wind of components known to fit.
+__device__ __forceinline__ uint32_t pack_fields(int32_t x, int32_t y, int32_t z)
+{
+    return kPackZero + (uint32_t)x + ((uint32_t)y << 10) + ((uint32_t)z << 20);
+}
+
+// The share of the home group's extent in the filter's error bound: times the
+// largest |p_i|^2 / 2 of the group (see small_bounds for the rest).
+constexpr float kSmallTol = 0.505f * 1.25f / (1 << 24) * 156.0f;
+
+// A system's table entry, read through the scalar cache (nothing writes it
+// while the kernel runs).
+using SysConst = const __attribute__((address_space(4))) SysDev;
+__device__ __forceinline__ SysConst *sys_const(const SysDev *p)
+{
+    return (SysConst *)(uintptr_t)p;
+}
+
+// The largest of the lanes' non-negative values, on the last lane.
+__device__ __forceinline__ float wave_max_f32(float x)
+{
+    int v = __builtin_bit_cast(int, x);   // non-negative floats order as their bits
+    v = max(v, dpp_or_zero<0x111>(v));
+    v = max(v, dpp_or_zero<0x112>(v));
+    v = max(v, dpp_or_zero<0x114>(v));
+    v = max(v, dpp_or_zero<0x118>(v));
+    v = max(v, dpp_or_zero<0x142, 0xa>(v));
+    v = max(v, dpp_or_zero<0x143, 0xc>(v));
+    return __builtin_bit_cast(float, v);
+}
+
+// The 64-bit test of atoms i, j of a system (X: its positions) with packed cell
+// shift S: -1 for a hit, 1 otherwise (out of line, see tile_exact).
+__device__ __attribute__((noinline)) float small_exact(const double *X, const SysDev *sd, int i, int j, uint32_t S)
+{
+    X += 3 * sd->atom_base;
+    double r2 = 0.0;
+#pragma unroll 1
+    for (int k = 0; k < 3; ++k) {
+        // R = xj - xi + C' * S ; r^2 = dot(R, R)  (gpu_kernels.jl:89-92)
+        int32_t Sx, Sy, Sz;
+        unpack_wind(S, Sx, Sy, Sz);
+        const double *C = sd->C + 3 * k;
+        const double R = (X[3 * j + k] - X[3 * i + k]) + ((C[0] * (double)Sx + C[1] * (double)Sy) + C[2] * (double)Sz);
+        r2 = k == 0 ? R * R : r2 + R * R;
+    }
+    return r2 < sd->rc2 ? -1.0f : 1.0f;
+}
+
+// small_kernel's side of tile_rows.
+struct SmallEnv {
+    static constexpr bool kLimit = true;
+    const double *X;
+    const SysDev *sd;
+    const TAtom *a_;         // home atom 0
+    const TileCands &C;
+    const TileHomes &H;
+    const TAtom *all;
+
+    template <int MODE>
+    __device__ __forceinline__ float exact(int a, int g) const
+    {
+        uint32_t S;
+        if constexpr (MODE == kEntry4) {
+            const uint32_t c = (uint32_t)C.ent[g] >> 26;   // two bits per component: its low ones
+            S = kPackZero - kFieldsLow + (((c + 1) & 3u) | ((c + 4) & 12u) << 8 | ((c + 16) & 48u) << 16);
+        } else {
+            S = C.ct[g] - (uint32_t)__builtin_amdgcn_readlane((int)H.t, a);
+        }
+        const float d = small_exact(X, sd, sgpr(a_[a].j), all[C.li[g]].j, S);
+        return C.li[g] == kUnitAtoms ? 1.0f : d;
+    }
+};
+
+// A batch of segments against the home atoms of a system with windings beyond
+// +-128, whose packed differences could leave their fields: 64-bit tests, S
+// taken apart; an S beyond +-511 sends the build to 16-byte entries.  Lane:
+// ex, st, sh of a segment; fill of a home atom, returned.  ks: the self
+// candidate of home atom 0.
+__device__ __forceinline__ int32_t small_far(const SmallArgs &A, const SmallLDS &L, SysConst *sd, int total, int ex, int st,
+                                             uint32_t sh, int hb, int nh, int ks, int32_t fill)
+{
+    const int lane = lane_id();
+    const int64_t base = sd->atom_base;
+    for (int k0 = 0; k0 < total; k0 += kWave) {
+        const int k = k0 + lane;
+        int q = 0;   // the last segment that starts at or before candidate k
+#pragma unroll
+        for (int step = kWave / 2; step >= 1; step >>= 1)
+            if (__shfl(ex, q + step, kWave) <= k) q += step;
+        const int dl = __shfl(st - ex, q, kWave);
+        const uint32_t s = (uint32_t)__shfl((int)sh, q, kWave);
+        const int li = k < total ? k + dl : kUnitAtoms;
+        const int64_t j = L.a[li].j;
+        int32_t sx, sy, sz, wx, wy, wz;
+        unpack_wind(s, sx, sy, sz);
+        unpack_wind(L.w[li], wx, wy, wz);
+        const double cx = A.X[3 * (base + j)], cy = A.X[3 * (base + j) + 1], cz = A.X[3 * (base + j) + 2];
+        for (int a = 0; a < nh; ++a) {
+            const int64_t i = sgpr(L.a[hb + a].j);
+            int32_t ix, iy, iz;
+            unpack_wind((uint32_t)sgpr((int)L.w[hb + a]), ix, iy, iz);
+            // R = xj - xi + C' * S ; r^2 = dot(R, R)  (gpu_kernels.jl:89-92)
+            const int32_t Sx = sx - wx + ix, Sy = sy - wy + iy, Sz = sz - wz + iz;
+            double tx, ty, tz;
+            cell_shift(sd->C, Sx, Sy, Sz, tx, ty, tz);
+            const double Rx = (cx - A.X[3 * (base + i)]) + tx, Ry = (cy - A.X[3 * (base + i) + 1]) + ty,
+                         Rz = (cz - A.X[3 * (base + i) + 2]) + tz;
+            const double r2 = (Rx * Rx + Ry * Ry) + Rz * Rz;
+            const uint64_t m = __builtin_amdgcn_ballot_w64(r2 < sd->rc2 && k < total && k != ks + a);
+            const int32_t f = __builtin_amdgcn_readlane(fill, a);
+            const int rank = (f >> 3) + (int)mbcnt64(m);
+            if (((m >> lane) & 1) && rank < A.cap) {
+                const uint32_t spk = pack_wind(Sx, Sy, Sz);
+                if (spk & kWindBig) A.status->wide = 1;
+                reinterpret_cast<uint64_t *>(A.slots)[slot_row(base + i, A.cap) + rank] =
+                    (uint64_t)(uint32_t)j | (uint64_t)spk << 32;
+            }
+            fill = write_lane(f + 8 * (int)__popcll(m), a, fill);
+        }
+    }
+    return fill;
 }
 
 template <typename TI>
@@ -1683,24 +1703,24 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
     const int32_t C0 = A.sys_cell_base[s0];
     const int M_u = A.sys_cell_base[s0 + ns] - C0;
     for (int k = tid; k <= ns; k += kSmallThreads) {
-        L.sys_cell0[k] = A.sys_cell_base[s0 + k] - C0;
-        L.sys_atom0[k] = (int32_t)(A.sys_atom_base[s0 + k] - A0);
+        L.sys_cell0[k] = (int16_t)(A.sys_cell_base[s0 + k] - C0);
+        L.sys_atom0[k] = (int16_t)(A.sys_atom_base[s0 + k] - A0);
         if (k < ns) {
             const SysDev &sd = A.sys[s0 + k];
             L.sys_row8[k] = (sd.nxyz[0] > 1 || sd.nxyz[1] > 1 || sd.nxyz[2] > 1) ? 1 : 0;
+            L.sys_far[k] = 0;
+            L.sys_geo[k] = (uint32_t)(sd.n[0] | sd.n[1] << 9 | sd.n[2] << 18) | (uint32_t)sd.pbc << 27;
+            L.sys_reach[k] = (uint8_t)(sd.nxyz[0] | sd.nxyz[1] << 2 | sd.nxyz[2] << 4);
             // candidates per home atom: the system's mean cell occupancy times its neighbour cells
             const int nseg = (2 * sd.nxyz[0] + 1) * (2 * sd.nxyz[1] + 1) * (2 * sd.nxyz[2] + 1);
             const int chunks = max(1, (int)((nseg * (int64_t)sd.nat / max(sd.M, 1) + kWave - 1) / kWave));
-            L.sys_group[k] = min(kWave, max(kMinGroup, kItemTests / chunks));
+            L.sys_group[k] = (uint8_t)min(kWave, max(kMinGroup, A.item_tests / chunks));
         }
     }
     for (int c = tid; c < M_u; c += kSmallThreads) L.u.s.fill[c] = 0;
     if (tid == 0) {
-        LAtom f;
-        f.x = f.y = f.z = kFar;
-        f.j = 0;
-        f.t = kPackZero;
-        L.a[kUnitAtoms] = f;
+        L.a[kUnitAtoms] = TAtom{kFar32, 0.0f, 0.0f, 0};
+        L.w[kUnitAtoms] = kPackZero;
         L.next_item = kSmallThreads / kWave;   // wave w starts at the part's item w
     }
     __syncthreads();
@@ -1708,7 +1728,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
     // cell_list.jl:66-74, 141-147), atoms per cell
     bool bad = false, big = false;
     for (int i = tid; i < nat_u; i += kSmallThreads) {
-        const int k = find_sys(L.sys_atom0, ns, (int32_t)i);
+        const int k = unit_sys(L.sys_atom0, ns, i);
         const SysDev &sd = A.sys[s0 + k];
         const int64_t g = A0 + i;
         int32_t c[3], w[3];
@@ -1719,6 +1739,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
         L.u.s.wk[i] = wp;
         L.u.s.sy[i] = (uint8_t)k;
         if (wp != kPackZero) L.sys_row8[k] = 1;
+        if ((unsigned)(w[0] + 128) > 256u || (unsigned)(w[1] + 128) > 256u || (unsigned)(w[2] + 128) > 256u) L.sys_far[k] = 1;
         big |= (wp & kWindBig) != 0;
         atomicAdd(&L.u.s.fill[key], 1);
         if (writer) A.atom_sys[g] = s0 + k;   // the fill kernel's map of atoms to systems
@@ -1726,16 +1747,23 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
     if (bad) atomicOr(&A.status->bad_position, 1);
     if (big) atomicOr(&A.status->small_fallback, 1);   // the general pipeline redoes the build
     __syncthreads();
-    {   // cell starts: exclusive scan of the counts, two cells per thread
-        const int c = 2 * tid;
-        const int v0 = c < M_u ? L.u.s.fill[c] : 0, v1 = c + 1 < M_u ? L.u.s.fill[c + 1] : 0;
+    {   // cell starts: exclusive scan of the counts, kThreadCells cells per thread
+        const int c0 = kThreadCells * tid;
+        int v[kThreadCells], sum = 0;
+#pragma unroll
+        for (int m = 0; m < kThreadCells; ++m) {
+            v[m] = c0 + m < M_u ? L.u.s.fill[c0 + m] : 0;
+            sum += v[m];
+            if (c0 + m < M_u) L.u.s.fill[c0 + m] = 0;
+        }
         int64_t tot;
-        const int ex = (int)block_excl_scan_n<kSmallThreads>(v0 + v1, tot);   // its barriers end every read of fill
-        if (c < M_u) L.cs[c] = ex;
-        if (c + 1 < M_u) L.cs[c + 1] = ex + v0;
-        if (tid == 0) L.cs[M_u] = (int32_t)tot;
-        if (c < M_u) L.u.s.fill[c] = 0;
-        if (c + 1 < M_u) L.u.s.fill[c + 1] = 0;
+        int ex = (int)block_excl_scan_n<kSmallThreads>(sum, tot);
+#pragma unroll
+        for (int m = 0; m < kThreadCells; ++m) {
+            if (c0 + m < M_u) L.cs[c0 + m] = (int16_t)ex;
+            ex += v[m];
+        }
+        if (tid == 0) L.cs[M_u] = (int16_t)tot;
     }
     __syncthreads();
     for (int i = tid; i < nat_u; i += kSmallThreads) {   // atoms grouped by cell
@@ -1753,32 +1781,43 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
         const int p = st + rank;
         const int k = L.u.s.sy[i];
         const int64_t g = A0 + i;
-        LAtom la;
-        la.x = A.X[3 * g];
-        la.y = A.X[3 * g + 1];
-        la.z = A.X[3 * g + 2];
-        la.j = i - L.sys_atom0[k];
-        la.t = L.u.s.wk[i];
-        L.a[p] = la;
+        const SysDev &sd = A.sys[s0 + k];
+        const double x = A.X[3 * g], y = A.X[3 * g + 1], z = A.X[3 * g + 2];
+        const uint32_t wk = L.u.s.wk[i];
+        double ux = x - 0.5 * (sd.C[0] + sd.C[1] + sd.C[2]), uy = y - 0.5 * (sd.C[3] + sd.C[4] + sd.C[5]),
+               uz = z - 0.5 * (sd.C[6] + sd.C[7] + sd.C[8]);
+        if (wk != kPackZero) {
+            int32_t wx, wy, wz;
+            unpack_wind(wk, wx, wy, wz);
+            double cx, cy, cz;
+            cell_shift(sd.C, wx, wy, wz, cx, cy, cz);
+            ux -= cx;
+            uy -= cy;
+            uz -= cz;
+        }
+        const int32_t jl = i - L.sys_atom0[k];
+        L.a[p] = TAtom{(float)ux, (float)uy, (float)uz, jl};
+        L.w[p] = wk;
         if (writer) {
             Rec r;
-            r.x = la.x;
-            r.y = la.y;
-            r.z = la.z;
-            r.j = la.j;
-            r.w = la.t;
+            r.x = x;
+            r.y = y;
+            r.z = z;
+            r.j = jl;
+            r.w = wk;
             A.rec[A0 + p] = r;
-            store_ti<TI>(A.perm_out, A0 + p, (int64_t)la.j + 1);
+            store_ti<TI>(A.perm_out, A0 + p, (int64_t)jl + 1);
             store_ti<TI>(A.cell_id_out, A0 + p, (int64_t)(key - L.sys_cell0[k]) + 1);
         }
     }
+    __syncthreads();   // the sorted atoms are complete; the sort's LDS now holds the count's
     // cell offsets: per system, 1-based, its cells then a trailing entry;
     // the system and the grid coordinates of every cell for the count
     for (int c = tid; c < M_u; c += kSmallThreads) {
-        const int k = find_sys(L.sys_cell0, ns, (int32_t)c);
-        const int lc = c - L.sys_cell0[k], n0 = A.sys[s0 + k].n[0], n1 = A.sys[s0 + k].n[1];
-        L.cell_info[c] = (uint32_t)k | (uint32_t)(lc % n0) << 8 | (uint32_t)((lc / n0) % n1) << 16 |
-                         (uint32_t)(lc / (n0 * n1)) << 24;
+        const int k = unit_sys(L.sys_cell0, ns, c);
+        const int lc = c - L.sys_cell0[k], n0 = (int)(L.sys_geo[k] & 511u), n1 = (int)((L.sys_geo[k] >> 9) & 511u);
+        L.u.c.cell_info[c] = (uint32_t)k | (uint32_t)(lc % n0) << 8 | (uint32_t)((lc / n0) % n1) << 16 |
+                             (uint32_t)(lc / (n0 * n1)) << 24;
         const int64_t gc = (int64_t)C0 + c + s0 + k;
         if (writer) {
             store_ti<TI>(A.cell_offsets_out, gc, (int64_t)(L.cs[c] - L.sys_atom0[k]) + 1);
@@ -1786,82 +1825,123 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
                 store_ti<TI>(A.cell_offsets_out, gc + 1, (int64_t)(L.sys_atom0[k + 1] - L.sys_atom0[k]) + 1);
         }
     }
-    __syncthreads();   // cell starts, cell info and the sorted atoms are complete
+    __syncthreads();
     {   // count work items, numbered in cell order: the cells' item counts, scanned
-        const int c = 2 * tid;
-        int v0 = 0, v1 = 0;
-        if (c < M_u) {
-            const int g = L.sys_group[L.cell_info[c] & 255u];
-            v0 = (L.cs[c + 1] - L.cs[c] + g - 1) / g;
-        }
-        if (c + 1 < M_u) {
-            const int g = L.sys_group[L.cell_info[c + 1] & 255u];
-            v1 = (L.cs[c + 2] - L.cs[c + 1] + g - 1) / g;
+        const int c0 = kThreadCells * tid;
+        int v[kThreadCells], sum = 0;
+#pragma unroll
+        for (int m = 0; m < kThreadCells; ++m) {
+            v[m] = 0;
+            if (c0 + m < M_u) {
+                const int g = L.sys_group[L.u.c.cell_info[c0 + m] & 255u];
+                v[m] = (L.cs[c0 + m + 1] - L.cs[c0 + m] + g - 1) / g;
+            }
+            sum += v[m];
         }
         int64_t tot;
-        const int ex = (int)block_excl_scan_n<kSmallThreads>(v0 + v1, tot);
-        if (c < M_u) L.item0[c] = (int16_t)ex;
-        if (c + 1 < M_u) L.item0[c + 1] = (int16_t)(ex + v0);
-        if (tid == 0) L.item0[M_u] = (int16_t)tot;
-        __syncthreads();
-        for (int t = 0; t < v0; ++t) L.item_cell[ex + t] = (int16_t)c;
-        for (int t = 0; t < v1; ++t) L.item_cell[ex + v0 + t] = (int16_t)(c + 1);
+        int ex = (int)block_excl_scan_n<kSmallThreads>(sum, tot);
+#pragma unroll
+        for (int m = 0; m < kThreadCells; ++m) {
+            if (c0 + m < M_u) L.u.c.item0[c0 + m] = (int16_t)ex;
+            for (int t = 0; t < v[m]; ++t) L.u.c.item_cell[ex + t] = (int16_t)(c0 + m);
+            ex += v[m];
+        }
+        if (tid == 0) L.u.c.item0[M_u] = (int16_t)tot;
     }
-    __syncthreads();   // the items are numbered; the sort's LDS now holds the waves' segment maps
-    const int nitems_u = L.item0[M_u];
-    SmallRows &Rw = L.u.r[wv];
+    __syncthreads();   // the items are numbered
+    const int nitems_u = L.u.c.item0[M_u];
+    SmallRows &Rw = L.u.c.r[wv];
     uint8_t *fl = reinterpret_cast<uint8_t *>(Rw.flag);
+    // (dx, dy, dz) of segment `lane` where the reach is one cell on every axis
+    const int ndz = lane / 9 - 1, ndy = lane / 3 - 3 * (lane / 9) - 1, ndx = lane - 3 * (lane / 3) - 1;
     for (int it = part + parts * wv; it < nitems_u; it = part + parts * take_next(&L.next_item)) {
-        const int hc = sgpr(L.item_cell[it]);
-        const int ig = it - sgpr(L.item0[hc]);   // the item's group of home atoms in its cell
+        const int hc = sgpr(L.u.c.item_cell[it]);
+        const int ig = it - sgpr(L.u.c.item0[hc]);   // the item's group of home atoms in its cell
         const int h0 = sgpr(L.cs[hc]), nha_c = sgpr(L.cs[hc + 1]) - h0;
-        const uint32_t info = (uint32_t)sgpr((int)L.cell_info[hc]);
+        const uint32_t info = (uint32_t)sgpr((int)L.u.c.cell_info[hc]);
         const int k = (int)(info & 255u);
         const int grp = sgpr(L.sys_group[k]);
         const int hg0 = ig * grp, nha = min(nha_c, hg0 + grp);   // home atoms [hg0, nha) of the cell
-        const SysDev &sd = A.sys[s0 + k];
+        const SysConst *sd = sys_const(A.sys + s0 + k);
         const int cb = sgpr(L.sys_cell0[k]);
-        const int n0 = sd.n[0], n1 = sd.n[1], n2 = sd.n[2];
+        const uint32_t geo = (uint32_t)sgpr((int)L.sys_geo[k]), rch = (uint32_t)sgpr((int)L.sys_reach[k]);
+        const int n0 = (int)(geo & 511u), n1 = (int)((geo >> 9) & 511u), n2 = (int)((geo >> 18) & 511u);
+        const bool p0 = (geo >> 27 & 1) != 0, p1 = (geo >> 28 & 1) != 0, p2 = (geo >> 29 & 1) != 0;
+        const int nx0 = (int)(rch & 3u), nx1 = (int)((rch >> 2) & 3u), nx2 = (int)(rch >> 4);
         const int ci0 = (int)((info >> 8) & 255u) + 1, ci1 = (int)((info >> 16) & 255u) + 1, ci2 = (int)(info >> 24) + 1;
-        const int nx0 = sd.nxyz[0], nx1 = sd.nxyz[1], nx2 = sd.nxyz[2];
         const int sxn = 2 * nx0 + 1, syn = 2 * nx1 + 1;
-        // quotients of the small integers below by float reciprocals: exact,
-        // as every numerator is within a few hundred of zero and a half away
-        // from a multiple of the divisor
-        const float rsx = 1.0f / (float)sxn, rsy = 1.0f / (float)syn;
-        const float rn0 = 1.0f / (float)n0, rn1 = 1.0f / (float)n1, rn2 = 1.0f / (float)n2;
         const int nseg = sxn * syn * (2 * nx2 + 1);
         const int center = (nx2 * syn + nx1) * sxn + nx0;   // (dx, dy, dz) = 0: the home cell, zero shift
-        const bool p0 = (sd.pbc & 1) != 0, p1 = (sd.pbc & 2) != 0, p2 = (sd.pbc & 4) != 0;
-        const bool narrow = sgpr(L.sys_row8[k]) == 0;   // every S in [-1, 1]^3: 4-byte slot entries
+        const bool row8 = sgpr(L.sys_row8[k]) != 0, far = sgpr(L.sys_far[k]) != 0;
+        const bool near = rch == 0x15u;   // a reach of one cell on every axis
+        // the home cell's centre, from the system's
+        const auto &C32 = sd->C32;
+        const float f0 = ((float)ci0 - 0.5f) * __builtin_amdgcn_rcpf((float)n0) - 0.5f,
+                    f1 = ((float)ci1 - 0.5f) * __builtin_amdgcn_rcpf((float)n1) - 0.5f,
+                    f2 = ((float)ci2 - 0.5f) * __builtin_amdgcn_rcpf((float)n2) - 0.5f;
+        const float ox = C32[0] * f0 + C32[1] * f1 + C32[2] * f2, oy = C32[3] * f0 + C32[4] * f1 + C32[5] * f2,
+                    oz = C32[6] * f0 + C32[7] * f1 + C32[8] * f2;
         for (int hg = hg0; hg < nha; hg += kWave) {
             const int nh = sgpr(min(kWave, nha - hg));
             const int hb = h0 + hg;
             const int hl = hb + (lane < nh ? lane : 0);
-            const uint32_t ht_l = kPackNeg - L.a[hl].t;   // pack(-w_i)
-            const int32_t hj_l = L.a[hl].j;
-            int32_t cnt_l = 0;
+            const TAtom h = L.a[hl];
+            TileHomes H;
+            H.nx = ox - h.x;
+            H.ny = oy - h.y;
+            H.nz = oz - h.z;
+            const float hq = 0.5f * __builtin_fmaf(H.nz, H.nz, __builtin_fmaf(H.ny, H.ny, H.nx * H.nx));
+            H.ai = hq - sd->rc2half;
+            const int64_t ha = sd->atom_base + h.j;
+            H.row = (reinterpret_cast<uint64_t>(A.slots) + 8ull * (uint64_t)slot_row(ha, A.cap)) |
+                    (uint64_t)(row8 ? 8 : 4) << 48;
+            H.t = 2 * kPackZero - L.w[hl];   // t'_i = -w_i
+            H.fill = 0;
+            // the filter's error bound (small_bounds); beyond any sane scale, 64-bit tests for all
+            const float hm = readlane_f32(wave_max_f32(hq), kWave - 1);
+            const float tol = hm < 1.0e30f ? __builtin_fmaf(hm, kSmallTol, sd->small_tol) : kFar32 * kFar32;
             for (int sb = 0; sb < nseg; sb += kWave) {
                 // lane: neighbour cell sb + lane in the reference order, its
                 // sorted atoms and cell shift (_is_cell_in_bounds,
                 // _get_neighbor_cell, gpu_kernels.jl:20-47)
                 const int gs = sb + lane;
                 int st = 0, len = 0;
-                uint32_t shp = kPackZero;
+                SegShift v;
                 if (gs < nseg) {
-                    const int t2 = (int)(((float)gs + 0.5f) * rsx), t3 = (int)(((float)t2 + 0.5f) * rsy);
-                    const int dx = gs - t2 * sxn - nx0, dy = t2 - t3 * syn - nx1, dz = t3 - nx2;
+                    int dx = ndx, dy = ndy, dz = ndz;
+                    if (!near) {
+                        // quotients of small integers by float reciprocals: exact, as every
+                        // numerator is within a few hundred of zero and a half away from a
+                        // multiple of the divisor
+                        const int t2 = (int)(((float)gs + 0.5f) * __builtin_amdgcn_rcpf((float)sxn));
+                        const int t3 = (int)(((float)t2 + 0.5f) * __builtin_amdgcn_rcpf((float)syn));
+                        dx = gs - t2 * sxn - nx0;
+                        dy = t2 - t3 * syn - nx1;
+                        dz = t3 - nx2;
+                    }
                     const int a0 = ci0 + dx, a1 = ci1 + dy, a2 = ci2 + dz;
-                    if ((p0 || (a0 >= 1 && a0 <= n0)) && (p1 || (a1 >= 1 && a1 <= n1)) &&
-                        (p2 || (a2 >= 1 && a2 <= n2))) {
+                    if ((p0 || (unsigned)(a0 - 1) < (unsigned)n0) && (p1 || (unsigned)(a1 - 1) < (unsigned)n1) &&
+                        (p2 || (unsigned)(a2 - 1) < (unsigned)n2)) {
                         int32_t c0, c1, c2, s0x, s0y, s0z;
-                        wrap_small(a0, n0, rn0, p0, c0, s0x);
-                        wrap_small(a1, n1, rn1, p1, c1, s0y);
-                        wrap_small(a2, n2, rn2, p2, c2, s0z);
-                        const int uc = cb + (c0 - 1) + (c1 - 1) * n0 + (c2 - 1) * n0 * n1;
+                        if (near) {   // in bounds, or periodic: at most one wrap
+                            wrap_near(a0, n0, c0, s0x);
+                            wrap_near(a1, n1, c1, s0y);
+                            wrap_near(a2, n2, c2, s0z);
+                        } else {
+                            wrap_small(a0, n0, p0, c0, s0x);
+                            wrap_small(a1, n1, p1, c1, s0y);
+                            wrap_small(a2, n2, p2, c2, s0z);
+                        }
+                        const int uc = cb + (c0 - 1) + ((c1 - 1) + (c2 - 1) * n1) * n0;
                         st = L.cs[uc];
                         len = L.cs[uc + 1] - st;
-                        shp = pack_wind(s0x, s0y, s0z);
+                        // a 4-byte system: the S code of every atom of the segment (w = 0)
+                        v.s = row8 ? pack_fields(s0x, s0y, s0z)
+                                   : (uint32_t)((s0x & 3) | (s0y & 3) << 2 | (s0z & 3) << 4) << 26;
+                        const float fx = (float)s0x, fy = (float)s0y, fz = (float)s0z;
+                        v.x = __builtin_fmaf(C32[0], fx, __builtin_fmaf(C32[1], fy, __builtin_fmaf(C32[2], fz, -ox)));
+                        v.y = __builtin_fmaf(C32[3], fx, __builtin_fmaf(C32[4], fy, __builtin_fmaf(C32[5], fz, -oy)));
+                        v.z = __builtin_fmaf(C32[6], fx, __builtin_fmaf(C32[7], fy, __builtin_fmaf(C32[8], fz, -oz)));
                     }
                 }
                 const int incl = wave_incl_scan(len);
@@ -1871,43 +1951,57 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
                 const int q = (int)mbcnt64(__builtin_amdgcn_ballot_w64(ne));
                 if (ne) {
                     Rw.dl[q] = st - ex;
-                    Rw.sh[q] = shp;
+                    Rw.sv[q] = v;
                 }
                 // home atom hg + a is candidate ex(center) + hg + a of the
                 // center segment, when that segment is in this batch
                 const int cl = center - sb;
-                const int self0 = (cl >= 0 && cl < kWave) ? __builtin_amdgcn_readlane(ex, cl) : -(1 << 28);
-                for (int k0 = 0; k0 < total; k0 += kPassCands) {
-                    const int nch = sgpr(min(kBrickChunks, (total - k0 + kWave - 1) / kWave));
+                const int self0 = (cl >= 0 && cl < kWave) ? __builtin_amdgcn_readlane(ex, cl) : 1 << 28;
+                if (far) {
+                    H.fill = small_far(A, L, sd, total, ex, st, v.s, hb, nh, self0 + hg, H.fill);
+                    continue;
+                }
+                for (int k0 = 0; k0 < total; k0 += kTileCands) {
+                    const int nch = sgpr(min(kTileChunks, (total - k0 + kWave - 1) / kWave));
                     // marks where a non-empty segment other than the first starts
-                    if (lane < kPassCands / 4) Rw.flag[lane] = 0u;
+                    Rw.flag[lane] = 0u;
                     const int pp = ex - k0;
-                    if (ne && q > 0 && pp > 0 && pp < kPassCands) fl[pp] = 1;
-                    int acc = (int)__popcll(__builtin_amdgcn_ballot_w64(ne && q > 0 && pp <= 0));
-                    double cx[kBrickChunks], cy[kBrickChunks], cz[kBrickChunks];
-                    uint64_t ent[kBrickChunks];
+                    if (ne && q > 0 && pp > 0 && pp < kTileCands) fl[pp] = 1;
+                    int acc = k0 == 0 ? 0 : (int)__popcll(__builtin_amdgcn_ballot_w64(ne && q > 0 && pp <= 0));
+                    TileCands C;
 #pragma unroll
-                    for (int g = 0; g < kBrickChunks; ++g) {
+                    for (int g = 0; g < kTileChunks; ++g) {
                         const uint64_t bm = __builtin_amdgcn_ballot_w64(fl[g * kWave + lane] != 0);
                         const int qk = acc + (int)(bm & 1u) + (int)mbcnt64(bm >> 1);
                         acc += (int)__popcll(bm);
                         const int kk = k0 + g * kWave + lane;
-                        const int li = kk < total ? kk + Rw.dl[qk] : kUnitAtoms;   // else the far sentinel
-                        const uint32_t sh = Rw.sh[qk];
-                        const LAtom c = L.a[li];
-                        cx[g] = c.x;
-                        cy[g] = c.y;
-                        cz[g] = c.z;
-                        const uint32_t t = sh - c.t + kPackZero;   // pack(s - w_j)
-                        const uint32_t code = (t & 3u) | ((t >> 8) & 12u) | ((t >> 16) & 48u);
-                        const uint32_t lo = narrow ? ((uint32_t)c.j | code << 26) : (uint32_t)c.j;
-                        ent[g] = (uint64_t)lo | ((uint64_t)t << 32);
+                        C.li[g] = kk < total ? kk + Rw.dl[qk] : kUnitAtoms;   // else the far sentinel
+                        const SegShift t = Rw.sv[qk];
+                        const TAtom c = L.a[C.li[g]];
+                        C.bx[g] = c.x + t.x;
+                        C.by[g] = c.y + t.y;
+                        C.bz[g] = c.z + t.z;
+                        C.bq[g] = 0.5f * __builtin_fmaf(C.bz[g], C.bz[g], __builtin_fmaf(C.by[g], C.by[g], C.bx[g] * C.bx[g]));
+                        C.ent[g] = row8 ? c.j : c.j | (int)t.s;
+                        if (row8) C.ct[g] = t.s - L.w[C.li[g]] + 2 * kPackZero;
                     }
-                    pass_home_atoms<false>(narrow, nch, cx, cy, cz, ent, L.a + hb, nh, ht_l, hj_l, self0 + hg - k0,
-                                           sd.C, sd.rc2, sd.atom_base, A.slots, A.cap, A.status, cnt_l);
+                    // entries that the pass's chunks may store: what it starts with left, so
+                    // a row runs over by less than a pass (kSlotSlack)
+                    H.left = max(0, min(kWave, A.cap - (H.fill >> (row8 ? 3 : 2))));
+                    const SmallEnv E{A.X, A.sys + s0 + k, L.a + hb, C, H, L.a};
+                    const int kp = self0 + hg - k0;   // home atom hg + a is candidate kp + a of this pass
+                    if (row8) {
+                        if (nch == 4) tile_pass<4, kEntry8>(E, tol, C, nh, kp, H);
+                        else if (nch == 3) tile_pass<3, kEntry8>(E, tol, C, nh, kp, H);
+                        else tile_pass<2, kEntry8>(E, tol, C, nh, kp, H);
+                    } else {
+                        if (nch == 4) tile_pass<4, kEntry4>(E, tol, C, nh, kp, H);
+                        else if (nch == 3) tile_pass<3, kEntry4>(E, tol, C, nh, kp, H);
+                        else tile_pass<2, kEntry4>(E, tol, C, nh, kp, H);
+                    }
                 }
             }
-            if (lane < nh) A.pair_count[sd.atom_base + hj_l] = cnt_l | (narrow ? 0 : kRow8Bit);
+            if (lane < nh) A.pair_count[ha] = row8 ? (H.fill >> 3) | kRow8Bit : H.fill >> 2;
         }
     }
 }
@@ -1917,7 +2011,7 @@ static void small_launch(const PipelineBufs &b, hipStream_t st)
 {
     SmallArgs A{b.X,          b.sys,     b.sys_atom_base, b.sys_cell_base, b.units,  b.unit_order,
                 b.atom_sys,   b.rec,     b.perm_out,      b.cell_id_out,   b.cell_offsets_out,
-                b.pair_count, b.slots,   b.slot_cap,      b.status};
+                b.pair_count, b.slots,   b.slot_cap,      b.item_tests,    b.status};
     hipLaunchKernelGGL((small_kernel<TI>), dim3((unsigned)b.nitems), dim3(kSmallThreads), 0, st, A);
 }
 

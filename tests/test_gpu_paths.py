@@ -182,3 +182,74 @@ def test_R_after_the_positions_are_gone(n):
         R = np.empty((m.value, 3))
         _lib.check(L.nlh_copy_pairlist(h.ptr, None, None, None, None, R.ctypes.data))
         assert m.value == ref.npairs() and np.array_equal(_bits(R), _bits(ref.R))
+
+
+def _check_batch(systems, int_type=np.int32, want_R=False):
+    bits = 32 if int_type == np.int32 else 64
+    got = nlhip.BatchBuilder(int_type=int_type).run(systems, want_R=want_R)
+    for k, y in enumerate(systems):
+        ref = oracle.neighbour_list(y.X, y.cutoff, y.cell, y.pbc, ti_bits=bits, want_R=want_R)
+        nl = got.pairlist(k)
+        assert np.array_equal(nl.first, ref.first), k
+        assert np.array_equal(nl.i, ref.i) and np.array_equal(nl.j, ref.j) and np.array_equal(nl.S, ref.S), k
+
+
+@pytest.mark.parametrize("shell", [0.5, 1.0, 1.5])
+@pytest.mark.parametrize("eps", [0.0, 3e-16, -3e-16, 1e-7, -1e-7])
+@pytest.mark.parametrize("scale", [1.0, 1e-10, 1e6])
+def test_batch_cutoff_on_a_shell(shell, eps, scale):
+    """Perfect crystals with the cutoff at a neighbour distance, in units from
+    metres to micrometres per metre: every pair of that shell is decided by
+    the 64-bit test."""
+    systems = []
+    for k in range(70):
+        X, cell = workloads.fcc(3.61, (1 + k % 3, 1 + k % 5, 1 + k % 4))
+        systems.append(workloads.System((X + 0.1 * (k % 7)) * scale, cell * scale, (True, k % 2 == 0, True),
+                                        3.61 * scale * np.sqrt(shell) * (1.0 + eps)))
+    print(f"batch shell {shell} {eps} {scale}", flush=True)
+    _check_batch(systems)
+
+
+@pytest.mark.parametrize("wind", [0, 1, 128, 129, 300, 511, 512])
+@pytest.mark.parametrize("pbc", [(True, True, True), (True, False, True), (False, False, False)])
+def test_batch_windings_and_far_atoms(wind, pbc):
+    """Atoms moved by lattice vectors: inside the packed differences, beyond
+    them, and beyond the packed windings; along open axes they lie far
+    outside the cell."""
+    rng = np.random.default_rng(wind)
+    systems = []
+    for k in range(72):
+        n = [1, 2, 7, 63, 64, 65, 200, 900][k % 8]
+        cell = (np.eye(3) + 0.1 * rng.random((3, 3))) * (n / 0.06) ** (1 / 3) * (1.0, 1.0, 0.6 + 0.2 * (k % 5))
+        X = rng.random((n, 3)) @ cell
+        X += (rng.integers(-wind, wind + 1, (n, 3)) * (rng.random((n, 1)) < 0.2)) @ cell
+        systems.append(workloads.System(X, cell, pbc, 3.0 + 0.3 * (k % 6)))
+    print(f"batch windings {wind} {pbc}", flush=True)
+    _check_batch(systems, np.int64 if wind % 2 else np.int32)
+
+
+@pytest.mark.parametrize("sizes", [[2048] * 64, [1] * 700 + [2048], [2047, 1, 0, 1] * 20, [0] * 70 + [3], [2049] + [5] * 70])
+def test_batch_unit_edges(sizes):
+    """Units of one full system, of hundreds of atoms of their own system, of
+    systems without atoms; one system beyond a unit (the general pipeline)."""
+    systems = []
+    for k, n in enumerate(sizes):
+        y = workloads.random_cubic(max(n, 1), density=0.05, seed=k, cutoff=3.5 + 0.1 * (k % 9))
+        systems.append(dataclasses.replace(y, X=y.X[:n]))
+    print(f"batch units {len(sizes)}", flush=True)
+    _check_batch(systems)
+
+
+@pytest.mark.parametrize("n", [40, 400, 2000])
+def test_batch_rows_that_overflow(n):
+    """Clusters whose atoms outgrow the estimated slot rows by far, the last
+    atoms of the batch among them, in cells whose images are neighbours too."""
+    rng = np.random.default_rng(n)
+    systems = []
+    for k in range(66):
+        cell = np.eye(3) * (6.0 if k % 3 == 0 else 40.0)
+        X = rng.random((n if k % 3 else 20, 3)) * 40.0
+        X[-min(n, 30):] = 20.0 + 0.5 * rng.random((len(X[-min(n, 30):]), 3))
+        systems.append(workloads.System(X, cell, (True, True, k % 2 == 0), 5.0))
+    print(f"batch overflow {n}", flush=True)
+    _check_batch(systems)
