@@ -550,6 +550,7 @@ void filter_bounds(nlh::SysDev &sd, const nlh_geometry &g)
     const bool ok = H < 1000 * rc && P < 1e6 * rc && rc > 1e-14 && rc < 1e9;
     sd.rc2half = (float)(0.5 * g.cutoff_sq);
     sd.tol = (float)(0.505 * tol);
+    sd.tol64 = (float)(1.6e-11 * rc * sum);
     sd.h2half = (float)(0.499 * H * H);
     sd.pmax2 = ok ? (float)(0.999 * P * P) : -1.0f;
 }

@@ -107,8 +107,9 @@ struct SysDev {
     // with every brick atom within sqrt(pmax2) of the brick's origin and every
     // home atom within sqrt(2 h2half) of its group's, the filter's value of
     // (r^2 - rc^2) / 2 has the sign of the 64-bit test wherever it is at least
-    // tol away from zero.  pmax2 < 0: the system does not use the filter.
-    float rc2half, tol, h2half, pmax2;
+    // tol away from zero (further out: see far_tol, which takes the 64-bit
+    // roundings' share from tol64).  pmax2 < 0: the system does not use the filter.
+    float rc2half, tol, h2half, pmax2, tol64;
     float small_tol;       // ... in small_kernel, less its home group's share (set by small_bounds)
     float C32[9];          // C in 32 bits
     int32_t run;           // home cells along x that share a candidate list (tile_kernel): 1 or 2

@@ -270,15 +270,28 @@ __device__ __forceinline__ Cand load_candidate(const PairsArgs &A, int k, int to
     return c;
 }
 
+// Home atoms of a cell from which the waves of its brick share it (10k atoms
+// clamped into a quarter of an open cell: 294 us unshared, 174 shared).
+constexpr int kShareHome = 32;
+
 // Per-wave count of one home cell from global memory: test every (home
 // atom, chunk) and append hits to the slots (the brick path's fallback, and
 // the path for neighbour reach beyond one cell).
 template <bool WIDE>
 __device__ __forceinline__ void count_cell(const PairsArgs &A, const SysDev &sd, int cell, int32_t *__restrict__ pair_count,
-                                        const SlotArgs &O)
+                                        const SlotArgs &O, int turn, int part, int parts)
 {
     HomeCell H;
     home_cell(A, sd, cell, H);
+    // a cell that atoms were clamped into may hold thousands: all `parts`
+    // waves share its home atoms; a smaller cell is one wave's, in turn
+    const int n = H.he - H.hs;
+    if (n > kShareHome) {
+        H.he = H.hs + (int)((int64_t)n * (part + 1) / parts);
+        H.hs += (int)((int64_t)n * part / parts);
+    } else if (turn % parts != part) {
+        return;
+    }
     if (H.hs >= H.he) return;
     const int lane = lane_id();
     const double *__restrict__ Cm = sd.C;
@@ -883,8 +896,8 @@ __global__ __launch_bounds__(BT) void count_kernel(
     if (!lds) {
         const SlotArgs O{slots, cap, status};
         const int wv0 = sgpr((int)(threadIdx.x >> 6));
-        for (int hc = wv0; hc < B.nhome; hc += BrickShape<BT>::waves)
-            count_cell<true>(A, *B.sd, brick_cell_id(B, hc), pair_count, O);
+        for (int hc = 0; hc < B.nhome; ++hc)
+            count_cell<true>(A, *B.sd, brick_cell_id(B, hc), pair_count, O, hc, wv0, BrickShape<BT>::waves);
         return;
     }
     const SysDev &sd = *B.sd;
@@ -1011,6 +1024,7 @@ struct TileLDS {
     int32_t next_item;              // the next work item a wave takes
     int32_t total, flag;
     int32_t row8;                   // some shift needs 8-byte slot entries
+    int32_t far2;                   // largest |p|^2 beyond the system's pmax2 (its bits), or 0
 };
 
 constexpr float kFar32 = 1.0e18f;   // sentinel position: |p|^2 / 2 = 5e35, never a hit
@@ -1045,8 +1059,7 @@ __device__ __forceinline__ void tile_run(const Brick &B, const TileRuns &T, int 
 
 // Stage the brick and its halo in LDS.  Returns false (for every thread of
 // the block) when the brick must take the global-memory path: more halo
-// atoms than the LDS holds, windings beyond +-128, or atoms further out than
-// the filter's bounds allow (clamped into the grid from far outside).
+// atoms than the LDS holds, or windings beyond +-128.
 template <int BT>
 __device__ bool tile_load(const PairsArgs &A, const Brick &B, const TileRuns &T, TileLDS<BT> &L, const double *Csh)
 {
@@ -1089,6 +1102,7 @@ __device__ bool tile_load(const PairsArgs &A, const Brick &B, const TileRuns &T,
         L.hoff[B.nhalo] = tot;
         L.next_item = Sh::waves;
         L.flag = 0;
+        L.far2 = 0;
         L.row8 = sd.nat > kNarrowMaxAtoms ? 1 : 0;
         L.a[Sh::cap] = TAtom{kFar32, 0.0f, 0.0f, 0};
         L.t[Sh::cap] = kPackZero;
@@ -1146,7 +1160,9 @@ __device__ bool tile_load(const PairsArgs &A, const Brick &B, const TileRuns &T,
                 dz += cz;
             }
             const float fx = (float)dx, fy = (float)dy, fz = (float)dz;
-            bad |= !(fx * fx + fy * fy + fz * fz <= sd.pmax2);
+            // an atom clamped into the grid from far outside (non-negative floats order as their bits)
+            const float f2 = fx * fx + fy * fy + fz * fz;
+            if (!(f2 <= sd.pmax2)) atomicMax(&L.far2, __builtin_bit_cast(int, f2));
             // 4-byte slot entries need every S = t'_j - t'_i within [-1, 1]^3: home
             // atoms with t' = 0 and halo atoms with |t'_k| <= 1
             const uint32_t c = t - 511u * kFieldsLow;   // fields 0, 1, 2 then
@@ -1224,6 +1240,33 @@ struct TileHomes {
 __device__ __forceinline__ float readlane_f32(float v, int l)
 {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
+
+// The largest of the lanes' non-negative values, on the last lane.
+__device__ __forceinline__ float wave_max_f32(float x)
+{
+    int v = __builtin_bit_cast(int, x);   // non-negative floats order as their bits
+    v = max(v, dpp_or_zero<0x111>(v));
+    v = max(v, dpp_or_zero<0x112>(v));
+    v = max(v, dpp_or_zero<0x114>(v));
+    v = max(v, dpp_or_zero<0x118>(v));
+    v = max(v, dpp_or_zero<0x142, 0xa>(v));
+    v = max(v, dpp_or_zero<0x143, 0xc>(v));
+    return __builtin_bit_cast(float, v);
+}
+
+// The filter's error bound (filter_bounds) for home atoms within H of their
+// centre and brick atoms up to |p|^2 of bits far2 beyond the system's pmax2.
+// Beyond any sane scale every value is decided by the 64-bit test.  (1,000 atoms
+// centred on the corner of an open cell, count kernel: bricks with such atoms
+// on the 64-bit per-wave path 684 us, with a bound of their own 68; 64-bit LDS
+// path 235.)
+__device__ __forceinline__ float far_tol(const SysDev &sd, float H, int far2)
+{
+    const float P = __builtin_sqrtf(fmaxf(sd.pmax2, __builtin_bit_cast(float, far2))), rc = __builtin_sqrtf(2.0f * sd.rc2half);
+    const float a = 2.0f * H + rc, b = H + rc;
+    const float e = 10.0f * (a * a + rc * rc) + 7.0f * b * b + 4.0f * rc * rc + 7.2f * (P + a) * rc;
+    return H + P < 1.0e15f ? 0.505f * (1.25f / (1 << 24) * e + sd.tol64) : kFar32 * kFar32;
 }
 
 // Slot entries of a pass: 4 or 8 bytes.
@@ -1348,12 +1391,14 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(5))) void ti
     const int wv = sgpr((int)(threadIdx.x >> 6));
     if (!lds) {
         const SlotArgs O{slots, cap, status};
-        for (int hc = copy + copies * wv; hc < B.nhome; hc += copies * BrickShape<BT>::waves)
-            count_cell<false>(A, *B.sd, brick_cell_id(B, hc), pair_count, O);
+        for (int hc = 0; hc < B.nhome; ++hc)
+            count_cell<false>(A, *B.sd, brick_cell_id(B, hc), pair_count, O, hc, copy + copies * wv,
+                              copies * BrickShape<BT>::waves);
         return;
     }
     const SysDev &sd = *B.sd;
     const bool narrow = sgpr(L.row8) == 0;   // the brick writes 4-byte slot entries
+    const int far2 = sgpr(L.far2);
     // L.a[].j holds j | S code << 26 whenever every j fits in 26 bits
     const uint32_t hjmask = sd.nat <= kNarrowMaxAtoms ? (uint32_t)(kNarrowMaxAtoms - 1) : 0xffffffffu;
     const uint32_t jmask = narrow ? 0xffffffffu : hjmask;   // entry low word: j | code << 26, or j
@@ -1400,9 +1445,10 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(5))) void ti
                     (uint64_t)(narrow ? 4 : 8) << 48;
             H.t = L.t[hl];
             H.fill = 0;
-            // a home atom further from the run's centre than the bounds assume
-            // (clamped into its cell): 64-bit tests for all
-            const float tol = __builtin_amdgcn_ballot_w64(!(hq <= sd.h2half)) != 0 ? kFar32 * kFar32 : sd.tol;
+            // atoms further out than the system's bounds assume: the brick's own
+            float tol = sd.tol;
+            if (__builtin_amdgcn_ballot_w64(!(hq <= sd.h2half)) != 0 || far2 != 0)
+                tol = far_tol(sd, __builtin_sqrtf(2.0f * readlane_f32(wave_max_f32(hq), kWave - 1)), far2);
             for (int k0 = 0; k0 < total; k0 += kTileCands) {
                 const int nch = sgpr(min(kTileChunks, (total - k0 + kWave - 1) / kWave));
                 // marks where a non-empty row other than the first starts (see row_map)
@@ -1581,19 +1627,6 @@ using SysConst = const __attribute__((address_space(4))) SysDev;
 __device__ __forceinline__ SysConst *sys_const(const SysDev *p)
 {
     return (SysConst *)(uintptr_t)p;
-}
-
-// The largest of the lanes' non-negative values, on the last lane.
-__device__ __forceinline__ float wave_max_f32(float x)
-{
-    int v = __builtin_bit_cast(int, x);   // non-negative floats order as their bits
-    v = max(v, dpp_or_zero<0x111>(v));
-    v = max(v, dpp_or_zero<0x112>(v));
-    v = max(v, dpp_or_zero<0x114>(v));
-    v = max(v, dpp_or_zero<0x118>(v));
-    v = max(v, dpp_or_zero<0x142, 0xa>(v));
-    v = max(v, dpp_or_zero<0x143, 0xc>(v));
-    return __builtin_bit_cast(float, v);
 }
 
 // The 64-bit test of atoms i, j of a system (X: its positions) with packed cell

@@ -253,3 +253,18 @@ def test_batch_rows_that_overflow(n):
         systems.append(workloads.System(X, cell, (True, True, k % 2 == 0), 5.0))
     print(f"batch overflow {n}", flush=True)
     _check_batch(systems)
+
+
+@pytest.mark.parametrize("n", [50, 1200, 20000])
+@pytest.mark.parametrize("shift", [0.25, 0.5, 30.0, 1e7])
+@pytest.mark.parametrize("pbc", [(False, False, False), (True, True, False), (False, True, True)])
+def test_open_axes_far_from_the_cell(n, shift, pbc):
+    """Positions shifted against the cell by parts and multiples of it along
+    open axes, so that edge cells hold atoms from far outside (up to all of
+    them, more than a brick stages)."""
+    if n == 20000 and sum(pbc) < 2 and shift > 0.25:
+        pytest.skip("a few cells hold every atom: slow in the oracle")
+    s = workloads.random_cubic(n, density=0.05, seed=n, cutoff=4.0)
+    X = s.X - np.where(pbc, 0.0, shift) * np.diag(np.asarray(s.cell))
+    print(f"open {n} {shift} {pbc}", flush=True)
+    _check(X, 4.0, s.cell, pbc)
