@@ -1047,6 +1047,25 @@ void settle(nlh_handle *h)
     h->inflight = false;
 }
 
+// Whether every destination (one at least) is plain memory of `device`,
+// aligned to its elements.
+bool on_device(const nlh::CopyList &c, int device)
+{
+    bool any = false;
+    for (int a = 0; a < nlh::CopyList::n; ++a) {
+        if (c.bytes[a] == 0) continue;
+        hipPointerAttribute_t at{};
+        if (hipPointerGetAttributes(&at, c.dst[a]) != hipSuccess) {
+            (void)hipGetLastError();   // memory the runtime does not know
+            return false;
+        }
+        if (at.type != hipMemoryTypeDevice || at.isManaged || at.device != device) return false;
+        if ((reinterpret_cast<uintptr_t>(c.dst[a]) & 3) != 0) return false;
+        any = true;
+    }
+    return any;
+}
+
 // The status of the stages just launched: early from the fill when it
 // publishes (not while phases are being timed: their events need the whole
 // stream), else after the stream.
@@ -1895,9 +1914,23 @@ int nlh_copy_pairlist(nlh_handle *h, void *i, void *j, void *S, void *first, dou
         if (!h) throw Error(NLH_EINVAL, "handle is NULL");
         if (!h->materialized) throw Error(NLH_ESTATE, "no materialised pair list");
         HIPC(hipSetDevice(h->device));
+        const size_t P = (size_t)h->npairs, ti = (size_t)h->ti_bytes;
+        const size_t nfirst = ((size_t)h->nat + h->nsys) * ti;
+        const nlh::CopyList c = {{i, j, S, first, R},
+                                 {h->i.p, h->j.p, h->S.p, h->first.p, h->R.p},
+                                 {i ? P * ti : 0, j ? P * ti : 0, S ? 3 * P * ti : 0, first ? nfirst : 0, R ? 24 * P : 0}};
+        if ((!R || P == 0 || h->have_R) && on_device(c, h->device)) {
+            // one kernel behind the fill.  The copies it replaces were ordered
+            // after the default stream, which may still use the memory: waited for.
+            HIPD(hipStreamSynchronize(nullptr));
+            nlh::launch_copy_list(c, h->stream);
+            HIPC(hipGetLastError());
+            HIPC(hipStreamSynchronize(h->stream));
+            h->inflight = false;
+            return;
+        }
         settle(h);
         HIPC(hipStreamSynchronize(h->stream));
-        const size_t P = (size_t)h->npairs, ti = (size_t)h->ti_bytes;
         if (P > 0) {
             if (i) HIPD(hipMemcpy(i, h->i.p, P * ti, hipMemcpyDefault));
             if (j) HIPD(hipMemcpy(j, h->j.p, P * ti, hipMemcpyDefault));
@@ -1907,7 +1940,7 @@ int nlh_copy_pairlist(nlh_handle *h, void *i, void *j, void *S, void *first, dou
                 HIPD(hipMemcpy(R, h->R.p, 3 * P * 8, hipMemcpyDefault));
             }
         }
-        if (first) HIPD(hipMemcpy(first, h->first.p, ((size_t)h->nat + h->nsys) * ti, hipMemcpyDefault));
+        if (first) HIPD(hipMemcpy(first, h->first.p, nfirst, hipMemcpyDefault));
     });
 }
 

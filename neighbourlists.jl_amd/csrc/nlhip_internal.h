@@ -300,6 +300,15 @@ struct PipelineBufs {
     int count_block;         // threads per count-pass brick workgroup (256 or 512)
 };
 
+// The arrays of a pair list copied out by one kernel (0 bytes: not copied).
+struct CopyList {
+    static constexpr int n = 5;
+    void *dst[n];
+    const void *src[n];
+    size_t bytes[n];   // multiples of 4, as the addresses are
+};
+void launch_copy_list(const CopyList &c, hipStream_t st);
+
 void launch_clear_status(const PipelineBufs &b, hipStream_t st);
 // Zero n 8-byte words by a kernel (no memset node: safe under graph capture).
 void launch_zero_words(uint64_t *p, int64_t n, hipStream_t st);

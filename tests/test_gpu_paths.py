@@ -268,3 +268,38 @@ def test_open_axes_far_from_the_cell(n, shift, pbc):
     X = s.X - np.where(pbc, 0.0, shift) * np.diag(np.asarray(s.cell))
     print(f"open {n} {shift} {pbc}", flush=True)
     _check(X, 4.0, s.cell, pbc)
+
+
+@pytest.mark.parametrize("n", [0, 1, 3, 500, 5000])
+@pytest.mark.parametrize("int_type", [np.int32, np.int64])
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+def test_copy_to_device_memory(n, int_type, shift):
+    """Lists copied to device memory of any element alignment, all arrays and
+    some, while the default stream still writes that memory."""
+    s = workloads.random_cubic(max(n, 1), density=0.05, seed=n, cutoff=5.0)
+    X = s.X[:n]
+    ref = nlhip.neighbour_list(X, 5.0, s.cell, s.pbc, int_type=int_type, want_R=True)
+    td = torch.int32 if int_type == np.int32 else torch.int64
+    h = _lib.Handle()
+    geom = _lib.geometry(s.cell, 5.0, s.pbc, 4 if int_type == np.int32 else 8)
+    m = ctypes.c_int64()
+    print(f"copy {n} {shift}", flush=True)
+    L = _lib.lib()
+    _lib.check(L.nlh_neighbour_list(h.ptr, X.ctypes.data, n, ctypes.byref(geom), _lib.NLH_WANT_R, ctypes.byref(m)))
+    P = m.value
+    for skip in [None, 0, 2, 4]:
+        out = [torch.zeros(k + 8, dtype=t, device="cuda") for k, t in
+               ((P, td), (P, td), (3 * P, td), (n + 1, td), (3 * P, torch.float64))]
+        big = torch.empty(1 << 26, device="cuda")
+        for _ in range(4):
+            big.fill_(1.0)
+        for o in out:
+            o.fill_(-7)
+        ptrs = [None if k == skip else o[shift:].data_ptr() for k, o in enumerate(out)]
+        _lib.check(L.nlh_copy_pairlist(h.ptr, *ptrs))
+        for k, (o, r) in enumerate(zip(out, (ref.i, ref.j, ref.S, ref.first, ref.R))):
+            o, r = o.cpu().numpy(), np.asarray(r).reshape(-1)
+            want = np.full(o.shape, -7, o.dtype)
+            if k != skip:
+                want[shift:shift + r.size] = r
+            assert np.array_equal(o, want), (k, skip)
