@@ -11,6 +11,7 @@
 //     bucket_scatter_kernel atoms grouped by bucket
 //     bucket_place_kernel   one workgroup per bucket: cell_start / cell_offsets,
 //                           stable in-cell rank -> perm, cell_id, sorted records
+//     (up to kBlockSortAtoms atoms of one system: block_sort_kernel, all of it)
 //   atomic
 //     bin_kernel            cell id + winding, cell histogram by global atomics
 //     scan (cells)          cell_start / cell_offsets
@@ -23,6 +24,22 @@
 #include "device_util.h"
 
 namespace nlh {
+
+// Zero the build status (when given) and n scan descriptors, by every thread
+// of a launch.
+__device__ __forceinline__ void clear_status(Status *__restrict__ status, uint64_t *__restrict__ lookback, int64_t n)
+{
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (status && g < (int64_t)(sizeof(Status) / 4)) reinterpret_cast<int32_t *>(status)[g] = 0;
+    for (int64_t i = g; i < n; i += (int64_t)gridDim.x * blockDim.x) lookback[i] = 0;
+}
+
+// A kernel rather than a memset, so the pipeline can be captured into a HIP
+// graph and replayed.
+__global__ void clear_status_kernel(Status *__restrict__ status, uint64_t *__restrict__ lookback, int64_t n)
+{
+    clear_status(status, lookback, n);
+}
 
 // ---------------------------------------------------------------------------
 // 0. batches: the system of every atom and every cell, once per build, for
@@ -503,15 +520,15 @@ __global__ __launch_bounds__(256) void sorted_positions_kernel(const Rec *__rest
 __global__ __launch_bounds__(kBinThreads) void bucket_count_kernel(
     const double *__restrict__ X, const SysDev *__restrict__ sys, const int32_t *__restrict__ atom_sys, int nsys,
     int64_t nat, SortPlan P, int32_t *__restrict__ key, int32_t *__restrict__ slot, int32_t *__restrict__ bmat,
-    Status *__restrict__ status)
+    Status *__restrict__ status, uint64_t *__restrict__ lookback, int64_t nlook)
 {
     extern __shared__ int32_t hist[];   // P.nb counters
+    clear_status(status, lookback, nlook);
     for (int b = threadIdx.x; b < P.nb; b += kBinThreads) hist[b] = 0;
     __syncthreads();
     const uint32_t lb = xcd_remap(blockIdx.x, gridDim.x);   // consecutive blocks on one XCD
     const int64_t a0 = (int64_t)lb * P.apb;
     const int64_t a1 = a0 + P.apb < nat ? a0 + P.apb : nat;
-    bool bad = false;
     for (int64_t g0 = a0 + threadIdx.x; g0 < a1; g0 += kBinThreads * kBinUnroll) {
         double x[kBinUnroll], y[kBinUnroll], z[kBinUnroll];
         int sy[kBinUnroll];
@@ -533,7 +550,7 @@ __global__ __launch_bounds__(kBinThreads) void bucket_count_kernel(
             if (g < a1) {
                 const SysDev &sd = sys[sy[u]];
                 int32_t c[3], w[3];
-                bad |= !cell_and_winding(sd, x[u], y[u], z[u], c, w);
+                cell_and_winding(sd, x[u], y[u], z[u], c, w);   // positions it cannot place: reported by place_one
                 const int32_t k = sd.cell_base + (c[0] - 1) + (c[1] - 1) * sd.n[0] + (c[2] - 1) * sd.n[0] * sd.n[1];
                 // read once more, by the scatter: streamed past the caches like the
                 // sort's other whole-line scratch traffic (the pair pass later relies
@@ -543,7 +560,6 @@ __global__ __launch_bounds__(kBinThreads) void bucket_count_kernel(
             }
         }
     }
-    if (bad) atomicOr(&status->bad_position, 1);
     __syncthreads();
     for (int b = threadIdx.x; b < P.nb; b += kBinThreads) bmat[(int64_t)b * P.na + lb] = hist[b];
 }
@@ -626,9 +642,9 @@ __device__ __forceinline__ int2 load_ke(const int2 *p)
 // kBucketLdsAtoms atoms keeps its cells, indices and groups in LDS; a larger
 // one (clustered atoms) works from global memory (bke and tmp, its own range).
 // The sorted record, perm and cell_id of atom e (global index) of cell k at
-// sorted place p.
+// sorted place p.  Returns whether its position was one.
 template <typename TI>
-__device__ __forceinline__ void place_one(int32_t k, int32_t e, int32_t p, const double *__restrict__ X,
+__device__ __forceinline__ bool place_one(int32_t k, int32_t e, int32_t p, const double *__restrict__ X,
                                           const SysDev *__restrict__ sys, const int32_t *__restrict__ cell_sys, int nsys,
                                           Rec *__restrict__ rec, int32_t *__restrict__ wbig, void *__restrict__ perm_out,
                                           void *__restrict__ cell_id_out)
@@ -637,7 +653,7 @@ __device__ __forceinline__ void place_one(int32_t k, int32_t e, int32_t p, const
     const SysDev &sd = sys[si];
     const double x = X[3 * (int64_t)e], y = X[3 * (int64_t)e + 1], z = X[3 * (int64_t)e + 2];
     int32_t cc[3], w[3];
-    cell_and_winding(sd, x, y, z, cc, w);
+    const bool ok = cell_and_winding(sd, x, y, z, cc, w);
     const int32_t j = (int32_t)(e - sd.atom_base);
     Rec o;
     o.x = x;
@@ -653,6 +669,7 @@ __device__ __forceinline__ void place_one(int32_t k, int32_t e, int32_t p, const
     }
     store_ti<TI>(perm_out, p, (int64_t)j + 1);
     store_ti<TI>(cell_id_out, p, (int64_t)(k - sd.cell_base) + 1);
+    return ok;
 }
 
 template <typename TI>
@@ -660,7 +677,8 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_place_kernel(
     const int2 *__restrict__ bke, const double *__restrict__ X, const int32_t *__restrict__ boff, SortPlan P,
     int64_t nat, int32_t M, const SysDev *__restrict__ sys, const int32_t *__restrict__ cell_sys, int nsys,
     int32_t *__restrict__ tmp, int32_t *__restrict__ cell_start, void *__restrict__ offsets_out,
-    Rec *__restrict__ rec, int32_t *__restrict__ wbig, void *__restrict__ perm_out, void *__restrict__ cell_id_out)
+    Rec *__restrict__ rec, int32_t *__restrict__ wbig, void *__restrict__ perm_out, void *__restrict__ cell_id_out,
+    Status *__restrict__ status)
 {
     __shared__ int32_t kl[kBucketLdsAtoms], el[kBucketLdsAtoms], grp[kBucketLdsAtoms];
     extern __shared__ int32_t lds[];
@@ -760,10 +778,13 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_place_kernel(
                 el[pq[u]] = eq[u];
             }
         __syncthreads();
+        bool bad = false;
         for (int q = threadIdx.x; q < n; q += kBucketThreads)
-            place_one<TI>(kl[q], el[q], bs + q, X, sys, cell_sys, nsys, rec, wbig, perm_out, cell_id_out);
+            bad |= !place_one<TI>(kl[q], el[q], bs + q, X, sys, cell_sys, nsys, rec, wbig, perm_out, cell_id_out);
+        if (bad) atomicOr(&status->bad_position, 1);
         return;
     }
+    bool bad = false;
     for (int i = threadIdx.x; i < n; i += kBucketThreads) {
         int32_t k, e;
         {
@@ -776,18 +797,105 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_place_kernel(
         int32_t rank = 0;
         for (int t = s0; t < s1; ++t) rank += grpg[t] < e;
         const int32_t p = bs + s0 + rank;
-        place_one<TI>(k, e, p, X, sys, cell_sys, nsys, rec, wbig, perm_out, cell_id_out);
+        bad |= !place_one<TI>(k, e, p, X, sys, cell_sys, nsys, rec, wbig, perm_out, cell_id_out);
     }
+    if (bad) atomicOr(&status->bad_position, 1);
 }
 
-// Zero the build status (when given) and n scan descriptors.  A kernel
-// rather than a memset, so the pipeline can be captured into a HIP graph and
-// replayed.
-__global__ void clear_status_kernel(Status *__restrict__ status, uint64_t *__restrict__ lookback, int64_t n)
+// The whole cell sort of one small system in one workgroup, everything in LDS.
+// Bound by the latency of its few steps, as each of the five launches it
+// replaces was (status clear, count, scan, scatter, place): 1,000 atoms 13.9 us of
+// kernels and their gaps / 5.9 us; per build with the gaps 96 atoms 74 / 67 us,
+// 1,000 54 / 42, 2,000 58 / 52, 3,000 57 / 57: kBlockSortAtoms.
+template <typename TI>
+__global__ __launch_bounds__(kBlockSortThreads) void block_sort_kernel(
+    const double *__restrict__ X, const SysDev *__restrict__ sys, int n, int M, Status *__restrict__ status,
+    uint64_t *__restrict__ lookback, int64_t nlook, int32_t *__restrict__ cell_start, void *__restrict__ offsets_out,
+    Rec *__restrict__ rec, int32_t *__restrict__ wbig, void *__restrict__ perm_out, void *__restrict__ cell_id_out)
 {
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (status && g < (int64_t)(sizeof(Status) / 4)) reinterpret_cast<int32_t *>(status)[g] = 0;
-    for (int64_t i = g; i < n; i += (int64_t)gridDim.x * blockDim.x) lookback[i] = 0;
+    constexpr int kPer = kBlockSortAtoms / kBlockSortThreads, kCells = kBlockSortCells / kBlockSortThreads;
+    __shared__ int32_t co[kBlockSortCells + 1], fill[kBlockSortCells];
+    __shared__ int16_t grp[kBlockSortAtoms];
+    const int tid = (int)threadIdx.x;
+    const SysDev &sd = sys[0];
+    double x[kPer], y[kPer], z[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const int i = u * kBlockSortThreads + tid;
+        x[u] = y[u] = z[u] = 0.0;
+        if (i < n) {
+            x[u] = X[3 * i];
+            y[u] = X[3 * i + 1];
+            z[u] = X[3 * i + 2];
+        }
+    }
+    clear_status(status, lookback, nlook);
+#pragma unroll
+    for (int m = 0; m < kCells; ++m) fill[m * kBlockSortThreads + tid] = 0;
+    __syncthreads();
+    int32_t k[kPer], q[kPer], w[kPer][3];
+    bool bad = false;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        k[u] = q[u] = 0;
+        if (u * kBlockSortThreads + tid < n) {
+            int32_t c[3];
+            bad |= !cell_and_winding(sd, x[u], y[u], z[u], c, w[u]);
+            k[u] = (c[0] - 1) + (c[1] - 1) * sd.n[0] + (c[2] - 1) * sd.n[0] * sd.n[1];
+            q[u] = atomicAdd(&fill[k[u]], 1);   // arrival rank in the cell
+        }
+    }
+    __syncthreads();
+    int v[kCells], sum = 0, tot;
+#pragma unroll
+    for (int m = 0; m < kCells; ++m) {
+        v[m] = fill[kCells * tid + m];
+        sum += v[m];
+    }
+    int run = block_excl_scan32<kBlockSortThreads>(sum, tot);
+#pragma unroll
+    for (int m = 0; m < kCells; ++m) {
+        const int c = kCells * tid + m;
+        co[c] = run;
+        if (c <= M) {   // cell M: the trailing entries
+            cell_start[c] = run;
+            store_ti<TI>(offsets_out, c, (int64_t)run + 1);
+        }
+        run += v[m];
+    }
+    if (tid == 0) {
+        co[kBlockSortCells] = tot;
+        if (M == kBlockSortCells) {
+            cell_start[M] = tot;
+            store_ti<TI>(offsets_out, M, (int64_t)tot + 1);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPer; ++u)
+        if (u * kBlockSortThreads + tid < n) grp[co[k[u]] + q[u]] = (int16_t)(u * kBlockSortThreads + tid);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const int i = u * kBlockSortThreads + tid;
+        if (i < n) {
+            const int s0 = co[k[u]], s1 = co[k[u] + 1];
+            int p = s0;   // ties of the cell keep ascending index
+            for (int t = s0; t < s1; ++t) p += grp[t] < i;
+            Rec o;
+            o.x = x[u];
+            o.y = y[u];
+            o.z = z[u];
+            o.j = i;
+            o.w = pack_wind(w[u][0], w[u][1], w[u][2]);
+            rec[p] = o;
+            if (o.w & kWindBig)
+                for (int m = 0; m < 3; ++m) wbig[3 * p + m] = w[u][m];
+            store_ti<TI>(perm_out, p, (int64_t)i + 1);
+            store_ti<TI>(cell_id_out, p, (int64_t)k[u] + 1);
+        }
+    }
+    if (bad) atomicOr(&status->bad_position, 1);   // cleared before the barriers above
 }
 
 // ---------------------------------------------------------------------------
@@ -796,8 +904,15 @@ __global__ void clear_status_kernel(Status *__restrict__ status, uint64_t *__res
 
 static inline unsigned blocks_for(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
+// Whether the whole sort is one workgroup's (block_sort_kernel).
+static bool block_sort(const PipelineBufs &b)
+{
+    return b.nsys == 1 && b.sort.bw >= 0 && b.nat <= kBlockSortAtoms && b.M <= kBlockSortCells;
+}
+
 void launch_clear_status(const PipelineBufs &b, hipStream_t st)
 {
+    if (b.nunits == 0 && b.sort.bw >= 0) return;   // by the bucketed sort's first kernel
     const int64_t n = lookback_entries(b.sort.n_sort, b.nat);
     hipLaunchKernelGGL(clear_status_kernel, dim3(std::min(blocks_for(n, 256), 64u)), dim3(256), 0, st, b.status,
                        b.lookback, n);
@@ -832,7 +947,8 @@ static void launch_bucket_sort(const PipelineBufs &b, hipStream_t st)
 {
     const SortPlan &P = b.sort;
     hipLaunchKernelGGL(bucket_count_kernel, dim3((unsigned)P.na), dim3(kBinThreads), (size_t)P.nb * 4, st, b.X, b.sys,
-                       b.atom_sys, b.nsys, b.nat, P, b.key, b.slot, b.bmat, b.status);
+                       b.atom_sys, b.nsys, b.nat, P, b.key, b.slot, b.bmat, b.status, b.lookback,
+                       lookback_entries(P.n_sort, b.nat));
     hipLaunchKernelGGL(scan_inplace_kernel, dim3((unsigned)scan_tiles(P.n_sort)), dim3(kScanThreads), 0, st, b.bmat,
                        P.n_sort, b.lookback, b.status);
     hipLaunchKernelGGL(bucket_scatter_kernel, dim3((unsigned)P.na), dim3(kBinThreads), 0, st, b.nat, P, b.key, b.slot,
@@ -842,7 +958,7 @@ static void launch_bucket_sort(const PipelineBufs &b, hipStream_t st)
                                        (size_t)(2 * (1 << P.bw) + 1) * 4, st, b.bke, b.X, b.bmat, P, b.nat, b.M,
                                        b.sys, b.nsys > 1 ? b.atom_sys + b.nat : nullptr, b.nsys, b.tmp,
                                        b.cell_start, b.cell_offsets_out, b.rec, b.wbig, b.perm_out,
-                                       b.cell_id_out));
+                                       b.cell_id_out, b.status));
 }
 
 void launch_build(const PipelineBufs &b, hipStream_t st)
@@ -851,6 +967,14 @@ void launch_build(const PipelineBufs &b, hipStream_t st)
     if (b.nsys > 1)
         hipLaunchKernelGGL(sys_map_kernel, dim3(blocks_for(b.nat + b.M, 256)), dim3(256), 0, st, b.sys_atom_base,
                            b.sys_cell_base, b.nsys, b.nat, (int64_t)b.M, b.atom_sys);
+    if (block_sort(b)) {
+        NLH_TI_DISPATCH(b.ti_bytes,
+                        hipLaunchKernelGGL(block_sort_kernel<TI>, dim3(1), dim3(kBlockSortThreads), 0, st, b.X, b.sys,
+                                           (int)b.nat, b.M, b.status, b.lookback,
+                                           lookback_entries(b.sort.n_sort, b.nat), b.cell_start, b.cell_offsets_out,
+                                           b.rec, b.wbig, b.perm_out, b.cell_id_out));
+        return;
+    }
     if (b.sort.bw >= 0) {
         launch_bucket_sort(b, st);
         return;

@@ -45,6 +45,9 @@ constexpr int kBucketLdsAtoms = 4096;     // buckets up to this size are ordered
 constexpr int kBucketMaxShift = 12;       // at most 4096 cells per bucket
 constexpr int kBucketMaxCount = 8192;     // buckets (LDS counters of a count block)
 constexpr int kBucketBytes = 8;           // scratch per atom: (cell, index)
+constexpr int kBlockSortThreads = 1024;   // one system of up to kBlockSortAtoms atoms and kBlockSortCells cells:
+constexpr int kBlockSortAtoms = 2048;     // its whole sort in one workgroup
+constexpr int kBlockSortCells = 4096;
 struct SortPlan {
     int32_t bw;     // log2 cells per bucket; -1: atomic histogram sort
     int32_t nb;     // buckets
@@ -309,6 +312,8 @@ struct CopyList {
 };
 void launch_copy_list(const CopyList &c, hipStream_t st);
 
+// Clears the status and the scan descriptors of a build that launch_build
+// follows (whose bucketed sort does it by itself).
 void launch_clear_status(const PipelineBufs &b, hipStream_t st);
 // Zero n 8-byte words by a kernel (no memset node: safe under graph capture).
 void launch_zero_words(uint64_t *p, int64_t n, hipStream_t st);

@@ -303,3 +303,33 @@ def test_copy_to_device_memory(n, int_type, shift):
             if k != skip:
                 want[shift:shift + r.size] = r
             assert np.array_equal(o, want), (k, skip)
+
+
+@pytest.mark.parametrize("int_type,bits", [(np.int32, 32), (np.int64, 64)])
+@pytest.mark.parametrize("n,per_cell,wind", [(1, 1.0, 0), (2, 0.001, 0), (1023, 6.0, 700), (1024, 0.25, 0), (1025, 0.2501, 3),
+                                             (2047, 2047.0, 0), (2048, 0.5, 0), (2048, 0.49, 0), (2049, 0.5, 0),
+                                             (4096, 4096.0, 1), (300, 300.0, 0), (5000, 5000.0, 2)])
+def test_cell_list_sort_forms(n, per_cell, wind, int_type, bits):
+    """The cell list of one system around the sizes (atoms, cells) up to which
+    one workgroup sorts it, from empty cells to all atoms in one; a position
+    that is none is refused in each form."""
+    rc = 2.0
+    cells = max(1, int(round(n / per_cell)))
+    shape = (cells, 1, 1) if cells < 64 else (16, 16, max(1, cells // 256))
+    cell = np.diag([(k + 0.01) * rc for k in shape])
+    rng = np.random.default_rng(n)
+    X = rng.random((n, 3)) @ cell
+    X[::5] += wind * cell[0]
+    print(f"sort {n} {shape} {wind}", flush=True)
+    pbc = (True, True, True)
+    cl = nlhip.build_cell_list(X, rc, cell, pbc, int_type=int_type)
+    ids = oracle.cell_ids(X, rc, cell, pbc, ti_bits=bits)[0]
+    perm = np.argsort(ids, kind="stable")
+    assert np.array_equal(cl.perm, perm + 1) and np.array_equal(cl.cell_id, ids[perm])
+    assert np.array_equal(cl.cell_offsets, np.searchsorted(ids[perm], np.arange(1, int(np.prod(shape)) + 2)) + 1)
+    assert np.array_equal(cl.X, X[perm])
+    if per_cell <= 10.0:
+        _check(X, rc, cell, pbc, int_type)
+    X[n // 2, 1] = np.nan
+    with pytest.raises(nlhip.NLHInvalidError):
+        nlhip.build_cell_list(X, rc, cell, pbc, int_type=int_type)
