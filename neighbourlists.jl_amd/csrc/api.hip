@@ -15,6 +15,7 @@
 
 #include "../../include/nlhip.h"
 #include "../../include/nlhip_device.h"
+#include "host_copy.h"
 #include "nlhip_internal.h"
 
 namespace {
@@ -1066,6 +1067,46 @@ bool on_device(const nlh::CopyList &c, int device)
     return any;
 }
 
+// A copier of the process for one copy.
+struct BorrowedCopier {
+    std::unique_ptr<nlh::HostCopier> c;
+    explicit BorrowedCopier(int device) : c(nlh::host_copiers().borrow(device)) {}
+    ~BorrowedCopier()
+    {
+        auto end = nlh::host_copiers().give_back(std::move(c));
+        if (end) device_wide([&] { end.reset(); });
+    }
+};
+
+// The arrays of c to the caller's memory of any kind, complete on return: by
+// several threads where all of it is pageable and there is enough of it.
+void copy_out(nlh_handle *h, const nlh::CopyList &c)
+{
+    size_t bytes = 0;
+    bool pageable = true;
+    std::vector<nlh::HostCopier::Piece> arrays;
+    for (int a = 0; a < nlh::CopyList::n; ++a) {
+        if (c.bytes[a] == 0) continue;
+        bytes += c.bytes[a];
+        arrays.push_back({static_cast<char *>(c.dst[a]), static_cast<char *>(const_cast<void *>(c.src[a])), c.bytes[a]});
+        pageable = pageable && nlh::HostCopier::pageable(c.dst[a]);
+    }
+    if (pageable && bytes >= nlh::HostCopier::kWorthIt) {
+        BorrowedCopier b(h->device);
+        hipError_t ready = hipSuccess;
+        device_wide([&] { ready = b.c->prepare(bytes); });
+        if (ready == hipSuccess) {
+            HIPC(b.c->to_host(h->stream, arrays));
+            h->inflight = false;   // the copies came behind everything else on the stream
+            return;
+        }
+        (void)hipGetLastError();   // no pinned memory to be had: the runtime's way
+    }
+    settle(h);
+    HIPC(hipStreamSynchronize(h->stream));
+    for (const auto &a : arrays) HIPD(hipMemcpy(a.host, a.device, a.bytes, hipMemcpyDefault));
+}
+
 // The status of the stages just launched: early from the fill when it
 // publishes (not while phases are being timed: their events need the whole
 // stream), else after the stream.
@@ -1743,6 +1784,7 @@ int nlh_create(nlh_handle **out)
             delete h;
             throw;
         }
+        nlh::host_copiers().handle_made();
         *out = h;
     });
 }
@@ -1766,6 +1808,7 @@ int nlh_destroy(nlh_handle *h)
                           &h->nr_count, &h->nr_off,    &h->nr_j,       &h->nr_R,         &h->nr_S};
         for (DevBuf *b : bufs) b->release(h->stream);
         device_wide([&] {
+            nlh::host_copiers().handle_gone();
             if (h->status_host) (void)hipHostFree(h->status_host);
             if (h->staging) (void)hipHostFree(h->staging);
             if (h->xstage) (void)hipHostFree(h->xstage);
@@ -1929,18 +1972,8 @@ int nlh_copy_pairlist(nlh_handle *h, void *i, void *j, void *S, void *first, dou
             h->inflight = false;
             return;
         }
-        settle(h);
-        HIPC(hipStreamSynchronize(h->stream));
-        if (P > 0) {
-            if (i) HIPD(hipMemcpy(i, h->i.p, P * ti, hipMemcpyDefault));
-            if (j) HIPD(hipMemcpy(j, h->j.p, P * ti, hipMemcpyDefault));
-            if (S) HIPD(hipMemcpy(S, h->S.p, 3 * P * ti, hipMemcpyDefault));
-            if (R) {
-                if (!h->have_R) throw Error(NLH_ESTATE, "R was not requested (NLH_WANT_R)");
-                HIPD(hipMemcpy(R, h->R.p, 3 * P * 8, hipMemcpyDefault));
-            }
-        }
-        if (first) HIPD(hipMemcpy(first, h->first.p, nfirst, hipMemcpyDefault));
+        if (R && P > 0 && !h->have_R) throw Error(NLH_ESTATE, "R was not requested (NLH_WANT_R)");
+        copy_out(h, c);
     });
 }
 
@@ -2041,9 +2074,8 @@ int nlh_neighbours_range(nlh_handle *h, int32_t sys, int64_t i_first, int64_t n,
         const int64_t total = h->nr_off_host[n];
         if (total > 0 && total <= cap) {
             const size_t ti = (size_t)h->ti_bytes;
-            if (j) HIPD(hipMemcpy(j, h->nr_j.p, (size_t)total * ti, hipMemcpyDeviceToHost));
-            if (R) HIPD(hipMemcpy(R, h->nr_R.p, (size_t)total * 24, hipMemcpyDeviceToHost));
-            if (S) HIPD(hipMemcpy(S, h->nr_S.p, (size_t)total * 3 * ti, hipMemcpyDeviceToHost));
+            const size_t t = (size_t)total;
+            copy_out(h, {{j, R, S}, {h->nr_j.p, h->nr_R.p, h->nr_S.p}, {j ? t * ti : 0, R ? t * 24 : 0, S ? 3 * t * ti : 0}});
         }
     });
 }

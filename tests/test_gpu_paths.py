@@ -333,3 +333,34 @@ def test_cell_list_sort_forms(n, per_cell, wind, int_type, bits):
     X[n // 2, 1] = np.nan
     with pytest.raises(nlhip.NLHInvalidError):
         nlhip.build_cell_list(X, rc, cell, pbc, int_type=int_type)
+
+
+@pytest.mark.parametrize("n", [3900, 5300, 43690, 43691, 120000])
+@pytest.mark.parametrize("int_type,bits", [(np.int32, 32), (np.int64, 64)])
+def test_lists_in_host_memory(n, int_type, bits):
+    """Positions and lists around the sizes from which several threads copy
+    them, on one handle (threads and pinned memory kept) and a fresh one, and
+    two handles at once from two threads."""
+    import threading
+
+    s = workloads.random_cubic(n, density=0.05, seed=n, cutoff=5.0)
+    ref = oracle.neighbour_list(s.X, 5.0, s.cell, s.pbc, ti_bits=bits, want_R=True, nthreads=8)
+    print(f"host list {n} {bits}", flush=True)
+    bad = []
+
+    def work():
+        h = _lib.Handle()
+        for want_R in (False, True, True):
+            nl = nlhip.neighbour_list(s.X, 5.0, s.cell, s.pbc, int_type=int_type, want_R=want_R, handle=h)
+            ok = (np.array_equal(nl.i, ref.i) and np.array_equal(nl.j, ref.j) and np.array_equal(nl.S, ref.S)
+                  and np.array_equal(nl.first, ref.first) and (not want_R or np.array_equal(_bits(nl.R), _bits(ref.R))))
+            if not ok:
+                bad.append(want_R)
+
+    work()
+    threads = [threading.Thread(target=work) for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
