@@ -145,6 +145,7 @@ struct nlh_handle {
     // (unit, then part | parts << 16), in the tables
     std::vector<int32_t> units_host, order_host;
     int32_t nunits = 0, nitems = 0, item_tests = 0;
+    bool keep_X = false;                  // the build's sort copies X to Xr
     int32_t *units_d = nullptr, *order_d = nullptr;
     bool small_ok = true;   // cleared when a fused build met a winding beyond +-511
     std::vector<char> tables_host;        // bytes of the last upload
@@ -238,6 +239,7 @@ struct nlh_handle {
         b.cell_offsets_out = cell_offsets.p;
         b.pair_count = pair_count.as<int32_t>();
         b.slots = slots.p;
+        b.X_keep = keep_X ? Xr.as<double>() : nullptr;
         b.Xr = X_dev == X.as<double>() ? X.as<double>() : Xr.as<double>();
         b.slot_cap = slot_cap;
         b.pair_off = pair_off.as<int64_t>();
@@ -871,8 +873,13 @@ void stage_positions(nlh_handle *h, const double *X, size_t bytes)
 void upload_positions(nlh_handle *h, const double *X, uint32_t flags)
 {
     if (h->nat > 0 && X == nullptr) throw Error(NLH_EINVAL, "X is NULL");
+    h->keep_X = false;
     if (flags & NLH_X_DEVICE) {
         h->X_dev = X;
+        if (flags & NLH_WANT_R) {
+            h->Xr.ensure(h->stream, (size_t)std::max<int64_t>(h->nat, 1) * 24);
+            h->keep_X = true;
+        }
     } else {
         h->X.ensure(h->stream, (size_t)std::max<int64_t>(h->nat, 1) * 24);
         if (h->nat > 0) stage_positions(h, X, (size_t)h->nat * 24);
@@ -1873,6 +1880,7 @@ int nlh_materialize(nlh_handle *h, uint32_t flags, int64_t *npairs)
         if (!h) throw Error(NLH_EINVAL, "handle is NULL");
         HIPC(hipSetDevice(h->device));
         settle(h);
+        h->keep_X = false;   // the build may have been another sort's: positions out of its records
         materialize(h, flags);
         if (npairs) *npairs = h->npairs;
     });

@@ -423,7 +423,8 @@ __global__ __launch_bounds__(1024) void range_scan_kernel(const int32_t *__restr
 // pair bases.  System s owns entries [atom_base[s] + s, atom_base[s+1] + s] of
 // the concatenated first arrays: thread g writes the entry of atom g (its
 // system from atom_sys) and, for g in [1, nsys], the trailing entry of
-// system g - 1 (its pair count + 1).
+// system g - 1 (its pair count + 1).  (As blocks of the fill kernel it cost more
+// than its launch: 4,096 systems, fill 210 -> 230 us against 7.7.)
 template <typename TI>
 __global__ __launch_bounds__(256) void batch_first_kernel(const int64_t *__restrict__ pair_off, int64_t nat,
                                                           const int64_t *__restrict__ sys_atom_base,
@@ -520,7 +521,7 @@ __global__ __launch_bounds__(256) void sorted_positions_kernel(const Rec *__rest
 __global__ __launch_bounds__(kBinThreads) void bucket_count_kernel(
     const double *__restrict__ X, const SysDev *__restrict__ sys, const int32_t *__restrict__ atom_sys, int nsys,
     int64_t nat, SortPlan P, int32_t *__restrict__ key, int32_t *__restrict__ slot, int32_t *__restrict__ bmat,
-    Status *__restrict__ status, uint64_t *__restrict__ lookback, int64_t nlook)
+    Status *__restrict__ status, uint64_t *__restrict__ lookback, int64_t nlook, double *__restrict__ X_keep)
 {
     extern __shared__ int32_t hist[];   // P.nb counters
     clear_status(status, lookback, nlook);
@@ -548,6 +549,11 @@ __global__ __launch_bounds__(kBinThreads) void bucket_count_kernel(
         for (int u = 0; u < kBinUnroll; ++u) {
             const int64_t g = g0 + (int64_t)u * kBinThreads;
             if (g < a1) {
+                if (X_keep) {
+                    X_keep[3 * g] = x[u];
+                    X_keep[3 * g + 1] = y[u];
+                    X_keep[3 * g + 2] = z[u];
+                }
                 const SysDev &sd = sys[sy[u]];
                 int32_t c[3], w[3];
                 cell_and_winding(sd, x[u], y[u], z[u], c, w);   // positions it cannot place: reported by place_one
@@ -811,7 +817,8 @@ template <typename TI>
 __global__ __launch_bounds__(kBlockSortThreads) void block_sort_kernel(
     const double *__restrict__ X, const SysDev *__restrict__ sys, int n, int M, Status *__restrict__ status,
     uint64_t *__restrict__ lookback, int64_t nlook, int32_t *__restrict__ cell_start, void *__restrict__ offsets_out,
-    Rec *__restrict__ rec, int32_t *__restrict__ wbig, void *__restrict__ perm_out, void *__restrict__ cell_id_out)
+    Rec *__restrict__ rec, int32_t *__restrict__ wbig, void *__restrict__ perm_out, void *__restrict__ cell_id_out,
+    double *__restrict__ X_keep)
 {
     constexpr int kPer = kBlockSortAtoms / kBlockSortThreads, kCells = kBlockSortCells / kBlockSortThreads;
     __shared__ int32_t co[kBlockSortCells + 1], fill[kBlockSortCells];
@@ -827,6 +834,11 @@ __global__ __launch_bounds__(kBlockSortThreads) void block_sort_kernel(
             x[u] = X[3 * i];
             y[u] = X[3 * i + 1];
             z[u] = X[3 * i + 2];
+            if (X_keep) {
+                X_keep[3 * i] = x[u];
+                X_keep[3 * i + 1] = y[u];
+                X_keep[3 * i + 2] = z[u];
+            }
         }
     }
     clear_status(status, lookback, nlook);
@@ -948,7 +960,7 @@ static void launch_bucket_sort(const PipelineBufs &b, hipStream_t st)
     const SortPlan &P = b.sort;
     hipLaunchKernelGGL(bucket_count_kernel, dim3((unsigned)P.na), dim3(kBinThreads), (size_t)P.nb * 4, st, b.X, b.sys,
                        b.atom_sys, b.nsys, b.nat, P, b.key, b.slot, b.bmat, b.status, b.lookback,
-                       lookback_entries(P.n_sort, b.nat));
+                       lookback_entries(P.n_sort, b.nat), b.X_keep);
     hipLaunchKernelGGL(scan_inplace_kernel, dim3((unsigned)scan_tiles(P.n_sort)), dim3(kScanThreads), 0, st, b.bmat,
                        P.n_sort, b.lookback, b.status);
     hipLaunchKernelGGL(bucket_scatter_kernel, dim3((unsigned)P.na), dim3(kBinThreads), 0, st, b.nat, P, b.key, b.slot,
@@ -972,7 +984,7 @@ void launch_build(const PipelineBufs &b, hipStream_t st)
                         hipLaunchKernelGGL(block_sort_kernel<TI>, dim3(1), dim3(kBlockSortThreads), 0, st, b.X, b.sys,
                                            (int)b.nat, b.M, b.status, b.lookback,
                                            lookback_entries(b.sort.n_sort, b.nat), b.cell_start, b.cell_offsets_out,
-                                           b.rec, b.wbig, b.perm_out, b.cell_id_out));
+                                           b.rec, b.wbig, b.perm_out, b.cell_id_out, b.X_keep));
         return;
     }
     if (b.sort.bw >= 0) {

@@ -276,6 +276,7 @@ struct PipelineBufs {
     void *cell_offsets_out;     // M + nsys, TI, 1-based per system
     // pairs
     int32_t *pair_count;
+    double *X_keep;             // Xr where the bucketed sort's first kernel makes that copy, else null
     double *Xr;                 // 3 * nat (R requested): positions the fill reads; X itself, or a copy out of rec
     void *slots;                // nat * slot_cap slot entries
     int32_t slot_cap;
