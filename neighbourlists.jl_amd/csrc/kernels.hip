@@ -96,9 +96,11 @@ __global__ __launch_bounds__(256) void bin_kernel(const double *__restrict__ X, 
 // A block takes its tile from the ticket, so every tile it waits for belongs
 // to a block that started before it and is running or done.  The tickets of
 // a launch are atomics on one address, about 8 ns each (1M atoms: 17 us with
-// them, 13 without), so a launch of up to kOrderlessTiles blocks goes without:
-// that many blocks are on the device together, and whichever starts last
-// starts.  The descriptors are zero before a launch (cleared with the
+// them, 13 without; 1.6M 20 and 15), so a launch of up to kOrderlessTiles blocks goes without:
+// that many blocks (four per CU, of the eight that fit) are on the device
+// together; where other work holds them up, each XCD starts its blocks in order,
+// so the first unfinished one is never among those that wait to start.  The
+// descriptors are zero before a launch (cleared with the
 // status at the start of a build, or by clear_lookback before a repeated
 // pair scan).
 

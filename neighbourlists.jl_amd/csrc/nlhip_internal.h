@@ -25,7 +25,7 @@ constexpr int kMinFillPairs = 128;        // smallest fill tile (pairs per fill 
 // items): the cell sort's scan (n_sort items), then the pair scan's.
 inline int64_t scan_tiles(int64_t n) { return n > 0 ? (n + kScanTile - 1) / kScanTile : 1; }
 constexpr int64_t kLookbackTiles = 2048;  // single-pass scans up to this many tiles
-constexpr unsigned kOrderlessTiles = 256; // single-pass scans whose blocks (one per CU) are on the device together
+constexpr unsigned kOrderlessTiles = 1024; // single-pass scans whose blocks (four per CU) are on the device together
 constexpr int64_t kSortLookbackTiles = 128;   // tiles of the bucketed sort's count scan at most
 inline int64_t lookback_cells(int64_t n_sort) { return scan_tiles(n_sort) + 1; }
 inline int64_t lookback_entries(int64_t n_sort, int64_t nat) { return lookback_cells(n_sort) + scan_tiles(nat) + 1; }
