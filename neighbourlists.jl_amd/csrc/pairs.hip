@@ -3,7 +3,7 @@
 // (src/gpu_kernels.jl:132-180) around the inner loop _for_each_neighbor_pair
 // (src/gpu_kernels.jl:58-101).
 //
-// tile_kernel (count_kernel when R is wanted or shifts are wide) -- work
+// tile_kernel (count_kernel for 16-byte slot entries) -- work
 // unit: a brick of up to 4x4x4 home cells per 256-thread (or 512-thread)
 // workgroup, the bricks launched largest first.  The brick and its one-cell
 // halo are staged in LDS in one load phase (every global load of the phase in
@@ -25,7 +25,7 @@
 // fill_kernel -- one wave per tile of consecutive output pairs, one lane per
 // pair: the tile's first atom comes from the pair scan's tile table, and
 // the lanes copy the slot-row entries of the atoms the tile covers into the
-// PairList arrays (i, j, S and optionally R), so every store is linear.
+// PairList arrays (i, j, S, and R from the positions), so every store is linear.
 #include <algorithm>
 
 #include "device_util.h"
@@ -1357,7 +1357,7 @@ struct TileEnv {
 //
 // Bound by instruction issue: a home atom against four chunks is 39 vector and
 // 30 scalar instructions; at 1M atoms the vector unit issues for 73% of the
-// time (61.5 instructions per home atom, 45 scalar; 73.9 and 64 in the 64-bit
+// time (62.8 instructions per home atom, 46 scalar; 73.9 and 64 in the 64-bit
 // kernel, whose 32-byte atoms also held a CU to four bricks, now five).  The
 // tests as matrix instructions (4 x 4 x 1 in 32 bits, 16 blocks: four home atoms
 // by 64 candidates) took 12 cycles of the wave's SIMD each, more than the
