@@ -171,6 +171,10 @@ struct nlh_handle {
     int64_t pair_capacity = 0;
     bool pair_lookback_clean = false;   // the pair scan's descriptors are zero
     int32_t slot_cap = 0;       // neighbour slots per atom
+    int32_t slot_cap_max = 0;   // ... the most that a build had to grow to
+    int64_t seen_nat = 0;       // a single system's last builds of seen_nat atoms and estimate
+    int32_t seen_est = 0;       // seen_est: their largest count
+    int32_t seen_max = 0;
     bool wide = false;          // 16-byte slot entries (cell shifts beyond +-511)
     const double *X_dev = nullptr;
     std::vector<nlh::SysDev> sys_host;
@@ -203,6 +207,23 @@ struct nlh_handle {
     // count-pass workgroup: 4 waves per brick unless tuned (four 39 KB
     // bricks share a CU; 8-wave bricks of 76 KB fit two)
     int count_block() const { return tune.count_block ? tune.count_block : 256; }
+
+    // Slot rows: 8 slot_cap bytes apart, or packed, the 4-byte rows 4 slot_cap
+    // bytes apart and the 8-byte ones after them all.  Packed rows share their
+    // lines, which is what lets a list of 42 neighbours per atom stay in the
+    // last-level cache between count and fill (1M FCC slab, rows 512 bytes
+    // apart 225 us of fill, 192 bytes apart 174); a list that stays there
+    // anyway gains nothing (1M cube), so rows are packed only where the last
+    // builds' counts are known and they fit what is allocated.
+    bool slot_packed = false;
+    size_t slot_off8() const
+    {
+        return slot_packed ? ((size_t)std::max<int64_t>(nat, 1) * slot_cap * 4 + 127) / 128 * 128 : 0;
+    }
+    size_t slot_bytes() const
+    {
+        return slot_off8() + (size_t)std::max<int64_t>(nat, 1) * slot_cap * (wide ? 16 : 8) + nlh::kSlotSlack;
+    }
 
     nlh::PipelineBufs bufs() const
     {
@@ -241,6 +262,8 @@ struct nlh_handle {
         b.slots = slots.p;
         b.X_keep = keep_X ? Xr.as<double>() : nullptr;
         b.Xr = X_dev == X.as<double>() ? X.as<double>() : Xr.as<double>();
+        b.slot_off8 = slot_off8();
+        b.slot_row4 = (slot_packed ? 4 : 8) * slot_cap;
         b.slot_cap = slot_cap;
         b.pair_off = pair_off.as<int64_t>();
         b.tile_atom = tiles.as<int32_t>();
@@ -964,9 +987,25 @@ int32_t estimate_slot_cap(const nlh_handle *h)
 
 void ensure_slots(nlh_handle *h, int32_t cap)
 {
-    h->slot_cap = std::max(h->slot_cap, cap);
-    const size_t n1 = (size_t)std::max<int64_t>(h->nat, 1) * (size_t)h->slot_cap;
-    h->slots.ensure(h->stream, n1 * (h->wide ? 16 : 8) + nlh::kSlotSlack);
+    h->slot_cap = cap;
+    h->slot_packed = false;
+    h->slots.ensure(h->stream, h->slot_bytes());
+}
+
+// The slot rows of a new build: what the densities say, never less than the
+// handle had to use.  A single system that builds one by one (no captured
+// pipeline to make again) and whose last builds of this size and density are
+// known takes rows of what their largest count needs, packed, where that fits (a
+// build that outgrows them grows the rows, and the next ones know).
+void plan_slots(nlh_handle *h)
+{
+    const int32_t est = estimate_slot_cap(h), cap = std::max(h->slot_cap_max, est);
+    if (h->nsys == 1 && h->nat >= kReplayMaxAtoms && !h->wide && h->seen_nat == h->nat && h->seen_est == est) {
+        h->slot_cap = std::min(cap, round_slot_cap(std::max(h->seen_max, 1)));
+        h->slot_packed = true;
+        if (h->slot_bytes() <= h->slots.cap) return;
+    }
+    ensure_slots(h, cap);
 }
 
 void ensure_pair_outputs(nlh_handle *h, int64_t cap, bool want_R)
@@ -1142,9 +1181,8 @@ void finish_pairs(nlh_handle *h, bool want_R);
 void check_pair_buffers(const nlh_handle *h, bool want_R)
 {
     const size_t n1 = (size_t)std::max<int64_t>(h->nat, 1);
-    const size_t ent = (size_t)h->slot_cap * n1;
     const size_t ti = (size_t)h->ti_bytes, cap = (size_t)std::max<int64_t>(h->pair_capacity, 0);
-    bool ok = h->slot_cap > 0 && h->slots.p && h->slots.cap >= ent * (h->wide ? 16 : 8) + nlh::kSlotSlack;
+    bool ok = h->slot_cap > 0 && h->slots.p && h->slots.cap >= h->slot_bytes();
     ok = ok && h->pair_count.cap >= n1 * 4 && h->pair_off.cap >= (n1 + 1) * 8;
     ok = ok && h->first.cap >= (n1 + h->nsys) * ti && h->sys_pair_base.cap >= (size_t)(h->nsys + 1) * 8;
     ok = ok && h->i.cap >= cap * ti && h->j.cap >= cap * ti && h->S.cap >= cap * 3 * ti;
@@ -1179,7 +1217,7 @@ void materialize(nlh_handle *h, uint32_t flags)
         return;
     }
     ensure_pair_outputs(h, std::max(h->pair_capacity, estimate_pairs(h)), want_R);
-    ensure_slots(h, std::max(h->slot_cap, estimate_slot_cap(h)));
+    plan_slots(h);
     check_pair_buffers(h, want_R);
     nlh::PipelineBufs b = h->bufs();
     mark(h, 1);
@@ -1211,8 +1249,10 @@ void materialize(nlh_handle *h, uint32_t flags)
         // (the counts, offsets and totals of the first pass stay valid)
         if (st.wide) h->wide = true;
         ensure_pair_outputs(h, std::max<int64_t>(st.npairs, 1), want_R);
-        h->slots.release(h->stream);
-        ensure_slots(h, round_slot_cap(std::max(st.max_count, 1)));
+        const int32_t cap = std::max(h->slot_cap, round_slot_cap(std::max(st.max_count, 1)));
+        h->slot_cap = h->slot_cap_max = std::max(h->slot_cap_max, cap);
+        if (h->slots.cap < h->slot_bytes()) h->slots.release(h->stream);
+        ensure_slots(h, h->slot_cap);
         check_pair_buffers(h, want_R);
         b = h->bufs();
         nlh::launch_count(b, want_R, h->wide, h->stream);
@@ -1232,6 +1272,13 @@ void finish_pairs(nlh_handle *h, bool want_R)
 {
     h->npairs = h->status_host->npairs;
     h->have_R = want_R;
+    if (h->nsys == 1) {
+        const int32_t est = estimate_slot_cap(h);
+        if (h->seen_nat != h->nat || h->seen_est != est) h->seen_max = 0;
+        h->seen_nat = h->nat;
+        h->seen_est = est;
+        h->seen_max = std::max(h->seen_max, h->status_host->max_count);
+    }
     // per-system pair offsets
     h->pair_offsets_host.resize(h->nsys + 1);
     h->offsets_stale = false;
@@ -1294,7 +1341,7 @@ bool rebuild_graph(nlh_handle *h, bool want_R)
     // and not at the build that sized them)
     ensure_pair_buffers(h);
     ensure_pair_outputs(h, std::max(h->pair_capacity, estimate_pairs(h)), want_R);
-    ensure_slots(h, std::max(h->slot_cap, estimate_slot_cap(h)));
+    plan_slots(h);
     check_pair_buffers(h, want_R);
     const nlh::PipelineBufs b = h->bufs();
     // the slot-entry width is baked into the captured count and fill: a build
@@ -1564,6 +1611,8 @@ size_t carve_noalloc(char *base, const NoAllocPlan &P, int ti, int32_t cap, bool
     const size_t rows = n1 * (size_t)cap;
     b.slots = c.take<void>(std::max(rows * (wide ? 16 : 8), n1 * nlh::kBucketBytes));
     b.bke = reinterpret_cast<int2 *>(b.slots);
+    b.slot_off8 = 0;            // every row 8 cap bytes: the limit's layout
+    b.slot_row4 = 8 * cap;
     b.slot_cap = cap;
     if (want_R) c.take<void>(rows * 24);
     b.Xr = const_cast<double *>(X);   // the call ends after its fill

@@ -278,7 +278,9 @@ struct PipelineBufs {
     int32_t *pair_count;
     double *X_keep;             // Xr where the bucketed sort's first kernel makes that copy, else null
     double *Xr;                 // 3 * nat (R requested): positions the fill reads; X itself, or a copy out of rec
-    void *slots;                // nat * slot_cap slot entries
+    void *slots;                // nat rows of slot_cap entries: 4-byte rows, and from slot_off8 on 8-byte rows
+    int64_t slot_off8;          // bytes
+    int32_t slot_row4;          // bytes between 4-byte rows
     int32_t slot_cap;
     int64_t *pair_off;          // nat + 1
     int32_t *tile_atom;         // 2 tile_cap: atom owning pair t * fill_pairs, its pairs before it

@@ -1375,7 +1375,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(5))) void ti
     const SysDev *__restrict__ sys, const int32_t *__restrict__ sys_cell_base, const int32_t *__restrict__ sys_brick_base,
     int nsys, int copies, int32_t M, int64_t nat, const int32_t *__restrict__ cell_start,
     const Rec *__restrict__ rec, const int32_t *__restrict__ wbig, int32_t *__restrict__ pair_count,
-    void *__restrict__ slots, int32_t cap, Status *__restrict__ status)
+    void *__restrict__ slots, int64_t off8, int32_t row4, int32_t cap, Status *__restrict__ status)
 {
     __shared__ TileLDS<BT> L;
     __shared__ double Csh[9];
@@ -1390,7 +1390,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(5))) void ti
     const int lane = lane_id();
     const int wv = sgpr((int)(threadIdx.x >> 6));
     if (!lds) {
-        const SlotArgs O{slots, cap, status};
+        const SlotArgs O{reinterpret_cast<char *>(slots) + off8, cap, status};
         for (int hc = 0; hc < B.nhome; ++hc)
             count_cell<false>(A, *B.sd, brick_cell_id(B, hc), pair_count, O, hc, copy + copies * wv,
                               copies * BrickShape<BT>::waves);
@@ -1441,7 +1441,8 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(5))) void ti
             H.nz = oz - h.z;
             const float hq = 0.5f * __builtin_fmaf(H.nz, H.nz, __builtin_fmaf(H.ny, H.ny, H.nx * H.nx));
             H.ai = hq - sd.rc2half;
-            H.row = (reinterpret_cast<uint64_t>(slots) + 8ull * (uint64_t)slot_row(sd.atom_base + hj_l, cap)) |
+            H.row = (reinterpret_cast<uint64_t>(slots) + (narrow ? 0 : off8) +
+                     (uint64_t)slot_row(sd.atom_base + hj_l, narrow ? row4 : 8 * cap)) |
                     (uint64_t)(narrow ? 4 : 8) << 48;
             H.t = L.t[hl];
             H.fill = 0;
@@ -1591,7 +1592,8 @@ struct SmallArgs {
     void *__restrict__ cell_offsets_out;
     int32_t *__restrict__ pair_count;
     void *__restrict__ slots;
-    int32_t cap, item_tests;
+    int64_t off8;
+    int32_t row4, cap, item_tests;
     Status *__restrict__ status;
 };
 
@@ -1713,7 +1715,7 @@ __device__ __forceinline__ int32_t small_far(const SmallArgs &A, const SmallLDS 
             if (((m >> lane) & 1) && rank < A.cap) {
                 const uint32_t spk = pack_wind(Sx, Sy, Sz);
                 if (spk & kWindBig) A.status->wide = 1;
-                reinterpret_cast<uint64_t *>(A.slots)[slot_row(base + i, A.cap) + rank] =
+                reinterpret_cast<uint64_t *>(reinterpret_cast<char *>(A.slots) + A.off8)[slot_row(base + i, A.cap) + rank] =
                     (uint64_t)(uint32_t)j | (uint64_t)spk << 32;
             }
             fill = write_lane(f + 8 * (int)__popcll(m), a, fill);
@@ -1926,7 +1928,8 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
             const float hq = 0.5f * __builtin_fmaf(H.nz, H.nz, __builtin_fmaf(H.ny, H.ny, H.nx * H.nx));
             H.ai = hq - sd->rc2half;
             const int64_t ha = sd->atom_base + h.j;
-            H.row = (reinterpret_cast<uint64_t>(A.slots) + 8ull * (uint64_t)slot_row(ha, A.cap)) |
+            H.row = (reinterpret_cast<uint64_t>(A.slots) + (row8 ? A.off8 : 0) +
+                     (uint64_t)slot_row(ha, row8 ? 8 * A.cap : A.row4)) |
                     (uint64_t)(row8 ? 8 : 4) << 48;
             H.t = 2 * kPackZero - L.w[hl];   // t'_i = -w_i
             H.fill = 0;
@@ -2044,7 +2047,8 @@ static void small_launch(const PipelineBufs &b, hipStream_t st)
 {
     SmallArgs A{b.X,          b.sys,     b.sys_atom_base, b.sys_cell_base, b.units,  b.unit_order,
                 b.atom_sys,   b.rec,     b.perm_out,      b.cell_id_out,   b.cell_offsets_out,
-                b.pair_count, b.slots,   b.slot_cap,      b.item_tests,    b.status};
+                b.pair_count, b.slots,   b.slot_off8,     b.slot_row4,     b.slot_cap,
+                b.item_tests, b.status};
     hipLaunchKernelGGL((small_kernel<TI>), dim3((unsigned)b.nitems), dim3(kSmallThreads), 0, st, A);
 }
 
@@ -2091,15 +2095,16 @@ struct RawEntry<true> {
 };
 
 template <bool WIDE>
-__device__ __forceinline__ RawEntry<WIDE> load_entry(const void *__restrict__ slots, int64_t rs, int r, bool row8)
+__device__ __forceinline__ RawEntry<WIDE> load_entry(const void *__restrict__ slots, int64_t off8, int32_t row4, int32_t cap,
+                                                     uint32_t row, int r, bool row8)
 {
     RawEntry<WIDE> x;
     if constexpr (WIDE) {
-        x.e = reinterpret_cast<const int4 *>(slots)[rs + r];
+        x.e = reinterpret_cast<const int4 *>(slots)[slot_row(row, cap) + r];
     } else {
-        // 8-byte rows: entry rs + r; 4-byte rows: 4-byte entry 2 rs + r of
-        // the same row (the 8 bytes read stay inside the row: 4 r + 8 <= 8 cap)
-        const int64_t byte = 8 * rs + ((int64_t)r << (row8 ? 3 : 2));
+        // a 4-byte row's last entry is read with the 4 bytes after it (the next
+        // row's, or the 8-byte rows')
+        const int64_t byte = (row8 ? off8 : 0) + slot_row(row, row8 ? 8 * cap : row4) + (r << (row8 ? 3 : 2));
         __builtin_memcpy(&x.e, reinterpret_cast<const char *>(slots) + byte, 8);
         x.w8 = row8;
     }
@@ -2196,7 +2201,7 @@ __global__ __launch_bounds__(1024) void fill_kernel(
     const double *__restrict__ X, const SysDev *__restrict__ sys, const int64_t *__restrict__ sys_atom_base,
     const int32_t *__restrict__ atom_sys, int nsys, int64_t nat, const int32_t *__restrict__ pair_count,
     const int64_t *__restrict__ pair_off, const int32_t *__restrict__ tile_atom, int64_t tile_cap,
-    const void *__restrict__ slots, const Status *__restrict__ status,
+    const void *__restrict__ slots, int64_t off8, int32_t row4, const Status *__restrict__ status,
     Status *__restrict__ status_pub, int32_t cap, int64_t pair_capacity, TI *__restrict__ i_out,
     TI *__restrict__ j_out, TI *__restrict__ S_out, double *__restrict__ R_out)
 {
@@ -2286,10 +2291,10 @@ __global__ __launch_bounds__(1024) void fill_kernel(
             // pairs past the tile's end read entry 0 of row 0 (in bounds, never
             // stored): no branch around the load
             const int r = live ? q - f[u] : 0;
-            const int64_t rs = live ? (A0 + s[u]) * (int64_t)cap : 0;
+            const uint32_t row = live ? (uint32_t)(A0 + s[u]) : 0u;
             const bool w8 = ((row8 >> s[u]) & 1) != 0;
             is[u] = batch ? __shfl(il, s[u], kWave) : (int32_t)(A0 + s[u] + 1);
-            e[u] = load_entry<WIDE>(slots, rs, r, w8);
+            e[u] = load_entry<WIDE>(slots, off8, row4, cap, row, r, w8);
         }
         if constexpr (!WANT_R) {
 #pragma unroll
@@ -2345,7 +2350,7 @@ __global__ __launch_bounds__(1024) void fill_kernel(
         const int r = (int)(P - pair_off[lo]);
         const int ls = nsys > 1 ? atom_sys[lo] : 0;
         const int32_t isv = (int32_t)(lo - (nsys > 1 ? sys_atom_base[ls] : 0) + 1);
-        const RawEntry<WIDE> e = load_entry<WIDE>(slots, lo * (int64_t)cap, r, (pair_count[lo] & kRow8Bit) != 0);
+        const RawEntry<WIDE> e = load_entry<WIDE>(slots, off8, row4, cap, (uint32_t)lo, r, (pair_count[lo] & kRow8Bit) != 0);
         int32_t j, Sx, Sy, Sz;
         decode_entry<WIDE>(e, j, Sx, Sy, Sz);
         fill_store_pairs<TI>(isv, j, Sx, Sy, Sz, pos0, n, i_out, j_out, S_out, lds);
@@ -2375,6 +2380,7 @@ __global__ __launch_bounds__(256) void fill_R_kernel(const double *__restrict__ 
                                                      int64_t nat, const Rec *__restrict__ rec,
                                                      const int32_t *__restrict__ pair_count,
                                                      const int64_t *__restrict__ pair_off, const void *__restrict__ slots,
+                                                     int64_t off8, int32_t row4,
                                                      const Status *__restrict__ status, int32_t cap,
                                                      int64_t pair_capacity, double *__restrict__ R_out)
 {
@@ -2411,7 +2417,7 @@ __global__ __launch_bounds__(256) void fill_R_kernel(const double *__restrict__ 
         const int r = live ? q - fs : 0;
         const int64_t ga = (int64_t)(int)__shfl((int)gi, s, kWave);
         const int64_t o = (int64_t)shfl64((uint64_t)off, s) + r;
-        const RawEntry<false> e = load_entry<false>(slots, live ? ga * cap : 0, r, (row8 >> s) & 1);
+        const RawEntry<false> e = load_entry<false>(slots, off8, row4, cap, live ? (uint32_t)ga : 0u, r, (row8 >> s) & 1);
         int32_t j, Sx, Sy, Sz;
         decode_entry<false>(e, j, Sx, Sy, Sz);
         const int64_t gj = live ? j : ga;
@@ -2467,7 +2473,7 @@ static void count_launch(const PipelineBufs &b, bool wide, hipStream_t st)
     else
         hipLaunchKernelGGL(tile_kernel<BT>, dim3((unsigned)(b.nbricks * b.brick_copies)), dim3(BT), 0, st, b.sys,
                            b.sys_cell_base, b.sys_brick_base, b.nsys, b.brick_copies, b.M, b.nat, b.cell_start, b.rec,
-                           b.wbig, b.pair_count, b.slots, b.slot_cap, b.status);
+                           b.wbig, b.pair_count, b.slots, b.slot_off8, b.slot_row4, b.slot_cap, b.status);
 }
 
 void launch_count(const PipelineBufs &b, bool want_R, bool wide, hipStream_t st)
@@ -2492,7 +2498,7 @@ static bool fill_launch(const PipelineBufs &b, hipStream_t st)
     const unsigned nblk = (unsigned)((waves * kWave + bs - 1) / bs);
     const size_t lds = R || sizeof(TI) == 8 ? bs / kWave * kTripleBytes : 0;
     hipLaunchKernelGGL((fill_kernel<R, W, TI, TW>), dim3(nblk), dim3(bs), lds, st, b.Xr, b.sys, b.sys_atom_base,
-                       b.atom_sys, b.nsys, b.nat, b.pair_count, b.pair_off, b.tile_atom, b.tile_cap, b.slots, b.status,
+                       b.atom_sys, b.nsys, b.nat, b.pair_count, b.pair_off, b.tile_atom, b.tile_cap, b.slots, b.slot_off8, b.slot_row4, b.status,
                        b.status_pub, b.slot_cap, b.pair_capacity, (TI *)b.i_out, (TI *)b.j_out, (TI *)b.S_out, b.R_out);
     return true;
 }
@@ -2511,8 +2517,8 @@ static bool fill_dispatch(const PipelineBufs &b, bool want_R, bool wide, hipStre
     if (want_R && b.nsys == 1 && !wide && b.nat > kRCellOrder) {
         const bool launched = fill_tiles<false, false, TI>(b, st);
         hipLaunchKernelGGL(fill_R_kernel, dim3((unsigned)((b.nat + 4 * kRAtoms - 1) / (4 * kRAtoms))), dim3(256), 0, st,
-                           b.Xr, b.sys, b.nat, b.rec, b.pair_count, b.pair_off, b.slots, b.status, b.slot_cap,
-                           b.pair_capacity, b.R_out);
+                           b.Xr, b.sys, b.nat, b.rec, b.pair_count, b.pair_off, b.slots, b.slot_off8, b.slot_row4, b.status,
+                           b.slot_cap, b.pair_capacity, b.R_out);
         return launched;
     }
     if (want_R) return wide ? fill_tiles<true, true, TI>(b, st) : fill_tiles<true, false, TI>(b, st);

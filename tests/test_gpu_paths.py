@@ -364,3 +364,31 @@ def test_lists_in_host_memory(n, int_type, bits):
     for t in threads:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("n", [12288, 30000])
+@pytest.mark.parametrize("int_type,bits", [(np.int32, 32), (np.int64, 64)])
+def test_slot_rows_follow_the_last_builds(n, int_type, bits):
+    """Repeated builds on one handle: a crystal whose rows shrink to its counts,
+    atoms that outgrow them (4-byte rows, 8-byte rows of unwrapped atoms), 16-byte
+    rows, another density and cutoff, and back."""
+    X, cell = workloads.fcc(3.61, (15, 15, (n + 899) // 900))
+    X, rng = X[:n], np.random.default_rng(n)
+    pbc = (True, True, False)
+    close = X.copy()
+    close[-60:] = X[50] + rng.random((60, 3))
+    moved = X.copy()
+    moved[::4] += cell[0] * rng.integers(-3, 4, (len(X[::4]), 1))
+    wide = X.copy()
+    wide[::9] += 600 * cell[1]
+    h = _lib.Handle()
+    for k, (Y, rc) in enumerate([(X, 4.9), (X, 4.9), (X, 4.9), (moved, 4.9), (close, 4.9), (X, 4.9), (X, 6.0), (X, 4.9),
+                                 (X * 0.9, 4.9), (wide, 4.9), (moved, 4.9), (X, 4.9)]):
+        print(f"slot rows {n} {bits} {k}", flush=True)
+        for want_R in ((False, True) if k in (2, 4) else (False,)):
+            ref = oracle.neighbour_list(Y, rc, cell, pbc, ti_bits=bits, want_R=want_R, nthreads=8)
+            nl = nlhip.neighbour_list(Y, rc, cell, pbc, int_type=int_type, want_R=want_R, handle=h)
+            assert np.array_equal(nl.first, ref.first)
+            assert np.array_equal(nl.i, ref.i) and np.array_equal(nl.j, ref.j) and np.array_equal(nl.S, ref.S)
+            if want_R:
+                assert np.array_equal(_bits(nl.R), _bits(ref.R))
