@@ -1261,8 +1261,8 @@ void materialize(nlh_handle *h, uint32_t flags)
         h->status_pub_pending = nlh::launch_fill(b, want_R, h->wide, h->stream);
         HIPC(hipGetLastError());
         wait_status(h);
-        if (h->status_host->npairs > h->pair_capacity || h->status_host->max_count > h->slot_cap)
-            throw Error(NLH_EDEVICE, "pair capacity still exceeded after growth");
+        if (st.npairs > h->pair_capacity || st.max_count > h->slot_cap || (st.wide && !h->wide))
+            throw Error(NLH_EDEVICE, "internal: pair capacity or slot entries still too small after growth");
     }
     finish_pairs(h, want_R);
 }

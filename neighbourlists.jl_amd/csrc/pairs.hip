@@ -144,15 +144,17 @@ __device__ __forceinline__ void emit_hits(const SlotArgs &O, uint64_t mask, int6
     if (mask == 0) return;   // wave-uniform
     const int lane = lane_id();
     const int32_t rank = ca + (int32_t)mbcnt64(mask);
-    if (((mask >> lane) & 1) && rank < O.cap) {
+    if ((mask >> lane) & 1) {
         const int64_t sidx = sbase + rank;
         if (WIDE) {
-            reinterpret_cast<int4 *>(O.slots)[sidx] = make_int4(cj, tx + wix, ty + wiy, tz + wiz);
+            if (rank < O.cap) reinterpret_cast<int4 *>(O.slots)[sidx] = make_int4(cj, tx + wix, ty + wiy, tz + wiz);
         } else {
-            // S = s_loop + w_i - w_j = t + w_i  (gpu_kernels.jl:88)
+            // S = s_loop + w_i - w_j = t + w_i  (gpu_kernels.jl:88).  Entries past a
+            // row's end count too: the repeat on longer rows is the last one
             const uint32_t spk = wzero ? t_pk : pack_wind(tx + wix, ty + wiy, tz + wiz);
             if (spk & kWindBig) O.status->wide = 1;
-            reinterpret_cast<uint64_t *>(O.slots)[sidx] = (uint64_t)(uint32_t)cj | ((uint64_t)spk << 32);
+            if (rank < O.cap)
+                reinterpret_cast<uint64_t *>(O.slots)[sidx] = (uint64_t)(uint32_t)cj | ((uint64_t)spk << 32);
         }
     }
     ca += __popcll(mask);
@@ -1712,11 +1714,12 @@ __device__ __forceinline__ int32_t small_far(const SmallArgs &A, const SmallLDS 
             const uint64_t m = __builtin_amdgcn_ballot_w64(r2 < sd->rc2 && k < total && k != ks + a);
             const int32_t f = __builtin_amdgcn_readlane(fill, a);
             const int rank = (f >> 3) + (int)mbcnt64(m);
-            if (((m >> lane) & 1) && rank < A.cap) {
+            if ((m >> lane) & 1) {
                 const uint32_t spk = pack_wind(Sx, Sy, Sz);
-                if (spk & kWindBig) A.status->wide = 1;
-                reinterpret_cast<uint64_t *>(reinterpret_cast<char *>(A.slots) + A.off8)[slot_row(base + i, A.cap) + rank] =
-                    (uint64_t)(uint32_t)j | (uint64_t)spk << 32;
+                if (spk & kWindBig) A.status->wide = 1;   // past the row's end too (see emit_hits)
+                if (rank < A.cap)
+                    reinterpret_cast<uint64_t *>(reinterpret_cast<char *>(A.slots) + A.off8)[slot_row(base + i, A.cap) + rank] =
+                        (uint64_t)(uint32_t)j | (uint64_t)spk << 32;
             }
             fill = write_lane(f + 8 * (int)__popcll(m), a, fill);
         }
