@@ -112,7 +112,10 @@ int nlh_geometry_init(const double cell[9], double cutoff, const uint8_t pbc[3],
  * (src/cell_list.jl:647-679) -- _compute_cell_ids (:684 / gpu_kernels.jl:378),
  * _get_sortperm (:706 / :711) and _compute_cell_offsets (:724 /
  * gpu_kernels.jl:386).  X is nat x 3 float64 (host, or device with
- * NLH_X_DEVICE; a device X must stay valid while the handle uses it). */
+ * NLH_X_DEVICE).  Lazy queries read a device X (X_orig) as it is when they
+ * are called, against the cells of the build, so it must stay valid until
+ * the last of them; nlh_materialize and nlh_copy_celllist's X_sorted take
+ * the positions of the build. */
 int nlh_build_cell_list(nlh_handle *h, const double *X, int64_t nat, const nlh_geometry *geom, uint32_t flags);
 
 /* Two-pass pair materialisation: replaces materialize_pairlist

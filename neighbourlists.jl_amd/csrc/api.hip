@@ -1469,8 +1469,7 @@ void neighbours_range(nlh_handle *h, int32_t sys, int64_t i_first, int64_t n)
     q.i_first = i_first - 1;
     q.n = n;
     q.X = h->X_dev;
-    q.rec = h->rec.as<nlh::Rec>();
-    q.wbig = h->wbig.as<int32_t>();
+    q.perm = h->perm.p;
     q.cell_offsets = h->cell_offsets.p;
     q.count = h->nr_count.as<int32_t>();
     q.off = h->nr_off.as<int64_t>();

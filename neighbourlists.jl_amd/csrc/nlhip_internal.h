@@ -335,9 +335,8 @@ struct LazyRange {
     const SysDev *sys;          // the system
     int32_t isys;
     int64_t i_first, n;
-    const double *X;            // positions of the whole build
-    const Rec *rec;
-    const int32_t *wbig;
+    const double *X;            // positions of the whole build, as they are now
+    const void *perm;           // of the whole build, TI, 1-based per system
     const void *cell_offsets;   // of the whole build, TI, 1-based per system
     int32_t *count;             // n
     int64_t *off;               // n + 1: first neighbour of each atom, then the total

@@ -241,7 +241,9 @@ struct Cand {
     bool zero_shift, valid;
 };
 
-__device__ __forceinline__ Cand load_candidate(const PairsArgs &A, int k, int total, int excl, int start_g, uint32_t shp)
+// Candidate k of a segment batch: its place in the sorted order (below the
+// batch's end only for k < its total) and its segment's packed shift.
+__device__ __forceinline__ int candidate_place(int k, int excl, int start_g, uint32_t shp, uint32_t &shm)
 {
     int m = 0;
 #pragma unroll
@@ -249,8 +251,14 @@ __device__ __forceinline__ Cand load_candidate(const PairsArgs &A, int k, int to
         const int e2 = __shfl(excl, m + step, kWave);
         if (e2 <= k) m += step;
     }
-    const int p = __shfl(start_g, m, kWave) + (k - __shfl(excl, m, kWave));
-    const uint32_t shm = __shfl(shp, m, kWave);
+    shm = __shfl(shp, m, kWave);
+    return __shfl(start_g, m, kWave) + (k - __shfl(excl, m, kWave));
+}
+
+__device__ __forceinline__ Cand load_candidate(const PairsArgs &A, int k, int total, int excl, int start_g, uint32_t shp)
+{
+    uint32_t shm;
+    const int p = candidate_place(k, excl, start_g, shp, shm);
     Cand c;
     c.valid = k < total;
     int32_t wjx = 0, wjy = 0, wjz = 0;
@@ -375,19 +383,24 @@ __device__ __forceinline__ void count_cell(const PairsArgs &A, const SysDev &sd,
 // counted, with it they are written from off[a] on (nothing when the total
 // off[n] exceeds cap: the host grows the outputs and runs it again).
 //
+// Every position, the home atom's and the candidates', is read from X, as
+// nlh_for_each_neighbour (nlhip_device.h) reads it: the caller may have moved
+// atoms since the build, and R_ij = -R_ji and the one-atom query hold all the
+// same.
+//
 // Latency-bound: a query of a few thousand atoms is one wave per SIMD.  With
-// one thread per atom walking the cells through perm and the positions the
-// two passes over 4,096 atoms of a 50,000-atom cube took 248 us each; a
-// wave per atom reading the sorted records takes 9 and 10 us.
+// one thread per atom walking the cells the two passes over 4,096 atoms of a
+// 50,000-atom cube took 248 us each; a wave per atom takes 12 and 15 us.
 template <typename TI, bool FILL>
 __global__ __launch_bounds__(kPairsBlock) void lazy_range_kernel(LazyRange Q)
 {
     const int64_t a = (int64_t)blockIdx.x * kWavesPerPairsBlock + sgpr((int)(threadIdx.x / kWave));
     if (a >= Q.n) return;   // wave-uniform
-    int64_t run = 0;
+    int64_t run = 0, end = 0;
     if (FILL) {
         if (Q.off[Q.n] > Q.cap) return;
         run = Q.off[a];
+        end = Q.off[a + 1];   // never past the atom's own run, whatever becomes of X between the passes
     }
     const SysDev &sd = *Q.sys;
     const int64_t il = Q.i_first + a;   // 0-based, local to the system
@@ -398,7 +411,7 @@ __global__ __launch_bounds__(kPairsBlock) void lazy_range_kernel(LazyRange Q)
     HomeCell H;
     home_grid(sd, ci[0], ci[1], ci[2], H);
     const TI *co = static_cast<const TI *>(Q.cell_offsets) + (int64_t)sd.cell_base + Q.isys;
-    const PairsArgs A{Q.sys, nullptr, 1, sd.M, sd.nat, nullptr, Q.rec, Q.wbig};
+    const TI *perm = static_cast<const TI *>(Q.perm);
     const int lane = lane_id();
     const double rc2 = sd.rc2;
     for (int sb = 0; sb < H.nseg; sb += kWave) {
@@ -410,17 +423,27 @@ __global__ __launch_bounds__(kPairsBlock) void lazy_range_kernel(LazyRange Q)
             n = (int)((int64_t)co[c + 1] - s0);
         });
         for (int k0 = 0; k0 < total; k0 += kWave) {
-            const Cand c = load_candidate(A, k0 + lane, total, excl, start_g, shp);
-            const int32_t Sx = c.tx + wi[0], Sy = c.ty + wi[1], Sz = c.tz + wi[2];
+            uint32_t shm;
+            const int p = candidate_place(k0 + lane, excl, start_g, shp, shm);
+            const bool valid = k0 + lane < total;
+            const int32_t j = valid ? (int32_t)perm[p] - 1 : 0;   // 0-based, local to the system
+            const double *xj = Q.X + 3 * (sd.atom_base + j);
+            const double x = xj[0], y = xj[1], z = xj[2];
+            int32_t cj[3], wj[3], s[3];
+            cell_and_winding(sd, x, y, z, cj, wj);
+            unpack_wind(shm, s[0], s[1], s[2]);
+            // S = s_loop + w_i - w_j  (gpu_kernels.jl:88)
+            const int32_t Sx = s[0] + wi[0] - wj[0], Sy = s[1] + wi[1] - wj[1], Sz = s[2] + wi[2] - wj[2];
             double cx, cy, cz;
             cell_shift(sd.C, Sx, Sy, Sz, cx, cy, cz);
-            const double Rx = (c.x - hx) + cx, Ry = (c.y - hy) + cy, Rz = (c.z - hz) + cz;
+            const double Rx = (x - hx) + cx, Ry = (y - hy) + cy, Rz = (z - hz) + cz;
             const double r2 = (Rx * Rx + Ry * Ry) + Rz * Rz;
-            const bool hit = c.valid & (r2 < rc2) & !(c.zero_shift & (c.j == (int32_t)il));
+            const bool self = j == (int32_t)il && (s[0] | s[1] | s[2]) == 0;
+            const bool hit = valid & (r2 < rc2) & !self;
             const uint64_t m = __ballot(hit);
-            if (FILL && hit) {
-                const int64_t q = run + mbcnt64(m);
-                static_cast<TI *>(Q.j)[q] = (TI)(c.j + 1);
+            const int64_t q = run + mbcnt64(m);
+            if (FILL && hit && q < end) {
+                static_cast<TI *>(Q.j)[q] = (TI)(j + 1);
                 double *R = Q.R + 3 * q;
                 R[0] = Rx;
                 R[1] = Ry;

@@ -77,3 +77,37 @@ def test_wide_entries_behind_short_rows_of_a_batch():
     got = nlhip.BatchBuilder().run(systems)
     for k, y in enumerate(systems):
         _same(got.pairlist(k), oracle.neighbour_list(y.X, y.cutoff, y.cell, y.pbc))
+
+
+@pytest.mark.parametrize("int_type,bits", [(np.int32, 32), (np.int64, 64)])
+@pytest.mark.parametrize("n,density,moved", [(40, 0.05, 1.0), (3000, 0.05, 0.3), (3000, 0.01, 1.0), (20000, 0.05, 0.02)])
+def test_lazy_queries_read_the_positions_as_they_are(n, density, moved, int_type, bits):
+    """Device positions moved in place between the build and the queries: a
+    range query sees for every atom what the one-atom query sees."""
+    s = workloads.random_cubic(n, density=density, seed=n, cutoff=5.0, pbc=(True, n != 3000, True))
+    X = torch.as_tensor(s.X).cuda()
+    cl = nlhip.build_cell_list(X, 5.0, s.cell, s.pbc, int_type=int_type)
+    print(f"lazy, moved {n} {moved} {bits}", flush=True)
+    rng = np.random.default_rng(n)
+    before = nlhip.neighbours_range(cl, 1, min(n, 500))
+    Y = s.X + 0.4 * rng.standard_normal((n, 3)) * (rng.random((n, 1)) < moved)
+    Y[::50] += np.asarray(s.cell)[0]
+    X.copy_(torch.as_tensor(Y))
+    torch.cuda.synchronize()
+    first, m = 2, min(n - 1, 600)
+    offs, j, R, S = nlhip.neighbours_range(cl, first, m)
+    L, h = _lib.lib(), cl._handle
+    dt = np.int32 if bits == 32 else np.int64
+    for a in range(0, m, 1 if n < 1000 else 7):
+        c = ctypes.c_int64()
+        j1, R1, S1 = np.empty(4096, dt), np.empty((4096, 3)), np.empty((4096, 3), dt)
+        _lib.check(L.nlh_neighbours(h.ptr, 0, first + a, 4096, j1.ctypes.data, R1.ctypes.data, S1.ctypes.data,
+                                    ctypes.byref(c)))
+        q, k = slice(offs[a], offs[a + 1]), c.value
+        assert offs[a + 1] - offs[a] == k and np.array_equal(j[q], j1[:k]) and np.array_equal(S[q], S1[:k])
+        assert np.array_equal(_bits(R[q]), _bits(R1[:k]))
+    # and the positions as they were give the first answer again
+    X.copy_(torch.as_tensor(s.X))
+    torch.cuda.synchronize()
+    for u, v in zip(nlhip.neighbours_range(cl, 1, min(n, 500)), before):
+        assert np.array_equal(u, v)
