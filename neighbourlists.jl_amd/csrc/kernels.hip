@@ -93,19 +93,25 @@ __global__ __launch_bounds__(256) void bin_kernel(const double *__restrict__ X, 
 // acquire and release each access also wrote back and invalidated the L2
 // (bucket counts of 1M atoms, 118 tiles: 8.5 -> 4.4 us).
 //
-// A block takes its tile from the ticket, so every tile it waits for belongs
-// to a block that started before it and is running or done.  The tickets of
-// a launch are atomics on one address, about 8 ns each (1M atoms: 17 us with
-// them, 13 without; 1.6M 20 and 15), so a launch of up to kOrderlessTiles blocks goes without:
-// that many blocks (four per CU, of the eight that fit) are on the device
-// together; where other work holds them up, each XCD starts its blocks in order,
-// so the first unfinished one is never among those that wait to start.  The
-// descriptors are zero before a launch (cleared with the
-// status at the start of a build, or by clear_lookback before a repeated
-// pair scan).
+// A block waits for tiles before its own, whose blocks may not have started
+// (other launches' waiting blocks can hold their places).  The pair scan's
+// blocks then help themselves: a wave that has waited kHelpSpins turns sums
+// the counts of the tiles it waits for, so every block that runs ends by
+// itself, whatever else runs.  The other two scans write over their input:
+// they take their tile from the ticket, so that every tile a block waits for
+// belongs to one that started before it and is running or done, except for
+// launches too small to block one another (kOrderlessTiles).  Tickets are
+// atomics on one address, about 8 ns each (pair counts of 1M atoms: 17 us with
+// them, 13 without; 1.6M 20 and 15).  The descriptors are zero before a launch
+// (cleared with the status at the start of a build, or by clear_lookback
+// before a repeated pair scan).
 
 constexpr uint64_t kDescAgg = 1ull << 62, kDescInc = 2ull << 62, kDescVal = kDescAgg - 1;
 constexpr int kLookbackSpins = 1 << 20;   // about a second: reached only if an invariant is broken
+#ifndef NLH_HELP_SPINS
+#define NLH_HELP_SPINS 256                // some 0.2 ms, a hundred times what a running block waits
+#endif
+constexpr int kHelpSpins = NLH_HELP_SPINS;
 
 __device__ __forceinline__ void load_tile(const int32_t *__restrict__ in, int64_t n, int64_t base, int32_t v[kScanItems],
                                           int32_t mask = -1)
@@ -175,8 +181,8 @@ __global__ __launch_bounds__(kScanThreads) void scan_partials_kernel(int64_t *__
 }
 
 // The tile of this block: its index when no block waits for another (tile
-// sums given: three-kernel scan) or all of them are on the device together,
-// else by ticket.  Returns -1 for a block with no tile (see scan_ticket).
+// sums given: three-kernel scan) or they are few (kOrderlessTiles), else by
+// ticket.  Returns -1 for a block with no tile (see scan_ticket).
 __device__ __forceinline__ int64_t scan_tile_begin(uint64_t *__restrict__ desc, const int64_t *__restrict__ partials,
                                                    Status *__restrict__ status)
 {
@@ -200,6 +206,15 @@ __device__ __forceinline__ int64_t wave_sum64(int64_t v)
     return v;
 }
 
+// The sum of tile t's counts, by one wave.
+__device__ __forceinline__ int64_t wave_tile_sum(const int32_t *__restrict__ counts, int64_t n, int32_t mask, int64_t t)
+{
+    const int64_t b0 = t * kScanTile, b1 = b0 + kScanTile < n ? b0 + kScanTile : n;
+    int64_t s = 0;
+    for (int64_t i = b0 + lane_id(); i < b1; i += kWave) s += counts[i] & mask;
+    return wave_sum64(s);
+}
+
 // Exclusive prefix of tile `tile` whose own sum is `agg`.  The block
 // publishes the aggregate, then reads the descriptors of the kScanThreads
 // preceding tiles at once (thread t: tile - 1 - t).  Each wave waits until
@@ -208,10 +223,14 @@ __device__ __forceinline__ int64_t wave_sum64(int64_t v)
 // and the block moves kScanThreads tiles further back if none did.  Then it
 // publishes its own inclusive prefix.  (One wave looking back 64 tiles at a
 // time took eight dependent steps for the last of 489 tiles.)
-// Waits are bounded: a wave that waits too long sets status->scan_error (the
-// host reports it) rather than spin for ever.
+// With HELP, counts[0 .. n) (each & mask) is the scan's input, which nothing
+// writes: a wave that has waited kHelpSpins turns for a tile sums it from there.
+// Without, waits are bounded: a wave that waits too long sets
+// status->scan_error (the host reports it) rather than spin for ever.
+template <bool HELP = false>
 __device__ __forceinline__ int64_t scan_lookback(uint64_t *__restrict__ desc, int64_t tile, int64_t agg,
-                                                 Status *__restrict__ status)
+                                                 Status *__restrict__ status, const int32_t *__restrict__ counts = nullptr,
+                                                 int64_t n = 0, int32_t mask = -1)
 {
     constexpr int kW = kScanThreads / kWave;
     __shared__ int64_t wsum[kW];
@@ -232,7 +251,16 @@ __device__ __forceinline__ int64_t scan_lookback(uint64_t *__restrict__ desc, in
             inc = __builtin_amdgcn_ballot_w64((v >> 62) == 2);
             const uint64_t need = inc ? (inc & (~inc + 1)) - 1 : ~0ull;
             if ((__builtin_amdgcn_ballot_w64(pending) & need) == 0) break;
-            if (++spins > kLookbackSpins) {
+            ++spins;
+            if (HELP && spins > kHelpSpins) {
+                for (uint64_t todo = __builtin_amdgcn_ballot_w64(pending) & need; todo; todo &= todo - 1) {
+                    const int l = __builtin_ctzll(todo);
+                    const int64_t s = wave_tile_sum(counts, n, mask, top - (int64_t)(wv * kWave + l));
+                    if (lane == l) v = kDescAgg | (uint64_t)s;
+                }
+                continue;
+            }
+            if (spins > kLookbackSpins) {
                 if (lane == 0) status->scan_error = 1;
                 if (pending) v = kDescInc;   // give up on it: an inclusive zero
                 inc = __builtin_amdgcn_ballot_w64((v >> 62) == 2);
@@ -267,6 +295,7 @@ __device__ __forceinline__ int64_t scan_lookback(uint64_t *__restrict__ desc, in
 // One padding slot per 8 items keeps the blocked accesses off shared banks.
 __device__ __forceinline__ int tile_slot(int i) { return i + (i >> 3); }
 constexpr int kTileSlots = kScanTile + kScanTile / 8;
+static_assert(kTileSlots * 12 + 1024 <= 160 * 1024 / kScanBlocksPerCu, "kScanBlocksPerCu scan blocks fit a CU's LDS");
 
 // Cell histogram -> cell_start (0-based), the caller-facing 1-based
 // cell_offsets per system; the histogram is cleared for the next build.
@@ -324,8 +353,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_pairs_kernel(
     int64_t *__restrict__ pair_off, int nsys, void *__restrict__ first_out, Status *__restrict__ status,
     int64_t capacity, int32_t *__restrict__ tile_atom, int64_t tile_cap, int tile_shift)
 {
-    const int64_t tile = scan_tile_begin(desc, partials, status);
-    if (tile < 0) return;
+    const int64_t tile = blockIdx.x;
     int32_t v[kScanItems];
     const int64_t base = tile * kScanTile;
     load_tile(counts, nat, base, v, kCountMask);   // bit 30: slot-row format
@@ -334,7 +362,8 @@ __global__ __launch_bounds__(kScanThreads) void scan_pairs_kernel(
     for (int q = 0; q < kScanItems; ++q) s += v[q];
     int64_t tot;
     const int64_t ex = block_excl_scan(s, tot);
-    const int64_t boff = partials ? partials[tile] : scan_lookback(desc, tile, tot, status);
+    const int64_t boff =
+        partials ? partials[tile] : scan_lookback<true>(desc, tile, tot, status, counts, nat, kCountMask);
     if (!partials && tile == (int64_t)gridDim.x - 1 && threadIdx.x == 0) {   // the last tile sees the total
         status->npairs = boff + tot;
         status->overflow = boff + tot > capacity ? 1 : 0;
@@ -578,8 +607,8 @@ __global__ __launch_bounds__(kScanThreads) void scan_inplace_kernel(int32_t *__r
                                                                     uint64_t *__restrict__ desc,
                                                                     Status *__restrict__ status)
 {
-    static_assert(kSortLookbackTiles <= kOrderlessTiles, "the tiles are on the device together");
-    const int64_t tile = blockIdx.x;
+    const int64_t tile = scan_tile_begin(desc, nullptr, status);
+    if (tile < 0) return;
     int32_t v[kScanItems];
     const int64_t base = tile * kScanTile;
     load_tile(a, n, base, v);

@@ -38,9 +38,11 @@ def hipcc() -> str:
     return "hipcc"
 
 
-USER_KERNEL_DIR = os.path.join(REPO, "tests", "user_kernel")
-USER_KERNEL_SRC = os.path.join(USER_KERNEL_DIR, "user_kernel.hip")
-USER_KERNEL_OUT = os.path.join(USER_KERNEL_DIR, "libnlh_user_kernel.so")
+# test-only libraries: a user kernel over include/nlhip_device.h, and the pair
+# scan with blocks that help themselves at once
+TEST_DIR = os.path.join(REPO, "tests", "user_kernel")
+TEST_LIBS = {os.path.join(TEST_DIR, src): os.path.join(TEST_DIR, out) for src, out in
+             (("user_kernel.hip", "libnlh_user_kernel.so"), ("scan_help.hip", "libnlh_scan_help.so"))}
 
 
 def _compile(srcs, out, verbose):
@@ -58,11 +60,11 @@ def _compile(srcs, out, verbose):
 
 
 def build(verbose: bool = False) -> str:
-    """libnlhip.so, then the test-only user kernel that exercises the
-    device-side header include/nlhip_device.h."""
+    """libnlhip.so, then the test-only libraries."""
     out = _compile([os.path.join(CSRC, s) for s in SOURCES], OUT, verbose)
-    if os.path.exists(USER_KERNEL_SRC):
-        _compile([USER_KERNEL_SRC], USER_KERNEL_OUT, verbose)
+    for src, lib in TEST_LIBS.items():
+        if os.path.exists(src):
+            _compile([src], lib, verbose)
     return out
 
 
