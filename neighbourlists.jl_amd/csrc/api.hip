@@ -172,9 +172,7 @@ struct nlh_handle {
     bool pair_lookback_clean = false;   // the pair scan's descriptors are zero
     int32_t slot_cap = 0;       // neighbour slots per atom
     int32_t slot_cap_max = 0;   // ... the most that a build had to grow to
-    int64_t seen_nat = 0;       // a single system's last builds of seen_nat atoms and estimate
-    int32_t seen_est = 0;       // seen_est: their largest count
-    int32_t seen_max = 0;
+    nlh::SlotHistory seen;      // single systems: the last builds' largest counts
     bool wide = false;          // 16-byte slot entries (cell shifts beyond +-511)
     const double *X_dev = nullptr;
     std::vector<nlh::SysDev> sys_host;
@@ -962,13 +960,6 @@ int64_t estimate_pairs(const nlh_handle *h)
     return (int64_t)std::min<long double>(est, 4.0e11L) + 1024;
 }
 
-// Slot rows hold a multiple of 16 entries, so every row starts on a 128-byte
-// line (8-byte entries) and a row of up to 32 4-byte entries fills one line.
-int32_t round_slot_cap(double c)
-{
-    return (int32_t)((c + 15) / 16) * 16;
-}
-
 // Expected neighbours per atom, largest over the batch (a slot-size guess;
 // an underestimate costs one repeat of the count and fill passes).
 int32_t estimate_slot_cap(const nlh_handle *h)
@@ -982,7 +973,7 @@ int32_t estimate_slot_cap(const nlh_handle *h)
         mx = std::max(mx, nat / vol * 4.18879020478639 * g.cutoff * g.cutoff * g.cutoff);
     }
     const double c = std::min(mx * 1.5 + 16.0, 1.0e6);
-    return round_slot_cap(c);
+    return nlh::round_slot_cap(c);
 }
 
 void ensure_slots(nlh_handle *h, int32_t cap)
@@ -995,13 +986,13 @@ void ensure_slots(nlh_handle *h, int32_t cap)
 // The slot rows of a new build: what the densities say, never less than the
 // handle had to use.  A single system that builds one by one (no captured
 // pipeline to make again) and whose last builds of this size and density are
-// known takes rows of what their largest count needs, packed, where that fits (a
-// build that outgrows them grows the rows, and the next ones know).
+// known takes rows for their largest count (SlotHistory), packed, where that
+// fits (a build that outgrows them grows the rows, and the next ones know).
 void plan_slots(nlh_handle *h)
 {
     const int32_t est = estimate_slot_cap(h), cap = std::max(h->slot_cap_max, est);
-    if (h->nsys == 1 && h->nat >= kReplayMaxAtoms && !h->wide && h->seen_nat == h->nat && h->seen_est == est) {
-        h->slot_cap = std::min(cap, round_slot_cap(std::max(h->seen_max, 1)));
+    if (h->nsys == 1 && h->nat >= kReplayMaxAtoms && !h->wide && h->seen.knows(h->nat, est)) {
+        h->slot_cap = std::min(cap, h->seen.rows());
         h->slot_packed = true;
         if (h->slot_bytes() <= h->slots.cap) return;
     }
@@ -1249,7 +1240,7 @@ void materialize(nlh_handle *h, uint32_t flags)
         // (the counts, offsets and totals of the first pass stay valid)
         if (st.wide) h->wide = true;
         ensure_pair_outputs(h, std::max<int64_t>(st.npairs, 1), want_R);
-        const int32_t cap = std::max(h->slot_cap, round_slot_cap(std::max(st.max_count, 1)));
+        const int32_t cap = std::max(h->slot_cap, nlh::round_slot_cap(std::max(st.max_count, 1)));
         h->slot_cap = h->slot_cap_max = std::max(h->slot_cap_max, cap);
         if (h->slots.cap < h->slot_bytes()) h->slots.release(h->stream);
         ensure_slots(h, h->slot_cap);
@@ -1272,13 +1263,7 @@ void finish_pairs(nlh_handle *h, bool want_R)
 {
     h->npairs = h->status_host->npairs;
     h->have_R = want_R;
-    if (h->nsys == 1) {
-        const int32_t est = estimate_slot_cap(h);
-        if (h->seen_nat != h->nat || h->seen_est != est) h->seen_max = 0;
-        h->seen_nat = h->nat;
-        h->seen_est = est;
-        h->seen_max = std::max(h->seen_max, h->status_host->max_count);
-    }
+    if (h->nsys == 1) h->seen.note(h->nat, estimate_slot_cap(h), h->status_host->max_count);
     // per-system pair offsets
     h->pair_offsets_host.resize(h->nsys + 1);
     h->offsets_stale = false;
@@ -1634,7 +1619,7 @@ int32_t slot_cap_for(const nlh_geometry &g, int64_t nat)
     const double vol = std::fabs(det3(g.cell));
     double mx = 0;
     if (nat > 0 && vol > 0) mx = nat / vol * 4.18879020478639 * g.cutoff * g.cutoff * g.cutoff;
-    return round_slot_cap(std::min(mx * 1.5 + 16.0, 1.0e6));
+    return nlh::round_slot_cap(std::min(mx * 1.5 + 16.0, 1.0e6));
 }
 
 // Wait for the stream and read the device status back.
@@ -1723,7 +1708,7 @@ void neighbour_list_noalloc(hipStream_t st, const double *X, int64_t nat, const 
         // longer or wider slot rows, then count, scan and fill again (the
         // cell list stays where it is: the slot rows are the layout's tail)
         wide = wide || s.wide;
-        cap = std::max(cap, round_slot_cap(std::max(s.max_count, 1)));
+        cap = std::max(cap, nlh::round_slot_cap(std::max(s.max_count, 1)));
         need = carve_noalloc(nullptr, P, ti, cap, wide, want_R, pair_capacity, X, i_out, j_out, S_out, first_out,
                              R_out, b);
         if (need > kScratchBytes) scratch_too_small(need);

@@ -1,0 +1,58 @@
+"""Host rules of the library that need no device, run in a small C++ program
+over the library's own headers."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "neighbourlists.jl_amd", "csrc")
+
+
+def run_cpp(tmp_path, body, includes=("nlhip_internal.h",)):
+    """Compile and run main() { body }; returns what it printed."""
+    if not shutil.which("g++"):
+        pytest.skip("no host compiler")
+    src, exe = tmp_path / "t.cpp", tmp_path / "t"
+    src.write_text("".join(f'#include "{i}"\n' for i in includes) +
+                   "#include <cstdio>\nusing namespace nlh;\nint main()\n{\n" + body + "\nreturn 0;\n}\n")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", CSRC, "-I", "/opt/rocm/include", str(src),
+                    "-o", str(exe), "-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib", "-lamdhip64", "-lpthread"],
+                   check=True, capture_output=True, text=True)
+    return subprocess.run([str(exe)], check=True, capture_output=True, text=True, timeout=60).stdout
+
+
+def _overflows(tmp_path, counts):
+    """Builds whose largest count does not fit the rows that the builds before
+    them suggest, and the last rows."""
+    out = run_cpp(tmp_path, "SlotHistory s; int over = 0;\nfor (int m : {" + ", ".join(map(str, counts)) +
+                  "}) { if (s.knows(1000, 96) && m > s.rows()) ++over; s.note(1000, 96, m); }\n"
+                  'printf("%d %d %d", over, (int)s.knows(1000, 96), s.rows());')
+    return tuple(int(x) for x in out.split())
+
+
+@pytest.mark.parametrize("counts,over", [
+    # largest counts of fcc crystals of 13,500 and 108,000 atoms heating up, at
+    # cutoffs of 5.0 and 5.4, and of random gases, build after build
+    ([42, 42, 44, 46, 47, 47, 48, 49, 50, 49, 50, 50, 52, 52, 52, 51, 52], 0),
+    ([42, 42, 45, 46, 48, 48, 49, 49, 50, 50, 51, 51, 52, 52, 53], 0),
+    ([54, 54, 54, 54, 55, 57, 57, 59, 59, 59, 61, 61, 62, 62, 64, 63, 64, 65], 0),
+    ([44, 51, 48, 47, 48, 47, 49, 49, 50, 51, 48], 0),
+    ([52, 50, 52, 51, 50, 53, 50, 52, 55, 52, 50, 51, 53, 58, 54], 0),
+    ([46, 47, 48, 49, 50, 51], 0),
+    # a jump that nothing announced
+    ([42, 42, 42, 100, 101], 1)])
+def test_slot_rows_leave_room_for_moving_atoms(tmp_path, counts, over):
+    got, knows, rows = _overflows(tmp_path, counts)
+    assert got == over and knows and rows >= max(counts)
+
+
+def test_slot_rows_of_static_atoms(tmp_path):
+    """Counts that never rise: rows of the next multiple of 16, from the third
+    build on; another size starts over."""
+    for m in (1, 15, 16, 17, 42, 48):
+        assert _overflows(tmp_path, [m, m, m]) == (0, 1, (m + 15) // 16 * 16)
+    assert _overflows(tmp_path, [42])[1] == 0
+    out = run_cpp(tmp_path, "SlotHistory s; s.note(10, 32, 5); s.note(10, 32, 9); s.note(11, 32, 40); s.note(11, 32, 40);\n"
+                  'printf("%d %d %d", (int)s.knows(10, 32), (int)s.knows(11, 32), s.rows());')
+    assert out == "0 1 48"
