@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
+#include <cstddef>
 #include <cstring>
 #include <functional>
 #include <memory>
@@ -63,13 +64,15 @@ public:
             if (e) (void)hipEventDestroy(e);
     }
 
-    // Frees the pinned memory if there is more of it than `bytes`.
-    void trim(size_t bytes)
+    // Frees the pinned memory if there is more of it than `bytes`; returns what is left.
+    size_t trim(size_t bytes)
     {
-        if (ring_bytes_ <= bytes) return;
-        (void)hipHostFree(ring_);
-        ring_ = nullptr;
-        ring_bytes_ = 0;
+        if (ring_bytes_ > bytes) {
+            (void)hipHostFree(ring_);
+            ring_ = nullptr;
+            ring_bytes_ = 0;
+        }
+        return ring_bytes_;
     }
 
     const int device;
@@ -210,27 +213,39 @@ private:
 };
 
 // The process's copiers.  A copy borrows one (its own, whatever other threads
-// do); one idle copier is kept for the next, with at most 32 MB of pinned memory,
-// and once no handle is left, with at most 8 MB.  (Starting one costs 60 us, its
-// pinned memory up to 300: more than a list of 10k atoms saves, on a handle
-// made for one list.)
+// do), and those given back are kept for the next copies: as many as were in use
+// at once, up to kKept, with the pinned memory they came to need (at most 32 MB
+// each), and once no handle is left, with at most 8 MB together.  (Starting one
+// costs 60 us, its pinned memory up to 300: more than a list of 10k atoms saves.)
 class HostCopierPool {
 public:
+    static constexpr size_t kKept = 4;
+
     std::unique_ptr<HostCopier> borrow(int device)
     {
         {
             std::lock_guard<std::mutex> lk(m_);
-            if (idle_ && idle_->device == device) return std::move(idle_);
+            for (size_t k = idle_.size(); k-- > 0;)   // the last one used first
+                if (idle_[k]->device == device) {
+                    std::unique_ptr<HostCopier> c = std::move(idle_[k]);
+                    idle_.erase(idle_.begin() + (std::ptrdiff_t)k);
+                    return c;
+                }
         }
         return std::make_unique<HostCopier>(device);
     }
 
-    // Returns the copier that is not kept, for the caller to end.
+    // Returns a copier that is not kept, if there is one, for the caller to end.
     std::unique_ptr<HostCopier> give_back(std::unique_ptr<HostCopier> c)
     {
         std::lock_guard<std::mutex> lk(m_);
-        std::swap(idle_, c);
-        return c;
+        std::unique_ptr<HostCopier> out;
+        if (idle_.size() == kKept) {
+            out = std::move(idle_.front());
+            idle_.erase(idle_.begin());
+        }
+        idle_.push_back(std::move(c));   // room for kKept: reserved
+        return out;
     }
 
     void handle_made()
@@ -241,12 +256,16 @@ public:
     void handle_gone()
     {
         std::lock_guard<std::mutex> lk(m_);
-        if (--handles_ == 0 && idle_) idle_->trim(8 << 20);
+        if (--handles_ > 0) return;
+        size_t left = 8 << 20;
+        for (auto &c : idle_) left -= c->trim(left);
     }
+
+    HostCopierPool() { idle_.reserve(kKept); }
 
 private:
     std::mutex m_;
-    std::unique_ptr<HostCopier> idle_;
+    std::vector<std::unique_ptr<HostCopier>> idle_;   // by time of their last use
     int64_t handles_ = 0;
 };
 

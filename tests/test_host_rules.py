@@ -56,3 +56,31 @@ def test_slot_rows_of_static_atoms(tmp_path):
     out = run_cpp(tmp_path, "SlotHistory s; s.note(10, 32, 5); s.note(10, 32, 9); s.note(11, 32, 40); s.note(11, 32, 40);\n"
                   'printf("%d %d %d", (int)s.knows(10, 32), (int)s.knows(11, 32), s.rows());')
     assert out == "0 1 48"
+
+
+def test_copiers_in_use_at_once_are_kept(tmp_path):
+    """Copies that overlap find the copiers of the last ones that did, each
+    device its own, and no more than the limit stay."""
+    out = run_cpp(tmp_path, """
+HostCopierPool p;
+p.handle_made();
+auto a = p.borrow(0), b = p.borrow(0);
+HostCopier *pa = a.get(), *pb = b.get();
+bool ended = p.give_back(std::move(a)) || p.give_back(std::move(b));
+for (int turn = 0; turn < 3; ++turn) {
+    auto c = p.borrow(0), d = p.borrow(0);
+    bool same = (c.get() == pa || c.get() == pb) && (d.get() == pa || d.get() == pb) && c != d;
+    printf("%d ", (int)same);
+    ended = ended || p.give_back(std::move(c)) || p.give_back(std::move(d));
+}
+auto other = p.borrow(1);
+printf("%d %d ", (int)ended, (int)(other.get() != pa && other.get() != pb));
+std::vector<std::unique_ptr<HostCopier>> many;
+many.push_back(std::move(other));
+for (int k = 0; k < 9; ++k) many.push_back(p.borrow(0));
+int gone = 0;
+for (auto &m : many) gone += p.give_back(std::move(m)) != nullptr;
+p.handle_gone();
+printf("%d", gone);
+""", includes=("host_copy.h",))
+    assert out == f"1 1 1 0 1 {10 - 4}"
