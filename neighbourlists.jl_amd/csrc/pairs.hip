@@ -84,7 +84,7 @@ __device__ __forceinline__ void rec_winding(const Rec &r, const int32_t *__restr
     }
 }
 
-constexpr int kChunksPerPass = 2;   // candidate chunks a lane holds at once (per-wave path)
+constexpr int kChunksPerPass = 3;   // candidate chunks a lane holds at once (per-wave path)
 constexpr double kFar = 1.0e200;    // invalid candidate: r^2 overflows to +inf, never a hit
 
 struct PairsArgs {
@@ -134,12 +134,10 @@ struct SlotArgs {
 
 // Append the hits of one (home atom, chunk) ballot to the home atom's slot.
 // sbase = sorted index of the home atom * cap; ca = its running count
-// (wave-uniform).  t_pk: this lane's packed s - w_j (valid when tfits);
-// (tx, ty, tz) the same unpacked; w_i the home atom's winding, wzero when 0.
+// (wave-uniform); (sx, sy, sz) this lane's S.
 template <bool WIDE>
 __device__ __forceinline__ void emit_hits(const SlotArgs &O, uint64_t mask, int64_t sbase, int32_t &ca, int32_t cj,
-                                          uint32_t t_pk, int32_t tx, int32_t ty, int32_t tz, int32_t wix, int32_t wiy,
-                                          int32_t wiz, bool wzero)
+                                          int32_t sx, int32_t sy, int32_t sz)
 {
     if (mask == 0) return;   // wave-uniform
     const int lane = lane_id();
@@ -147,17 +145,16 @@ __device__ __forceinline__ void emit_hits(const SlotArgs &O, uint64_t mask, int6
     if ((mask >> lane) & 1) {
         const int64_t sidx = sbase + rank;
         if (WIDE) {
-            if (rank < O.cap) reinterpret_cast<int4 *>(O.slots)[sidx] = make_int4(cj, tx + wix, ty + wiy, tz + wiz);
+            if (rank < O.cap) reinterpret_cast<int4 *>(O.slots)[sidx] = make_int4(cj, sx, sy, sz);
         } else {
-            // S = s_loop + w_i - w_j = t + w_i  (gpu_kernels.jl:88).  Entries past a
-            // row's end count too: the repeat on longer rows is the last one
-            const uint32_t spk = wzero ? t_pk : pack_wind(tx + wix, ty + wiy, tz + wiz);
+            // entries past a row's end count too: the repeat on longer rows is the last one
+            const uint32_t spk = pack_wind(sx, sy, sz);
             if (spk & kWindBig) O.status->wide = 1;
             if (rank < O.cap)
                 reinterpret_cast<uint64_t *>(O.slots)[sidx] = (uint64_t)(uint32_t)cj | ((uint64_t)spk << 32);
         }
     }
-    ca += __popcll(mask);
+    ca += (int32_t)__popcll(mask);
 }
 
 // ---------------------------------------------------------------------------
@@ -165,7 +162,6 @@ __device__ __forceinline__ void emit_hits(const SlotArgs &O, uint64_t mask, int6
 // ---------------------------------------------------------------------------
 
 struct HomeCell {
-    int32_t hs, he;             // sorted atom range
     int ci0, ci1, ci2;          // 1-based cell coordinates
     int n0, n1, n2, nx0, nx1, nx2, sx, sy, nseg;
     bool p0, p1, p2;
@@ -189,14 +185,6 @@ __device__ __forceinline__ void home_grid(const SysDev &sd, int ci0, int ci1, in
     H.sy = 2 * H.nx1 + 1;
     H.nseg = H.sx * H.sy * (2 * H.nx2 + 1);
     H.p0 = sd.pbc & 1; H.p1 = (sd.pbc >> 1) & 1; H.p2 = (sd.pbc >> 2) & 1;
-}
-
-__device__ __forceinline__ void home_cell(const PairsArgs &A, const SysDev &sd, int cell, HomeCell &H)
-{
-    H.hs = A.cell_start[cell];
-    H.he = A.cell_start[cell + 1];
-    const int lc = cell - sd.cell_base;
-    home_grid(sd, lc % sd.n[0] + 1, (lc / sd.n[0]) % sd.n[1] + 1, lc / (sd.n[0] * sd.n[1]) + 1, H);
 }
 
 // Neighbour cells sb .. sb+63 of the home cell, one per lane, in the
@@ -280,96 +268,76 @@ __device__ __forceinline__ Cand load_candidate(const PairsArgs &A, int k, int to
     return c;
 }
 
-// Home atoms of a cell from which the waves of its brick share it (10k atoms
-// clamped into a quarter of an open cell: 294 us unshared, 174 shared).
-constexpr int kShareHome = 32;
-
-// Per-wave count of one home cell from global memory: test every (home
-// atom, chunk) and append hits to the slots (the brick path's fallback, and
-// the path for neighbour reach beyond one cell).
+// Per-wave count of the home atoms hs .. he - 1 (up to a wave of them) of one
+// cell from global memory: test every (home atom, chunk) and append hits to
+// the slots (the brick path's fallback, and the path for neighbour reach
+// beyond one cell).
 template <bool WIDE>
-__device__ __forceinline__ void count_cell(const PairsArgs &A, const SysDev &sd, int cell, int32_t *__restrict__ pair_count,
-                                        const SlotArgs &O, int turn, int part, int parts)
+__device__ __forceinline__ void count_group(const PairsArgs &A, const SysDev &sd, int lc, int32_t hg, int nh,
+                                            int32_t *__restrict__ pair_count, const SlotArgs &O)
 {
     HomeCell H;
-    home_cell(A, sd, cell, H);
-    // a cell that atoms were clamped into may hold thousands: all `parts`
-    // waves share its home atoms; a smaller cell is one wave's, in turn
-    const int n = H.he - H.hs;
-    if (n > kShareHome) {
-        H.he = H.hs + (int)((int64_t)n * (part + 1) / parts);
-        H.hs += (int)((int64_t)n * part / parts);
-    } else if (turn % parts != part) {
-        return;
-    }
-    if (H.hs >= H.he) return;
+    home_grid(sd, lc % sd.n[0] + 1, (lc / sd.n[0]) % sd.n[1] + 1, lc / (sd.n[0] * sd.n[1]) + 1, H);
     const int lane = lane_id();
     const double *__restrict__ Cm = sd.C;
     const double rc2 = sd.rc2;
-    for (int32_t hg = H.hs; hg < H.he; hg += kWave) {
-        const int nh = sgpr(min(kWave, H.he - hg));
-        const int32_t hj_lane = lane < nh ? A.rec[hg + lane].j : 0;
-        int32_t cnt_lane = 0;   // lane a: running count of home atom hg + a
-        for (int sb = 0; sb < H.nseg; sb += kWave) {
-            int excl, start_g;
-            uint32_t shp;
-            const int total = segment_batch(H, sb, excl, start_g, shp, [&](int c, int &st, int &n) {
-                st = A.cell_start[H.cbase + c];
-                n = A.cell_start[H.cbase + c + 1] - st;
-            });
-            for (int k0 = 0; k0 < total; k0 += kChunksPerPass * kWave) {
-                const int nch = sgpr(min(kChunksPerPass, (total - k0 + kWave - 1) / kWave));
-                Cand c[kChunksPerPass];
-                uint32_t tpk[kChunksPerPass];
-                int32_t key[kChunksPerPass];
+    const int32_t hj_lane = lane < nh ? A.rec[hg + lane].j : 0;
+    int32_t cnt_lane = 0;   // lane a: running count of home atom hg + a
+    for (int sb = 0; sb < H.nseg; sb += kWave) {
+        int excl, start_g;
+        uint32_t shp;
+        const int total = segment_batch(H, sb, excl, start_g, shp, [&](int c, int &st, int &n) {
+            st = A.cell_start[H.cbase + c];
+            n = A.cell_start[H.cbase + c + 1] - st;
+        });
+        for (int k0 = 0; k0 < total; k0 += kChunksPerPass * kWave) {
+            const int nch = sgpr(min(kChunksPerPass, (total - k0 + kWave - 1) / kWave));
+            Cand c[kChunksPerPass];
+            uint64_t own[kChunksPerPass];   // candidates with no cell shift: the home atom's own is one of them
+#pragma unroll
+            for (int g = 0; g < kChunksPerPass; ++g) {
+                own[g] = 0;
+                if (g < nch) {
+                    c[g] = load_candidate(A, k0 + g * kWave + lane, total, excl, start_g, shp);
+                    if (!c[g].valid) c[g].x = c[g].y = c[g].z = kFar;
+                    own[g] = __builtin_amdgcn_ballot_w64(c[g].zero_shift);
+                } else {
+                    c[g].x = c[g].y = c[g].z = kFar;
+                    c[g].j = -1;
+                    c[g].tx = c[g].ty = c[g].tz = 0;
+                }
+            }
+            double cx[kChunksPerPass], cy[kChunksPerPass], cz[kChunksPerPass];
+            uint32_t wcache = 0xffffffffu;
+            int32_t wix = 0, wiy = 0, wiz = 0;
+            for (int a = 0; a < nh; ++a) {
+                const Rec h = A.rec[hg + a];   // wave-uniform: scalar loads
+                if (h.w != wcache || (h.w & kWindBig)) {
+                    rec_winding(h, A.wbig, hg + a, wix, wiy, wiz);
+#pragma unroll
+                    for (int g = 0; g < kChunksPerPass; ++g)
+                        cell_shift(Cm, c[g].tx + wix, c[g].ty + wiy, c[g].tz + wiz, cx[g], cy[g], cz[g]);
+                    wcache = h.w;
+                }
+                int32_t ca = __builtin_amdgcn_readlane(cnt_lane, a);
+                const int64_t sbase = (H.abase + __builtin_amdgcn_readlane(hj_lane, a)) * (int64_t)O.cap;
 #pragma unroll
                 for (int g = 0; g < kChunksPerPass; ++g) {
                     if (g < nch) {
-                        c[g] = load_candidate(A, k0 + g * kWave + lane, total, excl, start_g, shp);
-                        if (!c[g].valid) c[g].x = c[g].y = c[g].z = kFar;
-                        tpk[g] = pack_wind(c[g].tx, c[g].ty, c[g].tz);
-                        key[g] = (c[g].valid && c[g].zero_shift) ? c[g].j : -3;
-                    } else {
-                        c[g].x = c[g].y = c[g].z = kFar;
-                        c[g].j = -1;
-                        c[g].tx = c[g].ty = c[g].tz = 0;
-                        tpk[g] = 0;
-                        key[g] = -3;
+                        const double Rx = (c[g].x - h.x) + cx[g];
+                        const double Ry = (c[g].y - h.y) + cy[g];
+                        const double Rz = (c[g].z - h.z) + cz[g];
+                        const double r2 = (Rx * Rx + Ry * Ry) + Rz * Rz;
+                        const uint64_t mask = __builtin_amdgcn_ballot_w64(r2 < rc2) &
+                                              ~(__builtin_amdgcn_ballot_w64(c[g].j == h.j) & own[g]);
+                        emit_hits<WIDE>(O, mask, sbase, ca, c[g].j, c[g].tx + wix, c[g].ty + wiy, c[g].tz + wiz);
                     }
                 }
-                double cx[kChunksPerPass], cy[kChunksPerPass], cz[kChunksPerPass];
-                uint32_t wcache = 0xffffffffu;
-                int32_t wix = 0, wiy = 0, wiz = 0;
-                for (int a = 0; a < nh; ++a) {
-                    const Rec h = A.rec[hg + a];   // wave-uniform: scalar loads
-                    if (h.w != wcache || (h.w & kWindBig)) {
-                        rec_winding(h, A.wbig, hg + a, wix, wiy, wiz);
-#pragma unroll
-                        for (int g = 0; g < kChunksPerPass; ++g)
-                            cell_shift(Cm, c[g].tx + wix, c[g].ty + wiy, c[g].tz + wiz, cx[g], cy[g], cz[g]);
-                        wcache = h.w;
-                    }
-                    const bool wzero = (wix | wiy | wiz) == 0;
-                    int32_t ca = __builtin_amdgcn_readlane(cnt_lane, a);
-                    const int64_t sbase = (H.abase + __builtin_amdgcn_readlane(hj_lane, a)) * (int64_t)O.cap;
-#pragma unroll
-                    for (int g = 0; g < kChunksPerPass; ++g) {
-                        if (g < nch) {
-                            const double Rx = (c[g].x - h.x) + cx[g];
-                            const double Ry = (c[g].y - h.y) + cy[g];
-                            const double Rz = (c[g].z - h.z) + cz[g];
-                            const double r2 = (Rx * Rx + Ry * Ry) + Rz * Rz;
-                            const uint64_t mask = __ballot((r2 < rc2) & (key[g] != h.j));
-                            emit_hits<WIDE>(O, mask, sbase, ca, c[g].j, tpk[g], c[g].tx, c[g].ty, c[g].tz, wix, wiy, wiz,
-                                            wzero);
-                        }
-                    }
-                    cnt_lane = lane == a ? ca : cnt_lane;
-                }
+                cnt_lane = lane == a ? ca : cnt_lane;
             }
         }
-        if (lane < nh) pair_count[H.abase + hj_lane] = cnt_lane | kRow8Bit;
     }
+    if (lane < nh) pair_count[H.abase + hj_lane] = cnt_lane | kRow8Bit;
 }
 
 // ---------------------------------------------------------------------------
@@ -565,6 +533,42 @@ __device__ __forceinline__ int brick_cell_id(const Brick &B, int hc)
     const SysDev &sd = *B.sd;
     const int ix = hc % B.nh[0], iy = (hc / B.nh[0]) % B.nh[1], iz = hc / (B.nh[0] * B.nh[1]);
     return sd.cell_base + (B.b0[0] - 1 + ix) + (B.b0[1] - 1 + iy) * sd.n[0] + (B.b0[2] - 1 + iz) * sd.n[0] * sd.n[1];
+}
+
+// A brick's home cells from global memory: each cell's home atoms in groups,
+// all groups dealt to the `parts` waves in turn, so that a cell which atoms
+// were clamped into (thousands of them) or the one cell of a brick is shared,
+// and no cell is looked at twice.  Every group loads the cell's candidates:
+// groups smaller than a wave only where they must be (100k atoms shifted by a
+// quarter of an open axis, whole builds: groups of 16 above 32 atoms 368 us, of
+// 48 above 64 336; 10k in a corner of an open cell 263 with either).
+constexpr int kShareGroup = 48;
+template <bool WIDE>
+__device__ __forceinline__ void count_cells(const PairsArgs &A, const Brick &B, int32_t *__restrict__ pair_count,
+                                            const SlotArgs &O, int part, int parts)
+{
+    const SysDev &sd = *B.sd;
+    const int lane = lane_id();
+    int st = 0, n = 0, cell = 0;   // home cell `lane`
+    if (lane < B.nhome) {
+        cell = brick_cell_id(B, lane);
+        st = A.cell_start[cell];
+        n = A.cell_start[cell + 1] - st;
+    }
+    // home atoms of a group: a cell's own, an even share of a large one, or, where
+    // the waves outnumber the cells, a wave's share
+    const int shares = (n + kShareGroup - 1) / kShareGroup;
+    int gs = n > kWave ? (n + shares - 1) / shares : kWave;
+    if (B.nhome < parts) gs = min(gs, max(1, (int)(((int64_t)n * B.nhome + parts - 1) / parts)));
+    const int g = (n + gs - 1) / gs, incl = wave_incl_scan(g);
+    const int items = __builtin_amdgcn_readlane(incl, kWave - 1);
+    for (int it = part; it < items; it += parts) {
+        const int c = (int)__popcll(__builtin_amdgcn_ballot_w64(incl <= it));   // the item's cell
+        const int cg = __builtin_amdgcn_readlane(gs, c);
+        const int o = (it - (__builtin_amdgcn_readlane(incl, c) - __builtin_amdgcn_readlane(g, c))) * cg;
+        count_group<WIDE>(A, sd, __builtin_amdgcn_readlane(cell, c) - sd.cell_base, __builtin_amdgcn_readlane(st, c) + o,
+                          min(cg, __builtin_amdgcn_readlane(n, c) - o), pair_count, O);
+    }
 }
 
 // One halo atom in LDS, 32 bytes: a candidate is two 16-byte reads.
@@ -921,8 +925,7 @@ __global__ __launch_bounds__(BT) void count_kernel(
     if (!lds) {
         const SlotArgs O{slots, cap, status};
         const int wv0 = sgpr((int)(threadIdx.x >> 6));
-        for (int hc = 0; hc < B.nhome; ++hc)
-            count_cell<true>(A, *B.sd, brick_cell_id(B, hc), pair_count, O, hc, wv0, BrickShape<BT>::waves);
+        count_cells<true>(A, B, pair_count, O, wv0, BrickShape<BT>::waves);
         return;
     }
     const SysDev &sd = *B.sd;
@@ -1416,9 +1419,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(5))) void ti
     const int wv = sgpr((int)(threadIdx.x >> 6));
     if (!lds) {
         const SlotArgs O{reinterpret_cast<char *>(slots) + off8, cap, status};
-        for (int hc = 0; hc < B.nhome; ++hc)
-            count_cell<false>(A, *B.sd, brick_cell_id(B, hc), pair_count, O, hc, copy + copies * wv,
-                              copies * BrickShape<BT>::waves);
+        count_cells<false>(A, B, pair_count, O, copy + copies * wv, copies * BrickShape<BT>::waves);
         return;
     }
     const SysDev &sd = *B.sd;

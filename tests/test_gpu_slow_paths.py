@@ -1,0 +1,73 @@
+"""Systems that leave the pair search's fast path: results against the oracle
+at the edges of its other paths, and their times against an ordinary system's.
+"""
+import ctypes
+import time
+
+import numpy as np
+import pytest
+import torch
+
+import nlhip
+import oracle
+from nlhip import _lib, workloads
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(a):
+    return np.asarray(a).view(np.int64)
+
+
+def _check(X, rc, cell, pbc, want_R=False):
+    ref = oracle.neighbour_list(X, rc, cell, pbc, want_R=want_R, nthreads=8)
+    nl = nlhip.neighbour_list(X, rc, cell, pbc, want_R=want_R)
+    assert np.array_equal(nl.first, ref.first)
+    assert np.array_equal(nl.i, ref.i) and np.array_equal(nl.j, ref.j) and np.array_equal(nl.S, ref.S)
+    if want_R:
+        assert np.array_equal(_bits(nl.R), _bits(ref.R))
+
+
+def _time(X, rc, cell, pbc):
+    """Median time of a build of device positions on a handle that knows them (us)."""
+    L, h, m = _lib.lib(), _lib.Handle(), ctypes.c_int64()
+    g = _lib.geometry(cell, rc, pbc, 4)
+    D = torch.as_tensor(np.ascontiguousarray(X)).cuda()
+    torch.cuda.synchronize()
+    t = []
+    for _ in range(30):
+        t0 = time.perf_counter()
+        _lib.check(L.nlh_neighbour_list(h.ptr, D.data_ptr(), len(X), ctypes.byref(g), _lib.NLH_X_DEVICE, ctypes.byref(m)))
+        _lib.check(L.nlh_synchronize(h.ptr))
+        t.append(time.perf_counter() - t0)
+    return 1e6 * float(np.median(t[5:]))
+
+
+@pytest.mark.parametrize("reach", [1, 2])
+@pytest.mark.parametrize("sizes", [(1, 1, 1), (47, 48, 49, 63, 64, 65), (96, 97, 144, 145, 0, 200), (3, 0, 0, 130, 7, 1)])
+def test_cells_counted_from_global_memory(sizes, reach):
+    """A row of cells of given sizes, dense enough or of a reach that takes
+    them to the per-wave count: groups of home atoms up to a wave, shares of
+    larger cells, more waves than cells."""
+    rng = np.random.default_rng(sum(sizes))
+    rc = 2.0 if reach == 1 else 2.9   # along z: one cell of 2.02
+    cell = np.diag([len(sizes) * rc * 1.01, 2.0 * rc * 1.01, 2.02])
+    parts = []
+    for k, n in enumerate(sizes):
+        for y in range(2):
+            parts.append((np.array([k, y, 0]) + rng.random((n, 3))) * [rc * 1.01, rc * 1.01, 2.02])
+    print(f"per-wave {sizes} {reach}", flush=True)
+    for pbc in [(True, True, True), (False, True, True)]:
+        _check(np.concatenate(parts), rc, cell, pbc, want_R=True)
+
+
+def test_time_of_a_reach_of_two_cells():
+    """A plate one cell thick with a reach of two across it (few cells, none of
+    them in the LDS path): its bricks of one cell keep all their waves busy.
+    It took twice an ordinary system's time, and takes 1.3 of it."""
+    n = 3000
+    s = workloads.random_cubic(n, density=0.05, seed=n, cutoff=5.0)
+    L = (n / 0.05 / 6) ** 0.5
+    y = workloads.random_in_cell(n, np.diag([6.0, L, L]), seed=n, cutoff=7.0)
+    print("plate", flush=True)
+    assert _time(y.X, 7.0, y.cell, (True,) * 3) < 1.65 * _time(s.X, 5.0, s.cell, (True,) * 3)
