@@ -540,7 +540,7 @@ constexpr double kHaloFill = 0.9;
 //   7.2 u (P + 2 H + rc) rc      positions rounded to 32 bits, |p| <= P, then
 //                                taken from c
 //   1.6e-11 rc (|a1| + |a2| + |a3|)   the 64-bit roundings on both sides, for
-//                                windings within +-128 (nine times their bound)
+//                                windings within +-511 (six times their bound)
 // and by less than its distance from zero for candidates further away.  A
 // quarter is added for what the line above leaves out (second-order terms).
 void filter_bounds(nlh::SysDev &sd, const nlh_geometry &g)

@@ -46,6 +46,18 @@ __device__ __forceinline__ int take_next(int32_t *ctr)
     return __builtin_amdgcn_readfirstlane(t);
 }
 
+// The largest of the lanes' non-negative values, on the last lane.
+__device__ __forceinline__ int wave_max_pos(int v)
+{
+    v = max(v, dpp_or_zero<0x111>(v));
+    v = max(v, dpp_or_zero<0x112>(v));
+    v = max(v, dpp_or_zero<0x114>(v));
+    v = max(v, dpp_or_zero<0x118>(v));
+    v = max(v, dpp_or_zero<0x142, 0xa>(v));
+    v = max(v, dpp_or_zero<0x143, 0xc>(v));
+    return v;
+}
+
 // v with lane `lane` (wave-uniform) set to the wave-uniform x: one
 // v_writelane, no exec-mask or compare work.
 __device__ __forceinline__ int32_t write_lane(int32_t x, int lane, int32_t v)
@@ -1085,9 +1097,51 @@ __device__ __forceinline__ void tile_run(const Brick &B, const TileRuns &T, int 
     w = min(T.w, B.nh[0] - ix);
 }
 
+// Whether the S = t'_j - t'_i of any two of the brick's atoms packs (then each
+// t' relative to the origin atom's did): the windings of all of them are
+// packed ones, and their s - w span at most 510 along each axis.  Looked at
+// only where some winding is beyond +-128, as in trajectories whose positions
+// were never wrapped.
+template <int BT>
+__device__ bool tile_windings_near(const PairsArgs &A, TileLDS<BT> &L, int total)
+{
+    using Sh = BrickShape<BT>;
+    const int tid = threadIdx.x;
+    int32_t *far = &L.rowdl[0][0];   // per axis the largest of 1100 + (s - w) and of 1100 - (s - w), then a mark
+    if (tid < 7) far[tid] = 0;
+    __syncthreads();
+    int m[6] = {0, 0, 0, 0, 0, 0};
+    bool big = false;
+    for (int idx = tid; idx < total; idx += BT) {
+        const int h = L.owner[idx];
+        const uint32_t w = A.rec[L.hstart[h] + (idx - L.hoff[h])].w;
+        big |= (w & kWindBig) != 0;
+        int32_t s[3], v[3];
+        unpack_wind(L.hshift[h] & ~kHomeCell, s[0], s[1], s[2]);
+        unpack_wind(w, v[0], v[1], v[2]);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            m[k] = max(m[k], 1100 + s[k] - v[k]);
+            m[3 + k] = max(m[3 + k], 1100 - s[k] + v[k]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        const int v = wave_max_pos(m[k]);
+        if (lane_id() == kWave - 1) atomicMax(far + k, v);
+    }
+    if (big) far[6] = 1;
+    __syncthreads();
+    bool near = far[6] == 0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) near = near && far[k] + far[3 + k] <= 2200 + 510;
+    __syncthreads();   // read before the waves use the space
+    return near;
+}
+
 // Stage the brick and its halo in LDS.  Returns false (for every thread of
 // the block) when the brick must take the global-memory path: more halo
-// atoms than the LDS holds, or windings beyond +-128.
+// atoms than the LDS holds, or windings too far apart.
 template <int BT>
 __device__ bool tile_load(const PairsArgs &A, const Brick &B, const TileRuns &T, TileLDS<BT> &L, const double *Csh)
 {
@@ -1145,8 +1199,9 @@ __device__ bool tile_load(const PairsArgs &A, const Brick &B, const TileRuns &T,
     const int po = sgpr(L.hstart[ho] + (im - L.hoff[ho]));
     const Rec ro = A.rec[po];
     const double ox = ro.x, oy = ro.y, oz = ro.z;
-    // pack(t') of an atom = its cell shift's pack - its winding's + tb (no
-    // field leaves its 10 bits while every winding is within +-128)
+    // pack(t') of an atom = its cell shift's pack - its winding's + tb (no field
+    // leaves its 10 bits while every winding is within +-128, or as
+    // tile_windings_near finds)
     const uint32_t to = (L.hshift[ho] & ~kHomeCell) - ro.w, tb = kPackZero - to;
     // halo atoms: all loads of a thread in flight together
     int pg[Sh::unroll];
@@ -1216,7 +1271,7 @@ __device__ bool tile_load(const PairsArgs &A, const Brick &B, const TileRuns &T,
     }
     if (bad) L.flag = 1;
     __syncthreads();
-    return L.flag == 0;
+    return L.flag == 0 || tile_windings_near(A, L, total);
 }
 
 // The 64-bit test of home atom hl (LDS index) against candidate li: -1 for
@@ -1270,17 +1325,9 @@ __device__ __forceinline__ float readlane_f32(float v, int l)
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
 
-// The largest of the lanes' non-negative values, on the last lane.
-__device__ __forceinline__ float wave_max_f32(float x)
+__device__ __forceinline__ float wave_max_f32(float x)   // non-negative floats order as their bits
 {
-    int v = __builtin_bit_cast(int, x);   // non-negative floats order as their bits
-    v = max(v, dpp_or_zero<0x111>(v));
-    v = max(v, dpp_or_zero<0x112>(v));
-    v = max(v, dpp_or_zero<0x114>(v));
-    v = max(v, dpp_or_zero<0x118>(v));
-    v = max(v, dpp_or_zero<0x142, 0xa>(v));
-    v = max(v, dpp_or_zero<0x143, 0xc>(v));
-    return __builtin_bit_cast(float, v);
+    return __builtin_bit_cast(float, wave_max_pos(__builtin_bit_cast(int, x)));
 }
 
 // The filter's error bound (filter_bounds) for home atoms within H of their

@@ -71,3 +71,26 @@ def test_time_of_a_reach_of_two_cells():
     y = workloads.random_in_cell(n, np.diag([6.0, L, L]), seed=n, cutoff=7.0)
     print("plate", flush=True)
     assert _time(y.X, 7.0, y.cell, (True,) * 3) < 1.65 * _time(s.X, 5.0, s.cell, (True,) * 3)
+
+
+@pytest.mark.parametrize("n", [65, 3000, 40000])
+@pytest.mark.parametrize("base", [(0, 0, 0), (200, -300, 400), (511, -512, 511)])
+@pytest.mark.parametrize("spread", [0, 127, 128, 200, 254, 255, 256, 500])
+def test_windings_of_a_brick(spread, base, n):
+    """Atoms that drifted together by hundreds of cells, some of them apart by
+    up to twice `spread`: the brick path as long as the windings of a brick span
+    no more than its entries hold, and the paths beyond."""
+    s = workloads.random_in_cell(n, np.array([[1.0, 0.1, 0.0], [0.2, 1.1, 0.1], [0.0, 0.1, 0.9]]) * (n / 0.05) ** (1 / 3),
+                                 seed=n, cutoff=4.0)
+    rng = np.random.default_rng(spread)
+    w = rng.choice([-spread, 0, 0, spread], size=(n, 3)) + np.array(base) * (1 if spread < 300 else 0)
+    print(f"brick windings {spread} {base} {n}", flush=True)
+    _check(s.X + w.astype(float) @ s.cell, 4.0, s.cell, (True, True, True), want_R=n == 3000)
+
+
+def test_time_of_positions_that_were_never_wrapped():
+    """Positions hundreds of cells from the cell they are described in: twice an
+    ordinary system's time it was, and is the same."""
+    s = workloads.random_cubic(500000, density=0.05, seed=1, cutoff=5.0)
+    print("drifted", flush=True)
+    assert _time(s.X + 200 * np.asarray(s.cell).sum(0), 5.0, s.cell, s.pbc) < 1.5 * _time(s.X, 5.0, s.cell, s.pbc)
