@@ -460,15 +460,20 @@ void drop_graph(nlh_handle *h)
 // whose halo atoms, expected at this system's mean atom density per cell,
 // stay within the budget (clipped to the cell grid), or, where the grid is
 // too coarse for that to fill the device, the smallest whose bricks still
-// run together (`slots` of them).  Count kernel on MI355X, event timed: 1k
+// run together (`slots` of them), and at most 2 x 2 x 2 where those of the
+// next larger shape would fill less than four fifths: smaller halos leave room
+// for local densities above the mean.  Count kernel on MI355X, event timed: 1k
 // atoms, 125 bricks of one cell against 27 of 2 x 2 x 2, 10.4 / 18.2 us; 10k,
 // 2 x 1 x 1 (666 bricks) 13.0 us, 1 x 1 x 1 (1331, two rounds) 17.2, 2 x 2 x 2
-// 17.5; 100k, 4 x 2 x 2 (1183) 31.6, 2 x 2 x 2 (2197) 32.6.
+// 17.5; 100k, 4 x 2 x 2 (1183) 31.6, 2 x 2 x 2 (2197) 32.6.  Whole builds, 2 x
+// 2 x 2 (1331) against 4 x 2 x 2 (726): 30k uniform atoms 68 / 73, with half of
+// them in an eighth of the cell 79 / 166 (halos over the LDS).
 void choose_brick(const nlh_geometry &g, int64_t nat, int32_t budget, int32_t halo_max, int64_t slots, int32_t out[3])
 {
     static const int32_t ladder[][3] = {{4, 4, 4}, {4, 4, 2}, {4, 2, 2}, {2, 2, 2}, {2, 2, 1}, {2, 1, 1}, {1, 1, 1}};
     const double per_cell = g.ncells_total > 0 ? (double)nat / (double)g.ncells_total : 0.0;
     bool found = false;
+    int64_t found_nb = 0;
     for (const auto &b : ladder) {
         int32_t d[3];
         double halo = 1.0;
@@ -478,10 +483,11 @@ void choose_brick(const nlh_geometry &g, int64_t nat, int32_t budget, int32_t ha
             halo *= (double)(d[k] + 2);
             nb *= (g.ncells[k] + d[k] - 1) / d[k];
         }
-        if (found && nb > slots) return;
+        if (found && nb > slots && (found_nb >= slots * 4 / 5 || (int64_t)out[0] * out[1] * out[2] <= 8)) return;
         if (halo * per_cell <= (double)budget && halo <= (double)halo_max) {
             std::memcpy(out, d, sizeof d);
             found = true;
+            found_nb = nb;
         }
     }
     if (!found) out[0] = out[1] = out[2] = 1;

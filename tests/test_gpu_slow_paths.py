@@ -94,3 +94,14 @@ def test_time_of_positions_that_were_never_wrapped():
     s = workloads.random_cubic(500000, density=0.05, seed=1, cutoff=5.0)
     print("drifted", flush=True)
     assert _time(s.X + 200 * np.asarray(s.cell).sum(0), 5.0, s.cell, s.pbc) < 1.5 * _time(s.X, 5.0, s.cell, s.pbc)
+
+
+@pytest.mark.parametrize("n", [27000, 33000])
+def test_time_of_a_dense_region(n):
+    """Half of the atoms in an eighth of the cell: 1.2 of a uniform system's time,
+    with bricks whose halos fit the LDS there (2.2 to 2.6 with the next larger ones)."""
+    s = workloads.random_cubic(n, density=0.02, seed=n, cutoff=5.0)
+    X, c = s.X.copy(), np.diag(np.asarray(s.cell)) / 2
+    X[::2] = c + (X[::2] - c) * 0.5
+    print(f"dense region {n}", flush=True)
+    assert _time(X, 5.0, s.cell, s.pbc) < 1.7 * _time(s.X, 5.0, s.cell, s.pbc)
