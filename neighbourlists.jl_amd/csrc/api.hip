@@ -592,7 +592,8 @@ void filter_bounds(nlh::SysDev &sd, const nlh_geometry &g)
 //   u rc (8 H + 4 rc + 10 (A + O))
 // (home atom u (|o| + 2 H); candidate u (2 (H + rc) + |s - o|) and, for s - o
 // itself, u (4 A + 3 |o|)); with 2 H rc <= H^2 + rc^2 the sum of all terms is at
-// most u (78 H^2 + 66 rc^2 + 10 (A + O) rc), of which the kernel adds the first.
+// most u (78 H^2 + 66 rc^2 + 10 (A + O) rc), of which the kernel adds the first;
+// the 64-bit roundings' share is filter_bounds'.
 void small_bounds(nlh::SysDev &sd, const nlh_geometry &g)
 {
     constexpr double u = 1.0 / (1 << 24);

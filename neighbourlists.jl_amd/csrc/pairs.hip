@@ -1344,6 +1344,30 @@ __device__ __forceinline__ float far_tol(const SysDev &sd, float H, int far2)
     return H + P < 1.0e15f ? 0.505f * (1.25f / (1 << 24) * e + sd.tol64) : kFar32 * kFar32;
 }
 
+// Home atoms that lie far from their cell's centre (along an open axis; above
+// kFarHome rc^2 / 2 for half the square of their distance) are taken from the
+// first of them instead, which keeps the filter's error at their own extent's
+// (whole builds, us: a sheet of 200,000 atoms 1,000 A away from its cell 245 from
+// the cell's centre, 117 from an atom; 200 systems of 500 to 2,000 atoms 300
+// cells away 1,326 and 199).
+constexpr float kFarHome = 32.0f;
+__device__ __forceinline__ void home_centre(const TAtom &h, float &ox, float &oy, float &oz)
+{
+    ox = readlane_f32(h.x, 0);
+    oy = readlane_f32(h.y, 0);
+    oz = readlane_f32(h.z, 0);
+}
+
+// The home atoms' side of the tests from the centre o; half the squares of
+// their distances from it.
+__device__ __forceinline__ float tile_home(TileHomes &H, const TAtom &h, float ox, float oy, float oz)
+{
+    H.nx = ox - h.x;
+    H.ny = oy - h.y;
+    H.nz = oz - h.z;
+    return 0.5f * __builtin_fmaf(H.nz, H.nz, __builtin_fmaf(H.ny, H.ny, H.nx * H.nx));
+}
+
 // Slot entries of a pass: 4 or 8 bytes.
 enum { kEntry4, kEntry8 };
 
@@ -1488,7 +1512,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(5))) void ti
         const int hc = ix + B.hd[0] * ((iy + 1) + B.hd[1] * (iz + 1));   // halo cell before the run's first
         const int h0 = sgpr(L.hoff[hc + 1]), nha = sgpr(L.hoff[hc + 1 + w]) - h0;
         if (nha <= 0) continue;
-        const float ox = L.ctr[rn][0], oy = L.ctr[rn][1], oz = L.ctr[rn][2];
+        float ox = L.ctr[rn][0], oy = L.ctr[rn][1], oz = L.ctr[rn][2];
         // candidates: nine rows of w + 2 cells, each contiguous in LDS
         const int rst = L.hoff[hc + roff];
         const int len = lane < 9 ? L.hoff[hc + roff + w + 2] - rst : 0;
@@ -1509,20 +1533,24 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(5))) void ti
             const TAtom h = L.a[hl];
             const int32_t hj_l = (int32_t)((uint32_t)h.j & hjmask);
             TileHomes H;
-            H.nx = ox - h.x;
-            H.ny = oy - h.y;
-            H.nz = oz - h.z;
-            const float hq = 0.5f * __builtin_fmaf(H.nz, H.nz, __builtin_fmaf(H.ny, H.ny, H.nx * H.nx));
+            float hq = tile_home(H, h, ox, oy, oz);
+            // atoms further out than the system's bounds assume: the brick's own
+            float tol = sd.tol;
+            if (__builtin_amdgcn_ballot_w64(!(hq <= sd.h2half)) != 0 || far2 != 0) {
+                float hm = readlane_f32(wave_max_f32(hq), kWave - 1);
+                if (hm > kFarHome * sd.rc2half) {
+                    home_centre(h, ox, oy, oz);
+                    hq = tile_home(H, h, ox, oy, oz);
+                    hm = readlane_f32(wave_max_f32(hq), kWave - 1);
+                }
+                tol = far_tol(sd, __builtin_sqrtf(2.0f * hm), far2);
+            }
             H.ai = hq - sd.rc2half;
             H.row = (reinterpret_cast<uint64_t>(slots) + (narrow ? 0 : off8) +
                      (uint64_t)slot_row(sd.atom_base + hj_l, narrow ? row4 : 8 * cap)) |
                     (uint64_t)(narrow ? 4 : 8) << 48;
             H.t = L.t[hl];
             H.fill = 0;
-            // atoms further out than the system's bounds assume: the brick's own
-            float tol = sd.tol;
-            if (__builtin_amdgcn_ballot_w64(!(hq <= sd.h2half)) != 0 || far2 != 0)
-                tol = far_tol(sd, __builtin_sqrtf(2.0f * readlane_f32(wave_max_f32(hq), kWave - 1)), far2);
             for (int k0 = 0; k0 < total; k0 += kTileCands) {
                 const int nch = sgpr(min(kTileChunks, (total - k0 + kWave - 1) / kWave));
                 // marks where a non-empty row other than the first starts (see row_map)
@@ -1695,6 +1723,8 @@ __device__ __forceinline__ uint32_t pack_fields(int32_t x, int32_t y, int32_t z)
 // The share of the home group's extent in the filter's error bound: times the
 // largest |p_i|^2 / 2 of the group (see small_bounds for the rest).
 constexpr float kSmallTol = 0.505f * 1.25f / (1 << 24) * 156.0f;
+// ... and that of a centre beyond the system's cell: times its distance and the cutoff.
+constexpr float kSmallTolFar = 0.505f * 1.25f / (1 << 24) * 10.0f;
 
 // A system's table entry, read through the scalar cache (nothing writes it
 // while the kernel runs).
@@ -1988,18 +2018,25 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
         const float f0 = ((float)ci0 - 0.5f) * __builtin_amdgcn_rcpf((float)n0) - 0.5f,
                     f1 = ((float)ci1 - 0.5f) * __builtin_amdgcn_rcpf((float)n1) - 0.5f,
                     f2 = ((float)ci2 - 0.5f) * __builtin_amdgcn_rcpf((float)n2) - 0.5f;
-        const float ox = C32[0] * f0 + C32[1] * f1 + C32[2] * f2, oy = C32[3] * f0 + C32[4] * f1 + C32[5] * f2,
-                    oz = C32[6] * f0 + C32[7] * f1 + C32[8] * f2;
+        float ox = C32[0] * f0 + C32[1] * f1 + C32[2] * f2, oy = C32[3] * f0 + C32[4] * f1 + C32[5] * f2,
+              oz = C32[6] * f0 + C32[7] * f1 + C32[8] * f2;
         for (int hg = hg0; hg < nha; hg += kWave) {
             const int nh = sgpr(min(kWave, nha - hg));
             const int hb = h0 + hg;
             const int hl = hb + (lane < nh ? lane : 0);
             const TAtom h = L.a[hl];
             TileHomes H;
-            H.nx = ox - h.x;
-            H.ny = oy - h.y;
-            H.nz = oz - h.z;
-            const float hq = 0.5f * __builtin_fmaf(H.nz, H.nz, __builtin_fmaf(H.ny, H.ny, H.nx * H.nx));
+            float hq = tile_home(H, h, ox, oy, oz);
+            // the filter's error bound (small_bounds); beyond any sane scale, 64-bit tests for all
+            float hm = readlane_f32(wave_max_f32(hq), kWave - 1), so = 0.0f;
+            if (hm > kFarHome * sd->rc2half) {
+                home_centre(h, ox, oy, oz);
+                hq = tile_home(H, h, ox, oy, oz);
+                hm = readlane_f32(wave_max_f32(hq), kWave - 1);
+                so = __builtin_sqrtf(2.0f * sd->rc2half * (ox * ox + oy * oy + oz * oz));
+            }
+            const float tol = hm + so < 1.0e30f ? __builtin_fmaf(so, kSmallTolFar, __builtin_fmaf(hm, kSmallTol, sd->small_tol))
+                                                : kFar32 * kFar32;
             H.ai = hq - sd->rc2half;
             const int64_t ha = sd->atom_base + h.j;
             H.row = (reinterpret_cast<uint64_t>(A.slots) + (row8 ? A.off8 : 0) +
@@ -2007,9 +2044,6 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
                     (uint64_t)(row8 ? 8 : 4) << 48;
             H.t = 2 * kPackZero - L.w[hl];   // t'_i = -w_i
             H.fill = 0;
-            // the filter's error bound (small_bounds); beyond any sane scale, 64-bit tests for all
-            const float hm = readlane_f32(wave_max_f32(hq), kWave - 1);
-            const float tol = hm < 1.0e30f ? __builtin_fmaf(hm, kSmallTol, sd->small_tol) : kFar32 * kFar32;
             for (int sb = 0; sb < nseg; sb += kWave) {
                 // lane: neighbour cell sb + lane in the reference order, its
                 // sorted atoms and cell shift (_is_cell_in_bounds,

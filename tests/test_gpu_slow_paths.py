@@ -43,6 +43,22 @@ def _time(X, rc, cell, pbc):
     return 1e6 * float(np.median(t[5:]))
 
 
+def _time_batch(systems):
+    """Median time of a rebuild of a batch of device positions (us)."""
+    B = nlhip.BatchBuilder()
+    X = np.concatenate([y.X for y in systems])
+    D = torch.as_tensor(X).cuda()
+    torch.cuda.synchronize()
+    B.run(systems, X_device=D, copy=False)
+    t = []
+    for _ in range(30):
+        t0 = time.perf_counter()
+        B.rebuild(X, X_device=D, copy=False)
+        _lib.check(_lib.lib().nlh_synchronize(B.handle.ptr))
+        t.append(time.perf_counter() - t0)
+    return 1e6 * float(np.median(t[5:]))
+
+
 @pytest.mark.parametrize("reach", [1, 2])
 @pytest.mark.parametrize("sizes", [(1, 1, 1), (47, 48, 49, 63, 64, 65), (96, 97, 144, 145, 0, 200), (3, 0, 0, 130, 7, 1)])
 def test_cells_counted_from_global_memory(sizes, reach):
@@ -105,3 +121,50 @@ def test_time_of_a_dense_region(n):
     X[::2] = c + (X[::2] - c) * 0.5
     print(f"dense region {n}", flush=True)
     assert _time(X, 5.0, s.cell, s.pbc) < 1.7 * _time(s.X, 5.0, s.cell, s.pbc)
+
+
+@pytest.mark.parametrize("off", [0.0, 30.0, 1e3, 1e5, -1e7])
+@pytest.mark.parametrize("shell", [0.5, 1.0])
+@pytest.mark.parametrize("eps", [0.0, 3e-16, 1e-7, -1e-7])
+def test_crystals_far_from_an_open_cell(shell, eps, off):
+    """Crystal slabs away from their cell along its open axis, the cutoff at a
+    neighbour distance: single builds and a fused batch, where the home atoms'
+    own position is the tests' centre."""
+    rc = 3.61 * np.sqrt(shell) * (1.0 + eps)
+    systems = []
+    for k in range(66):
+        X, cell = workloads.fcc(3.61, (2 + k % 3, 2 + k % 2, 1 + k % 4))
+        systems.append(workloads.System(X + 0.1 + np.array([0.0, 0.0, off * (1 + k % 2)]), cell, (True, True, False), rc))
+    X, cell = workloads.fcc(3.61, (14, 13, 2))
+    print(f"far crystals {shell} {eps} {off}", flush=True)
+    _check(X + np.array([0.1, 0.1, off]), rc, cell, (True, True, False), want_R=True)
+    got = nlhip.BatchBuilder().run(systems)
+    for k, y in enumerate(systems):
+        ref = oracle.neighbour_list(y.X, y.cutoff, y.cell, y.pbc)
+        nl = got.pairlist(k)
+        assert np.array_equal(nl.first, ref.first), k
+        assert np.array_equal(nl.i, ref.i) and np.array_equal(nl.j, ref.j) and np.array_equal(nl.S, ref.S), k
+
+
+def test_time_of_a_sheet_far_from_its_cell():
+    """A sheet one cell thick 1,000 A along its open axis from the cell: twice the
+    time of one inside it was, and is the same."""
+    L = (200000 / 0.05 / 10) ** 0.5
+    s = workloads.random_in_cell(200000, np.diag([L, L, 10.0]), seed=1, cutoff=5.0)
+    pbc = (True, True, False)
+    print("sheet", flush=True)
+    assert _time(s.X + [0.0, 0.0, 1000.0], 5.0, s.cell, pbc) < 1.5 * _time(s.X, 5.0, s.cell, pbc)
+
+
+def test_time_of_a_batch_far_from_its_cells():
+    """A fused batch 300 cells along its open axes from its cells: as long as 3
+    cells away (it took six times as long)."""
+    t = []
+    for w in (3, 300):
+        systems = []
+        for k in range(200):
+            s = workloads.random_cubic(500 + 7 * k, density=0.05, seed=k, cutoff=5.0)
+            systems.append(workloads.System(s.X + [0.0, 0.0, w * s.cell[2][2]], s.cell, (True, True, False), 5.0))
+        t.append(_time_batch(systems))
+    print("far batch", t, flush=True)
+    assert t[1] < 1.5 * t[0]
