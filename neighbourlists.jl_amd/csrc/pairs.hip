@@ -1659,7 +1659,7 @@ struct SmallLDS {
     uint8_t sys_reach[kUnitSystems];  // nxyz: x | y << 2 | z << 4
     uint8_t sys_group[kUnitSystems];  // home atoms per count work item
     uint8_t sys_row8[kUnitSystems];   // 8-byte slot rows: some winding, or reach beyond one cell
-    uint8_t sys_far[kUnitSystems];    // some winding beyond +-128
+    uint8_t sys_far[kUnitSystems];    // windings too far apart for packed differences
     union {
         SmallSort s;
         SmallCount c;
@@ -1777,8 +1777,8 @@ struct SmallEnv {
     }
 };
 
-// A batch of segments against the home atoms of a system with windings beyond
-// +-128, whose packed differences could leave their fields: 64-bit tests, S
+// A batch of segments against the home atoms of a system whose windings lie so
+// far apart that packed differences could leave their fields: 64-bit tests, S
 // taken apart; an S beyond +-511 sends the build to 16-byte entries.  Lane:
 // ex, st, sh of a segment; fill of a home atom, returned.  ks: the self
 // candidate of home atom 0.
@@ -1878,7 +1878,6 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
         L.u.s.wk[i] = wp;
         L.u.s.sy[i] = (uint8_t)k;
         if (wp != kPackZero) L.sys_row8[k] = 1;
-        if ((unsigned)(w[0] + 128) > 256u || (unsigned)(w[1] + 128) > 256u || (unsigned)(w[2] + 128) > 256u) L.sys_far[k] = 1;
         big |= (wp & kWindBig) != 0;
         atomicAdd(&L.u.s.fill[key], 1);
         if (writer) A.atom_sys[g] = s0 + k;   // the fill kernel's map of atoms to systems
@@ -1933,6 +1932,15 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs A)
             ux -= cx;
             uy -= cy;
             uz -= cz;
+        }
+        const uint32_t w0 = L.u.s.wk[L.sys_atom0[k]];
+        if (wk != w0) {
+            // every S = s - w_j + w_i packs while the windings are within 252 of the first atom's
+            int32_t wx, wy, wz, vx, vy, vz;
+            unpack_wind(wk, wx, wy, wz);
+            unpack_wind(w0, vx, vy, vz);
+            if ((unsigned)(wx - vx + 252) > 504u || (unsigned)(wy - vy + 252) > 504u || (unsigned)(wz - vz + 252) > 504u)
+                L.sys_far[k] = 1;
         }
         const int32_t jl = i - L.sys_atom0[k];
         L.a[p] = TAtom{(float)ux, (float)uy, (float)uz, jl};

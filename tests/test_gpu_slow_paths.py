@@ -168,3 +168,41 @@ def test_time_of_a_batch_far_from_its_cells():
         t.append(_time_batch(systems))
     print("far batch", t, flush=True)
     assert t[1] < 1.5 * t[0]
+
+def _batch(nsys, lo, hi, move, seed):
+    rng = np.random.default_rng(seed)
+    out = []
+    for k in range(nsys):
+        n = int(rng.integers(lo, hi + 1))
+        s = workloads.random_cubic(n, density=0.05, seed=seed + k, cutoff=4.0 + 0.5 * (k % 3))
+        out.append(workloads.System(s.X + move(rng, k, n).astype(float) @ np.asarray(s.cell), s.cell,
+                                    (True, k % 5 != 1, True), s.cutoff))
+    return out
+
+
+@pytest.mark.parametrize("want_R", [False, True])
+@pytest.mark.parametrize("base", [0, 300, -511])
+@pytest.mark.parametrize("spread", [1, 128, 251, 252, 253, 256])
+def test_batch_windings_of_a_system(spread, base, want_R):
+    """Systems of a fused batch that drifted by up to 511 cells, with atoms apart
+    by one to twice `spread`, R included."""
+    def move(rng, k, n):
+        w = rng.choice([0, 0, spread if base <= 0 else -spread, -spread if base == 0 and k % 2 else 0], size=(n, 3))
+        return w + base * (k % 3 != 2)
+    print(f"batch windings {spread} {base} {want_R}", flush=True)
+    systems = _batch(70, 1, 300, move, 17)
+    got = nlhip.BatchBuilder().run(systems, want_R=want_R)
+    for k, y in enumerate(systems):
+        ref = oracle.neighbour_list(y.X, y.cutoff, y.cell, y.pbc, want_R=want_R)
+        nl = got.pairlist(k)
+        assert np.array_equal(nl.first, ref.first), k
+        assert np.array_equal(nl.i, ref.i) and np.array_equal(nl.j, ref.j) and np.array_equal(nl.S, ref.S), k
+        if want_R:
+            assert np.array_equal(_bits(nl.R), _bits(ref.R)), k
+
+
+def test_time_of_a_batch_that_was_never_wrapped():
+    """A fused batch of drifted systems: twice an ordinary batch's time it was, and is the same."""
+    t = [_time_batch(_batch(200, 500, 2000, lambda rng, k, n: np.full((n, 3), w), 5)) for w in (0, 200)]
+    print("drifted batch", t, flush=True)
+    assert t[1] < 1.5 * t[0]
