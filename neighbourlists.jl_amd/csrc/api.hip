@@ -536,6 +536,12 @@ constexpr int64_t kReplayMaxAtoms = 12288;
 // counted from global memory instead).
 constexpr double kHaloFill = 0.9;
 
+// The distance that cutoff_sq, which decides, stands for (a caller fills both).
+double search_radius(const nlh_geometry &g)
+{
+    return std::max(g.cutoff, std::sqrt(g.cutoff_sq));
+}
+
 // Bounds of the 32-bit distance filter (SysDev; tile_kernel in pairs.hip).
 // With u = 2^-24, c the centre of a run of home cells, |p_i - c| <= H for
 // its home atoms and |p_j - c| <= H + rc for any candidate within the cutoff,
@@ -552,7 +558,7 @@ constexpr double kHaloFill = 0.9;
 void filter_bounds(nlh::SysDev &sd, const nlh_geometry &g)
 {
     constexpr double u = 1.0 / (1 << 24);
-    const double rc = g.cutoff;
+    const double rc = search_radius(g);
     double step[3][3], len[3], sum = 0.0, P = rc;
     for (int k = 0; k < 3; ++k) {
         double l2 = 0.0;
@@ -597,7 +603,7 @@ void filter_bounds(nlh::SysDev &sd, const nlh_geometry &g)
 void small_bounds(nlh::SysDev &sd, const nlh_geometry &g)
 {
     constexpr double u = 1.0 / (1 << 24);
-    const double rc = g.cutoff;
+    const double rc = search_radius(g);
     double sum = 0.0, A = 0.0;
     for (int k = 0; k < 3; ++k) {
         double l2 = 0.0;
@@ -634,7 +640,11 @@ int32_t plan_search(nlh::SysDev &sd, const nlh_geometry &g, bool single, int cus
     int64_t bricks = 1;
     for (int k = 0; k < 3; ++k) bricks *= (sd.n[k] + sd.brick[k] - 1) / sd.brick[k];
     const int cells = sd.brick[0] * sd.brick[1] * sd.brick[2];
-    sd.run = sd.brick[0] > 1 && per_cell <= 8.0 && bricks > 2 * slots ? 2 : 1;
+    // ... and only where a cell is a cutoff high, so that cells two apart hold no
+    // neighbours (a caller's own cell counts may be finer)
+    const double *inv = g.inv_cell;
+    const double height = 1.0 / (std::sqrt(inv[0] * inv[0] + inv[1] * inv[1] + inv[2] * inv[2]) * sd.n[0]);
+    sd.run = sd.brick[0] > 1 && per_cell <= 8.0 && bricks > 2 * slots && height >= search_radius(g) * (1.0 - 1e-9) ? 2 : 1;
     sd.split = cells == 1 ? 2 : (cells == 2 ? 1 : 0);
     int32_t copies = 1;
     while (single && sd.split > 0 && sd.split < 6 && per_cell >= 4 << sd.split && bricks * copies * 2 <= slots) {

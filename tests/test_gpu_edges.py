@@ -111,3 +111,27 @@ def test_lazy_queries_read_the_positions_as_they_are(n, density, moved, int_type
     torch.cuda.synchronize()
     for u, v in zip(nlhip.neighbours_range(cl, 1, min(n, 500)), before):
         assert np.array_equal(u, v)
+
+
+@pytest.mark.parametrize("cells,square", [(56, 25.0), (34, 25.0), (56, 30.0)])
+def test_cells_smaller_than_the_cutoff(cells, square):
+    """A caller's own cell counts with a reach of one cell, and its own square of
+    the cutoff: the 27 cells around an atom and no more, whatever the pair search
+    shares between home cells."""
+    n = 250000
+    s = workloads.random_cubic(n, density=0.05, seed=1, cutoff=5.0)
+    g = _lib.geometry(s.cell, 5.0, s.pbc, 4)
+    for k in range(3):
+        g.ncells[k], g.nxyz[k] = cells, 1
+    g.ncells_total = cells ** 3
+    g.cutoff_sq = square
+    L, h, m = _lib.lib(), _lib.Handle(), ctypes.c_int64()
+    print(f"cells {cells} {square}", flush=True)
+    _lib.check(L.nlh_neighbour_list(h.ptr, s.X.ctypes.data, n, ctypes.byref(g), 0, ctypes.byref(m)))
+    j, first, S = np.empty(m.value, np.int32), np.empty(n + 1, np.int32), np.empty((m.value, 3), np.int32)
+    _lib.check(L.nlh_copy_pairlist(h.ptr, None, j.ctypes.data, S.ctypes.data, first.ctypes.data, None))
+    for i in range(1, n + 1, 997):
+        c, j1, S1 = ctypes.c_int64(), np.empty(256, np.int32), np.empty((256, 3), np.int32)
+        _lib.check(L.nlh_neighbours(h.ptr, 0, i, 256, j1.ctypes.data, None, S1.ctypes.data, ctypes.byref(c)))
+        a, b = first[i - 1] - 1, first[i] - 1
+        assert b - a == c.value and np.array_equal(j[a:b], j1[:c.value]) and np.array_equal(S[a:b], S1[:c.value])
