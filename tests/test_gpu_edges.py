@@ -135,3 +135,40 @@ def test_cells_smaller_than_the_cutoff(cells, square):
         _lib.check(L.nlh_neighbours(h.ptr, 0, i, 256, j1.ctypes.data, None, S1.ctypes.data, ctypes.byref(c)))
         a, b = first[i - 1] - 1, first[i] - 1
         assert b - a == c.value and np.array_equal(j[a:b], j1[:c.value]) and np.array_equal(S[a:b], S1[:c.value])
+
+
+def _edge_batches():
+    """name -> systems: units at their limits, systems without atoms, one beyond a
+    unit, rows that overflow, atoms far outside open cells."""
+    def cubes(sizes):
+        out = []
+        for k, n in enumerate(sizes):
+            y = workloads.random_cubic(max(n, 1), density=0.05, seed=k, cutoff=3.5 + 0.1 * (k % 9))
+            out.append(workloads.System(y.X[:n], y.cell, y.pbc, y.cutoff))
+        return out
+
+    rng = np.random.default_rng(8)
+    clusters, far = [], []
+    for k in range(66):
+        n = [30, 300, 900][k % 3]
+        cell = np.eye(3) * (6.0 if k % 3 == 0 else 40.0)
+        X = rng.random((n, 3)) * 40.0
+        X[-30:] = 20.0 + 0.5 * rng.random((30, 3))
+        clusters.append(workloads.System(X, cell, (True, True, k % 2 == 0), 5.0))
+        y = workloads.random_cubic(150 + k, density=0.05, seed=k, cutoff=4.0)
+        pbc = (k % 2 == 0, k % 3 == 0, False)
+        far.append(workloads.System(y.X + np.where(pbc, 0.0, [0.3, 17.0, 1e6][k % 3]) * y.cell[0][0], y.cell, pbc, 4.0))
+    return {"full units": cubes([2048] * 64), "one large": cubes([1] * 700 + [2048]), "empty": cubes([2047, 1, 0, 1] * 20),
+            "almost empty": cubes([0] * 70 + [3]), "beyond a unit": cubes([2049] + [5] * 70), "clusters": clusters,
+            "far": far}
+
+
+@pytest.mark.parametrize("int_type,bits", [(np.int32, 32), (np.int64, 64)])
+@pytest.mark.parametrize("name", sorted(_edge_batches()))
+def test_R_of_batches_at_their_edges(name, int_type, bits):
+    """R of batches at the limits of the fused build, against the oracle bit for bit."""
+    systems = _edge_batches()[name]
+    print(f"R batch edges {name} {bits}", flush=True)
+    got = nlhip.BatchBuilder(int_type=int_type).run(systems, want_R=True)
+    for k, y in enumerate(systems):
+        _same(got.pairlist(k), oracle.neighbour_list(y.X, y.cutoff, y.cell, y.pbc, ti_bits=bits, want_R=True), True)
