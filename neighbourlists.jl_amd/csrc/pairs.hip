@@ -29,6 +29,7 @@
 #include <algorithm>
 
 #include "device_util.h"
+#include "filter_bounds.h"
 
 namespace nlh {
 
@@ -1067,7 +1068,6 @@ struct TileLDS {
     int32_t far2;                   // largest |p|^2 beyond the system's pmax2 (its bits), or 0
 };
 
-constexpr float kFar32 = 1.0e18f;   // sentinel position: |p|^2 / 2 = 5e35, never a hit
 constexpr uint32_t kFieldsLow = 1u | (1u << 10) | (1u << 20);
 
 // The runs of a brick: sd.run home cells next to each other along x, the last
@@ -1330,20 +1330,6 @@ __device__ __forceinline__ float wave_max_f32(float x)   // non-negative floats 
     return __builtin_bit_cast(float, wave_max_pos(__builtin_bit_cast(int, x)));
 }
 
-// The filter's error bound (filter_bounds) for home atoms within H of their
-// centre and brick atoms up to |p|^2 of bits far2 beyond the system's pmax2.
-// Beyond any sane scale every value is decided by the 64-bit test.  (1,000 atoms
-// centred on the corner of an open cell, count kernel: bricks with such atoms
-// on the 64-bit per-wave path 684 us, with a bound of their own 68; 64-bit LDS
-// path 235.)
-__device__ __forceinline__ float far_tol(const SysDev &sd, float H, int far2)
-{
-    const float P = __builtin_sqrtf(fmaxf(sd.pmax2, __builtin_bit_cast(float, far2))), rc = __builtin_sqrtf(2.0f * sd.rc2half);
-    const float a = 2.0f * H + rc, b = H + rc;
-    const float e = 10.0f * (a * a + rc * rc) + 7.0f * b * b + 4.0f * rc * rc + 7.2f * (P + a) * rc;
-    return H + P < 1.0e15f ? 0.505f * (1.25f / (1 << 24) * e + sd.tol64) : kFar32 * kFar32;
-}
-
 // Home atoms that lie far from their cell's centre (along an open axis; above
 // kFarHome rc^2 / 2 for half the square of their distance) are taken from the
 // first of them instead, which keeps the filter's error at their own extent's
@@ -1543,7 +1529,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(5))) void ti
                     hq = tile_home(H, h, ox, oy, oz);
                     hm = readlane_f32(wave_max_f32(hq), kWave - 1);
                 }
-                tol = far_tol(sd, __builtin_sqrtf(2.0f * hm), far2);
+                tol = far_tol(sd, __builtin_sqrtf(2.0f * hm), __builtin_bit_cast(float, far2));
             }
             H.ai = hq - sd.rc2half;
             H.row = (reinterpret_cast<uint64_t>(slots) + (narrow ? 0 : off8) +
@@ -1719,12 +1705,6 @@ __device__ __forceinline__ uint32_t pack_fields(int32_t x, int32_t y, int32_t z)
 {
     return kPackZero + (uint32_t)x + ((uint32_t)y << 10) + ((uint32_t)z << 20);
 }
-
-// The share of the home group's extent in the filter's error bound: times the
-// largest |p_i|^2 / 2 of the group (see small_bounds for the rest).
-constexpr float kSmallTol = 0.505f * 1.25f / (1 << 24) * 156.0f;
-// ... and that of a centre beyond the system's cell: times its distance and the cutoff.
-constexpr float kSmallTolFar = 0.505f * 1.25f / (1 << 24) * 10.0f;
 
 // A system's table entry, read through the scalar cache (nothing writes it
 // while the kernel runs).

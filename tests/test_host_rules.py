@@ -9,17 +9,23 @@ import pytest
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "neighbourlists.jl_amd", "csrc")
 
 
-def run_cpp(tmp_path, body, includes=("nlhip_internal.h",)):
-    """Compile and run main() { body }; returns what it printed."""
+def run_file(tmp_path, src):
+    """Compile and run a C++ program over the library's headers; returns what it printed."""
     if not shutil.which("g++"):
         pytest.skip("no host compiler")
-    src, exe = tmp_path / "t.cpp", tmp_path / "t"
+    exe = tmp_path / "t"
+    subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__", "-I", CSRC, "-I",
+                    "/opt/rocm/include", str(src), "-o", str(exe), "-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib",
+                    "-lamdhip64", "-lpthread"], check=True, capture_output=True, text=True)
+    return subprocess.run([str(exe)], check=True, capture_output=True, text=True, timeout=60).stdout
+
+
+def run_cpp(tmp_path, body, includes=("nlhip_internal.h",)):
+    """The same for main() { body }."""
+    src = tmp_path / "t.cpp"
     src.write_text("".join(f'#include "{i}"\n' for i in includes) +
                    "#include <cstdio>\nusing namespace nlh;\nint main()\n{\n" + body + "\nreturn 0;\n}\n")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", CSRC, "-I", "/opt/rocm/include", str(src),
-                    "-o", str(exe), "-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib", "-lamdhip64", "-lpthread"],
-                   check=True, capture_output=True, text=True)
-    return subprocess.run([str(exe)], check=True, capture_output=True, text=True, timeout=60).stdout
+    return run_file(tmp_path, src)
 
 
 def _overflows(tmp_path, counts):
@@ -84,3 +90,15 @@ p.handle_gone();
 printf("%d", gone);
 """, includes=("host_copy.h",))
     assert out == f"1 1 1 0 1 {10 - 4}"
+
+
+def test_filter_bounds(tmp_path):
+    """The 32-bit distance filter of both pair searches, emulated: over cells of
+    one to nine cutoffs, sheared, in units from 1e-10 to 1e6, with windings and
+    atoms far outside open cells, no pair beyond its error bound has another
+    sign than the 64-bit test, and no error near the cutoff exceeds the bound."""
+    out = run_file(tmp_path, os.path.join(os.path.dirname(os.path.abspath(__file__)), "filter_bounds_check.cpp"))
+    for line in out.splitlines():
+        pairs, wrong, worst, _ = line.split()
+        assert int(pairs) > 100000 and int(wrong) == 0 and float(worst) < 1.0, line
+    assert len(out.splitlines()) == 2
