@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256) void bin_kernel(const double *__restrict__ X, 
 // itself, whatever else runs.  The other two scans write over their input:
 // they take their tile from the ticket, so that every tile a block waits for
 // belongs to one that started before it and is running or done, except for
-// launches too small to block one another (kOrderlessTiles).  Tickets are
+// launches too small to block one another (kOrderlessBuckets, kOrderlessCells).  Tickets are
 // atomics on one address, about 8 ns each (pair counts of 1M atoms: 17 us with
 // them, 13 without; 1.6M 20 and 15).  The descriptors are zero before a launch
 // (cleared with the status at the start of a build, or by clear_lookback
@@ -181,12 +181,12 @@ __global__ __launch_bounds__(kScanThreads) void scan_partials_kernel(int64_t *__
 }
 
 // The tile of this block: its index when no block waits for another (tile
-// sums given: three-kernel scan) or they are few (kOrderlessTiles), else by
-// ticket.  Returns -1 for a block with no tile (see scan_ticket).
+// sums given: three-kernel scan) or there are no more blocks than `orderless`,
+// else by ticket.  Returns -1 for a block with no tile (see scan_ticket).
 __device__ __forceinline__ int64_t scan_tile_begin(uint64_t *__restrict__ desc, const int64_t *__restrict__ partials,
-                                                   Status *__restrict__ status)
+                                                   unsigned orderless, Status *__restrict__ status)
 {
-    return partials || gridDim.x <= kOrderlessTiles ? (int64_t)blockIdx.x : scan_ticket(desc, status);
+    return partials || gridDim.x <= orderless ? (int64_t)blockIdx.x : scan_ticket(desc, status);
 }
 
 __device__ __forceinline__ uint64_t desc_load(const uint64_t *p)
@@ -295,7 +295,7 @@ __device__ __forceinline__ int64_t scan_lookback(uint64_t *__restrict__ desc, in
 // One padding slot per 8 items keeps the blocked accesses off shared banks.
 __device__ __forceinline__ int tile_slot(int i) { return i + (i >> 3); }
 constexpr int kTileSlots = kScanTile + kScanTile / 8;
-static_assert(kTileSlots * 12 + 1024 <= 160 * 1024 / kScanBlocksPerCu, "kScanBlocksPerCu scan blocks fit a CU's LDS");
+static_assert(kTileSlots * 12 + 1024 <= 160 * 1024 / kCellScanBlocksPerCu, "their LDS");
 
 // Cell histogram -> cell_start (0-based), the caller-facing 1-based
 // cell_offsets per system; the histogram is cleared for the next build.
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_cells_kernel(
     int32_t *__restrict__ cell_start, const SysDev *__restrict__ sys, const int32_t *__restrict__ cell_sys,
     int nsys, void *__restrict__ offsets_out, Status *__restrict__ status)
 {
-    const int64_t tile = scan_tile_begin(desc, partials, status);
+    const int64_t tile = scan_tile_begin(desc, partials, kOrderlessCells, status);
     if (tile < 0) return;
     int32_t v[kScanItems];
     const int64_t base = tile * kScanTile;
@@ -603,11 +603,11 @@ __global__ __launch_bounds__(kBinThreads) void bucket_count_kernel(
 
 // Exclusive scan of n counts in place (the bucket counts, at most
 // kSortLookbackTiles tiles: sort_plan); tile prefixes by look-back.
-__global__ __launch_bounds__(kScanThreads) void scan_inplace_kernel(int32_t *__restrict__ a, int64_t n,
+__global__ __launch_bounds__(kScanThreads, kBucketScanBlocksPerCu) void scan_inplace_kernel(int32_t *__restrict__ a, int64_t n,
                                                                     uint64_t *__restrict__ desc,
                                                                     Status *__restrict__ status)
 {
-    const int64_t tile = scan_tile_begin(desc, nullptr, status);
+    const int64_t tile = scan_tile_begin(desc, nullptr, kOrderlessBuckets, status);
     if (tile < 0) return;
     int32_t v[kScanItems];
     const int64_t base = tile * kScanTile;

@@ -26,18 +26,21 @@ constexpr int kMinFillPairs = 128;        // smallest fill tile (pairs per fill 
 inline int64_t scan_tiles(int64_t n) { return n > 0 ? (n + kScanTile - 1) / kScanTile : 1; }
 constexpr int64_t kLookbackTiles = 2048;  // single-pass scans up to this many tiles
 
-// Scans that write over their input (sort and cell counts) take their tiles in
-// block order up to kOrderlessTiles blocks, by ticket beyond.  A block waits
+// Scans that write over their input (bucket and cell counts) take their tiles
+// in block order while they are this small, by ticket beyond.  A block waits
 // for the tiles before its own, and one of those may not have started: an
 // XCD starts a launch's blocks in order, but it may be full of other launches'
 // waiting blocks, which wait for blocks that other full XCDs do not start.
-// That cannot be while the waiting blocks of all other hardware queues, one
-// scan each, dealt to the XCDs in turn, leave a place on every XCD free.
+// That cannot be while a launch, dealt to the XCDs in turn, has no more blocks
+// on an XCD than fit one of its compute units: the waiting blocks of all other
+// hardware queues, one scan each, then leave a compute unit of it free.
 constexpr int kXcds = 8, kXcdCus = 32;
-constexpr int kScanBlocksPerCu = 5;       // scan blocks that fit a CU at least (LDS; see kernels.hip)
-constexpr int kHwQueues = 32;             // eight processes of the runtime's four
-constexpr unsigned kOrderlessTiles = kXcds * ((kXcdCus * kScanBlocksPerCu - 1) / (kHwQueues - 1));
-static_assert((kHwQueues - 1) * (kOrderlessTiles / kXcds) < kXcdCus * kScanBlocksPerCu, "a place is left");
+constexpr int kHwQueues = 32;                 // eight processes of the runtime's four
+constexpr int kBucketScanBlocksPerCu = 8;     // all 32 waves of a compute unit
+constexpr int kCellScanBlocksPerCu = 5;       // 28 KB of LDS each
+constexpr unsigned kOrderlessBuckets = kXcds * kBucketScanBlocksPerCu;
+constexpr unsigned kOrderlessCells = kXcds * kCellScanBlocksPerCu;
+static_assert(kHwQueues <= kXcdCus, "the other queues' scans leave a compute unit free");
 
 constexpr int64_t kSortLookbackTiles = 128;   // tiles of the bucketed sort's count scan at most
 inline int64_t lookback_cells(int64_t n_sort) { return scan_tiles(n_sort) + 1; }

@@ -33,27 +33,28 @@ def _constants():
     return k
 
 
-def _stuck(tiles, launches, places, xcds=8):
+def _stuck(tiles, launches, per_cu, cus=32, xcds=8):
     """Whether `launches` scans of `tiles` blocks in block order can wait for
     one another for ever: launch l's next block finds no place on XCD l mod m
     (an XCD starts a launch's blocks in order), and each such XCD is full of
     the other launches' blocks, all of which wait."""
     per_xcd = -(-tiles // xcds)
     for m in range(2, min(launches, xcds) + 1):
-        if all(per_xcd * sum(1 for l in range(launches) if l % m != x) >= places for x in range(m)):
+        if all(per_xcd * sum(1 for l in range(launches) if l % m != x) >= per_cu * cus for x in range(m)):
             return True
     return False
 
 
 def test_block_order_is_for_scans_that_cannot_block_one_another():
     """Scans without tickets leave a place on every XCD free, with every
-    hardware queue of several processes at one: at three scans of 1,024 tiles
-    they would not."""
+    hardware queue of several processes at one: three scans of 1,024 tiles
+    would not."""
     k = _constants()
-    places = k["kXcdCus"] * k["kScanBlocksPerCu"]
-    assert _stuck(1024, 3, places) and not _stuck(256, 4, places) and _stuck(256, 8, places)
-    for queues in range(2, 33):
-        assert not _stuck(k["kOrderlessTiles"], queues, places)
+    assert _stuck(1024, 3, 5) and not _stuck(256, 4, 5) and _stuck(256, 8, 5)
+    for limit, per_cu in ((8 * k["kBucketScanBlocksPerCu"], 8), (8 * k["kCellScanBlocksPerCu"], 5)):
+        for queues in range(2, k["kHwQueues"] + 1):
+            assert not _stuck(limit, queues, per_cu)
+    assert k["kXcds"] == 8 and k["kXcdCus"] == 32 and k["kHwQueues"] >= 32
 
 
 def _scan(counts, ti_bytes, reps):
