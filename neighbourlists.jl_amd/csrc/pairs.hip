@@ -18,9 +18,9 @@
 //     the atom's neighbours in exactly the reference traversal order.
 // tile_kernel tests 32-bit positions and decides what lies within their error
 // of the cutoff by the 64-bit test.  Bricks whose neighbour reach exceeds one
-// cell, whose halo does not fit LDS, or whose windings do not pack take a
-// per-wave path that reads global memory (one home cell per wave) with the
-// same enumeration and output.
+// cell, whose halo does not fit LDS, or whose windings lie too far apart take a
+// per-wave path that reads global memory (groups of home atoms dealt to the
+// waves) with the same enumeration and output.
 //
 // fill_kernel -- one wave per tile of consecutive output pairs, one lane per
 // pair: the tile's first atom comes from the pair scan's tile table, and
@@ -1442,13 +1442,13 @@ struct TileEnv {
 //
 // Bound by instruction issue: a home atom against four chunks is 39 vector and
 // 30 scalar instructions; at 1M atoms the vector unit issues for 73% of the
-// time (62.8 instructions per home atom, 46 scalar; 73.9 and 64 in the 64-bit
+// time (63.2 instructions per home atom, 47 scalar; 73.9 and 64 in the 64-bit
 // kernel, whose 32-byte atoms also held a CU to four bricks, now five).  The
 // tests as matrix instructions (4 x 4 x 1 in 32 bits, 16 blocks: four home atoms
 // by 64 candidates) took 12 cycles of the wave's SIMD each, more than the
 // vector instructions they replaced: 157 against 151 us.  Kernel times before
 // and after (MI355X): 96-atom crystal 66 / 12 us, 1k atoms 17.2 / 7.8, 100k 33 /
-// 28, 1M 193 / 151, 1M FCC slab 368 / 234 (there most bricks of atoms outside
+// 28, 1M 193 / 154, 1M FCC slab 368 / 231 (there most bricks of atoms outside
 // the cell wrote 8-byte rows; windings now count from the brick's own).
 //
 // A run of two home cells shares one candidate list, their nine rows of four
