@@ -147,10 +147,11 @@ struct SlotArgs {
 
 // Append the hits of one (home atom, chunk) ballot to the home atom's slot.
 // sbase = sorted index of the home atom * cap; ca = its running count
-// (wave-uniform); (sx, sy, sz) this lane's S.
+// (wave-uniform); (sx, sy, sz) this lane's S, spk the same packed if `packed`
+// (wave-uniform: most home atoms have no winding, and their S is s - w_j).
 template <bool WIDE>
 __device__ __forceinline__ void emit_hits(const SlotArgs &O, uint64_t mask, int64_t sbase, int32_t &ca, int32_t cj,
-                                          int32_t sx, int32_t sy, int32_t sz)
+                                          int32_t sx, int32_t sy, int32_t sz, bool packed, uint32_t spk)
 {
     if (mask == 0) return;   // wave-uniform
     const int lane = lane_id();
@@ -161,7 +162,7 @@ __device__ __forceinline__ void emit_hits(const SlotArgs &O, uint64_t mask, int6
             if (rank < O.cap) reinterpret_cast<int4 *>(O.slots)[sidx] = make_int4(cj, sx, sy, sz);
         } else {
             // entries past a row's end count too: the repeat on longer rows is the last one
-            const uint32_t spk = pack_wind(sx, sy, sz);
+            if (!packed) spk = pack_wind(sx, sy, sz);
             if (spk & kWindBig) O.status->wide = 1;
             if (rank < O.cap)
                 reinterpret_cast<uint64_t *>(O.slots)[sidx] = (uint64_t)(uint32_t)cj | ((uint64_t)spk << 32);
@@ -306,14 +307,17 @@ __device__ __forceinline__ void count_group(const PairsArgs &A, const SysDev &sd
         for (int k0 = 0; k0 < total; k0 += kChunksPerPass * kWave) {
             const int nch = sgpr(min(kChunksPerPass, (total - k0 + kWave - 1) / kWave));
             Cand c[kChunksPerPass];
+            uint32_t tpk[kChunksPerPass];
             uint64_t own[kChunksPerPass];   // candidates with no cell shift: the home atom's own is one of them
 #pragma unroll
             for (int g = 0; g < kChunksPerPass; ++g) {
                 own[g] = 0;
+                tpk[g] = 0;
                 if (g < nch) {
                     c[g] = load_candidate(A, k0 + g * kWave + lane, total, excl, start_g, shp);
                     if (!c[g].valid) c[g].x = c[g].y = c[g].z = kFar;
                     own[g] = __builtin_amdgcn_ballot_w64(c[g].zero_shift);
+                    tpk[g] = pack_wind(c[g].tx, c[g].ty, c[g].tz);
                 } else {
                     c[g].x = c[g].y = c[g].z = kFar;
                     c[g].j = -1;
@@ -332,6 +336,7 @@ __device__ __forceinline__ void count_group(const PairsArgs &A, const SysDev &sd
                         cell_shift(Cm, c[g].tx + wix, c[g].ty + wiy, c[g].tz + wiz, cx[g], cy[g], cz[g]);
                     wcache = h.w;
                 }
+                const bool wzero = (wix | wiy | wiz) == 0;
                 int32_t ca = __builtin_amdgcn_readlane(cnt_lane, a);
                 const int64_t sbase = (H.abase + __builtin_amdgcn_readlane(hj_lane, a)) * (int64_t)O.cap;
 #pragma unroll
@@ -343,7 +348,7 @@ __device__ __forceinline__ void count_group(const PairsArgs &A, const SysDev &sd
                         const double r2 = (Rx * Rx + Ry * Ry) + Rz * Rz;
                         const uint64_t mask = __builtin_amdgcn_ballot_w64(r2 < rc2) &
                                               ~(__builtin_amdgcn_ballot_w64(c[g].j == h.j) & own[g]);
-                        emit_hits<WIDE>(O, mask, sbase, ca, c[g].j, c[g].tx + wix, c[g].ty + wiy, c[g].tz + wiz);
+                        emit_hits<WIDE>(O, mask, sbase, ca, c[g].j, c[g].tx + wix, c[g].ty + wiy, c[g].tz + wiz, wzero, tpk[g]);
                     }
                 }
                 cnt_lane = lane == a ? ca : cnt_lane;
@@ -553,8 +558,8 @@ __device__ __forceinline__ int brick_cell_id(const Brick &B, int hc)
 // were clamped into (thousands of them) or the one cell of a brick is shared,
 // and no cell is looked at twice.  Every group loads the cell's candidates:
 // groups smaller than a wave only where they must be (100k atoms shifted by a
-// quarter of an open axis, whole builds: groups of 16 above 32 atoms 368 us, of
-// 48 above 64 336; 10k in a corner of an open cell 263 with either).
+// quarter of an open axis, whole builds: groups of 48 above 64 atoms 320 us, of
+// 16 above 32 a tenth more; 10k in a corner of an open cell 263 with either).
 constexpr int kShareGroup = 48;
 template <bool WIDE>
 __device__ __forceinline__ void count_cells(const PairsArgs &A, const Brick &B, int32_t *__restrict__ pair_count,
