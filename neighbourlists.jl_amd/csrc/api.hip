@@ -1071,7 +1071,7 @@ void copy_out(nlh_handle *h, const nlh::CopyList &c)
         hipError_t ready = hipSuccess;
         device_wide([&] { ready = b.c->prepare(bytes); });
         if (ready == hipSuccess) {
-            HIPC(b.c->to_host(h->stream, arrays));
+            HIPC(b.c->to_host(h->stream, arrays, nlh::host_copiers().threads()));
             h->inflight = false;   // the copies came behind everything else on the stream
             return;
         }

@@ -102,3 +102,20 @@ def test_filter_bounds(tmp_path):
         pairs, wrong, worst, _ = line.split()
         assert int(pairs) > 100000 and int(wrong) == 0 and float(worst) < 1.0, line
     assert len(out.splitlines()) == 2
+
+
+def test_copies_at_once_take_fewer_threads(tmp_path):
+    """Two copies have all their threads, three and more half of them each."""
+    out = run_cpp(tmp_path, """
+HostCopierPool p;
+std::vector<std::unique_ptr<HostCopier>> c;
+for (int k = 0; k < 4; ++k) {
+    c.push_back(p.borrow(0));
+    printf("%d ", p.threads());
+}
+for (auto &x : c) {
+    p.give_back(std::move(x));
+    printf("%d ", p.threads());
+}
+""", includes=("host_copy.h",))
+    assert out.split() == ["4", "4", "2", "2", "2", "4", "4", "4"]
